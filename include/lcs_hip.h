@@ -65,7 +65,7 @@ typedef struct lcs_schedule {
  * column symbols and none move between lanes.  The bytes are staged (two
  * small launches) for pairs of 2^22 cells or more, and at any size with
  * LCS_VARIANT_CHAIN_BYTES; the results are the same either way. */
-#define LCS_VARIANT_CHAIN_LDS 2  /* band chain with b staged through LDS      */
+#define LCS_VARIANT_CHAIN_LDS 2  /* band chain, four bands linked through LDS */
 /* Batches only: pairs of a batch with this variant are combed two per wave
  * with 16-bit strands (pair X in the low, pair Y in the high half of every
  * register, 5 VALU per 2 cells against 4 per cell; 4 per 2 cells when

@@ -28,9 +28,10 @@
 // checks, and all waves exit.
 //
 // Residuals (the reference's CPU fixup, src/lcs_grid.hpp:451-493) are handled
-// in the kernel: lanes whose column is outside [0, n) skip the cells, rows
-// beyond m in the last band never match and hold the smallest strand id, so
-// they pass every v strand through unchanged.
+// in the kernel: lanes whose column is outside [0, n) hold a symbol no row
+// matches and the largest strand (or, where no such symbol is known, skip the
+// cells), rows beyond m in the last band never match and hold the smallest
+// strand id; both pass every v strand through unchanged.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -324,6 +325,13 @@ __device__ __forceinline__ void band_steps8(const int32_t (&a)[TM], uint32_t (&h
         Q = qn;
         return;
     }
+    if constexpr (LCS_CHUNK_BLOCKS && C == 16 && !ROWMASK && !COLMASK && TM <= 16) {
+        // half a chunk of a linked band (cell_asm.h)
+        uint32_t qn;
+        cell_chunk16<TM>(a, h, sym, Q, v, qn);
+        Q = qn;
+        return;
+    }
     if constexpr (LCS_WORD_BLOCKS && !ROWMASK && !COLMASK && TM <= 16) {
         // the four steps of a symbol word in one asm block (cell_asm.h)
 #pragma unroll
@@ -345,6 +353,58 @@ __device__ __forceinline__ void band_steps8(const int32_t (&a)[TM], uint32_t (&h
     }
 }
 
+constexpr int kRingPolls = 8;    // ring polls per look at the abort flag and the clock
+
+// Linked bands (comb_group_kernel): the four bands of a workgroup hand
+// strands to each other through LDS.  Link w carries the strands leaving
+// wave w's band to wave w+1's as a ring of kLinkSlots column chunks guarded
+// by two progress words: the producer's last published chunk and the
+// consumer's last consumed one.
+constexpr int kGroupW = 4;       // bands (waves) per workgroup, one per SIMD
+constexpr int kLinkSlots = 16;   // column chunks in flight on one link
+struct GroupLds {
+    volatile int prog[kGroupW];   // prog[w]: last column chunk wave w published (-1: none)
+    volatile int cons[kGroupW];   // cons[w]: last chunk wave w took from wave w-1
+    volatile unsigned stop;       // set by a wave whose wait expired
+};
+typedef __attribute__((address_space(3))) GroupLds lds_group;
+typedef __attribute__((address_space(3))) volatile uint32_t lds_word;
+
+// A linked wave's ends: its position in the group and the rings on both
+// sides (in: from wave w-1, out: to wave w+1).
+struct BandLink {
+    lds_group *G;
+    lds_word *in, *out;
+    int w;
+    bool first, last;   // wave-uniform: reads the global ring / has no consumer in the group
+};
+
+// Spins until *word >= target (LDS).  When the stop word is set or the time
+// runs out (then both abort words are raised) `dead` is set instead; a dead
+// wave waits for nothing any more and runs its band to the end on whatever
+// it holds, so no wait has an exit that the band loop would have to carry.
+// A wave in step with the one above it comes here every chunk, so most polls
+// read nothing else: the clock is a memory round trip away.
+constexpr int kFastPolls = 64;
+__device__ __forceinline__ void lds_wait_ge(__attribute__((address_space(3))) volatile int *word, int target,
+                                            lds_group *G, const ChainArgs &A, int &dead)
+{
+    unsigned long long t_start = 0;
+#pragma nounroll
+    for (int i = 1; !dead; ++i) {
+        if (__builtin_amdgcn_readfirstlane(*word) >= target) return;
+        if (A.poll_sleep) __builtin_amdgcn_s_sleep(1);
+        if (i % kFastPolls == 0) {
+            const unsigned long long now = __builtin_amdgcn_s_memrealtime();
+            if (t_start == 0) t_start = now;
+            const bool late = A.timeout_ticks == 0 || now - t_start > A.timeout_ticks;
+            if (late) raise_abort(A.abort_flag);
+            if (late) G->stop = 1u;
+            dead = __builtin_amdgcn_readfirstlane(G->stop) != 0;
+        }
+    }
+}
+
 // Every band runs the same sequence of memory operations: it reads its top
 // edge from ring slot g&1 (tag g) and writes its bottom edge to slot (g+1)&1
 // (tag g+1).  The prep kernel seeds slot 0 with the grid's top edge (tag 0)
@@ -358,13 +418,47 @@ __device__ __forceinline__ void band_steps8(const int32_t (&a)[TM], uint32_t (&h
 // needed.
 constexpr uint32_t kPadRow16 = 0xffffu, kPadCol16 = 0xfffeu;
 
+// What a band's column symbols are: 32-bit words, bytes, or bytes whose
+// padding (255) no symbol of b equals.
+constexpr int kSymWords = 0, kSymBytes = 1, kSymBytesPadded = 2;
+
 // S8: the column symbols come from the byte copies of b (P.sym8) instead of
 // b; every lane loads its own C symbols of the next chunk (C/4 words from
 // the copy that starts its window on a word boundary) and no symbol
 // conveyor runs.
-template <int TM, int C, bool ROWMASK, bool PK, typename Desc, bool S8 = false, bool OH = false>
-__device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int g, int lane, int t_id)
+//
+// LK: a band of a linked group.  Its first wave reads the global ring and the
+// others the LDS link of the wave above; every wave also stores to the global
+// ring as an unlinked band does (only the last wave's words are read from
+// there, by the next group or the extract kernel), so that no path skips the
+// store and no wait for a load ever covers a store in flight.  A chunk's
+// outputs go to the link as soon as its steps are done, and the next chunk's
+// inputs are read from the link halfway through the chunk: a lag of 64 + 32 +
+// 16 steps against the global hand-off's 64 + 32 + 32 (its load is issued a
+// chunk ahead, which hides the trip through memory).  The link's reads,
+// progress words and branches cost more than those 16 steps: m = n = 16384
+// at 4 rows per lane 0.94 ms against the chain's 0.85 (1.24 and 1.09 before
+// the groups shared band_pass), so only LCS_VARIANT_CHAIN_LDS comes here.
+//
+// The first and last chunks of a band (some lane's column outside [0, n))
+// run the same unmasked steps as the others where a symbol exists that no
+// row of the band can match (PAD): lanes outside [0, n) then carry that
+// symbol and the strand ~0, which every row lets pass unchanged
+// (hn = min(h, ~0) = h, v' = ~0).  The packed chain has its pad symbols, the
+// byte copies are padded with 255 (kSym8Has255 in the flag word keeps the
+// masked steps for a b that holds it), and the 32-bit path looks for a value
+// that none of the band's rows holds.  A masked step takes several times an
+// unmasked one's time, and the first 96 steps of a band lie between its first
+// input and its first output, so masked ramps set the band-to-band lag of the
+// whole chain: m = n = 16384 at 4 rows per lane, one strip, took 1.09 ms with
+// masked ramps and 0.91 without; with the wait loops and the publish below
+// as they are now, 0.85 (2 rows per lane: 1.18, 0.93, 0.73).
+template <int TM, int C, bool ROWMASK, bool PK, typename Desc, int S8 = kSymWords, bool OH = false, bool LK = false>
+__device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int g, int lane, int t_id,
+                                          const BandLink &K = BandLink{})
 {
+    static_assert(!LK || (!PK && C == 32), "linked bands");
+    constexpr bool PAD = PK || S8 == kSymBytesPadded || (!S8 && !ROWMASK);
     const int m = P.m, n = P.n;
     const int r0 = g * (kWave * TM) + lane * TM;
     if (A.trace && t_id < A.trace_cap && lane == 0) A.trace[2 * (size_t)t_id] = __builtin_amdgcn_s_memrealtime();
@@ -395,6 +489,7 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
             // passes them unchanged and the band needs no row mask
             valid[k] = r < m;
             a[k] = valid[k] ? P.a[r] : -1;
+            if (S8 == kSymBytesPadded && a[k] == 255) a[k] = -1;   // b holds no 255
             h[k] = valid[k] ? (P.h_in ? (uint32_t)P.h_in[m - 1 - r] : (uint32_t)(m - 1 - r)) : 0u;
         } else {
             valid[k] = ROWMASK ? (r < m) : true;
@@ -402,13 +497,24 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
             h[k] = valid[k] ? (P.h_in ? (uint32_t)P.h_in[m - 1 - r] : (uint32_t)(m - 1 - r)) : 0u;
         }
     }
+    // the symbol of a column outside [0, n) (PAD): one that no row holds; the
+    // search ends within 64 TM + 1 values and nearly always at once
+    [[maybe_unused]] int32_t pad = OH ? 0 : (int32_t)(kPadCol16 << 16 | kPadCol16);
+    if constexpr (PAD && !PK && !S8) {
+        for (pad = -1;; --pad) {
+            bool hit = false;
+#pragma unroll
+            for (int k = 0; k < TM; ++k) hit = hit || a[k] == pad;
+            if (__builtin_amdgcn_ballot_w64(hit) == 0) break;
+        }
+    }
     const uint32_t tag_in = (uint32_t)g;
     const unsigned long long tag_out = (unsigned long long)(g + 1) << 32;
     gcword *Ein = (gcword *)(P.E + (size_t)(g & 1) * (size_t)n);
     gword *Eout = (gword *)(P.E + (size_t)((g + 1) & 1) * (size_t)n);
     const int nchunks = (n + kWave + C - 1) / C;
-    // the column symbol of column c (c in [0, n)): for the packed chain both
-    // pairs' symbols, each from a clamped in-bounds address
+    // the column symbol of column c (c >= 0; from n on the pad symbol or, with
+    // masked steps, any): always loaded from a clamped in-bounds address
     auto load_b = [&](auto c) -> int32_t {
         if constexpr (PK) {
             uint32_t x = 0;
@@ -420,12 +526,13 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
             }
             return (int32_t)x;
         } else {
-            return ((gsym *)P.b)[c];
+            const int32_t x = ((gsym *)P.b)[min((int)c, n - 1)];
+            return PAD && (int)c >= n ? pad : x;
         }
     };
 
     // Byte symbols: lane L combs column t - L at step t, the byte at
-    // x0 + t of the padded symbol string (x0 = kSym8Pad + col0 - L >= 65);
+    // x0 + t of the padded symbol string (x0 = kSym8Pad - L >= 65);
     // copy j = x0 % 4 holds it at byte x0 - j + t, a word boundary for
     // every chunk (t0 is a multiple of C).  The copies extend kSym8Pad
     // bytes past column n, beyond the last prefetch (t0 <= n + 64 + C).
@@ -433,7 +540,7 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     [[maybe_unused]] uint32_t sym[C / 4], psym[C / 4];
     [[maybe_unused]] gsym8 *sym_base = nullptr;
     if constexpr (S8) {
-        const int x0 = kSym8Pad + P.sym8_col0 - lane;
+        const int x0 = kSym8Pad - lane;
         const int j = x0 & 3;
         sym_base = (gsym8 *)P.sym8 + (size_t)j * (size_t)P.sym8_stride + ((x0 - j) >> 2);
     }
@@ -451,71 +558,106 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     // fetches C words, not 64.
     int32_t pB = 0;
     if constexpr (S8) load_sym(sym, 0);
-    else pB = load_b(min(lane & (C - 1), nm1));
-    unsigned long long pE = ld_relaxed(Ein + min(lane & (C - 1), nm1));
+    else pB = load_b(lane & (C - 1));
+    unsigned long long pE = 0;
+    if (!LK || K.first) pE = ld_relaxed(Ein + min(lane & (C - 1), nm1));
     // Publishes the C bottom-edge strands caught in O during the chunk that
-    // started at step t: O lanes [64-C, 64) hold columns t-64 .. t-64+C-1.
-    // Every lane stores every time, so no path skips the store and the waits
-    // for the prefetch loads can leave it in flight: lane L stores the word of
-    // lane 64-C + L%C (fetched by one bpermute), so the C/64 copies of each
-    // word carry the same value to the same address.  Columns outside [0, n)
-    // (the first and last chunks of a band) go to trash words past the ring.
-    // A chunk's words are published during the next chunk: publishing them
-    // right after their chunk (the upper half of O copied down by
-    // v_permlane32_swap instead of the bpermute) was measured slower, 146.1
-    // against 144.4 ms at m=n=2^20.
-    static_assert(C > 0 && (C & (C - 1)) == 0 && C <= kWave, "C must be a power of two <= 64");
-    gword *trash = (gword *)(P.E + 2 * (size_t)n);
-    // INSIDE: every column is known to be in [0, n), so the store needs no
-    // range check (the interior chunks below).
+    // started at step t: lanes 64-C .. 63 hold columns t-64 .. t-64+C-1.
+    // Inside the grid every lane stores (lane L the word of lane 64-C + L%C,
+    // which v_permlane32_swap brings down for C = 32): a lane mask would put
+    // a branch round the store, and the waits for the prefetch loads could
+    // then not leave it in flight.  The first and last chunks of a band leave
+    // columns outside [0, n) out.  A chunk's words are published at the start
+    // of the next chunk, behind that chunk's loads.
+    static_assert(C == kWave / 2, "publish moves the upper half of the wave to both halves");
+    auto both_halves = [](uint32_t x) {
+        return (uint32_t)__builtin_amdgcn_permlane32_swap((int)x, (int)x, false, false)[1];
+    };
+    // INSIDE: every column is known to be in [0, n) (the interior chunks below)
     auto publish = [&](uint32_t Ox, int t, auto inside) {
-        const int src = kWave - C + (lane & (C - 1));
-        const uint32_t x = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)Ox);
-        const int col = t + C - 2 * kWave + src;
-        if constexpr (decltype(inside)::value) {
+        const int col = t - kWave + (lane & (C - 1));
+        const uint32_t x = both_halves(Ox);
+        if (decltype(inside)::value || (col >= 0 && col < n))
             st_relaxed(Eout + (uint32_t)col, tag_out | (unsigned long long)x);
-        } else {
-            const bool mine = col >= 0 && col < n;
-            st_relaxed(mine ? Eout + col : trash + src, tag_out | (unsigned long long)x);
-        }
     };
     // Turns the prefetched ring words of the chunk starting at t into lane 0's
     // conveyor I (waiting, bounded in time, until they carry this band's tag).
     // INSIDE: the chunk's columns are known to be < n.
-    auto take_inputs = [&](int t, uint32_t &I, auto inside) -> bool {
+    // Set when a wait gave up: nothing is waited for after that, and the band
+    // runs to its end on whatever it holds.  An early return from each wait
+    // made the compiler carry the band's registers over every exit (about 20
+    // copies and several branches a chunk).
+    int dead = 0;
+    auto take_inputs = [&](int t, uint32_t &I, auto inside) {
         const int c = t + (lane & (C - 1));   // lanes >= C repeat lanes < C
-        const bool need = lane < C && (decltype(inside)::value || c < n);
+        const bool need = decltype(inside)::value || c < n;
         unsigned long long e = pE;
         // keeps the tag test (and so the wait for the prefetched word) after
         // the chunk's last step: I still holds the conveyor the chunk left,
         // which that step wrote, so the compare cannot be hoisted next to
         // the load to wait there for the whole round trip
         asm volatile("" : "+v"(e) : "v"(I));
-        bool ok = !need || (uint32_t)(e >> 32) == tag_in;
-        if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
-            // The band above is not that far yet: poll.  Every round also
-            // reads the abort flag and the clock; re-reading the ring words
-            // back to back without them was measured slower.
-            const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
-            do {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(need && (uint32_t)(e >> 32) != tag_in) != 0, 0)) {
+            // The band above is not that far yet: poll, looking at the abort
+            // flag and the clock every few rounds only (each is a memory
+            // round trip of its own).
+            unsigned long long t_start = 0;
+#pragma nounroll
+            for (int polls = 0; !dead; ++polls) {
                 // a wave that shares its SIMD with other launches' waves
                 // gives up its issue slots between polls
                 if (A.poll_sleep) __builtin_amdgcn_s_sleep(2);
-                if (__builtin_amdgcn_readfirstlane(ld_flag(A.abort_flag))) return false;
-                if (__builtin_amdgcn_s_memrealtime() - t_start > A.timeout_ticks) {
-                    raise_abort(A.abort_flag);
-                    return false;
+                e = ld_relaxed(Ein + min(c, nm1));
+                if (__builtin_amdgcn_ballot_w64(need && (uint32_t)(e >> 32) != tag_in) == 0) break;
+                if (polls % kRingPolls == 0) {
+                    const unsigned long long now = __builtin_amdgcn_s_memrealtime();
+                    if (polls == 0) t_start = now;
+                    const bool late = A.timeout_ticks == 0 || now - t_start > A.timeout_ticks;
+                    if (late) raise_abort(A.abort_flag);
+                    dead = late || __builtin_amdgcn_readfirstlane(ld_flag(A.abort_flag)) != 0;
                 }
-                if (!ok) e = ld_relaxed(Ein + min(c, nm1));
-                ok = !need || (uint32_t)(e >> 32) == tag_in;
-            } while (__builtin_amdgcn_ballot_w64(!ok) != 0);
+            }
         }
-        I = (uint32_t)e;
-        return true;
+        I = PAD && !need ? ~0u : (uint32_t)e;
     };
-    uint32_t v = 0, Q = 0, Osave = 0;
-    int32_t bq = 0, IB = pB;
-    if (!take_inputs(0, Q, std::false_type{})) return false;
+    // Linked bands: what a wave reads from LDS halfway through chunk j - 1
+    // (the producer's progress, then the words of column chunk j; LDS runs a
+    // wave's accesses in order, so the progress vouches for the words) and
+    // checks when chunk j starts.
+    [[maybe_unused]] int lk_prog = 0, lk_cons = 0;
+    [[maybe_unused]] uint32_t lk_in = 0;
+    [[maybe_unused]] const int lk_chunks = (n + C - 1) / C;   // column chunks that carry inputs
+    auto link_read = [&](int j) {
+        if (!K.first) {
+            if (lane == 0) K.G->cons[K.w] = j - 1;   // the chunk before is in registers
+            lk_prog = K.G->prog[K.w - 1];
+            lk_in = K.in[(j & (kLinkSlots - 1)) * C + (lane & (C - 1))];
+        }
+        if (!K.last) lk_cons = K.G->cons[K.w + 1];
+    };
+    auto link_take = [&](int j, uint32_t &I) {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(lk_prog) < j, 0)) {
+            lds_wait_ge(&K.G->prog[K.w - 1], j, K.G, A, dead);
+            lk_in = K.in[(j & (kLinkSlots - 1)) * C + (lane & (C - 1))];
+        }
+        I = lk_in;
+    };
+    // the outputs of column chunk j, in lanes 64-C .. 63 of Ox
+    auto link_put = [&](int j, uint32_t Ox) {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(lk_cons) < j - kLinkSlots, 0))
+            lds_wait_ge(&K.G->cons[K.w + 1], j - kLinkSlots, K.G, A, dead);
+        K.out[(j & (kLinkSlots - 1)) * C + (lane & (C - 1))] = both_halves(Ox);
+        if (lane == 0) K.G->prog[K.w] = j;
+    };
+    uint32_t v = PAD ? ~0u : 0u, Q = 0, Osave = 0;
+    int32_t bq = PAD ? pad : 0, IB = pB;
+    if (!LK || K.first) {
+        take_inputs(0, Q, std::false_type{});
+    } else {
+        link_read(0);
+        link_take(0, Q);
+        if (PAD && (lane & (C - 1)) >= n) Q = ~0u;
+    }
     // One chunk: prefetch chunk k+1, then publish chunk k-1 (the wait for the
     // loads at the end then leaves the store in flight), comb C steps, take
     // the next inputs.  The chunks run in three phases (ramp-in, interior,
@@ -527,33 +669,66 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     // faster.
     using Masked = std::integral_constant<bool, true>;
     using Full = std::integral_constant<bool, false>;
-    auto chunk = [&](auto colmask, int k) -> bool {
+    auto chunk = [&](auto colmask, int k) {
         const int t0 = k * C;
+        constexpr bool CM = decltype(colmask)::value && !PAD;   // masked steps
         if constexpr (S8) load_sym(psym, t0 + C);
         if constexpr (decltype(colmask)::value) {
-            const int c = min(t0 + C + (lane & (C - 1)), nm1);
+            const int c = t0 + C + (lane & (C - 1));
             if constexpr (!S8) pB = load_b(c);
-            pE = ld_relaxed(Ein + c);
+            if (!LK || K.first) pE = ld_relaxed(Ein + min(c, nm1));
         } else {   // an interior chunk: the next chunk's columns are inside [0, n)
             const uint32_t c = (uint32_t)(t0 + C + (lane & (C - 1)));
             if constexpr (!S8) pB = load_b(c);
-            pE = ld_relaxed(Ein + c);
+            if (!LK || K.first) pE = ld_relaxed(Ein + c);
         }
         publish(Osave, t0 - C, std::integral_constant<bool, !decltype(colmask)::value>{});
-        if constexpr (S8)
-            band_steps8<TM, C, ROWMASK, decltype(colmask)::value>(a, h, valid, v, Q, sym, t0, lane, n);
-        else
-            band_steps<TM, C, ROWMASK, decltype(colmask)::value, PK, OH>(a, h, valid, v, bq, Q, IB, t0, lane, n);
+        if constexpr (LK) {
+            // two halves, the link's words read between them
+            constexpr int H = C / 2;
+            if constexpr (S8) {
+                uint32_t lo[H / 4], hi[H / 4];
+#pragma unroll
+                for (int q = 0; q < H / 4; ++q) {
+                    lo[q] = sym[q];
+                    hi[q] = sym[H / 4 + q];
+                }
+                band_steps8<TM, H, ROWMASK, CM>(a, h, valid, v, Q, lo, t0, lane, n);
+                link_read(k + 1);
+                band_steps8<TM, H, ROWMASK, CM>(a, h, valid, v, Q, hi, t0 + H, lane, n);
+            } else {
+                band_steps<TM, H, ROWMASK, CM>(a, h, valid, v, bq, Q, IB, t0, lane, n);
+                link_read(k + 1);
+                band_steps<TM, H, ROWMASK, CM>(a, h, valid, v, bq, Q, IB, t0 + H, lane, n);
+            }
+        } else if constexpr (S8) {
+            band_steps8<TM, C, ROWMASK, CM>(a, h, valid, v, Q, sym, t0, lane, n);
+        } else {
+            band_steps<TM, C, ROWMASK, CM, PK, OH>(a, h, valid, v, bq, Q, IB, t0, lane, n);
+        }
         Osave = Q;
+        if constexpr (LK) {
+            // chunk k completes column chunk k - 64 / C; an interior chunk
+            // always completes one that carries outputs
+            const int jo = k - kWave / C;
+            if (!K.last && (!decltype(colmask)::value || (jo >= 0 && jo < lk_chunks)))
+                link_put(jo, Q);
+        }
         if (!decltype(colmask)::value || k + 1 < nchunks) {   // an interior chunk is never the last
             if constexpr (S8) {
 #pragma unroll
                 for (int q = 0; q < C / 4; ++q) sym[q] = psym[q];
             }
             IB = pB;
-            if (!take_inputs(t0 + C, Q, std::integral_constant<bool, !decltype(colmask)::value>{})) return false;
+            if (!LK || K.first) {
+                take_inputs(t0 + C, Q, std::integral_constant<bool, !decltype(colmask)::value>{});
+            } else if (!decltype(colmask)::value || k + 1 < lk_chunks) {
+                link_take(k + 1, Q);
+                if (PAD && decltype(colmask)::value && t0 + C + (lane & (C - 1)) >= n) Q = ~0u;
+            } else {
+                Q = ~0u;   // columns past n
+            }
         }
-        return true;
     };
     // Interior chunks: no lane's column leaves [0, n) (t0 >= 63, t0 + C <= n),
     // the next chunk's prefetch stays inside (t0 + 2C <= n) and so does the
@@ -562,14 +737,13 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     const int k_in = (kWave + C) / C;                      // first interior chunk
     const int k_out = max(k_in, min(n / C - 1, nchunks));  // first chunk after them
     int k = 0;
-    for (; k < min(k_in, nchunks); ++k)
-        if (!chunk(Masked{}, k)) return false;
-    for (; k + 1 < k_out; k += 2)
-        if (!chunk(Full{}, k) || !chunk(Full{}, k + 1)) return false;
-    for (; k < k_out; ++k)
-        if (!chunk(Full{}, k)) return false;
-    for (; k < nchunks; ++k)
-        if (!chunk(Masked{}, k)) return false;
+    for (; k < min(k_in, nchunks); ++k) chunk(Masked{}, k);
+    for (; k + 1 < k_out; k += 2) {
+        chunk(Full{}, k);
+        chunk(Full{}, k + 1);
+    }
+    for (; k < k_out; ++k) chunk(Full{}, k);
+    for (; k < nchunks; ++k) chunk(Masked{}, k);
     publish(Osave, (nchunks - 1) * C, std::false_type{});
     if constexpr (PK) {
 #pragma unroll
@@ -583,7 +757,26 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
             if (valid[k]) P.h_out[m - 1 - (r0 + k)] = (int32_t)h[k];
     }
     if (A.trace && t_id < A.trace_cap && lane == 0) A.trace[2 * (size_t)t_id + 1] = __builtin_amdgcn_s_memrealtime();
-    return true;
+    return !dead;
+}
+
+// One band of a pair, by what its column symbols are: bytes when the pair has
+// byte copies and all of b fits in a byte (they pad a partial band's rows
+// instead of masking them), else 32-bit words, masked in the band that has
+// rows past m (only a pair's last one does).
+template <int TM, int C, bool LK>
+__device__ __forceinline__ bool band_dispatch(const ChainArgs &A, const PairDesc &P, int g, int lane, int t_id,
+                                              const BandLink &K)
+{
+    const int flags = P.sym8 ? __builtin_amdgcn_readfirstlane(*P.sym8_flags) : kSym8Bad;
+    if (!(flags & kSym8Bad)) {
+        if (!(flags & kSym8Has255))
+            return band_pass<TM, C, false, false, PairDesc, kSymBytesPadded, false, LK>(A, P, g, lane, t_id, K);
+        return band_pass<TM, C, false, false, PairDesc, kSymBytes, false, LK>(A, P, g, lane, t_id, K);
+    }
+    const bool rowmask = (long long)(g + 1) * (kWave * TM) > (long long)P.m;
+    return rowmask ? band_pass<TM, C, true, false, PairDesc, kSymWords, false, LK>(A, P, g, lane, t_id, K)
+                   : band_pass<TM, C, false, false, PairDesc, kSymWords, false, LK>(A, P, g, lane, t_id, K);
 }
 
 template <int TM, int C>
@@ -599,16 +792,7 @@ __global__ __launch_bounds__(256) void comb_chain_kernel(ChainArgs A)
         const int2 task = A.tasks[t];
         const PairDesc P = A.pairs[task.x];
         const int g = task.y;
-        const bool rowmask = (long long)(g + 1) * (kWave * TM) > (long long)P.m;
-        // byte symbols when the pair has them and all of b fits in a byte
-        const bool s8 = P.sym8 != nullptr && __builtin_amdgcn_readfirstlane(*P.sym8_bad) == 0;
-        bool ok;
-        if (s8)   // byte symbols pad a partial band's rows instead of masking them
-            ok = band_pass<TM, C, false, false, PairDesc, true>(A, P, g, lane, (int)t);
-        else
-            ok = rowmask ? band_pass<TM, C, true, false>(A, P, g, lane, (int)t)
-                         : band_pass<TM, C, false, false>(A, P, g, lane, (int)t);
-        if (!ok) break;
+        if (!band_dispatch<TM, C, false>(A, P, g, lane, (int)t, BandLink{})) break;
     }
 }
 
@@ -626,237 +810,29 @@ __global__ __launch_bounds__(256) void comb_chain16_kernel(ChainArgs A)
         const int2 task = A.tasks[t];
         const CoupleDesc D = A.couples[task.x];
         const bool ok = __builtin_amdgcn_readfirstlane(D.onehot)
-                            ? band_pass<TM, C, false, true, CoupleDesc, false, true>(A, D, task.y, lane, (int)t)
+                            ? band_pass<TM, C, false, true, CoupleDesc, kSymWords, true>(A, D, task.y, lane, (int)t)
                             : band_pass<TM, C, false, true>(A, D, task.y, lane, (int)t);
         if (!ok) break;
     }
 }
 
-// ---- LDS group variant -----------------------------------------------------
+// ---- linked groups ----------------------------------------------------------
 //
-// W consecutive bands of one pair share a workgroup, one wave per band (one
-// per SIMD of a CU).  Inside the group the bottom-edge strands go from wave w
-// to wave w+1 through an R-slot LDS ring guarded by two progress words (the
-// producer's last published chunk, the consumer's last consumed chunk), and
-// the b symbols are loaded once per group by wave 0 (coalesced, 64 B per
-// chunk) into an LDS ring that every wave reads.  Only the group's first wave
-// reads the global ring and only its last wave writes it.  Waves are not
-// lock-stepped: each waits only for the data it needs and for a free slot,
-// so the ring gives the same slack the global ring gives between bands,
-// while a hand-off costs an LDS round trip instead of a global one.  A wave
-// finishes chunk j-kShift's columns (kShift = 64/C: the lane skew) during its
-// chunk j.  Every wait is bounded in time; an expired wait raises the global
-// abort flag and an LDS stop word that every waiting wave checks.
-constexpr int kXferSlots = 8;   // LDS ring between consecutive waves (chunks)
-constexpr int kBRing = 64;      // b chunks staged in LDS
-
-struct GroupLds {
-    volatile int prog[4];   // prog[w]: last column chunk wave w published (-1: none)
-    volatile int cons[4];   // cons[w]: last chunk wave w took from wave w-1
-    volatile unsigned stop; // set by a wave whose wait expired
-};
-typedef __attribute__((address_space(3))) GroupLds lds_group;
-
-// Spins until *word >= target (LDS), the stop word is set, or the time runs
-// out (then raises both abort words).  Returns false when the wave must stop.
-__device__ __forceinline__ bool lds_wait_ge(__attribute__((address_space(3))) volatile int *word, int target,
-                                            lds_group *G, const ChainArgs &A)
-{
-    if (*word >= target) return true;
-    const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
-    while (*word < target) {
-        if (G->stop) return false;
-        if (__builtin_amdgcn_s_memrealtime() - t_start > A.timeout_ticks) {
-            G->stop = 1u;
-            raise_abort(A.abort_flag);
-            return false;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
-    return true;
-}
-
-// ROLE bit 1: the group's first wave (reads the global ring, stages b);
-// bit 2: its last wave (writes the global ring).  The role is a template
-// argument so each wave's loop is straight-line code: with the role as a
-// runtime branch the waits of the merged paths cover every outstanding load.
-constexpr int kFirst = 1, kLast = 2;
-
-template <int TM, int C, int W, bool ROWMASK, int ROLE>
-__device__ bool group_band(const ChainArgs &A, const PairDesc &P, int g, int w, int lane,
-                           uint32_t (*xfer_)[kXferSlots][C], int32_t (*bring_)[C], lds_group *G)
-{
-    constexpr int kShift = kWave / C;
-    static_assert((W - 1) * (kShift + kXferSlots + 1) + 2 <= kBRing, "b ring too short for the group's spread");
-    constexpr bool first = (ROLE & kFirst) != 0, last = (ROLE & kLast) != 0;
-    // Every LDS access of the hand-off is volatile: the compiler keeps them
-    // in program order and the LDS executes one wave's accesses in order, so
-    // a progress word read before a data word vouches for that data.
-    typedef __attribute__((address_space(3))) volatile uint32_t lds_u32;
-    typedef __attribute__((address_space(3))) volatile int32_t lds_i32;
-    lds_u32 *xfer_in = (lds_u32 *)(w > 0 ? &xfer_[w > 0 ? w - 1 : 0][0][0] : &xfer_[0][0][0]);
-    lds_u32 *xfer_out = (lds_u32 *)&xfer_[last ? 0 : w][0][0];
-    lds_i32 *bring = (lds_i32 *)&bring_[0][0];
-    const int m = P.m, n = P.n;
-    const int r0 = g * (kWave * TM) + lane * TM;
-    int32_t a[TM];
-    uint32_t h[TM];
-    bool valid[TM];
-    gsym *asym = (gsym *)P.a, *hin = (gsym *)P.h_in;
-#pragma unroll
-    for (int k = 0; k < TM; ++k) {
-        const int r = r0 + k;
-        valid[k] = ROWMASK ? (r < m) : true;
-        a[k] = valid[k] ? asym[r] : 0;
-        h[k] = valid[k] ? (hin ? (uint32_t)hin[m - 1 - r] : (uint32_t)(m - 1 - r)) : 0u;
-    }
-    // Let the row loads land here: left outstanding into the loop, the wait
-    // for them would sit before the cells of every chunk and also cover the
-    // last wave's in-flight ring store.
-    __builtin_amdgcn_s_waitcnt(0);
-    const uint32_t tag_in = (uint32_t)g;
-    const unsigned long long tag_out = (unsigned long long)(g + 1) << 32;
-    gcword *Ein = (gcword *)(P.E + (size_t)(g & 1) * (size_t)n);
-    gword *Eout = (gword *)(P.E + (size_t)((g + 1) & 1) * (size_t)n);
-    gword *trash = (gword *)(P.E + 2 * (size_t)n);
-    gsym *bsym = (gsym *)P.b;
-    const int nchunks = (n + kWave + C - 1) / C;
-    const int nin = (n + C - 1) / C;   // chunks whose columns carry inputs
-    const int nm1 = n - 1;
-    const int ql = lane & (C - 1);
-    // as in band_pass: every lane stores, C/64 copies of each word
-    auto publish = [&](uint32_t Ox, int t) {
-        const int src = kWave - C + ql;
-        const uint32_t x = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)Ox);
-        const int col = t + C - 2 * kWave + src;
-        st_relaxed(col >= 0 && col < n ? Eout + col : trash + src, tag_out | (unsigned long long)x);
-    };
-    unsigned long long pE = 0;
-    auto take_inputs = [&](int t, uint32_t &I) -> bool {
-        const int c = t + ql;
-        const bool need = lane < C && c < n;
-        unsigned long long e = pE;
-        bool ok = !need || (uint32_t)(e >> 32) == tag_in;
-        if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
-            // poll as band_pass does
-            const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
-            do {
-                if (A.poll_sleep) __builtin_amdgcn_s_sleep(2);
-                if (__builtin_amdgcn_readfirstlane(ld_flag(A.abort_flag)) || G->stop) return false;
-                if (__builtin_amdgcn_s_memrealtime() - t_start > A.timeout_ticks) {
-                    G->stop = 1u;
-                    raise_abort(A.abort_flag);
-                    return false;
-                }
-                if (!ok) e = ld_relaxed(Ein + min(c, nm1));
-                ok = !need || (uint32_t)(e >> 32) == tag_in;
-            } while (__builtin_amdgcn_ballot_w64(!ok) != 0);
-        }
-        I = (uint32_t)e;
-        return true;
-    };
-    // chunk j's inputs from wave w-1 (wave >= 1): read now, checked later
-    int32_t pn = 0;
-    uint32_t In = 0;
-    int32_t IBn = 0;
-    auto lds_prefetch = [&](int j) {
-        pn = G->prog[w - 1];
-        In = xfer_in[(j & (kXferSlots - 1)) * C + ql];
-        IBn = bring[(j & (kBRing - 1)) * C + ql];
-    };
-    auto lds_take = [&](int j, uint32_t &I, int32_t &IB) -> bool {
-        if (__builtin_amdgcn_readfirstlane(pn) < j) {
-            if (!lds_wait_ge(&G->prog[w - 1], j, G, A)) return false;
-            In = xfer_in[(j & (kXferSlots - 1)) * C + ql];
-            IBn = bring[(j & (kBRing - 1)) * C + ql];
-        }
-        I = In;
-        IB = IBn;
-        if (lane == 0) G->cons[w] = j;
-        return true;
-    };
-    int32_t cn = 0;   // consumer word of wave w+1, read a chunk ahead
-
-    uint32_t v = 0, Q = 0, Osave = 0;
-    int32_t bq = 0, IB = 0, pB = 0;
-    if constexpr (first) {
-        pB = bsym[min(ql, nm1)];
-        pE = ld_relaxed(Ein + min(ql, nm1));
-        if (!take_inputs(0, Q)) return false;
-        IB = pB;
-        if (lane < C) bring[lane] = pB;
-    } else {
-        lds_prefetch(0);
-        if (!lds_take(0, Q, IB)) return false;
-    }
-    for (int j = 0; j < nchunks; ++j) {
-        const int t0 = j * C;
-        // Order: global loads, then the ring store (so the wait for the
-        // loads at the end of the chunk leaves the store in flight), then the
-        // LDS prefetch (so the store's bpermute wait covers none of it).
-        if constexpr (first) {
-            if (j + 1 < nchunks) {
-                const int c = min(t0 + C + ql, nm1);
-                pB = bsym[c];
-                pE = ld_relaxed(Ein + c);
-            }
-        }
-        if constexpr (last) publish(Osave, t0 - C);
-        if constexpr (!first) {
-            if (j + 1 < nin) lds_prefetch(j + 1);
-        }
-        if constexpr (!last) cn = G->cons[w + 1];
-        if (t0 >= kWave - 1 && t0 + C <= n)
-            band_steps<TM, C, ROWMASK, false>(a, h, valid, v, bq, Q, IB, t0, lane, n);
-        else
-            band_steps<TM, C, ROWMASK, true>(a, h, valid, v, bq, Q, IB, t0, lane, n);
-        Osave = Q;
-        if constexpr (!last) {
-            if (j >= kShift && j - kShift < nin) {
-                const int jo = j - kShift;   // the column chunk O now completes
-                if (__builtin_amdgcn_readfirstlane(cn) < jo - kXferSlots &&
-                    !lds_wait_ge(&G->cons[w + 1], jo - kXferSlots, G, A))
-                    return false;
-                if (lane >= kWave - C) xfer_out[(jo & (kXferSlots - 1)) * C + lane - (kWave - C)] = Osave;
-                if (lane == 0) G->prog[w] = jo;
-            }
-        }
-        if constexpr (first) {
-            if (j + 1 < nchunks) {
-                IB = pB;
-                if (!take_inputs(t0 + C, Q)) return false;
-                if (lane < C) bring[((j + 1) & (kBRing - 1)) * C + lane] = pB;
-            }
-        } else {
-            if (j + 1 < nin) {
-                if (!lds_take(j + 1, Q, IB)) return false;
-            } else {
-                Q = 0;   // columns past n: no input
-                IB = 0;
-            }
-        }
-    }
-    if constexpr (last) publish(Osave, (nchunks - 1) * C);
-    gout *hout = (gout *)P.h_out;
-#pragma unroll
-    for (int k = 0; k < TM; ++k)
-        if (valid[k]) hout[m - 1 - (r0 + k)] = (int32_t)h[k];
-    return true;
-}
-
+// kGroupW consecutive bands of one pair share a workgroup, one wave per band
+// (one per SIMD of a CU), linked through LDS (band_pass, LK): three of four
+// hand-offs go through LDS instead of memory.
 // Ticket t runs band group tasks[t].y (bands W*y .. W*y+W-1) of pair
 // tasks[t].x.  The only barriers are the three per task, which every wave
 // passes whatever its band did.
-template <int TM, int C, int W>
-__global__ __launch_bounds__(kWave * W) void comb_group_kernel(ChainArgs A)
+template <int TM, int C>
+__global__ __launch_bounds__(kWave * kGroupW) void comb_group_kernel(ChainArgs A)
 {
-    static_assert(W >= 2 && W <= 4, "group of 2..4 waves");
-    __shared__ uint32_t xfer[W - 1][kXferSlots][C];
-    __shared__ int32_t bring[kBRing][C];
+    constexpr int W = kGroupW;
+    __shared__ uint32_t links[W - 1][kLinkSlots * C];
     __shared__ GroupLds group;
     __shared__ unsigned s_task, s_stop;
     const int lane = threadIdx.x & (kWave - 1);
-    const int w = (int)(threadIdx.x >> 6);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     lds_group *G = (lds_group *)&group;
     for (;;) {
         __syncthreads();  // every wave is done with the previous task's LDS
@@ -864,44 +840,27 @@ __global__ __launch_bounds__(kWave * W) void comb_group_kernel(ChainArgs A)
             const unsigned t = atomicAdd(A.ticket, 1u);
             s_task = t;
             s_stop = ((int)t >= A.ntasks || ld_flag(A.abort_flag)) ? 1u : 0u;
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < W; ++i) {
                 G->prog[i] = -1;
                 G->cons[i] = -1;
             }
             G->stop = 0u;
         }
         __syncthreads();
-        const unsigned t = s_task, stop = s_stop;
+        const unsigned t = __builtin_amdgcn_readfirstlane(s_task), stop = __builtin_amdgcn_readfirstlane(s_stop);
         __syncthreads();
         if (stop) break;
         const int2 task = A.tasks[t];
         const PairDesc P = A.pairs[task.x];
         const int g0 = task.y * W;
         const int wact = min(W, P.nbands - g0);
-        const int trace_id = (int)t * W + w;
-        const bool traced = A.trace && trace_id < A.trace_cap && lane == 0;
-        if (traced) A.trace[2 * (size_t)trace_id] = __builtin_amdgcn_s_memrealtime();
         if (w < wact) {
-            const int g = g0 + w;
-            // only a pair's last band has rows past m, and it is its group's last wave
-            const bool rowmask = (long long)(g + 1) * (kWave * TM) > (long long)P.m;
-            const int role = (w == 0 ? kFirst : 0) | (w == wact - 1 ? kLast : 0);
-            bool ok;
-            if (rowmask)
-                ok = role == (kFirst | kLast)
-                         ? group_band<TM, C, W, true, kFirst | kLast>(A, P, g, w, lane, xfer, bring, G)
-                         : group_band<TM, C, W, true, kLast>(A, P, g, w, lane, xfer, bring, G);
-            else if (role == (kFirst | kLast))
-                ok = group_band<TM, C, W, false, kFirst | kLast>(A, P, g, w, lane, xfer, bring, G);
-            else if (role == kFirst)
-                ok = group_band<TM, C, W, false, kFirst>(A, P, g, w, lane, xfer, bring, G);
-            else if (role == kLast)
-                ok = group_band<TM, C, W, false, kLast>(A, P, g, w, lane, xfer, bring, G);
-            else
-                ok = group_band<TM, C, W, false, 0>(A, P, g, w, lane, xfer, bring, G);
+            const int g = g0 + w, trace_id = (int)t * W + w;
+            const BandLink K = {G, (lds_word *)&links[w > 0 ? w - 1 : 0][0], (lds_word *)&links[w < W - 1 ? w : 0][0], w,
+                                w == 0, w == wact - 1};
+            const bool ok = band_dispatch<TM, C, true>(A, P, g, lane, trace_id, K);
             if (!ok && lane == 0) G->stop = 1u;  // let the group's other waves stop waiting
         }
-        if (traced) A.trace[2 * (size_t)trace_id + 1] = __builtin_amdgcn_s_memrealtime();
     }
 }
 
@@ -973,29 +932,34 @@ __global__ void lcsk_zero_kernel(int32_t *x, int32_t n)
     if (i < n) x[i] = 0;
 }
 
-// Byte symbols of b (the layout lcsk_sym8_stride describes): one thread per
-// word of the four copies; copy 0 (which covers every column) raises *bad
-// for a symbol outside [0, 255].
-__global__ void comb_sym8_kernel(const int32_t *b, int32_t n, uint32_t *out, int32_t stride, int32_t *bad)
+// Byte symbols of a string cut into strips of W columns (the layout
+// lcsk_sym8_stride describes, one set of copies per strip): one thread per
+// word; copy 0 of each strip (which covers every column) raises *flags for a
+// symbol outside [0, 255] or equal to the padding.
+__global__ void comb_sym8_kernel(const int32_t *b, int32_t n, int32_t W, uint32_t *out, int32_t stride, int32_t *flags)
 {
+    const int32_t col0 = (int32_t)blockIdx.y * W, ns = min(W, n - col0);
+    b += col0;
+    out += 4 * (size_t)stride * blockIdx.y;
     const long long total = 4LL * stride;
     const long long step = (long long)gridDim.x * blockDim.x;
     for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += step) {
         const int j = (int)(q / stride);
         const long long x = 4 * (q - (long long)j * stride) + j - kSym8Pad;   // column of byte 0
         uint32_t word = 0;
-        bool out_of_range = false;
+        int seen = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const long long c = x + i;
-            if (c >= 0 && c < n) {
-                const int32_t sym = b[c];
-                out_of_range |= (uint32_t)sym > 255u;
-                word |= ((uint32_t)sym & 0xffu) << (8 * i);
+            uint32_t sym = 255u;
+            if (c >= 0 && c < ns) {
+                sym = (uint32_t)b[c];
+                seen |= sym > 255u ? kSym8Bad : sym == 255u ? kSym8Has255 : 0;
             }
+            word |= (sym & 0xffu) << (8 * i);
         }
         out[q] = word;
-        if (out_of_range && j == 0) atomicOr(bad, 1);
+        if (seen && j == 0) atomicOr(flags, seen);
     }
 }
 
@@ -1092,7 +1056,6 @@ using namespace lcsk;
 // (m=n=2^20 at TM=16: the register chain 143.9 against 145.6 ms, the LDS
 // groups 154.7 against 166.0 ms; 8 and 64 steps are slower in both).
 constexpr int kChainChunk = 32;
-constexpr int kGroupChunk = 32;
 
 template <int TM>
 static int launch_chain_tm(const ChainArgs &args, int grid_blocks, int block_threads, hipStream_t stream)
@@ -1101,8 +1064,8 @@ static int launch_chain_tm(const ChainArgs &args, int grid_blocks, int block_thr
         comb_chain_kernel<TM, kChainChunk><<<dim3(grid_blocks), dim3(block_threads), 0, stream>>>(args);
         return 0;
     }
-    if (args.group_w == 4 && block_threads == 4 * kWave) {
-        comb_group_kernel<TM, kGroupChunk, 4><<<dim3(grid_blocks), dim3(block_threads), 0, stream>>>(args);
+    if (args.group_w == kGroupW && block_threads == kGroupW * kWave) {
+        comb_group_kernel<TM, kChainChunk><<<dim3(grid_blocks), dim3(block_threads), 0, stream>>>(args);
         return 0;
     }
     return -22;
@@ -1132,13 +1095,17 @@ int lcsk_launch_chain(const ChainArgs &args, const PairDesc *d_pairs, int npairs
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-int lcsk_launch_sym8(const int32_t *b, int32_t n, uint32_t *out, int32_t stride, int32_t *bad, hipStream_t stream)
+int lcsk_launch_sym8(const int32_t *b, int32_t n, int32_t W, uint32_t *out, int32_t stride, int32_t *flags,
+                     hipStream_t stream)
 {
-    if (n <= 0 || stride < lcsk_sym8_stride(n)) return -22;
-    hipLaunchKernelGGL(lcsk_zero_kernel, dim3(1), dim3(64), 0, stream, bad, 1);
+    if (n <= 0 || W <= 0 || stride < lcsk_sym8_stride(W)) return -22;
+    const int32_t strips = (n + W - 1) / W;
+    if (strips > 65535) return -34;
+    hipLaunchKernelGGL(lcsk_zero_kernel, dim3(1), dim3(64), 0, stream, flags, 1);
     const long long words = 4LL * stride;
-    const unsigned blocks = (unsigned)std::min<long long>((words + 255) / 256, 8192);
-    hipLaunchKernelGGL(comb_sym8_kernel, dim3(blocks), dim3(256), 0, stream, b, n, out, stride, bad);
+    const unsigned blocks = (unsigned)std::min<long long>((words + 255) / 256, std::max(1, 8192 / strips));
+    hipLaunchKernelGGL(comb_sym8_kernel, dim3(blocks, (unsigned)strips), dim3(256), 0, stream, b, n, W, out, stride,
+                       flags);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 

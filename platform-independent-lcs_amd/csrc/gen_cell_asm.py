@@ -364,6 +364,15 @@ if __name__ == "__main__":
     print('    else static_assert(R == 1 || R == 2 || R == 4 || R == 8 || R == 16, "rows per block");\n}\n')
     for R in (1, 2, 4, 8, 16):
         print(chunk_block(R, 8))
+    for R in (1, 2, 4, 8, 16):
+        print(chunk_block(R, 4))
+    print("// cell_chunk{R}x4 by template argument: half a chunk (16 steps)")
+    print("template <int R>\n__device__ __forceinline__ void cell_chunk16(const int32_t *a, uint32_t *h,"
+          " const uint32_t *sb, uint32_t q, uint32_t &vt, uint32_t &qo)\n{")
+    print("    if constexpr (R == 1) cell_chunk1x4(a, h, sb, q, vt, qo);")
+    for R in (2, 4, 8, 16):
+        print(f"    else if constexpr (R == {R}) cell_chunk{R}x4(a, h, sb, q, vt, qo);")
+    print('    else static_assert(R == 1 || R == 2 || R == 4 || R == 8 || R == 16, "rows per block");\n}\n')
     print("// cell_chunk{R}x8 by template argument: the 32 steps of a chunk")
     print("template <int R>\n__device__ __forceinline__ void cell_chunk32(const int32_t *a, uint32_t *h,"
           " const uint32_t *sb, uint32_t q, uint32_t &vt, uint32_t &qo)\n{")

@@ -385,19 +385,18 @@ bool use_sym8(int variant, int32_t m, int32_t n)
     if (!LCS_SYM8 || n <= 0 || n > kSym8MaxN) return false;
     return variant == LCS_VARIANT_CHAIN_BYTES || (double)m * (double)n >= kSym8MinCells;
 }
-int stage_sym8(lcs_ctx *ctx, const int32_t *d_b, int32_t n, std::vector<PairDesc> &pairs,
-               const std::vector<int32_t> &col0, hipStream_t stream)
+int stage_sym8(lcs_ctx *ctx, const int32_t *d_b, int32_t n, int32_t W, std::vector<PairDesc> &pairs,
+               hipStream_t stream)
 {
-    const int32_t stride = lcsk_sym8_stride(n);
-    const size_t bytes = (size_t)4 * 4 * (size_t)stride + 64;
+    const int32_t stride = lcsk_sym8_stride(W);
+    const size_t set = 4 * (size_t)stride, bytes = pairs.size() * set * 4 + 64;
     if (ctx->sym8.reserve(ctx, bytes) != LCS_OK) return LCS_OK;
     uint32_t *copies = (uint32_t *)ctx->sym8.ptr;
-    int32_t *bad = (int32_t *)(copies + (size_t)4 * stride);
-    if (lcsk_launch_sym8(d_b, n, copies, stride, bad, stream)) return LCS_EIO;
+    int32_t *flags = (int32_t *)(copies + pairs.size() * set);
+    if (lcsk_launch_sym8(d_b, n, W, copies, stride, flags, stream)) return LCS_EIO;
     for (size_t p = 0; p < pairs.size(); ++p) {
-        pairs[p].sym8 = copies;
-        pairs[p].sym8_bad = bad;
-        pairs[p].sym8_col0 = col0[p];
+        pairs[p].sym8 = copies + p * set;
+        pairs[p].sym8_flags = flags;
         pairs[p].sym8_stride = stride;
     }
     return LCS_OK;
@@ -438,10 +437,8 @@ int enqueue_strips(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d
         size[(size_t)s] = (int64_t)m + P.n;
         acc += size[(size_t)s];
     }
-    if (group_w == 1 && sym8) {
-        std::vector<int32_t> col0((size_t)S);
-        for (int s = 0; s < S; ++s) col0[(size_t)s] = s * W;
-        if ((rc = stage_sym8(ctx, d_b, n, pairs, col0, stream))) return rc;
+    if (sym8) {
+        if ((rc = stage_sym8(ctx, d_b, n, W, pairs, stream))) return rc;
     }
     if ((rc = enqueue_pairs(ctx, pairs, tm, wps, stream, group_w))) return rc;
     // enqueue_pairs staged the descriptors into ctx->descs; reuse them for the permutations
@@ -569,8 +566,8 @@ static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const i
     P.v_out = d_v;
     P.m = m;
     P.n = n;
-    if (group_w == 1 && sym8) {
-        const int rc = stage_sym8(ctx, d_b, n, pairs, std::vector<int32_t>(1, 0), stream);
+    if (sym8) {
+        const int rc = stage_sym8(ctx, d_b, n, n, pairs, stream);
         if (rc) return rc;
     }
     return enqueue_pairs(ctx, pairs, tm, wps, stream, group_w);

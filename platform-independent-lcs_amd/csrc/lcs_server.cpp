@@ -215,11 +215,10 @@ int launch_slot(lcs_server *S, Slot &slot)
             // byte symbols (register chain): the copies follow the ring in the block
             const int32_t stride = lcsk_sym8_stride(n);
             uint32_t *copies = (uint32_t *)(((uintptr_t)(E + lcsk_ring_words(n)) + kAlign - 1) & ~(uintptr_t)(kAlign - 1));
-            int32_t *bad = (int32_t *)(copies + (size_t)4 * stride);
-            if (lcsk_launch_sym8(db, n, copies, stride, bad, slot.stream)) return LCS_EIO;
+            int32_t *flags = (int32_t *)(copies + (size_t)4 * stride);
+            if (lcsk_launch_sym8(db, n, n, copies, stride, flags, slot.stream)) return LCS_EIO;
             P.sym8 = copies;
-            P.sym8_bad = bad;
-            P.sym8_col0 = 0;
+            P.sym8_flags = flags;
             P.sym8_stride = stride;
         }
         groups[(size_t)c].push_back(P);
