@@ -21,6 +21,29 @@ struct PairDesc {
     const uint32_t *sym8;
     const int32_t *sym8_flags;
     int32_t sym8_stride, pad;
+    // Nullable: the pair's permutation (row_to_col, m + n entries), written
+    // instead of h_out and v_out.
+    int32_t *perm;
+};
+
+// One pair cut into GR x GC tiles of H rows and W columns (the last ones may
+// be smaller), each combed from its own identity; described by value in the
+// launch arguments, so that a single-pair call uploads nothing.  Tile (i, j)
+// combs a[iH ..) against b[jW ..) with ring slot iGC + j of `pair.E` and the
+// byte copies of strip j of `pair.sym8`.  With one tile the pair's own
+// h_in, v_in, h_out and v_out are used; with more, each tile writes its
+// permutation at `perm` + tile_perm_off(i, j).
+struct TileGrid {
+    PairDesc pair;
+    int32_t H, W, GR, GC;
+    int32_t *perm;
+    int32_t *sym8_flags;   // pair.sym8_flags, cleared by the extract kernel for the next launch
+    __host__ __device__ int32_t rows(int32_t i) const { return pair.m - i * H < H ? pair.m - i * H : H; }
+    __host__ __device__ int32_t cols(int32_t j) const { return pair.n - j * W < W ? pair.n - j * W : W; }
+    __host__ __device__ int64_t perm_off(int32_t i, int32_t j) const
+    {
+        return (int64_t)i * ((int64_t)GC * H + pair.n) + (int64_t)j * (rows(i) + W);
+    }
 };
 
 // Byte symbols of a string b of n symbols: four copies (stride words each,
@@ -32,10 +55,8 @@ constexpr int32_t kSym8Pad = 128;
 // padding of the copies
 constexpr int32_t kSym8Bad = 1, kSym8Has255 = 2;
 inline int32_t lcsk_sym8_stride(int32_t n) { return (int32_t)((((int64_t)n + 2 * kSym8Pad + 15) / 16) * 4); }
-// Writes the four copies of each strip of W columns of b (the last strip may
-// be narrower) into `out`, 4 * stride words per strip, and b's flags.
-int lcsk_launch_sym8(const int32_t *b, int32_t n, int32_t W, uint32_t *out, int32_t stride, int32_t *flags,
-                     hipStream_t stream);
+// Writes the four copies of b into `out` (4 * stride words) and b's flags.
+int lcsk_launch_sym8(const int32_t *b, int32_t n, uint32_t *out, int32_t stride, int32_t *flags, hipStream_t stream);
 
 // Two pairs combed together by the 16-bit packed chain
 // (LCS_VARIANT_PACKED16): pair q (0 = X, low halves; 1 = Y, high halves)
@@ -62,7 +83,8 @@ inline size_t lcsk_ring_words(int32_t n) { return 2 * (size_t)n + 64; }
 // group_w*tasks[t].y .. +group_w-1 in one workgroup (group_w > 1).  Tasks must list every band after the
 // band above it (same pair), which makes every wait one on a resident wave.
 struct ChainArgs {
-    const PairDesc *pairs;       // the register chain and LDS groups
+    const PairDesc *pairs;       // the register chain and linked groups; null: the tiles of `grid`, task t being
+                                 // band (or group) t / (GR GC) of tile t % (GR GC)
     const CoupleDesc *couples;   // the packed chain (tasks[t].x indexes couples)
     const int2 *tasks;
     int32_t ntasks;
@@ -75,8 +97,12 @@ struct ChainArgs {
     int32_t poll_sleep;          // 1: a wave waiting for its inputs sleeps between polls (launches that
                                  // share SIMDs with other launches' waves)
     unsigned *sticky;            // nullable: the prep kernel ORs the abort flag into it before clearing it
+    TileGrid grid;               // when pairs is null
 };
 
+// The same for the tiles of args.grid, with the byte copies of b (when
+// grid.pair.sym8 is set) staged by the seeding kernel.
+int lcsk_launch_grid(const ChainArgs &args, int grid_blocks, int block_threads, hipStream_t stream);
 // Seeds the rings of pairs[0..npairs) and clears ticket/abort; then runs the
 // chain for tile height tile_m; then extracts v_out.  All on `stream`.
 int lcsk_launch_chain(const ChainArgs &args, const PairDesc *d_pairs, int npairs, int max_n, int tile_m,
@@ -105,6 +131,6 @@ int lcsk_launch_r2c_from_strands(const int32_t *h, int32_t m, const int32_t *v, 
 // dst[0..count) = src[0..count) (a kernel, so it can sit in a captured graph).
 int lcsk_launch_copy(int32_t *dst, const int32_t *src, long long count, hipStream_t stream);
 // Strands from a permutation (row_to_col, size m+n): h_out[l] = row of col
-// n+l, v_out[j] = row of col j.  scratch holds m+n words.
-int lcsk_launch_strands_from_perm(const int32_t *r2c, int32_t m, int32_t n, int32_t *scratch, int32_t *h_out,
-                                  int32_t *v_out, hipStream_t stream);
+// n+l, v_out[j] = row of col j.
+int lcsk_launch_strands_from_perm(const int32_t *r2c, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out,
+                                  hipStream_t stream);

@@ -754,7 +754,13 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     } else {
 #pragma unroll
         for (int k = 0; k < TM; ++k)
-            if (valid[k]) P.h_out[m - 1 - (r0 + k)] = (int32_t)h[k];
+            if (valid[k]) {
+                const int l = m - 1 - (r0 + k);
+                // ids are below m+n after a completed comb; the test keeps an
+                // aborted one (whose strands are undefined) from writing out of range
+                if (P.perm == nullptr) P.h_out[l] = (int32_t)h[k];
+                else if (h[k] < (uint32_t)(m + n)) P.perm[h[k]] = n + l;
+            }
     }
     if (A.trace && t_id < A.trace_cap && lane == 0) A.trace[2 * (size_t)t_id + 1] = __builtin_amdgcn_s_memrealtime();
     return !dead;
@@ -779,6 +785,38 @@ __device__ __forceinline__ bool band_dispatch(const ChainArgs &A, const PairDesc
                    : band_pass<TM, C, false, false, PairDesc, kSymWords, false, LK>(A, P, g, lane, t_id, K);
 }
 
+// Tile p of a grid as a pair of its own.
+__device__ __forceinline__ PairDesc tile_pair(const TileGrid &T, int p)
+{
+    PairDesc P = T.pair;
+    if (T.GR * T.GC > 1) {
+        const int i = p / T.GC, j = p - i * T.GC;
+        P.a += (size_t)i * T.H;
+        P.b += (size_t)j * T.W;
+        P.m = T.rows(i);
+        P.n = T.cols(j);
+        P.E += (size_t)p * (2 * (size_t)T.W + 64);
+        if (P.sym8) P.sym8 += (size_t)j * 4 * (size_t)P.sym8_stride;
+        P.perm = T.perm + T.perm_off(i, j);
+        P.nbands = (P.m + kWave * P.tile_m - 1) / (kWave * P.tile_m);
+    }
+    return P;
+}
+
+// The pair of task t and its band (or group); a grid's last tile row may have
+// fewer bands than the others (then P.nbands <= the band: no work).
+__device__ __forceinline__ PairDesc task_pair(const ChainArgs &A, unsigned t, int &unit)
+{
+    if (A.pairs) {
+        const int2 task = A.tasks[t];
+        unit = task.y;
+        return A.pairs[task.x];
+    }
+    const unsigned tiles = (unsigned)(A.grid.GR * A.grid.GC);
+    unit = (int)(t / tiles);
+    return tile_pair(A.grid, (int)(t % tiles));
+}
+
 template <int TM, int C>
 __global__ __launch_bounds__(256) void comb_chain_kernel(ChainArgs A)
 {
@@ -789,9 +827,9 @@ __global__ __launch_bounds__(256) void comb_chain_kernel(ChainArgs A)
         t = __builtin_amdgcn_readfirstlane(t);
         if ((int)t >= A.ntasks) break;
         if (__builtin_amdgcn_readfirstlane(ld_flag(A.abort_flag))) break;
-        const int2 task = A.tasks[t];
-        const PairDesc P = A.pairs[task.x];
-        const int g = task.y;
+        int g;
+        const PairDesc P = task_pair(A, t, g);
+        if (g >= P.nbands) continue;
         if (!band_dispatch<TM, C, false>(A, P, g, lane, (int)t, BandLink{})) break;
     }
 }
@@ -850,9 +888,9 @@ __global__ __launch_bounds__(kWave * kGroupW) void comb_group_kernel(ChainArgs A
         const unsigned t = __builtin_amdgcn_readfirstlane(s_task), stop = __builtin_amdgcn_readfirstlane(s_stop);
         __syncthreads();
         if (stop) break;
-        const int2 task = A.tasks[t];
-        const PairDesc P = A.pairs[task.x];
-        const int g0 = task.y * W;
+        int unit;
+        const PairDesc P = task_pair(A, t, unit);
+        const int g0 = unit * W;
         const int wact = min(W, P.nbands - g0);
         if (w < wact) {
             const int g = g0 + w, trace_id = (int)t * W + w;
@@ -864,6 +902,38 @@ __global__ __launch_bounds__(kWave * kGroupW) void comb_group_kernel(ChainArgs A
     }
 }
 
+// Byte symbols of a strip of ns columns at b (the layout lcsk_sym8_stride
+// describes), one thread per word; copy 0 (which covers every column) raises
+// *flags for a symbol outside [0, 255] or equal to the padding.
+__device__ __forceinline__ void stage_sym8(const int32_t *b, int32_t ns, uint32_t *out, int32_t stride, int32_t *flags)
+{
+    const long long total = 4LL * stride;
+    const long long step = (long long)gridDim.x * blockDim.x;
+    for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += step) {
+        const int j = (int)(q / stride);
+        const long long x = 4 * (q - (long long)j * stride) + j - kSym8Pad;   // column of byte 0
+        uint32_t word = 0;
+        int seen = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const long long c = x + i;
+            uint32_t sym = 255u;
+            if (c >= 0 && c < ns) {
+                sym = (uint32_t)b[c];
+                seen |= sym > 255u ? kSym8Bad : sym == 255u ? kSym8Has255 : 0;
+            }
+            word |= (sym & 0xffu) << (8 * i);
+        }
+        out[q] = word;
+        if (seen && j == 0) atomicOr(flags, seen);
+    }
+}
+
+__global__ void comb_sym8_kernel(const int32_t *b, int32_t n, uint32_t *out, int32_t stride, int32_t *flags)
+{
+    stage_sym8(b, n, out, stride, flags);
+}
+
 // Seeds the rings before a chain launch (blockIdx.y = pair): slot 0 holds
 // the grid's top edge (v_in[c], or the ids m+c) under tag 0 for band 0,
 // slot 1 holds a tag no band waits for.  A pair with no band (n == 0) gets
@@ -871,9 +941,8 @@ __global__ __launch_bounds__(kWave * kGroupW) void comb_group_kernel(ChainArgs A
 // folding the previous launch's abort flag into `sticky` (the context's
 // status word, read and cleared by the host).  A kernel, not
 // hipMemsetAsync, so the launch sequence can live inside a hipGraph.
-__global__ void comb_prep_kernel(const PairDesc *pairs, unsigned *ctrl, unsigned *sticky)
+__device__ __forceinline__ void prep_pair(const PairDesc &P, unsigned *ctrl, unsigned *sticky)
 {
-    const PairDesc P = pairs[blockIdx.y];
     // 64-bit indices: a grid-stride step past a size near 2^31 must not wrap
     const long long stride = (long long)gridDim.x * blockDim.x;
     for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.n; c += stride) {
@@ -889,6 +958,22 @@ __global__ void comb_prep_kernel(const PairDesc *pairs, unsigned *ctrl, unsigned
         ctrl[0] = 0u;
         ctrl[1] = 0u;
     }
+}
+
+__global__ void comb_prep_kernel(const PairDesc *pairs, unsigned *ctrl, unsigned *sticky)
+{
+    prep_pair(pairs[blockIdx.y], ctrl, sticky);
+}
+
+// The tiles of a grid (blockIdx.y = tile): rings, control words and, from the
+// first tile row, the byte copies of the strips.  The flags word is zero here:
+// the extract kernel of the launch before left it so.
+__global__ void comb_prep_grid_kernel(TileGrid T, unsigned *ctrl, unsigned *sticky)
+{
+    const PairDesc P = tile_pair(T, (int)blockIdx.y);
+    prep_pair(P, ctrl, sticky);
+    if (P.sym8 && (int)blockIdx.y < T.GC)
+        stage_sym8(P.b, P.n, (uint32_t *)P.sym8, P.sym8_stride, T.sym8_flags);
 }
 
 // Seeds the rings of the packed chain (blockIdx.y = couple): column c of
@@ -932,37 +1017,6 @@ __global__ void lcsk_zero_kernel(int32_t *x, int32_t n)
     if (i < n) x[i] = 0;
 }
 
-// Byte symbols of a string cut into strips of W columns (the layout
-// lcsk_sym8_stride describes, one set of copies per strip): one thread per
-// word; copy 0 of each strip (which covers every column) raises *flags for a
-// symbol outside [0, 255] or equal to the padding.
-__global__ void comb_sym8_kernel(const int32_t *b, int32_t n, int32_t W, uint32_t *out, int32_t stride, int32_t *flags)
-{
-    const int32_t col0 = (int32_t)blockIdx.y * W, ns = min(W, n - col0);
-    b += col0;
-    out += 4 * (size_t)stride * blockIdx.y;
-    const long long total = 4LL * stride;
-    const long long step = (long long)gridDim.x * blockDim.x;
-    for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += step) {
-        const int j = (int)(q / stride);
-        const long long x = 4 * (q - (long long)j * stride) + j - kSym8Pad;   // column of byte 0
-        uint32_t word = 0;
-        int seen = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const long long c = x + i;
-            uint32_t sym = 255u;
-            if (c >= 0 && c < ns) {
-                sym = (uint32_t)b[c];
-                seen |= sym > 255u ? kSym8Bad : sym == 255u ? kSym8Has255 : 0;
-            }
-            word |= (sym & 0xffu) << (8 * i);
-        }
-        out[q] = word;
-        if (seen && j == 0) atomicOr(flags, seen);
-    }
-}
-
 // Range check of the packed chain's symbols (blockIdx.y = string): bit 0 of
 // bad[item] for a symbol outside [0, 0xfffd], bit 1 for one above 15 (the
 // one-hot cells need every symbol in [0, 15]).
@@ -981,13 +1035,21 @@ __global__ void check16_kernel(const SymbolRange *ranges, int32_t *bad)
 }
 
 // v_out = the strands the last band left in its slot (blockIdx.y = pair).
-__global__ void comb_extract_kernel(const PairDesc *pairs)
+__device__ __forceinline__ void extract_pair(const PairDesc &P)
 {
-    const PairDesc P = pairs[blockIdx.y];
     const unsigned long long *slot = P.E + (size_t)(P.nbands & 1) * (size_t)P.n;
     const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.n; c += stride)
-        P.v_out[c] = (int32_t)(uint32_t)slot[c];
+    for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.n; c += stride) {
+        const uint32_t id = (uint32_t)slot[c];
+        if (P.perm == nullptr) P.v_out[c] = (int32_t)id;
+        else if (id < (uint32_t)(P.m + P.n)) P.perm[id] = (int32_t)c;   // always, after a completed comb
+    }
+}
+__global__ void comb_extract_kernel(const PairDesc *pairs) { extract_pair(pairs[blockIdx.y]); }
+__global__ void comb_extract_grid_kernel(TileGrid T)
+{
+    extract_pair(tile_pair(T, (int)blockIdx.y));
+    if (T.sym8_flags && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *T.sym8_flags = 0;
 }
 
 // row_to_col of each pair's permutation (blockIdx.y = pair): the strand that
@@ -1020,17 +1082,15 @@ __global__ void r2c_from_strands_kernel(const int32_t *h, int32_t m, const int32
     if (id < size) r2c[id] = (int32_t)(i < m ? n + i : i - m);
 }
 
-__global__ void invert_perm_kernel(const int32_t *r2c, int32_t size, int32_t *c2r)
+// h_out, v_out of a permutation: the strand that ends in column c < n leaves
+// column c at the bottom, in column n + l row l on the right.
+__global__ void strands_from_perm_kernel(const int32_t *r2c, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < size && (uint32_t)r2c[i] < (uint32_t)size) c2r[r2c[i]] = (int32_t)i;
-}
-
-__global__ void strands_from_c2r_kernel(const int32_t *c2r, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) v_out[i] = c2r[i];
-    else if (i < (long long)n + m) h_out[i - n] = c2r[i];
+    if (i >= (long long)m + n) return;
+    const uint32_t c = (uint32_t)r2c[i];
+    if (c < (uint32_t)n) v_out[c] = (int32_t)i;
+    else if (c < (uint32_t)(m + n)) h_out[c - (uint32_t)n] = (int32_t)i;
 }
 
 __global__ void copy_kernel(int32_t *dst, const int32_t *src, long long count)
@@ -1071,6 +1131,33 @@ static int launch_chain_tm(const ChainArgs &args, int grid_blocks, int block_thr
     return -22;
 }
 
+static int launch_bands(const ChainArgs &args, int tile_m, int grid_blocks, int block_threads, hipStream_t stream)
+{
+    switch (tile_m) {
+    case 1: return launch_chain_tm<1>(args, grid_blocks, block_threads, stream);
+    case 2: return launch_chain_tm<2>(args, grid_blocks, block_threads, stream);
+    case 4: return launch_chain_tm<4>(args, grid_blocks, block_threads, stream);
+    case 8: return launch_chain_tm<8>(args, grid_blocks, block_threads, stream);
+    case 16: return launch_chain_tm<16>(args, grid_blocks, block_threads, stream);
+    case 32: return launch_chain_tm<32>(args, grid_blocks, block_threads, stream);
+    default: return -22;
+    }
+}
+
+int lcsk_launch_grid(const ChainArgs &args, int grid_blocks, int block_threads, hipStream_t stream)
+{
+    const TileGrid &T = args.grid;
+    const unsigned tiles = (unsigned)(T.GR * T.GC);
+    if (tiles < 1 || tiles > 65535 || args.ntasks <= 0) return -22;
+    // one thread per ring column (and per word of the byte copies)
+    const unsigned fill = (unsigned)std::min<long long>(1024, ((long long)T.W + 255) / 256);
+    hipLaunchKernelGGL(comb_prep_grid_kernel, dim3(fill, tiles), dim3(256), 0, stream, T, args.ticket, args.sticky);
+    const int rc = launch_bands(args, T.pair.tile_m, grid_blocks, block_threads, stream);
+    if (rc) return rc;
+    hipLaunchKernelGGL(comb_extract_grid_kernel, dim3(fill, tiles), dim3(256), 0, stream, T);
+    return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
 int lcsk_launch_chain(const ChainArgs &args, const PairDesc *d_pairs, int npairs, int max_n, int tile_m,
                       int grid_blocks, int block_threads, hipStream_t stream)
 {
@@ -1079,33 +1166,19 @@ int lcsk_launch_chain(const ChainArgs &args, const PairDesc *d_pairs, int npairs
     hipLaunchKernelGGL(comb_prep_kernel, dim3(fill_blocks, npairs), dim3(256), 0, stream, d_pairs, args.ticket,
                        args.sticky);
     if (args.ntasks > 0) {
-        int rc;
-        switch (tile_m) {
-        case 1: rc = launch_chain_tm<1>(args, grid_blocks, block_threads, stream); break;
-        case 2: rc = launch_chain_tm<2>(args, grid_blocks, block_threads, stream); break;
-        case 4: rc = launch_chain_tm<4>(args, grid_blocks, block_threads, stream); break;
-        case 8: rc = launch_chain_tm<8>(args, grid_blocks, block_threads, stream); break;
-        case 16: rc = launch_chain_tm<16>(args, grid_blocks, block_threads, stream); break;
-        case 32: rc = launch_chain_tm<32>(args, grid_blocks, block_threads, stream); break;
-        default: rc = -22;
-        }
+        const int rc = launch_bands(args, tile_m, grid_blocks, block_threads, stream);
         if (rc) return rc;
     }
     hipLaunchKernelGGL(comb_extract_kernel, dim3(fill_blocks, npairs), dim3(256), 0, stream, d_pairs);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-int lcsk_launch_sym8(const int32_t *b, int32_t n, int32_t W, uint32_t *out, int32_t stride, int32_t *flags,
-                     hipStream_t stream)
+int lcsk_launch_sym8(const int32_t *b, int32_t n, uint32_t *out, int32_t stride, int32_t *flags, hipStream_t stream)
 {
-    if (n <= 0 || W <= 0 || stride < lcsk_sym8_stride(W)) return -22;
-    const int32_t strips = (n + W - 1) / W;
-    if (strips > 65535) return -34;
+    if (n <= 0 || stride < lcsk_sym8_stride(n)) return -22;
     hipLaunchKernelGGL(lcsk_zero_kernel, dim3(1), dim3(64), 0, stream, flags, 1);
-    const long long words = 4LL * stride;
-    const unsigned blocks = (unsigned)std::min<long long>((words + 255) / 256, std::max(1, 8192 / strips));
-    hipLaunchKernelGGL(comb_sym8_kernel, dim3(blocks, (unsigned)strips), dim3(256), 0, stream, b, n, W, out, stride,
-                       flags);
+    const unsigned blocks = (unsigned)std::min<long long>((4LL * stride + 255) / 256, 8192);
+    hipLaunchKernelGGL(comb_sym8_kernel, dim3(blocks), dim3(256), 0, stream, b, n, out, stride, flags);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -1163,14 +1236,13 @@ int lcsk_launch_r2c_from_strands(const int32_t *h, int32_t m, const int32_t *v, 
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-int lcsk_launch_strands_from_perm(const int32_t *r2c, int32_t m, int32_t n, int32_t *scratch, int32_t *h_out,
-                                  int32_t *v_out, hipStream_t stream)
+int lcsk_launch_strands_from_perm(const int32_t *r2c, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out,
+                                  hipStream_t stream)
 {
     const long long size = (long long)m + n;
     if (size == 0) return 0;
-    const dim3 grid((unsigned)((size + 255) / 256));
-    hipLaunchKernelGGL(invert_perm_kernel, grid, dim3(256), 0, stream, r2c, (int32_t)size, scratch);
-    hipLaunchKernelGGL(strands_from_c2r_kernel, grid, dim3(256), 0, stream, scratch, m, n, h_out, v_out);
+    hipLaunchKernelGGL(strands_from_perm_kernel, dim3((unsigned)((size + 255) / 256)), dim3(256), 0, stream, r2c, m, n,
+                       h_out, v_out);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 

@@ -249,7 +249,7 @@ int batch_core(lcs_ctx *ctx, Extras *X, int32_t npairs, const int32_t *da, const
     // launches) and the product's strands written to h_out, v_out.
     struct Striped {
         int32_t p, S, W;
-        size_t strip_h, permA, permB, core_ws, c2r, ws_words, perm_off;   // word offsets in merge_ws
+        size_t strip_h, permA, permB, core_ws, ws_words, perm_off;   // word offsets in merge_ws
     };
     std::vector<Striped> sp;
     std::vector<PairDesc> strip_descs;
@@ -270,7 +270,6 @@ int batch_core(lcs_ctx *ctx, Extras *X, int32_t npairs, const int32_t *da, const
         t.permA = take(perm_words);
         t.permB = take(perm_words);
         t.core_ws = take((size_t)std::max(1, t.S / 2) * t.ws_words);
-        t.c2r = take(mm + (size_t)n[p]);
         sp.push_back(t);
     }
     int rc;
@@ -471,8 +470,7 @@ int batch_core(lcs_ctx *ctx, Extras *X, int32_t npairs, const int32_t *da, const
         }
         for (size_t i = 0; i < sp.size(); ++i) {
             const int32_t p = sp[i].p;
-            if (lcsk_launch_strands_from_perm(cur[i].perm[0], m[p], n[p], mws + sp[i].c2r, dh + a_off[p],
-                                              dv + b_off[p], st))
+            if (lcsk_launch_strands_from_perm(cur[i].perm[0], m[p], n[p], dh + a_off[p], dv + b_off[p], st))
                 return LCS_EIO;
         }
         return LCS_OK;

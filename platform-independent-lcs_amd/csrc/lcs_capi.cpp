@@ -300,12 +300,6 @@ int prepare_pairs(lcs_ctx *ctx, std::vector<PairDesc> &pairs, int tm, int wps, u
     return LCS_OK;
 }
 
-int prepare_pairs_own_rings(lcs_ctx *ctx, std::vector<PairDesc> &pairs, int tm, int wps, DevBuf &descs,
-                            unsigned *ctrl, PreparedLaunch &L, hipStream_t stream, int group_w)
-{
-    return prepare_pairs(ctx, pairs, tm, wps, nullptr, descs, ctrl, L, stream, group_w);
-}
-
 // Prep, chain and extract kernels of a prepared launch (no copies or
 // memsets: capturable in a hipGraph).
 int launch_prepared(const PreparedLaunch &L, hipStream_t stream)
@@ -314,23 +308,6 @@ int launch_prepared(const PreparedLaunch &L, hipStream_t stream)
     if (L.packed)
         return lcsk_launch_chain16(L.args, L.args.couples, L.npairs, L.max_n, L.tile_m, L.blocks, L.threads, stream);
     return lcsk_launch_chain(L.args, L.args.pairs, L.npairs, L.max_n, L.tile_m, L.blocks, L.threads, stream);
-}
-
-// Launches the band chain over `pairs` on `stream` with the context's ring,
-// descriptor buffer and ticket words.
-int enqueue_pairs(lcs_ctx *ctx, std::vector<PairDesc> &pairs, int tm, int wps, hipStream_t stream, int group_w)
-{
-    int rc = ctx->ring.reserve(ctx, pairs_ring_words(pairs) * sizeof(unsigned long long));
-    if (rc) return rc;
-    PreparedLaunch L;
-    if ((rc = prepare_pairs(ctx, pairs, tm, wps, (unsigned long long *)ctx->ring.ptr, ctx->descs, ctx->ctrl, L,
-                            stream, group_w)))
-        return rc;
-    if (hipEventRecord(ctx->evc0, stream) != hipSuccess) return LCS_EIO;
-    if ((rc = launch_prepared(L, stream))) return rc;
-    if (hipEventRecord(ctx->evc1, stream) != hipSuccess) return LCS_EIO;
-    ctx->chain_timed = true;
-    return LCS_OK;
 }
 
 // Strips a single pair is cut into.  A thin pair (m <= kDefaultStripMaxM)
@@ -385,97 +362,132 @@ bool use_sym8(int variant, int32_t m, int32_t n)
     if (!LCS_SYM8 || n <= 0 || n > kSym8MaxN) return false;
     return variant == LCS_VARIANT_CHAIN_BYTES || (double)m * (double)n >= kSym8MinCells;
 }
-int stage_sym8(lcs_ctx *ctx, const int32_t *d_b, int32_t n, int32_t W, std::vector<PairDesc> &pairs,
-               hipStream_t stream)
+// How one pair is cut and combed.
+struct GridPlan {
+    int32_t tm, wps, group_w, GR, GC;
+    bool sym8;
+};
+
+// Words of one merge workspace (the largest product of the tree).
+static size_t grid_merge_ws(int32_t m, int32_t n, const GridPlan &G)
 {
-    const int32_t stride = lcsk_sym8_stride(W);
-    const size_t set = 4 * (size_t)stride, bytes = pairs.size() * set * 4 + 64;
-    if (ctx->sym8.reserve(ctx, bytes) != LCS_OK) return LCS_OK;
-    uint32_t *copies = (uint32_t *)ctx->sym8.ptr;
-    int32_t *flags = (int32_t *)(copies + pairs.size() * set);
-    if (lcsk_launch_sym8(d_b, n, W, copies, stride, flags, stream)) return LCS_EIO;
-    for (size_t p = 0; p < pairs.size(); ++p) {
-        pairs[p].sym8 = copies + p * set;
-        pairs[p].sym8_flags = flags;
-        pairs[p].sym8_stride = stride;
-    }
-    return LCS_OK;
+    size_t w = 0;
+    if (G.GC > 1) w = std::max(w, lcsb_multiply_ws_words(m + n, m + n, m));
+    if (G.GR > 1) w = std::max(w, lcsb_multiply_ws_words(m + n, m + n, n));
+    return w;
 }
 
-// One pair cut into `strips` column strips: comb the strips in one chain
-// launch, turn each into its permutation, merge them pairwise with the
-// steady ant (b-split, k = m), and read the strands off the product.
-int enqueue_strips(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_b, int32_t n, int strips, int tm,
-                   int wps, int group_w, bool sym8, int32_t *d_h, int32_t *d_v, hipStream_t stream)
+// Words of the tiles' permutations: every tile row holds its rows once per
+// tile column and the columns once.
+static size_t grid_perm_words(int32_t m, int32_t n, const GridPlan &G)
 {
-    const int32_t W = (n + strips - 1) / strips;
-    const int S = (n + W - 1) / W;
-    size_t perm_words = (size_t)S * m + n;
-    // one workspace per product of a merge-tree level (at most S/2 of them)
-    const size_t ws_words = lcsb_multiply_ws_words(m + n, m + n, m);
-    const size_t nws = (size_t)(S / 2 > 0 ? S / 2 : 1);
-    const size_t words = (size_t)S * m + n + 2 * perm_words + nws * ws_words + (size_t)(m + n) + 2 * (size_t)(S + 1);
-    int rc = ctx->strip_ws.reserve(ctx, words * 4);
-    if (rc) return rc;
-    int32_t *hs = (int32_t *)ctx->strip_ws.ptr, *vs = hs + (size_t)S * m;
-    int32_t *permA = vs + n, *permB = permA + perm_words, *mws = permB + perm_words;
-    int32_t *c2r = mws + nws * ws_words;
-    int64_t *d_off = (int64_t *)(((uintptr_t)(c2r + m + n) + 7) & ~(uintptr_t)7);
-    std::vector<PairDesc> pairs((size_t)S);
-    std::vector<int64_t> off((size_t)S), size((size_t)S);
-    int64_t acc = 0;
-    for (int s = 0; s < S; ++s) {
-        PairDesc &P = pairs[(size_t)s];
-        P = PairDesc{};
-        P.a = d_a;
-        P.b = d_b + (size_t)s * W;
-        P.m = m;
-        P.n = std::min<int32_t>(W, n - s * W);
-        P.h_out = hs + (size_t)s * m;
-        P.v_out = vs + (size_t)s * W;
-        off[(size_t)s] = acc;
-        size[(size_t)s] = (int64_t)m + P.n;
-        acc += size[(size_t)s];
-    }
-    if (sym8) {
-        if ((rc = stage_sym8(ctx, d_b, n, W, pairs, stream))) return rc;
-    }
-    if ((rc = enqueue_pairs(ctx, pairs, tm, wps, stream, group_w))) return rc;
-    // enqueue_pairs staged the descriptors into ctx->descs; reuse them for the permutations
-    if ((rc = upload(ctx, d_off, off.data(), off.size() * sizeof(int64_t), stream))) return rc;
-    if ((rc = lcsk_launch_from_strands((const PairDesc *)ctx->descs.ptr, S, m + W, permA, d_off, stream))) return rc;
-    // merge tree: the products of a level share one core launch
-    std::vector<int32_t *> cur((size_t)S);
-    std::vector<int64_t> cur_size = size;
-    for (int s = 0; s < S; ++s) cur[(size_t)s] = permA + off[(size_t)s];
+    return (size_t)G.GC * m + (size_t)G.GR * n;
+}
+
+// Merges the tiles' permutations to the whole pair's and writes its strands.
+// Every level joins neighbours along the shorter side of the current tiles
+// (two tiles side by side glue on their common rows, one above the other on
+// their common columns), all its products in one launch sequence.
+static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_t *ws, size_t ws_words, int32_t *d_h,
+                       int32_t *d_v, hipStream_t stream)
+{
+    const int32_t m = T.pair.m, n = T.pair.n;
+    struct Tile {
+        int32_t *p;
+        int32_t m, n;
+    };
+    int32_t gr = T.GR, gc = T.GC;
+    std::vector<Tile> cur((size_t)gr * gc);
+    for (int32_t i = 0; i < gr; ++i)
+        for (int32_t j = 0; j < gc; ++j) cur[(size_t)i * gc + j] = Tile{permA + T.perm_off(i, j), T.rows(i), T.cols(j)};
     int32_t *dst_base = permB;
-    while (cur.size() > 1) {
-        std::vector<int32_t *> nxt;
-        std::vector<int64_t> nxt_size;
+    while (gr * gc > 1) {
+        const bool side = gc > 1 && (gr == 1 || cur[0].m <= cur[0].n);   // glue columns of tiles (on rows) or rows
+        const int32_t nr = side ? gr : (gr + 1) / 2, nc = side ? (gc + 1) / 2 : gc;
+        std::vector<Tile> nxt((size_t)nr * nc);
         std::vector<MulSpec> specs;
         int32_t *dst = dst_base;
-        for (size_t i = 0; i + 1 < cur.size(); i += 2) {
-            const int64_t out_size = cur_size[i] + cur_size[i + 1] - m;
-            specs.push_back(MulSpec{cur[i], (int32_t)cur_size[i], cur[i + 1], (int32_t)cur_size[i + 1], m, 0, dst,
-                                    mws + specs.size() * ws_words});
-            nxt.push_back(dst);
-            nxt_size.push_back(out_size);
-            dst += out_size;
-        }
-        if ((rc = lcsb_multiply_many_device(specs.data(), (int)specs.size(), stream))) return rc;
-        if (cur.size() % 2) {
-            // carry the odd permutation over to the next buffer
-            if (hipMemcpyAsync(dst, cur.back(), (size_t)cur_size.back() * 4, hipMemcpyDeviceToDevice, stream) !=
-                hipSuccess)
-                return LCS_EIO;
-            nxt.push_back(dst);
-            nxt_size.push_back(cur_size.back());
-        }
+        for (int32_t i = 0; i < nr; ++i)
+            for (int32_t j = 0; j < nc; ++j) {
+                const Tile &p = cur[(size_t)(side ? i : 2 * i) * gc + (side ? 2 * j : j)];
+                Tile &o = nxt[(size_t)i * nc + j];
+                o = Tile{dst, p.m, p.n};
+                if (side ? 2 * j + 1 < gc : 2 * i + 1 < gr) {
+                    const Tile &q = side ? cur[(size_t)i * gc + 2 * j + 1] : cur[(size_t)(2 * i + 1) * gc + j];
+                    specs.push_back(MulSpec{p.p, p.m + p.n, q.p, q.m + q.n, side ? p.m : p.n, side ? 0 : 1, dst,
+                                            ws + specs.size() * ws_words});
+                    if (side) o.n += q.n;
+                    else o.m += q.m;
+                } else if (lcsk_launch_copy(dst, p.p, (long long)p.m + p.n, stream)) {
+                    return LCS_EIO;   // an odd tile moves on unchanged
+                }
+                dst += o.m + o.n;
+            }
+        const int rc = lcsb_multiply_many_device(specs.data(), (int)specs.size(), stream);
+        if (rc) return rc;
         cur.swap(nxt);
-        cur_size.swap(nxt_size);
-        dst_base = (dst_base == permB) ? permA : permB;
+        gr = nr;
+        gc = nc;
+        dst_base = dst_base == permB ? permA : permB;
     }
-    return lcsk_launch_strands_from_perm(cur[0], m, n, c2r, d_h, d_v, stream);
+    return lcsk_launch_strands_from_perm(cur[0].p, m, n, d_h, d_v, stream);
+}
+
+// Combs one pair as the tiles of `G` in one chain launch and merges them.
+// The launch is described by its arguments alone: nothing is uploaded.
+static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, hipStream_t stream)
+{
+    const int32_t m = pair.m, n = pair.n;
+    TileGrid T{};
+    T.pair = pair;
+    T.H = (m + G.GR - 1) / G.GR;
+    T.W = (n + G.GC - 1) / G.GC;
+    T.GR = G.GR = (m + T.H - 1) / T.H;   // no empty tile
+    T.GC = G.GC = (n + T.W - 1) / T.W;
+    const int32_t tiles = T.GR * T.GC;
+    T.pair.tile_m = G.tm;
+    T.pair.nbands = bands_of(T.H, T.W, G.tm);
+    int rc = ctx->ring.reserve(ctx, (size_t)tiles * lcsk_ring_words(T.W) * sizeof(unsigned long long));
+    if (rc) return rc;
+    T.pair.E = (unsigned long long *)ctx->ring.ptr;
+    if (G.sym8) {
+        const int32_t stride = lcsk_sym8_stride(T.W);
+        if (ctx->sym8.reserve(ctx, (size_t)T.GC * 16 * (size_t)stride) == LCS_OK) {
+            T.pair.sym8 = (const uint32_t *)ctx->sym8.ptr;
+            T.pair.sym8_stride = stride;
+            T.sym8_flags = (int32_t *)ctx->ctrl + kSym8FlagWord;
+            T.pair.sym8_flags = T.sym8_flags;
+        }
+    }
+    size_t perm_words = 0, ws_words = 0;
+    int32_t *ws = nullptr;
+    if (tiles > 1) {
+        perm_words = grid_perm_words(m, n, G);
+        ws_words = grid_merge_ws(m, n, G);
+        if ((rc = ctx->strip_ws.reserve(ctx, (2 * perm_words + (size_t)(tiles / 2) * ws_words) * 4))) return rc;
+        T.perm = (int32_t *)ctx->strip_ws.ptr;
+        ws = T.perm + 2 * perm_words;
+    }
+    ChainArgs A{};
+    const long long units = (T.pair.nbands + G.group_w - 1) / G.group_w * (long long)tiles;
+    if (units > 0x7fffffffLL) return LCS_ERANGE;
+    A.grid = T;
+    A.ntasks = (int32_t)units;
+    A.group_w = G.group_w;
+    A.ticket = ctx->ctrl;
+    A.abort_flag = ctx->ctrl + 1;
+    A.sticky = ctx->ctrl + kStickyWord;
+    A.timeout_ticks = ctx->timeout_ticks;
+    A.trace = ctx->band_trace;
+    A.trace_cap = ctx->band_trace_cap;
+    const long long per_cu = G.group_w == 1 ? 4LL : 1LL, resident = per_cu * ctx->num_cus * G.wps;
+    const long long blocks = (std::min(units, resident) + per_cu - 1) / per_cu;
+    if (hipEventRecord(ctx->evc0, stream) != hipSuccess) return LCS_EIO;
+    if ((rc = lcsk_launch_grid(A, (int)blocks, 256, stream))) return rc;
+    if (hipEventRecord(ctx->evc1, stream) != hipSuccess) return LCS_EIO;
+    ctx->chain_timed = true;
+    if (tiles == 1) return LCS_OK;
+    return merge_tiles(T, T.perm, T.perm + perm_words, ws, ws_words, pair.h_out, pair.v_out, stream);
 }
 
 int ws_acquire(lcs_ctx *ctx, hipStream_t s)
@@ -553,11 +565,8 @@ static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const i
     if (strips > 1 && (d_h_in || d_v_in)) return LCS_EINVAL;  // fixups use explicit strands: one strip
     if (strips > 1 && m > kMaxCoreK) return LCS_ERANGE;
     if (strips > n) strips = n;
-    const bool sym8 = use_sym8(sched ? sched->variant : LCS_VARIANT_AUTO, m, n);
-    if (strips > 1) return enqueue_strips(ctx, d_a, m, d_b, n, strips, tm, wps, group_w, sym8, d_h, d_v, stream);
-    std::vector<PairDesc> pairs(1);
-    PairDesc &P = pairs[0];
-    P = PairDesc{};
+    GridPlan G{tm, wps, group_w, 1, strips, use_sym8(sched ? sched->variant : LCS_VARIANT_AUTO, m, n)};
+    PairDesc P{};
     P.a = d_a;
     P.b = d_b;
     P.h_in = d_h_in;
@@ -566,11 +575,7 @@ static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const i
     P.v_out = d_v;
     P.m = m;
     P.n = n;
-    if (sym8) {
-        const int rc = stage_sym8(ctx, d_b, n, n, pairs, stream);
-        if (rc) return rc;
-    }
-    return enqueue_pairs(ctx, pairs, tm, wps, stream, group_w);
+    return enqueue_grid(ctx, P, G, stream);
 }
 
 // The abort flag of the last launch on the context's own ctrl words (the

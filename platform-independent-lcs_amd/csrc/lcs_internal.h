@@ -64,6 +64,9 @@ namespace lcs {
 // ctrl word that collects the abort flags of finished launches (folded in by
 // each launch's prep kernel); lcs_ctx_status reads and clears it
 constexpr int kStickyWord = 63;
+// ctrl word of the byte-symbol flags of single-pair launches; zero between
+// launches (each one's extract kernel clears it)
+constexpr int kSym8FlagWord = 62;
 }  // namespace lcs
 
 struct lcs_ctx {
@@ -127,9 +130,6 @@ int prepare_pairs(lcs_ctx *ctx, std::vector<PairDesc> &pairs, int tm, int wps, u
 // group width of a schedule variant (LCS_VARIANT_*), 0 if unknown
 int group_width(int variant);
 int launch_prepared(const PreparedLaunch &L, hipStream_t stream);
-int prepare_pairs_own_rings(lcs_ctx *ctx, std::vector<PairDesc> &pairs, int tm, int wps, DevBuf &descs,
-                            unsigned *ctrl, PreparedLaunch &L, hipStream_t stream, int group_w = 1);
-int enqueue_pairs(lcs_ctx *ctx, std::vector<PairDesc> &pairs, int tm, int wps, hipStream_t stream, int group_w = 1);
 // whether a single pair's register chain stages its b as byte symbols
 // (lcsk_launch_sym8): pairs of 2^22 cells or more, or LCS_VARIANT_CHAIN_BYTES
 bool use_sym8(int variant, int32_t m, int32_t n);

@@ -216,7 +216,7 @@ int launch_slot(lcs_server *S, Slot &slot)
             const int32_t stride = lcsk_sym8_stride(n);
             uint32_t *copies = (uint32_t *)(((uintptr_t)(E + lcsk_ring_words(n)) + kAlign - 1) & ~(uintptr_t)(kAlign - 1));
             int32_t *flags = (int32_t *)(copies + (size_t)4 * stride);
-            if (lcsk_launch_sym8(db, n, n, copies, stride, flags, slot.stream)) return LCS_EIO;
+            if (lcsk_launch_sym8(db, n, copies, stride, flags, slot.stream)) return LCS_EIO;
             P.sym8 = copies;
             P.sym8_flags = flags;
             P.sym8_stride = stride;
