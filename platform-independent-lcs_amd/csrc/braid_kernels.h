@@ -4,8 +4,8 @@
 #include <stdint.h>
 
 // Largest padded core (2^L): cores up to 2^11 run in one workgroup's LDS,
-// larger ones over the whole GPU (their grid of ant-walk boxes is sized
-// for nodes of at most 2^22 points).
+// larger ones over the whole GPU (their grid of boxes is sized for nodes of
+// at most 2^22 points).
 constexpr int kMaxCoreL = 22;
 constexpr int kMaxCoreK = 1 << kMaxCoreL;
 

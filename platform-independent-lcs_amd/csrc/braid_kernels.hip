@@ -15,19 +15,20 @@
 //    once -- and remembers where each point came from;
 //  * bottom-up, each depth lifts the children's products into the node's
 //    coordinates (the reference's inverse_mapping, :191-202) and runs the ant
-//    passage (:123-189) for all nodes at once.  The passage is cut into
-//    chunks of rows: the dominance-sum difference
+//    passage (:123-189) for all nodes at once.  The dominance-sum difference
 //        delta(r, c) = #{hi points: row < r, col < c} - #{lo points: row >= r, col >= c}
 //    is non-decreasing in r and c, so the ant leaves row r at the first
-//    column T(r) where delta >= 0.  Waves find T and delta at each chunk
-//    boundary with sweeps over the node's columns (and, in nodes of 256
-//    rows or more, where the ant crosses every rc-th column with sweeps
-//    over its rows); then one thread per piece walks it with the
-//    reference's incremental updates and places the good points.
-// The union of the children's points, the per-column view and the parents
-// of every depth's partition live in LDS (16-bit entries, the lo/hi flag in
-// bit 15), so the walks and the lifts run at LDS latency.  Cores up to
-// K = 2048 take this path (the parents alone are 4 K log2(K) bytes).
+//    column T(r) where delta >= 0, and the product's point of row r follows
+//    from T(r) and the row's own point alone: it is T(r) - 1 when T(r) > 0
+//    and the point is counted at T(r) (lo ? col >= T : col < T), else the
+//    point itself.  So nothing is walked: waves find T at every 64th row line
+//    and the row where the path crosses every 64th column line, and one wave
+//    per box finds T for its 64 rows, a lane each, from bit masks of the
+//    box's columns.
+// The last six depths (nodes of 64 points) run in one wave's registers.  The
+// union of the children's points, the per-column view and the parents of the
+// depths above live in LDS (16-bit entries, the lo/hi flag in bit 15) for
+// cores up to K = 2048.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -40,33 +41,21 @@
 namespace lcsb {
 
 constexpr int kThreads = 1024;
-// nodes of at least this many rows also cut their walks at column lines
-#ifndef LCS_COL_LINE_MIN_S
-#define LCS_COL_LINE_MIN_S 256
-#endif
-constexpr int kColLineMinS = LCS_COL_LINE_MIN_S;
-// rows per walked chunk of a node (nodes above 128 chunks take s / 128)
-#ifndef LCS_CORE_CHUNK_ROWS
-#define LCS_CORE_CHUNK_ROWS 8
-#endif
-constexpr int kChunkRows = LCS_CORE_CHUNK_ROWS;
-static_assert(kChunkRows >= 4 && kChunkRows <= 64 && (kChunkRows & (kChunkRows - 1)) == 0, "chunk rows");
 constexpr uint16_t kLoFlag = 0x8000u;
 constexpr uint16_t kIdx = 0x7fffu;
 // cores up to this size keep keys, products and parents in LDS
 // (braid_core_lds_kernel and the leaves of larger cores)
 constexpr int kLdsCoreL = 11;
 constexpr int kLdsCoreK = 1 << kLdsCoreL;
-// row chunks per node are at most 128 (chunk height max(kChunkRows, s/128)); each wave
-// keeps 2 x kMaxChunks bucket counters in LDS for the boundary sweeps
-constexpr int kMaxChunks = 128;
+constexpr int kBox = 64;   // side of a box: one wave, a lane per row
+constexpr int kMaxLeafLines = kLdsCoreK / kBox;   // grid lines of the largest node in LDS
 // dynamic LDS of a core of 2^L points: keys / U, CI, R, Rn (4K uint16), the
 // K/64+1 group counts of P and of Q, then the parents of P and of Q at each
-// depth (2 L K uint16)
+// depth above the 64-point nodes (2 (L - 6) K uint16)
 constexpr size_t lds_core_bytes(int L)
 {
     return (size_t)4 * (1 << L) * sizeof(uint16_t) + 2 * ((size_t)(1 << L) / 64 + 1) * 4 +
-           (size_t)2 * L * (1 << L) * sizeof(uint16_t);
+           (size_t)2 * (L - 6) * (1 << L) * sizeof(uint16_t);
 }
 
 // Inclusive prefix sum over the 64 lanes of a wave with DPP: four row_shr
@@ -83,20 +72,165 @@ __device__ __forceinline__ int wave_incl_scan(int x)
     return x;
 }
 
-// One bottom-up depth (node size s) of the core: lift the children's
-// products into node coordinates (the reference's inverse_mapping, :191-202)
-// and run the chunked ant passage (:123-189) for every node of the depth.
-// U, CI are in LDS; R (children's products) and Rn (this depth's) are
-// either global int32 or LDS uint16 arrays; pp, pq (LDS) map depth d+1
-// positions to depth d positions; bT, bD hold K/kChunkRows chunk entries.
-template <typename UT, typename RT, typename RNT>
-__device__ __forceinline__ void bottom_up_depth(UT *U, UT *CI, const RT *R, RNT *Rn, const uint16_t *pp,
-                                                const uint16_t *pq, int K, int s, int32_t *bT, int32_t *bD,
-                                                int32_t *cT, int *hist)
+// An entry of U or CI counts at line r: lo ? idx >= r : idx < r.  With the
+// lo flag in bit F of the entry and idx, r below 2^F this is bit F of e - r.
+template <int F>
+__device__ __forceinline__ uint32_t counted(uint32_t e, int r)
+{
+    return ((e - (uint32_t)r) >> F) & 1u;
+}
+
+// Position of the k-th set bit of w, of 2H bits (1 <= k <= popcount(w)).
+template <int H>
+__device__ __forceinline__ int select_bit(uint32_t w, int k)
+{
+    int pos = 0;
+#pragma unroll
+    for (int h = H; h >= 1; h >>= 1) {
+        const int c = __popc(w & ((1u << h) - 1));
+        const bool up = k > c;
+        k -= up ? c : 0;
+        w = up ? w >> h : w;
+        pos += up ? h : 0;
+    }
+    return pos;
+}
+__device__ __forceinline__ int select64(uint32_t lo, uint32_t hi, int k)
+{
+    const int c = __popc(lo);
+    const bool up = k > c;
+    return (up ? 32 : 0) + select_bit<16>(up ? hi : lo, up ? k - c : k);
+}
+
+// Bit c (of 16) = entry c counts at this lane's line, for 16 entries held by
+// the 16 lanes of each DPP row (lane l of the row: entry l), every entry and
+// line shifted so that the counted bit of their difference is bit 31.  Each of
+// the 16 rotations of the row subtracts and shifts one bit in (a v_sub with a
+// DPP operand and a v_alignbit); after them bit b is the entry of lane
+// (b + l + 1) mod 16.
+__device__ __forceinline__ uint32_t counted_row16(uint32_t up, uint32_t rr, int lane)
+{
+    uint32_t w = (up - rr) >> 31, t;
+    // in one block, as the compiler does not fold the rotation into the
+    // subtract; the s_nop covers a DPP read of an `up` written just before
+#define LCSB_ROR(I)                                                                     \
+    "v_sub_u32_dpp %[t], %[e], %[r] row_ror:" #I " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_alignbit_b32 %[w], %[w], %[t], 31\n\t"
+    asm("s_nop 1\n\t" LCSB_ROR(1) LCSB_ROR(2) LCSB_ROR(3) LCSB_ROR(4) LCSB_ROR(5) LCSB_ROR(6) LCSB_ROR(7) LCSB_ROR(8)
+            LCSB_ROR(9) LCSB_ROR(10) LCSB_ROR(11) LCSB_ROR(12) LCSB_ROR(13) LCSB_ROR(14) LCSB_ROR(15)
+        : [w] "+v"(w), [t] "=&v"(t)
+        : [e] "v"(up), [r] "v"(rr));
+#undef LCSB_ROR
+    return ((w | w << 16) >> (~lane & 15)) & 0xffffu;
+}
+
+__device__ __forceinline__ int lane_push(int dst, int x) { return __builtin_amdgcn_ds_permute(dst << 2, x); }
+__device__ __forceinline__ int lane_pull(int src, int x) { return __builtin_amdgcn_ds_bpermute(src << 2, x); }
+
+// The sticky product of 64 points in one wave: lane x holds row x's shared
+// column kp and column x's shared row kq; returns row x's column.  All six
+// depths stay in registers: the partitions and lifts move between lanes by
+// ds_permute, and a node's T(r) comes from one mask of its columns per lane
+// (each node is a single box entered at T(s) = 0).  Bound by VALU issue:
+// about 1000 instructions per 64 points, 12 us of a 2048-point core's 75.
+__device__ __forceinline__ int wave_product64(int kp, int kq, int lane)
+{
+    const unsigned long long lt = (1ull << lane) - 1;
+    int pp[6], pq[6];
+    auto split = [&](int &key, int s, int bit) {
+        const int b = (key >> bit) & 1, seg = lane & ~(s - 1);
+        const unsigned long long in = s == 64 ? ~0ull : ((1ull << (s & 63)) - 1) << seg, m = __ballot(b) & in;
+        const int before = __popcll(m & lt), ones = __popcll(m);
+        const int pos = b ? seg + s - ones + before : lane - before;
+        const int v = lane_push(pos, key << 6 | lane);
+        key = v >> 6;
+        return v & 63;
+    };
+#pragma unroll
+    for (int d = 0; d < 6; ++d) {
+        pp[d] = split(kp, 64 >> d, 5 - d);
+        pq[d] = split(kq, 64 >> d, 5 - d);
+    }
+    int R = 0;   // 1 x 1 nodes
+#pragma unroll
+    for (int d = 5; d >= 0; --d) {
+        const int s = 64 >> d, h = s >> 1;
+        const int p_pos = pp[d], q_pos = lane_pull((lane & ~(h - 1)) + R, pq[d]);
+        const int p0 = p_pos & ~(s - 1);
+        const uint32_t flag = (lane & h) ? 0u : 0x80u;
+        const uint32_t u = (uint32_t)lane_push(p_pos, (int)((uint32_t)(q_pos - p0) | flag));
+        const uint32_t ci = (uint32_t)lane_push(q_pos, (int)((uint32_t)(p_pos - p0) | flag));
+        const int v0 = lane & ~(s - 1), r = lane - v0;
+        const unsigned long long in = s == 64 ? ~0ull : ((1ull << (s & 63)) - 1) << v0;
+        const int need = __popcll(__ballot((u & 0x80u) != 0) & in & ~lt);   // lo rows >= r
+        // the node's columns 16 at a time: the lane's own DPP row and, in
+        // larger nodes, the rows that lane_pull brings alongside
+        const uint32_t up = ci << 24, rr = (uint32_t)r << 24;
+        int T = 0;
+        if (s <= 16) {
+            const uint32_t w = (counted_row16(up, rr, lane) >> (v0 & 15)) & ((1u << (s & 31)) - 1);
+            T = 1 + (s == 16 ? select_bit<8>(w, need) : s == 8 ? select_bit<4>(w, need) : s == 4 ? select_bit<2>(w, need)
+                                                                                     : select_bit<1>(w, need));
+        } else {
+            uint32_t q[4] = {};
+#pragma unroll
+            for (int i = 0; i < s / 16; ++i)
+                q[i] = counted_row16((uint32_t)lane_pull(v0 + 16 * i + (lane & 15), (int)up), rr, lane);
+            const uint32_t lo = q[0] | q[1] << 16;
+            T = 1 + (s == 32 ? select_bit<16>(lo, need) : select64(lo, q[2] | q[3] << 16, need));
+        }
+        T = need ? T : 0;
+        const int lc = (int)(u & 0x7fu);
+        R = T > 0 && counted<7>(u, T) ? T - 1 : lc;
+        R &= s - 1;   // in range whatever an aborted comb fed in
+    }
+    return R;
+}
+
+// One wave's box of kBox rows r_lo .. r_lo + 63 of a node (lane l: row r_lo +
+// l, entry u): the rows that the ant's path crosses with T in (cs, ce] (or T =
+// cs, from a row line), ce - cs <= 64.  From a row line (COL false) every row
+// is open and delta(r_lo + 64, cs) = 0; from a column line cs the rows up to
+// rho are, and delta(rho, cs) = -1.  -delta(r, cs) adds the rows from r down
+// to the line that count at cs; T(r) is the position after that many counted
+// columns.  entry(c) reads column c's entry, c < ce; the caller may lower ce
+// to T(r_lo), which no open row exceeds.  Returns the row's new column or -1.
+template <int F, bool COL, typename Entry>
+__device__ __forceinline__ int box_rows(uint32_t u, Entry entry, int r_lo, int rho, int cs, int ce, int lane)
+{
+    const int r = r_lo + lane;
+    const bool uc = counted<F>(u, cs);
+    const unsigned long long m = __ballot(COL ? uc && r < rho : uc);
+    const int need = (COL ? 1 : 0) + (int)__popcll(m >> lane);
+    const uint32_t rr = (uint32_t)r << (31 - F);
+    uint32_t q[4] = {};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int c = cs + 16 * i + (lane & 15);
+        if (cs + 16 * i < ce)   // uniform; past ce an entry that counts at no line
+            q[i] = counted_row16(c < ce ? (uint32_t)entry(c) << (31 - F) : 0x7fffffffu, rr, lane);
+    }
+    const uint32_t lo = q[0] | q[1] << 16, hi = q[2] | q[3] << 16;
+    const bool open = (!COL || r <= rho) && need <= __popc(lo) + __popc(hi);
+    const int T = need ? cs + 1 + select64(lo, hi, need) : cs;
+    return open && T > 0 && counted<F>(u, T) ? T - 1 : -1;
+}
+
+// One bottom-up depth (node size s >= 128) of a core in LDS: lift the
+// children's products into node coordinates (the reference's
+// inverse_mapping, :191-202), then the ant passage (:123-189) for every node:
+// counts per 64-entry block and line, the crossing of each line, the boxes.
+struct LeafLines {
+    uint16_t T[2][kMaxLeafLines];                      // [0] row lines, [1] column lines (T = rho + 1), per node nb
+    uint16_t lo[2][kMaxLeafLines];                     // lo entries per block of CI, of U
+    uint8_t cnt[2][kMaxLeafLines][kMaxLeafLines];      // [dir][block][j]: z_j entries of the block
+};
+__device__ __forceinline__ void bottom_up_depth(uint16_t *U, uint16_t *CI, const uint16_t *R, uint16_t *Rn,
+                                                const uint16_t *pp, const uint16_t *pq, int K, int s, LeafLines &B)
 {
     const int h = s >> 1;
     // lift the children's products into node coordinates
-#pragma unroll 4
+#pragma unroll 2
     for (int x = threadIdx.x; x < K; x += kThreads) {
         const int p_pos = pp[x];
         const int cseg = x & ~(h - 1);
@@ -106,243 +240,92 @@ __device__ __forceinline__ void bottom_up_depth(UT *U, UT *CI, const RT *R, RNT 
         const int lr = p_pos - v0, lc = q_pos - v0;
         U[p_pos] = (uint16_t)lc | lo;
         CI[v0 + lc] = (uint16_t)lr | lo;
-        Rn[p_pos] = lc;
+        Rn[p_pos] = (uint16_t)lc;
     }
     __syncthreads();
-    // chunk height: kChunkRows, or s/128 for big nodes, balancing the
-    // boundary scans (O(s) each) against the walks (O(rows) each)
-    // (nodes under 64 rows are one chunk: the boundary sweeps read 64 columns per round)
-    const int rc = s < 64 ? s : (s / 128 > kChunkRows ? s / 128 : kChunkRows);
-    const int rc_log = __builtin_ctz(rc);   // rc and s are powers of two
-    const int nch = s / rc;            // chunks per node
-    // chunk entry points: chunk j of a node covers rows [s-(j+1)rc, s-j rc).
-    // A node's first chunk (j = 0) enters at T = 0; its entry is computed in
-    // the walk, so only chunks j > 0 (nodes of 64 rows or more, at most
-    // K/kChunkRows chunks) store entries in bT, bD.  For chunk j > 0 entering at row
-    // Dr = s - j rc:
-    //   T(Dr) = min{ c : Z(c) >= Y }, Z(c) = #{c' < c : z(c')},
-    //   z(c) = hi(c) ? row(c) < Dr : row(c) >= Dr,  Y = #{lo rows >= Dr},
-    // and delta(Dr, T) = Z(T) - Y = 0.  With the row bucket of a column,
-    // b(c) = (s-1-row(c)) / rc, z_j(c) = lo ? b(c) < j : b(c) >= j, so one
-    // wave finds all of a node's boundaries in two sweeps over its columns
-    // (64 per round, conflict-free): the histogram of the round's buckets
-    // (lo and hi, wave-local LDS counters) and a scan over the buckets give
-    // every boundary's count at once; lane L keeps boundaries 2L and 2L+1.
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // Line j of a node (row line Dr = s - 64 j over the columns' entries CI,
+    // column line c = s - 64 j over the rows' entries U): with bucket b =
+    // (s-1-idx) / 64 of an entry, z_j = lo ? b < j : b >= j, Y_j = #{lo
+    // entries with b < j} and T_j = the first position with Y_j z_j entries
+    // before it.
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    constexpr int kWaves = kThreads / 64;
+    const int nb = s >> 6, blocks = K >> 6, nodes = K / s;
     const unsigned long long lt = (1ull << lane) - 1;
-    if (nch > 1) {
-        int *hlo = hist + wave * 2 * kMaxChunks, *hhi = hlo + kMaxChunks;   // this wave's counters
-        const int j0 = 2 * lane, j1 = 2 * lane + 1;
-        // Bucket counts of the columns [c_begin, c_end) of a node, as seen
-        // from boundaries j0 and j1: lo columns with bucket < j (lp) and
-        // columns with z_j (cnt).  The wave's LDS accesses run in order; the
-        // fences keep the compiler from moving counter stores, adds and loads
-        // across each other.
-        auto range_counts = [&](const UT *E, int v0, int c_begin, int c_end, int &lp0, int &lp1, int &cnt0,
-                                int &cnt1) {
-            hlo[j0] = 0;
-            hlo[j1] = 0;
-            hhi[j0] = 0;
-            hhi[j1] = 0;
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            for (int c0 = c_begin; c0 < c_end; c0 += 64) {
-                const uint16_t e = E[v0 + c0 + lane];
-                const int bk = (s - 1 - (e & kIdx)) >> rc_log;
-                atomicAdd((e & kLoFlag) ? &hlo[bk] : &hhi[bk], 1);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const int l0 = __hip_atomic_load(&hlo[j0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            const int l1 = __hip_atomic_load(&hlo[j1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            const int g0 = __hip_atomic_load(&hhi[j0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            const int g1 = __hip_atomic_load(&hhi[j1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            const int il = wave_incl_scan(l0 + l1), ih = wave_incl_scan(g0 + g1);
-            const int hi_total = __builtin_amdgcn_readlane(ih, 63);
-            lp0 = il - l0 - l1;
-            lp1 = lp0 + l0;
-            const int hp0 = ih - g0 - g1, hp1 = hp0 + g0;   // hi columns with bucket < j
-            cnt0 = lp0 + (hi_total - hp0);
-            cnt1 = lp1 + (hi_total - hp1);
-        };
-        // Running Z_j over [c_begin, c_end) in rounds of 64 columns for the
-        // open boundaries until Z_j reaches Y_j; T = the column where it does.
-        auto find_T = [&](const UT *E, int v0, int c_begin, int c_end, int Y0, int Y1, int Z0, int Z1, bool open0,
-                          bool open1, int &T0, int &T1) {
-            for (int c0 = c_begin; c0 < c_end && __ballot(open0 || open1); c0 += 64) {
-                hlo[j0] = 0;
-                hlo[j1] = 0;
-                hhi[j0] = 0;
-                hhi[j1] = 0;
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                const uint16_t e = E[v0 + c0 + lane];
-                const bool lo = (e & kLoFlag) != 0;
-                const int bk = (s - 1 - (e & kIdx)) >> rc_log;
-                atomicAdd(lo ? &hlo[bk] : &hhi[bk], 1);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                const int l0 = __hip_atomic_load(&hlo[j0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                const int l1 = __hip_atomic_load(&hlo[j1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                const int g0 = __hip_atomic_load(&hhi[j0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                const int g1 = __hip_atomic_load(&hhi[j1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                const int il = wave_incl_scan(l0 + l1), ih = wave_incl_scan(g0 + g1);
-                const int hi_total = __builtin_amdgcn_readlane(ih, 63);
-                const int lp0 = il - l0 - l1, lp1 = lp0 + l0;      // lo columns with bucket < j
-                const int hp0 = ih - g0 - g1, hp1 = hp0 + g0;      // hi columns with bucket < j
-                const int cnt0 = lp0 + (hi_total - hp0), cnt1 = lp1 + (hi_total - hp1);
-                const bool cross0 = open0 && Z0 + cnt0 >= Y0, cross1 = open1 && Z1 + cnt1 >= Y1;
-                if (open0 && !cross0) Z0 += cnt0;
-                if (open1 && !cross1) Z1 += cnt1;
-                // boundaries reaching Y in this round: find the exact column, one at a time
-                const unsigned long long todo = __ballot(cross0), todo1 = __ballot(cross1);
-                for (int which = 0; which < 2; ++which) {
-                    unsigned long long t = which ? todo1 : todo;
-                    while (t) {
-                        const int l = __ffsll((long long)t) - 1;
-                        t &= t - 1;
-                        const int jj = 2 * l + which;
-                        const int need = __shfl(which ? Y1 - Z1 : Y0 - Z0, l);   // 1-based rank in this round
-                        const bool z = lo ? bk < jj : bk >= jj;
-                        const unsigned long long zm = __ballot(z);
-                        const bool hit = z && __popcll(zm & lt) == need - 1;
-                        const int pos = __ffsll((long long)__ballot(hit));  // 1-based lane of the column
-                        if (lane == l) {
-                            if (which) T1 = c0 + pos; else T0 = c0 + pos;
-                        }
-                    }
-                }
-                if (cross0) open0 = false;
-                if (cross1) open1 = false;
-            }
-        };
-        // entries: enter row Dr-1, delta(Dr-1, T) = -[row Dr-1 counted at T]
-        auto entry = [&](int node, int v0, int j, int T) {
-            const int Dr = s - j * rc;
-            const uint16_t e = U[v0 + Dr - 1];
-            const int col = e & kIdx;
-            const int ch = node * nch + j;
-            bT[ch] = T;
-            bD[ch] = -((e & kLoFlag) ? (col >= T) : (col < T));
-        };
-        constexpr int kWaves = kThreads / 64;
-        const int nodes = K / s;
-        // dir 0: row lines from the columns' entries (CI); dir 1 (nodes of
-        // kColLineMinS rows or more): column lines from the rows' entries
-        // (U), the column line c = i rc being boundary nch - i, T = rho + 1
-        for (int dir = 0; dir < (s >= kColLineMinS ? 2 : 1); ++dir) {
-            const UT *E = dir ? U : CI;
-            auto store = [&](int node, int v0, int j, int T) {
-                if (dir) cT[node * nch + j] = T;
-                else entry(node, v0, j, T);
-            };
-            if (dir) __syncthreads();   // the row direction's counters are read
-            if (nodes >= kWaves || K < 64 * kWaves) {
-                // one wave per node: Y_j from the node's counts, then one sweep
-                for (int node = wave; node < nodes; node += kWaves) {
-                    const int v0 = node * s;
-                    int Y0, Y1, c0_, c1_;
-                    range_counts(E, v0, 0, s, Y0, Y1, c0_, c1_);
-                    int T0 = 0, T1 = 0;
-                    find_T(E, v0, 0, s, Y0, Y1, 0, 0, j0 >= 1 && j0 < nch && Y0 > 0, j1 < nch && Y1 > 0, T0, T1);
-                    if (j0 >= 1 && j0 < nch) store(node, v0, j0, T0);
-                    if (j1 < nch) store(node, v0, j1, T1);
-                }
-            } else {
-                // W = kWaves / nodes waves per node, each on s / W consecutive
-                // entries: every wave counts its segment, the segments' counts
-                // give Y_j and each segment's starting Z_j, and only the wave in
-                // whose segment Z_j reaches Y_j sweeps for T_j.
-                const int W = kWaves / nodes, node = wave / W, seg = wave % W, seg_len = s / W;
-                const int v0 = node * s, cb = seg * seg_len;
-                int lp0, lp1, cnt0, cnt1;
-                range_counts(E, v0, cb, cb + seg_len, lp0, lp1, cnt0, cnt1);
-                hlo[j0] = cnt0;
-                hlo[j1] = cnt1;
-                hhi[j0] = lp0;
-                hhi[j1] = lp1;
-                __syncthreads();
-                int Y0 = 0, Y1 = 0, Zs0 = 0, Zs1 = 0;
-                for (int w2 = 0; w2 < W; ++w2) {
-                    const int *other = hist + (node * W + w2) * 2 * kMaxChunks;
-                    Y0 += other[kMaxChunks + j0];
-                    Y1 += other[kMaxChunks + j1];
-                    if (w2 < seg) {
-                        Zs0 += other[j0];
-                        Zs1 += other[j1];
-                    }
-                }
-                __syncthreads();   // every wave has read the counts before they are reused
-                const bool mine0 = j0 >= 1 && j0 < nch && Y0 > 0 && Zs0 < Y0 && Y0 <= Zs0 + cnt0;
-                const bool mine1 = j1 < nch && Y1 > 0 && Zs1 < Y1 && Y1 <= Zs1 + cnt1;
-                int T0 = 0, T1 = 0;
-                find_T(E, v0, cb, cb + seg_len, Y0, Y1, Zs0, Zs1, mine0, mine1, T0, T1);
-                if (j0 >= 1 && j0 < nch && (mine0 || (Y0 == 0 && seg == 0))) store(node, v0, j0, T0);
-                if (j1 < nch && (mine1 || (Y1 == 0 && seg == 0))) store(node, v0, j1, T1);
-            }
+    for (int t = wave; t < 2 * blocks; t += kWaves) {
+        const int dir = t >= blocks, g = dir ? t - blocks : t;
+        const uint32_t e = (dir ? U : CI)[g * 64 + lane];
+        const unsigned long long los = __ballot((e & kLoFlag) != 0);
+        const int bk = (s - 1 - (int)(e & kIdx)) >> 6;
+        // lane j: the entries with bucket < j, from the buckets' bit planes
+        unsigned long long lt_j = 0, eq = ~0ull;
+        for (int p = nb >> 1; p; p >>= 1) {
+            const unsigned long long plane = __ballot((bk & p) != 0), mine = (lane & p) ? ~0ull : 0ull;
+            lt_j |= eq & ~plane & mine;
+            eq &= ~(plane ^ mine);
         }
+        if (lane < nb) B.cnt[dir][g][lane] = (uint8_t)(__popcll(los & lt_j) + __popcll(~los & ~lt_j));
+        if (lane == 0) B.lo[dir][g] = (uint16_t)__popcll(los);
     }
     __syncthreads();
-    // The walk (the reference's ant passage, :123-189) with the four entries
-    // it reads kept in registers: cl = CI[dc-1], cc = CI[dc], ud = U[dr],
-    // ur = U[dr-1].  A step right only needs the new CI[dc] and a step down
-    // only the new U[dr-1], so every step is one LDS read from a selected
-    // address, and the step is written with selects so that no lane of the
-    // wave branches on the direction.
-    // counted(e, r) = lo ? idx >= r : idx < r for an entry e = lo << 15 | idx:
-    // bit 15 of e - r, for idx in [0, 32768) and r in [0, 32768].
-    auto counted = [](uint32_t e, int r) { return (int)(((e - (uint32_t)r) >> 15) & 1u); };
-    // Pieces: chunk j (q = j < nch) starts at its row line; in nodes of
-    // kColLineMinS rows or more the walks are also cut at the column lines
-    // c = i rc (q = nch - 1 + i), so every piece stays in one rc x rc box
-    // and takes at most 2 rc + 1 steps, whatever the permutations look like
-    // (a strip permutation's long straight runs would otherwise fall to a
-    // few chunks).  Smaller nodes walk whole row chunks.
-    const bool boxes = s >= kColLineMinS && nch > 1;
-    const int per_node = boxes ? 2 * nch - 1 : nch, pieces = (K / s) * per_node;
-    for (int pc = threadIdx.x; pc < pieces; pc += kThreads) {
-        const int node = pc / per_node, q = pc % per_node, v0 = node * s;
-        int dr, dc, delta, r_lo, c_hi;
-        if (q < nch) {
-            const int j = q, r_hi = s - j * rc;
-            r_lo = r_hi - rc;
-            dr = r_hi - 1;
-            if (j == 0) {
-                // T(s) = 0, delta(s, 0) = 0; entering row s-1 subtracts it when it is lo
-                dc = 0;
-                delta = (U[v0 + s - 1] & kLoFlag) ? -1 : 0;
-            } else {
-                dc = min(max(bT[node * nch + j], 0), s);
-                delta = bD[node * nch + j];
-            }
-            const int cb = dc == 0 ? 0 : (dc - 1) >> rc_log;
-            c_hi = !boxes || cb >= nch - 1 ? s + 1 : (cb + 1) * rc + 1;
+    // lines, up to kLineBatch per wave at once so that their LDS reads overlap
+    constexpr int kLineBatch = 2 * kMaxLeafLines / kWaves;
+    int lY[kLineBatch], lc[kLineBatch];
+    uint32_t le[kLineBatch];
+#pragma unroll
+    for (int i = 0; i < kLineBatch; ++i) {
+        const int t = wave + i * kWaves, dir = t >= blocks, q = dir ? t - blocks : t, j = q & (nb - 1), b0 = q - j;
+        const bool on = t < 2 * blocks;
+        // Y_j: the lo entries of the other array's last j blocks (their idx is
+        // the position there)
+        lY[i] = on && lane >= nb - j && lane < nb ? B.lo[dir ^ 1][b0 + lane] : 0;
+        lc[i] = on && lane < nb ? B.cnt[dir][b0 + lane][j] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < kLineBatch; ++i) {
+        const int t = wave + i * kWaves, dir = t >= blocks, q = dir ? t - blocks : t;
+        const int Y = __builtin_amdgcn_readlane(wave_incl_scan(lY[i]), 63), incl = wave_incl_scan(lc[i]);
+        const unsigned long long reach = __ballot(lane < nb && incl >= Y);
+        const int g = reach ? __ffsll((long long)reach) - 1 : 0;
+        lY[i] = reach ? Y - __builtin_amdgcn_readlane(incl - lc[i], g) : 0;   // still needed in block g
+        lc[i] = g;
+        le[i] = t < 2 * blocks ? (dir ? U : CI)[(q & ~(nb - 1)) * 64 + g * 64 + lane] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < kLineBatch; ++i) {
+        const int t = wave + i * kWaves, dir = t >= blocks, q = dir ? t - blocks : t, j = q & (nb - 1);
+        const int bk = (s - 1 - (int)(le[i] & kIdx)) >> 6;
+        const bool z = (le[i] & kLoFlag) ? bk < j : bk >= j;
+        const unsigned long long zm = __ballot(z);
+        const unsigned long long hit = __ballot(z && (int)__popcll(zm & lt) == lY[i] - 1);
+        if (lane == 0 && t < 2 * blocks && j) B.T[dir][q] = (uint16_t)(hit ? lc[i] * 64 + __ffsll((long long)hit) : 0);
+    }
+    __syncthreads();
+    // boxes: piece q < nb of a node starts at row line j = q (q = 0: at T(s) =
+    // 0), q >= nb at column line i = q - nb + 1
+    const int per_node = 2 * nb - 1;
+    for (int t = wave; t < nodes * per_node; t += kWaves) {
+        const int node = t / per_node, q = t - node * per_node, v0 = node * s;
+        int r_lo, cs, ce, rho;
+        if (q < nb) {
+            r_lo = s - (q + 1) * 64;
+            rho = r_lo + 63;
+            cs = q == 0 ? 0 : min((int)B.T[0][node * nb + q], s);
+            ce = cs == 0 ? 64 : (((cs - 1) >> 6) + 1) << 6;
         } else {
-            // stepping right over column line c = i rc at row rho: delta = -1 + [CI(c) counted at rho]
-            const int i = q - nch + 1;
-            const int Tc = min(max(cT[node * nch + nch - i], 0), s);
+            const int i = q - nb + 1, Tc = min((int)B.T[1][node * nb + nb - i], s);
             if (Tc == 0) continue;   // the ant never reaches this column line
-            dr = Tc - 1;
-            dc = i * rc + 1;
-            delta = -1 + counted(CI[v0 + i * rc], dr);
-            r_lo = s - (((s - 1 - dr) >> rc_log) + 1) * rc;
-            c_hi = i == nch - 1 ? s + 1 : (i + 1) * rc + 1;
+            rho = Tc - 1;
+            r_lo = rho & ~63;
+            cs = i * 64;
+            ce = cs + 64;
         }
-        // entries outside the node (dc = 0 or s, dr = 0) are read clamped and never used
-        uint32_t cl = CI[v0 + max(dc - 1, 0)], cc = CI[v0 + min(dc, s - 1)];
-        uint32_t ud = U[v0 + dr], ur = U[v0 + max(dr - 1, 0)];
-        while (dr >= r_lo && dc < c_hi) {
-            const int d_left = delta - counted(cl, dr);
-            const int d_down = delta + counted(ud, dc);
-            if (dc > 0 && d_left < 0 && d_down > 0) Rn[v0 + dr] = dc - 1;
-            // delta(dr, s) >= 0 always; the dc < s test only bounds the walk
-            const bool right = delta < 0 && dc < s;
-            const int d_right = counted(cc, dr), d_up = dr > 0 ? counted(ur, dc) : 0;
-            delta = right ? delta + d_right : delta - d_up;
-            dc += right ? 1 : 0;
-            dr -= right ? 0 : 1;
-            cl = right ? cc : cl;
-            ud = right ? ud : ur;
-            const uint32_t nx = right ? CI[v0 + min(dc, s - 1)] : U[v0 + max(dr - 1, 0)];
-            cc = right ? nx : cc;
-            ur = right ? ur : nx;
-        }
+        if (r_lo) ce = min(ce, (int)B.T[0][node * nb + nb - (r_lo >> 6)]);   // T(r_lo): open rows stay below it
+        const uint32_t u = U[v0 + r_lo + lane];
+        auto entry = [&](int c) { return CI[v0 + c]; };
+        const int c = q < nb ? box_rows<15, false>(u, entry, r_lo, rho, cs, ce, lane)
+                             : box_rows<15, true>(u, entry, r_lo, rho, cs, ce, lane);
+        if (c >= 0) Rn[v0 + r_lo + lane] = (uint16_t)c;
     }
     __syncthreads();
 }
@@ -439,7 +422,7 @@ __device__ __forceinline__ void split_depth_pq(const uint16_t *keyP, uint16_t *k
 // big core reads its slice of the big core's keys).
 template <bool QKEY>
 __device__ __forceinline__ void core_lds_body(const int32_t *P, const int32_t *Q, int32_t *Rout, int k, int L,
-                                              uint16_t *lds, int32_t *bT, int32_t *bD, int32_t *cT, int *hist)
+                                              uint16_t *lds, LeafLines &B)
 {
     const int K = 1 << L, mask = K - 1;
     uint16_t *keyP = lds, *keyP2 = lds + K;                       // top-down
@@ -447,8 +430,8 @@ __device__ __forceinline__ void core_lds_body(const int32_t *P, const int32_t *Q
     uint16_t *U = lds, *CI = lds + K;                             // bottom-up (reuses the key space)
     uint16_t *R = lds + 2 * (size_t)K, *Rn = lds + 3 * (size_t)K;
     int32_t *gcP = (int32_t *)(lds + 4 * (size_t)K), *gcQ = gcP + (K / 64 + 1);
-    uint16_t *parP = lds + 4 * (size_t)K + 4 * ((size_t)K / 64 + 1);   // L * K
-    uint16_t *parQ = parP + (size_t)L * K;                              // L * K
+    uint16_t *parP = lds + 4 * (size_t)K + 4 * ((size_t)K / 64 + 1);   // (L - 6) * K
+    uint16_t *parQ = parP + (size_t)(L - 6) * K;                        // (L - 6) * K
 
     // P ordered by row (key = shared column), Q ordered by column (key = shared row)
     for (int x = threadIdx.x; x < K; x += kThreads) keyP[x] = (uint16_t)(x < k ? (P[x] & mask) : x);
@@ -461,16 +444,32 @@ __device__ __forceinline__ void core_lds_body(const int32_t *P, const int32_t *Q
             if ((uint32_t)Q[r] < (uint32_t)k) keyQ[Q[r]] = (uint16_t)r;
     }
     __syncthreads();
-    for (int d = 0; d < L; ++d) {
+    const int D = L - 6;   // depths above the 64-point nodes
+    for (int d = 0; d < D; ++d) {
         split_depth_pq(keyP, keyP2, parP + (size_t)d * K, keyQ, keyQ2, parQ + (size_t)d * K, gcP, gcQ, K, K >> d,
                        L - d - 1);
         uint16_t *t = keyP; keyP = keyP2; keyP2 = t;
         t = keyQ; keyQ = keyQ2; keyQ2 = t;
     }
-    for (int x = threadIdx.x; x < K; x += kThreads) R[x] = 0;  // depth L: 1x1 nodes
+    // the 64-point nodes, a wave each; R takes the place of Q's spare keys
+    // only once every wave has read its keys
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int kWaves = kThreads / 64, kPerWave = kLdsCoreK / 64 / kWaves;
+    int prod[kPerWave];
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+        const int node = wave + i * kWaves;
+        prod[i] = node < K / 64 ? wave_product64(keyP[node * 64 + lane] & 63, keyQ[node * 64 + lane] & 63, lane) : 0;
+    }
     __syncthreads();
-    for (int d = L - 1; d >= 0; --d) {
-        bottom_up_depth(U, CI, R, Rn, parP + (size_t)d * K, parQ + (size_t)d * K, K, K >> d, bT, bD, cT, hist);
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+        const int node = wave + i * kWaves;
+        if (node < K / 64) R[node * 64 + lane] = (uint16_t)prod[i];
+    }
+    __syncthreads();
+    for (int d = D - 1; d >= 0; --d) {
+        bottom_up_depth(U, CI, R, Rn, parP + (size_t)d * K, parQ + (size_t)d * K, K, K >> d, B);
         uint16_t *tmp = R; R = Rn; Rn = tmp;
     }
     for (int x = threadIdx.x; x < k; x += kThreads) Rout[x] = R[x];
@@ -480,22 +479,21 @@ __global__ __launch_bounds__(kThreads) void braid_core_lds_kernel(CoreBatch batc
 {
     const BraidCoreDesc D = batch.d[blockIdx.x];
     extern __shared__ uint16_t lds[];
-    __shared__ int32_t bT[kLdsCoreK / kChunkRows], bD[kLdsCoreK / kChunkRows], cT[kLdsCoreK / kChunkRows];
-    __shared__ int hist[(kThreads / 64) * 2 * kMaxChunks];
-    core_lds_body<false>(D.P, D.Q, D.R, D.k, D.L, lds, bT, bD, cT, hist);
+    __shared__ LeafLines lines;
+    core_lds_body<false>(D.P, D.Q, D.R, D.k, D.L, lds, lines);
 }
 
 // ---------------------------------------------------------------- big cores
 // Cores above kLdsCoreK run the same recursion spread over the whole GPU
-// (the one-workgroup core walks its top depths in the same box pieces):
+// (the one-workgroup core finishes its top depths in the same boxes):
 //  * the top d0 = L - L0 depths of the top-down split are device-wide
 //    stable partitions (count, scan, scatter per depth);
 //  * the 2^d0 nodes of depth d0 are independent sticky products of 2^L0
 //    points each, one workgroup per node (core_lds_body on their keys);
 //  * bottom-up, each top depth lifts the children's products into node
 //    coordinates (inverse_mapping, src/braid_multiplication.hpp:191-202)
-//    and runs the ant passage (:123-189) cut into pieces that a lane each
-//    walks in LDS.  The ant leaves row r at T(r) = min{c : delta(r, c) >= 0}
+//    and runs the ant passage (:123-189) cut into boxes that a wave each
+//    finishes.  The ant leaves row r at T(r) = min{c : delta(r, c) >= 0}
 //    (delta non-decreasing in r and c), so its path is fixed by where it
 //    crosses a grid of lines every g rows and every g columns of a node:
 //      - row line Dr (= s - j g): enters row Dr-1 at column T(Dr), with
@@ -512,31 +510,15 @@ __global__ __launch_bounds__(kThreads) void braid_core_lds_kernel(CoreBatch batc
 //    (T_j = rho + 1).  Block histograms (big_hist_kernel), a search over
 //    the blocks per boundary and a sweep of the one block where the count
 //    crosses (big_sweep_kernel) find every T_j.  A piece starts at a
-//    crossing and ends at the next one, so it stays inside one g x g box and
-//    takes at most 2g + 1 steps (big_walk_kernel).
+//    crossing and ends at the next one, so it stays inside one g x g box,
+//    whose rows' T follow from its columns' entries (big_box_kernel).
 // Entries of U (row -> column) and CI (column -> row) are node-local
 // indices with the lo flag in bit 31.
 constexpr int kBigBatch = 32;          // products per big-core launch
 constexpr int kSplitTile = 2048;       // elements per block of a device-wide partition
 constexpr int kMaxLines = 8192;        // grid lines per node and direction
-// Box side g of a node's grid: kBoxGSmall for nodes up to 2^kBoxSmallMaxL
-// points, kBoxG above (nodes above kMaxLines * g take g = s / kMaxLines).
-// Smaller boxes halve the walks and double the lines whose crossings the
-// sweeps find; the sweeps are cheap for small nodes.  Same box: the Zipf
-// pair's merges (nodes up to 2^14) 1.60 ms with boxes of 32 against 1.78
-// with 64; a k = 2^20 product 1.60 ms with 32 everywhere against 1.47.
-#ifndef LCS_BIG_BOX_G
-#define LCS_BIG_BOX_G 64
-#endif
-#ifndef LCS_BIG_BOX_G_SMALL
-#define LCS_BIG_BOX_G_SMALL 32
-#endif
-#ifndef LCS_BIG_BOX_SMALL_MAX_L
-#define LCS_BIG_BOX_SMALL_MAX_L 14
-#endif
-constexpr int kBoxG = LCS_BIG_BOX_G, kBoxGSmall = LCS_BIG_BOX_G_SMALL, kBoxSmallMaxL = LCS_BIG_BOX_SMALL_MAX_L;
-static_assert(kBoxG >= 16 && kBoxG <= 512 && (kBoxG & (kBoxG - 1)) == 0, "box side");
-static_assert(kBoxGSmall >= 16 && kBoxGSmall <= 512 && (kBoxGSmall & (kBoxGSmall - 1)) == 0, "box side");
+// Box side of a node's grid: one wave per box takes 64 rows and 64 columns
+// at a time, so 64 up to nodes of kMaxLines * 64 points, s / kMaxLines above.
 constexpr uint32_t kLo31 = 0x80000000u;
 
 struct BigCore {
@@ -575,8 +557,7 @@ __host__ __device__ inline BigDepth big_depth(int L, int d)
 {
     BigDepth D;
     D.s = 1 << (L - d);
-    const int g = L - d <= kBoxSmallMaxL ? kBoxGSmall : kBoxG;
-    D.nb = D.s / g < kMaxLines ? D.s / g : kMaxLines;
+    D.nb = D.s / kBox < kMaxLines ? D.s / kBox : kMaxLines;
     D.glog = __builtin_ctz((unsigned)(D.s / D.nb));
     D.w = 1 << big_w_log(L - d);
     if (D.w > D.s) D.w = D.s;
@@ -629,8 +610,6 @@ struct BigBatch {
     BigLayout Y;
     BigDepth D[kMaxCoreL];
 };
-
-__device__ __forceinline__ uint32_t counted31(uint32_t e, int r) { return ((e - (uint32_t)r) >> 31) & 1u; }
 
 __global__ void big_init_kernel(BigBatch B)
 {
@@ -767,10 +746,9 @@ __global__ __launch_bounds__(kThreads) void big_leaf_kernel(BigBatch B)
     const int32_t *keyP = C.ws + ((d0 & 1) ? Y.keyP2 : Y.keyP) + v0;
     const int32_t *keyQ = C.ws + ((d0 & 1) ? Y.keyQ2 : Y.keyQ) + v0;
     extern __shared__ uint16_t lds[];
-    __shared__ int32_t bT[kLdsCoreK / kChunkRows], bD[kLdsCoreK / kChunkRows], cT[kLdsCoreK / kChunkRows];
-    __shared__ int hist[(kThreads / 64) * 2 * kMaxChunks];
+    __shared__ LeafLines lines;
     // depth d0 of the big core's own recursion: the products go to R
-    core_lds_body<true>(keyP, keyQ, C.ws + Y.R + v0, s0, B.L0, lds, bT, bD, cT, hist);
+    core_lds_body<true>(keyP, keyQ, C.ws + Y.R + v0, s0, B.L0, lds, lines);
 }
 
 // lift the children's products into node coordinates (node size s).  The
@@ -978,93 +956,79 @@ __global__ __launch_bounds__(64 * kSweepWaves) void big_sweep_kernel(BigBatch B,
     if (lane == 0 && pos) *T = seg * D.w + pos;
 }
 
-// A box entry relative to the box: idx clamped to [base, top] minus base,
-// the lo flag in bit 15.  For r in (base, top], counted31(e, r) of the
-// absolute entry equals counted16 of this one at r - base.
-__device__ __forceinline__ uint16_t box_entry(uint32_t e, int base, int top)
-{
-    const int idx = (int)(e & ~kLo31);
-    return (uint16_t)(((e & kLo31) ? 0x8000u : 0u) | (uint32_t)(min(max(idx, base), top) - base));
-}
-__device__ __forceinline__ int counted16(uint32_t e, int r) { return (int)(((e - (uint32_t)r) >> 15) & 1u); }
-
-// One lane per piece of the ant's path.  Piece q < nb of a node starts at
-// row line j = q (q = 0: the start of the passage at (s-1, 0)), q >= nb at
-// column line i = q - nb + 1; it stays in one g x g box.  Each lane stages
-// its box -- rows r_lo-1 .. r_hi-1 of U and columns c_lo-1 .. c_hi-1 of CI,
-// clamped into the node -- in LDS as 16-bit entries relative to the box, then
-// walks it with the reference's incremental updates, placing the good
-// points.  In box coordinates R = dr - r_lo + 1 (1 .. g while in the box)
-// and X = dc - c_lo + 1 (1 .. nc - 1 before the exit line): U(dr) = bu[R],
-// U(dr-1) = bu[R-1], CI(dc) = bc[X], CI(dc-1) = bc[X-1].
-constexpr int kMaxBoxG = 512;   // g at the largest node (2^22 / kMaxLines)
-constexpr size_t walk_lds_bytes(int g) { return (size_t)64 * (2 * g + 3) * sizeof(uint16_t); }
-__global__ __launch_bounds__(64) void big_walk_kernel(BigBatch B, int d, int flip)
+// One wave per piece of the ant's path.  Piece q < nb of a node starts at
+// row line j = q (q = 0: the start of the passage at T(s) = 0), q >= nb at
+// column line i = q - nb + 1; it stays in one g x g box (box_rows above says
+// how its rows find T).  With g above 64 the rows go 64 at a time from the
+// line upwards, carrying the rows counted so far, and the columns 64 at a
+// time.  About 200 VALU and a few coalesced loads per wave; walking the boxes
+// one lane each took 21 us per depth of a k = 2^16 product, this 3.  Whole
+// products (random, kernel time, before and after boxes and wave_product64
+// took the walks' place): k = 2^11 142 and 100 us, 2^16 344 and 215, 2^20
+// 1419 and 1178.
+constexpr int kBoxWaves = 4;   // pieces per workgroup
+__global__ __launch_bounds__(64 * kBoxWaves) void big_box_kernel(BigBatch B, int d, int flip)
 {
     const BigCore &C = B.c[blockIdx.z];
     const BigLayout &Y = B.Y;
     const BigDepth &D = B.D[d];
     const int K = 1 << B.L, s = D.s, nodes = K / s, g = 1 << D.glog, nb = D.nb;
-    const int pieces = 2 * nb - 1;
-    const int t = blockIdx.x * 64 + threadIdx.x;
+    const int pieces = 2 * nb - 1, lane = threadIdx.x & 63;
+    const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * kBoxWaves + (threadIdx.x >> 6));
     if (t >= nodes * pieces) return;
-    const int node = t / pieces, q = t % pieces;
+    const int node = t / pieces, q = t - node * pieces;
     const size_t v0 = (size_t)node * s;
     const uint32_t *U = (const uint32_t *)(C.ws + Y.U) + v0, *CI = (const uint32_t *)(C.ws + Y.CI) + v0;
     int32_t *Rn = C.ws + (flip ? Y.R : Y.Rn) + v0;
-    const int32_t *Trow = C.ws + Y.T + (size_t)node * nb;
-    const int32_t *Tcol = C.ws + Y.T + (size_t)nodes * nb + (size_t)node * nb;
     // T lies in [0, s]; the clamps only keep every access inside the node
     // after an aborted comb fed undefined input
-    int dr, dc, r_lo, cb;
-    if (q < nb) {
-        const int Dr = s - q * g;
-        dc = q == 0 ? 0 : min(max(Trow[q], 0), s);
-        dr = Dr - 1;
-        r_lo = Dr - g;
-        cb = dc == 0 ? 0 : (dc - 1) >> D.glog;
+    int r_lo, rho, cs, ce;
+    const bool col = q >= nb;
+    if (!col) {
+        r_lo = s - (q + 1) * g;
+        rho = r_lo + g - 1;
+        cs = q == 0 ? 0 : min(max(C.ws[Y.T + (size_t)node * nb + q], 0), s);
+        ce = cs == 0 ? g : (((cs - 1) >> D.glog) + 1) << D.glog;
     } else {
         const int i = q - nb + 1;
-        const int Tc = min(max(Tcol[nb - i], 0), s);
+        const int Tc = min(max(C.ws[Y.T + (size_t)nodes * nb + (size_t)node * nb + nb - i], 0), s);
         if (Tc == 0) return;   // the ant never reaches this column line
-        dr = Tc - 1;
-        dc = i * g + 1;
-        r_lo = s - (((s - 1 - dr) >> D.glog) + 1) * g;
-        cb = i;
+        rho = Tc - 1;
+        r_lo = rho & ~(g - 1);
+        cs = i * g;
+        ce = cs + g;
     }
-    const int c_lo = cb ? cb * g + 1 : 0, c_hi = cb == nb - 1 ? s + 1 : (cb + 1) * g + 1;
-    const int nc = c_hi - c_lo + 1;   // at most g + 2
-    extern __shared__ uint16_t walk_lds[];
-    uint16_t *bu = walk_lds + (size_t)threadIdx.x * (2 * g + 3), *bc = bu + (g + 1);
-    // U entries hold columns, compared with dc in [c_lo, c_hi - 1]; CI
-    // entries hold rows, compared with dr in [r_lo, r_lo + g - 1]
-#pragma unroll 32
-    for (int i = 0; i <= g; ++i) bu[i] = box_entry(U[min(max(r_lo - 1 + i, 0), s - 1)], c_lo - 1, c_hi);
-#pragma unroll 32
-    for (int i = 0; i < nc; ++i) bc[i] = box_entry(CI[min(max(c_lo - 1 + i, 0), s - 1)], r_lo - 1, r_lo + g);
-    // entering row Dr-1 at T: delta = -[U(Dr-1) counted at T]; stepping right
-    // over column line c = i g at row rho: delta = -1 + [CI(c) counted at rho]
-    int R = dr - r_lo + 1, X = dc - c_lo + 1;
-    const int Xs = s - c_lo + 1;   // X < Xs <=> dc < s
-    int delta = q < nb ? -counted16(bu[R], X) : -1 + counted16(bc[0], R);
-    uint32_t cl = bc[X - 1], cc = bc[X], ud = bu[R], ur = bu[R - 1];
-    // the lanes of a wave take different directions, so each step is written
-    // with selects and reads one LDS entry from a selected index: the new
-    // CI(dc) after a step right, U(dr-1) after a step down
-    while (R >= 1 && X < nc) {
-        const int d_left = delta - counted16(cl, R);
-        const int d_down = delta + counted16(ud, X);
-        if (X + c_lo > 1 && d_left < 0 && d_down > 0) Rn[R + r_lo - 1] = X + c_lo - 2;
-        const bool right = delta < 0 && X < Xs;
-        const int d_right = counted16(cc, R), d_up = R + r_lo > 1 ? counted16(ur, X) : 0;
-        delta = right ? delta + d_right : delta - d_up;
-        X += right ? 1 : 0;
-        R -= right ? 0 : 1;
-        cl = right ? cc : cl;
-        ud = right ? ud : ur;
-        const uint32_t nx = bu[right ? g + 1 + min(X, nc - 1) : max(R - 1, 0)];
-        cc = right ? nx : cc;
-        ur = right ? ur : nx;
+    auto entry = [&](int c) { return CI[c]; };
+    if (g == kBox) {
+        if (r_lo) ce = min(ce, min(max(C.ws[Y.T + (size_t)node * nb + nb - (r_lo >> D.glog)], 0), s));
+        const uint32_t u = U[r_lo + lane];
+        const int c = col ? box_rows<31, true>(u, entry, r_lo, rho, cs, ce, lane)
+                          : box_rows<31, false>(u, entry, r_lo, rho, cs, ce, lane);
+        if (c >= 0) Rn[r_lo + lane] = c;
+        return;
+    }
+    int below = col ? 1 : 0;   // -delta(r, cs) just below the rows in hand
+    for (int rb = (rho & ~63); rb >= r_lo; rb -= 64) {
+        const int r = rb + lane;
+        const uint32_t u = U[r];
+        const bool uc = counted<31>(u, cs);
+        const unsigned long long m = __ballot(col ? uc && r < rho : uc);
+        int need = below + (int)__popcll(m >> lane);
+        below += (int)__popcll(m);
+        int T = need ? -1 : cs;
+        for (int c0 = cs; c0 < ce; c0 += 64) {
+            uint32_t q[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int c = c0 + 16 * i + (lane & 15);
+                q[i] = counted_row16(c < ce ? entry(c) : ~kLo31, (uint32_t)r, lane);
+            }
+            const uint32_t lo = q[0] | q[1] << 16, hi = q[2] | q[3] << 16;
+            const int cnt = __popc(lo) + __popc(hi);
+            if (T < 0 && need <= cnt) T = c0 + 1 + select64(lo, hi, need);
+            need -= cnt;
+        }
+        if ((!col || r <= rho) && T > 0 && counted<31>(u, T)) Rn[r] = T - 1;
     }
 }
 
@@ -1289,8 +1253,8 @@ static int launch_big(const BigBatch &B, int cnt, hipStream_t stream)
         hipLaunchKernelGGL(big_sweep_kernel, dim3((unsigned)((lines + kSweepWaves - 1) / kSweepWaves), 2, (unsigned)cnt),
                            dim3(64 * kSweepWaves), 0, stream,
                            B, d);
-        hipLaunchKernelGGL(big_walk_kernel, dim3((unsigned)((pieces + 63) / 64), 1, (unsigned)cnt), dim3(64),
-                           walk_lds_bytes(1 << D.glog), stream, B, d, flip);
+        hipLaunchKernelGGL(big_box_kernel, dim3((unsigned)((pieces + kBoxWaves - 1) / kBoxWaves), 1, (unsigned)cnt),
+                           dim3(64 * kBoxWaves), 0, stream, B, d, flip);
         flip ^= 1;
     }
     hipLaunchKernelGGL(big_out_kernel, lin, dim3(256), 0, stream, B, flip);
@@ -1307,9 +1271,7 @@ int lcsb_init(void)
         if (hipFuncSetAttribute((const void *)braid_core_lds_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds_core_bytes(kLdsCoreL)) != hipSuccess ||
             hipFuncSetAttribute((const void *)big_leaf_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds_core_bytes(kLdsCoreL)) != hipSuccess ||
-            hipFuncSetAttribute((const void *)big_walk_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)walk_lds_bytes(kMaxBoxG)) != hipSuccess)
+                                (int)lds_core_bytes(kLdsCoreL)) != hipSuccess)
             rc = -5;
     });
     return rc;
