@@ -194,7 +194,8 @@ __device__ __forceinline__ int wave_product64(int kp, int kq, int lane)
 // rho are, and delta(rho, cs) = -1.  -delta(r, cs) adds the rows from r down
 // to the line that count at cs; T(r) is the position after that many counted
 // columns.  entry(c) reads column c's entry, c < ce; the caller may lower ce
-// to T(r_lo), which no open row exceeds.  Returns the row's new column or -1.
+// to T(r_lo), which no open row exceeds.  Returns the row's column in the
+// product, or -1 for a row of another piece.
 template <int F, bool COL, typename Entry>
 __device__ __forceinline__ int box_rows(uint32_t u, Entry entry, int r_lo, int rho, int cs, int ce, int lane)
 {
@@ -213,7 +214,8 @@ __device__ __forceinline__ int box_rows(uint32_t u, Entry entry, int r_lo, int r
     const uint32_t lo = q[0] | q[1] << 16, hi = q[2] | q[3] << 16;
     const bool open = (!COL || r <= rho) && need <= __popc(lo) + __popc(hi);
     const int T = need ? cs + 1 + select64(lo, hi, need) : cs;
-    return open && T > 0 && counted<F>(u, T) ? T - 1 : -1;
+    const int c = T > 0 && counted<F>(u, T) ? T - 1 : (int)(u & ~(1u << F));
+    return open ? c : -1;
 }
 
 // One bottom-up depth (node size s >= 128) of a core in LDS: lift the
@@ -414,15 +416,53 @@ __device__ __forceinline__ void split_depth_pq(const uint16_t *keyP, uint16_t *k
     __syncthreads();
 }
 
-// The sticky product with keys, both products, the parents of every depth
-// and the chunk entries in LDS for cores up to K = kLdsCoreK, one workgroup
-// per core; the dynamic LDS is laid out as lds_core_bytes(L) says.  P holds
-// row -> shared column; Q holds shared row -> column, or (QKEY) column ->
-// shared row, the keys themselves.  Values are read modulo K (a leaf of a
-// big core reads its slice of the big core's keys).
-template <bool QKEY>
-__device__ __forceinline__ void core_lds_body(const int32_t *P, const int32_t *Q, int32_t *Rout, int k, int L,
-                                              uint16_t *lds, LeafLines &B)
+// One product p (.) q glued on k strands, as every kernel of the sequence
+// takes it (by value in the launch arguments).  The workspace holds q's
+// inverse, the rows of p and the columns of q that the core's strands stand
+// for, the block counts of the two slices, and the core's own words, which
+// begin with the keys: keyP[x] = shared strand of the core's row x, keyQ[x] =
+// shared strand of its column x.
+constexpr int kScanBlock = 256, kScanPer = 8, kScanTile = kScanBlock * kScanPer;
+constexpr int kMulBatch = 32;   // products per launch
+struct MulArgs {
+    const int32_t *p, *q;
+    int32_t *out, *ws;
+    int32_t p_size, q_size, k, row_glue, L, pad;
+    __host__ __device__ int32_t *q_c2r() const { return ws; }
+    __host__ __device__ int32_t *map_row() const { return ws + q_size; }
+    __host__ __device__ int32_t *map_col() const { return map_row() + k; }
+    __host__ __device__ int32_t blocks() const
+    {
+        return (p_size > q_size ? p_size : q_size) / kScanTile + 1;
+    }
+    __host__ __device__ int32_t *counts(int side) const { return map_col() + k + side * blocks(); }
+    __host__ __device__ int32_t *core() const { return counts(2); }
+    // row i of the core goes to column c: the product's point
+    // (braid_multiplication.hpp:353-401); the range tests only matter after an
+    // aborted comb fed undefined input
+    __device__ __forceinline__ void put(int i, int c) const
+    {
+        if (i >= k || (uint32_t)c >= (uint32_t)k) return;
+        const int row = map_row()[i], col = map_col()[c];
+        if ((uint32_t)row >= (uint32_t)p_size) return;
+        if (row_glue) out[q_size - k + row] = col;
+        else out[row] = col + p_size - k;
+    }
+};
+struct MulBatch {
+    MulArgs m[kMulBatch];
+};
+
+// The sticky product with keys, both products, the parents of the depths
+// above the 64-point nodes and the line tables in LDS for cores up to K =
+// kLdsCoreK, one workgroup per core; the dynamic LDS is laid out as
+// lds_core_bytes(L) says.  P holds row -> shared strand, Q column -> shared
+// strand, for the first k of K (the rest are fixed points); values are read
+// modulo K (a leaf of a big core reads its slice of the big core's keys).
+// done(x, c) receives row x's column.
+template <typename Done>
+__device__ __forceinline__ void core_lds_body(const int32_t *P, const int32_t *Q, int k, int L, uint16_t *lds,
+                                              LeafLines &B, Done done)
 {
     const int K = 1 << L, mask = K - 1;
     uint16_t *keyP = lds, *keyP2 = lds + K;                       // top-down
@@ -433,15 +473,10 @@ __device__ __forceinline__ void core_lds_body(const int32_t *P, const int32_t *Q
     uint16_t *parP = lds + 4 * (size_t)K + 4 * ((size_t)K / 64 + 1);   // (L - 6) * K
     uint16_t *parQ = parP + (size_t)(L - 6) * K;                        // (L - 6) * K
 
-    // P ordered by row (key = shared column), Q ordered by column (key = shared row)
-    for (int x = threadIdx.x; x < K; x += kThreads) keyP[x] = (uint16_t)(x < k ? (P[x] & mask) : x);
-    if (QKEY) {
-        for (int x = threadIdx.x; x < K; x += kThreads) keyQ[x] = (uint16_t)(Q[x] & mask);
-    } else {
-        for (int x = threadIdx.x; x < K; x += kThreads)
-            if (x >= k) keyQ[x] = (uint16_t)x;
-        for (int r = threadIdx.x; r < k; r += kThreads)
-            if ((uint32_t)Q[r] < (uint32_t)k) keyQ[Q[r]] = (uint16_t)r;
+    for (int x = threadIdx.x; x < K; x += kThreads) {
+        const int kp = x < k ? P[x] : x, kq = x < k ? Q[x] : x;
+        keyP[x] = (uint16_t)(kp & mask);
+        keyQ[x] = (uint16_t)(kq & mask);
     }
     __syncthreads();
     const int D = L - 6;   // depths above the 64-point nodes
@@ -472,15 +507,16 @@ __device__ __forceinline__ void core_lds_body(const int32_t *P, const int32_t *Q
         bottom_up_depth(U, CI, R, Rn, parP + (size_t)d * K, parQ + (size_t)d * K, K, K >> d, B);
         uint16_t *tmp = R; R = Rn; Rn = tmp;
     }
-    for (int x = threadIdx.x; x < k; x += kThreads) Rout[x] = R[x];
+    for (int x = threadIdx.x; x < K; x += kThreads) done(x, (int)R[x]);
 }
 
-__global__ __launch_bounds__(kThreads) void braid_core_lds_kernel(CoreBatch batch)
+__global__ __launch_bounds__(kThreads) void braid_core_lds_kernel(MulBatch B)
 {
-    const BraidCoreDesc D = batch.d[blockIdx.x];
+    const MulArgs &M = B.m[blockIdx.x];
     extern __shared__ uint16_t lds[];
     __shared__ LeafLines lines;
-    core_lds_body<false>(D.P, D.Q, D.R, D.k, D.L, lds, lines);
+    const int32_t *key = M.core();
+    core_lds_body(key, key + (1 << M.L), M.k, M.L, lds, lines, [&](int x, int c) { M.put(x, c); });
 }
 
 // ---------------------------------------------------------------- big cores
@@ -514,19 +550,12 @@ __global__ __launch_bounds__(kThreads) void braid_core_lds_kernel(CoreBatch batc
 //    whose rows' T follow from its columns' entries (big_box_kernel).
 // Entries of U (row -> column) and CI (column -> row) are node-local
 // indices with the lo flag in bit 31.
-constexpr int kBigBatch = 32;          // products per big-core launch
 constexpr int kSplitTile = 2048;       // elements per block of a device-wide partition
 constexpr int kMaxLines = 8192;        // grid lines per node and direction
 // Box side of a node's grid: one wave per box takes 64 rows and 64 columns
 // at a time, so 64 up to nodes of kMaxLines * 64 points, s / kMaxLines above.
 constexpr uint32_t kLo31 = 0x80000000u;
 
-struct BigCore {
-    const int32_t *P, *Q;   // k: row -> shared column, shared row -> column
-    int32_t *R;             // k: row -> column of the product
-    int32_t *ws;            // lcsb_big_ws_words(k, L0) words
-    int32_t k;
-};
 // grid of one top depth (node size s): lines every g = s / nb
 struct BigDepth {
     int32_t s, nb, glog, w, nsegs;   // w entries per histogram block, nsegs per node
@@ -565,9 +594,11 @@ __host__ __device__ inline BigDepth big_depth(int L, int d)
     return D;
 }
 
-// word offsets inside one product's workspace
+// word offsets inside one core's words; U and CI (64-bit pairs would not
+// coalesce with the row and column reads) alternate between two sets, as a
+// depth's boxes read one while they lift into the next depth's
 struct BigLayout {
-    size_t keyP, keyQ, keyP2, keyQ2, parP, parQ, R, Rn, U, CI, cnt, hist, T, total;
+    size_t keyP, keyQ, keyP2, keyQ2, parP, parQ, U[2], CI[2], cnt, hist, total;
 };
 
 __host__ __device__ inline BigLayout big_layout(int L, int L0)
@@ -582,49 +613,57 @@ __host__ __device__ inline BigLayout big_layout(int L, int L0)
     B.keyQ2 = o; o += K;
     B.parP = o; o += (size_t)d0 * K;
     B.parQ = o; o += (size_t)d0 * K;
-    B.R = o; o += K;
-    B.Rn = o; o += K;
-    B.U = o; o += K;
-    B.CI = o; o += K;
+    for (int i = 0; i < 2; ++i) {
+        B.U[i] = o; o += K;
+        B.CI[i] = o; o += K;
+    }
     B.cnt = o; o += 3 * 2 * (K / kSplitTile);   // tile counts of P and Q, three depths in rotation
-    size_t hist = 0, lines = 0;
+    size_t hist = 0;
     for (int d = 0; d < d0; ++d) {
         const BigDepth D = big_depth(L, d);
-        const size_t nodes = K / (size_t)D.s;
-        const size_t h = 2 * nodes * (size_t)D.nsegs * (size_t)(D.nb + 1);
+        const size_t h = 2 * (K / (size_t)D.s) * (size_t)D.nsegs * (size_t)(D.nb + 1);
         hist = h > hist ? h : hist;
-        lines = nodes * (size_t)D.nb > lines ? nodes * (size_t)D.nb : lines;
     }
     B.hist = o; o += hist;
-    B.T = o; o += 2 * lines;
     B.total = o;
     return B;
+}
+
+// Leaves of a core of 2^L points: one workgroup's LDS core each, of 2^10 points
+// up to 2^18 (the leaf is VALU-bound on its CU, and few leaves leave most CUs
+// idle), of 2^11 above (one device-wide depth less).  Kernel time with leaves
+// of 2^10 and 2^11: k = 2^12 106 and 127 us, 2^16 197 and 215, 2^18 355 and
+// 361, 2^20 1249 and 1178.
+constexpr int kBigMinL = 11;
+__host__ __device__ constexpr int big_leaf_L(int L) { return L > 18 ? 11 : 10; }
+static_assert(kLdsCoreL >= 11, "leaves fit the LDS core");
+// the tile counts' offset, for kernels without a BigBatch
+__host__ __device__ inline size_t big_layout_cnt(int L)
+{
+    return ((size_t)8 + 2 * (size_t)(L - big_leaf_L(L))) << L;
 }
 
 // The launch arguments of the big-core kernels: the products, and the
 // workspace layout and the grid of every top depth, computed once on the
 // host (per wave they were a loop of 64-bit divisions on the scalar unit).
 struct BigBatch {
-    BigCore c[kBigBatch];
+    MulArgs c[kMulBatch];
     int32_t L, L0;
     BigLayout Y;
     BigDepth D[kMaxCoreL];
 };
 
-__global__ void big_init_kernel(BigBatch B)
+// Row x of a node of depth d + 1 goes to its local column c (node at v0, size
+// h): its point in the parent, node size 2 h at depth d, written to that
+// depth's U (row -> column) and CI (column -> row).
+__device__ __forceinline__ void big_lift(const BigBatch &B, int32_t *w, int d, int v0, int h, int x, int c)
 {
-    const BigCore &C = B.c[blockIdx.z];
-    const BigLayout &Y = B.Y;
-    const int K = 1 << B.L, x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= K) return;
-    int32_t *keyP = C.ws + Y.keyP, *keyQ = C.ws + Y.keyQ;
-    keyP[x] = x < C.k ? C.P[x] : x;
-    if (x >= C.k) keyQ[x] = x;
-    else if ((uint32_t)C.Q[x] < (uint32_t)C.k) keyQ[C.Q[x]] = x;
-    // the tile counts of depths 1 and 2 are accumulated by the scatters
-    // before them and start at zero
-    const int ntiles = K / kSplitTile;
-    if (x < 2 * 2 * ntiles) C.ws[Y.cnt + 2 * (size_t)ntiles + x] = 0;
+    const size_t K = (size_t)1 << B.L;
+    const int p_pos = w[B.Y.parP + (size_t)d * K + x], q_pos = w[B.Y.parQ + (size_t)d * K + v0 + (c & (h - 1))];
+    const int p0 = p_pos & ~(2 * h - 1);
+    const uint32_t lo = (x & h) ? 0u : kLo31;
+    ((uint32_t *)w)[B.Y.U[d & 1] + p_pos] = (uint32_t)(q_pos - p0) | lo;
+    ((uint32_t *)w)[B.Y.CI[d & 1] + q_pos] = (uint32_t)(p_pos - p0) | lo;
 }
 
 // Depth-0 ones of the top bit per tile of kSplitTile keys (y = 0: P keys,
@@ -632,10 +671,10 @@ __global__ void big_init_kernel(BigBatch B)
 // accumulated by the scatter of the depth before.
 __global__ __launch_bounds__(256) void big_split_count_kernel(BigBatch B, int d)
 {
-    const BigCore &C = B.c[blockIdx.z];
+    int32_t *const w = B.c[blockIdx.z].core();
     const BigLayout &Y = B.Y;
     const int K = 1 << B.L, bit = B.L - d - 1, y = blockIdx.y;
-    const int32_t *key = C.ws + (y ? ((d & 1) ? Y.keyQ2 : Y.keyQ) : ((d & 1) ? Y.keyP2 : Y.keyP));
+    const int32_t *key = w + (y ? ((d & 1) ? Y.keyQ2 : Y.keyQ) : ((d & 1) ? Y.keyP2 : Y.keyP));
     const int base = blockIdx.x * kSplitTile + threadIdx.x * 8;
     int c = 0;
 #pragma unroll
@@ -645,7 +684,7 @@ __global__ __launch_bounds__(256) void big_split_count_kernel(BigBatch B, int d)
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
     __syncthreads();
     if (threadIdx.x == 0)
-        C.ws[Y.cnt + ((size_t)(d % 3) * 2 + y) * (K / kSplitTile) + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+        w[Y.cnt + ((size_t)(d % 3) * 2 + y) * (K / kSplitTile) + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
 // Stable partition of every segment of size s by bit `bit` (zeros first);
@@ -660,14 +699,14 @@ __global__ __launch_bounds__(256) void big_split_count_kernel(BigBatch B, int d)
 template <bool NEXT>
 __global__ __launch_bounds__(256) void big_split_scatter_kernel(BigBatch B, int d)
 {
-    const BigCore &C = B.c[blockIdx.z];
+    int32_t *const w = B.c[blockIdx.z].core();
     const BigLayout &Y = B.Y;
     const int K = 1 << B.L, s = K >> d, bit = B.L - d - 1, y = blockIdx.y;
     const int ntiles = K / kSplitTile;
-    const int32_t *key = C.ws + (y ? ((d & 1) ? Y.keyQ2 : Y.keyQ) : ((d & 1) ? Y.keyP2 : Y.keyP));
-    int32_t *key_new = C.ws + (y ? ((d & 1) ? Y.keyQ : Y.keyQ2) : ((d & 1) ? Y.keyP : Y.keyP2));
-    int32_t *par = C.ws + (y ? Y.parQ : Y.parP) + (size_t)d * K;
-    const int32_t *cnt = C.ws + Y.cnt + ((size_t)(d % 3) * 2 + y) * ntiles;
+    const int32_t *key = w + (y ? ((d & 1) ? Y.keyQ2 : Y.keyQ) : ((d & 1) ? Y.keyP2 : Y.keyP));
+    int32_t *key_new = w + (y ? ((d & 1) ? Y.keyQ : Y.keyQ2) : ((d & 1) ? Y.keyP : Y.keyP2));
+    int32_t *par = w + (y ? Y.parQ : Y.parP) + (size_t)d * K;
+    const int32_t *cnt = w + Y.cnt + ((size_t)(d % 3) * 2 + y) * ntiles;
     const int base = blockIdx.x * kSplitTile + threadIdx.x * 8;
     int32_t kv[8];
     int c = 0;
@@ -725,55 +764,30 @@ __global__ __launch_bounds__(256) void big_split_scatter_kernel(BigBatch B, int 
             atomicAdd(b ? &no[pos / kSplitTile - ot] : &nz[pos / kSplitTile - zt], 1);
     }
     if (NEXT) {
-        int32_t *next = C.ws + Y.cnt + ((size_t)((d + 1) % 3) * 2 + y) * ntiles;
+        int32_t *next = w + Y.cnt + ((size_t)((d + 1) % 3) * 2 + y) * ntiles;
         __syncthreads();
         if (threadIdx.x < 4) {
             const int v = threadIdx.x < 2 ? nz[threadIdx.x] : no[threadIdx.x - 2];
             const int tile = (threadIdx.x < 2 ? zt : ot) + (threadIdx.x & 1);
             if (v) atomicAdd(&next[tile], v);
         }
-        if (threadIdx.x == 0) C.ws[Y.cnt + ((size_t)((d + 2) % 3) * 2 + y) * ntiles + blockIdx.x] = 0;
+        if (threadIdx.x == 0) w[Y.cnt + ((size_t)((d + 2) % 3) * 2 + y) * ntiles + blockIdx.x] = 0;
     }
 }
 
-// the 2^d0 independent nodes of depth d0, one workgroup each
+// the 2^d0 independent nodes of depth d0, one workgroup each, lifted into
+// depth d0 - 1
 __global__ __launch_bounds__(kThreads) void big_leaf_kernel(BigBatch B)
 {
-    const BigCore &C = B.c[blockIdx.z];
+    int32_t *const w = B.c[blockIdx.z].core();
     const BigLayout &Y = B.Y;
-    const int d0 = B.L - B.L0, s0 = 1 << B.L0;
-    const size_t v0 = (size_t)blockIdx.x * s0;
-    const int32_t *keyP = C.ws + ((d0 & 1) ? Y.keyP2 : Y.keyP) + v0;
-    const int32_t *keyQ = C.ws + ((d0 & 1) ? Y.keyQ2 : Y.keyQ) + v0;
+    const int d0 = B.L - B.L0, s0 = 1 << B.L0, v0 = (int)blockIdx.x * s0;
+    const int32_t *keyP = w + ((d0 & 1) ? Y.keyP2 : Y.keyP) + v0;
+    const int32_t *keyQ = w + ((d0 & 1) ? Y.keyQ2 : Y.keyQ) + v0;
     extern __shared__ uint16_t lds[];
     __shared__ LeafLines lines;
-    // depth d0 of the big core's own recursion: the products go to R
-    core_lds_body<true>(keyP, keyQ, C.ws + Y.R + v0, s0, B.L0, lds, lines);
-}
-
-// lift the children's products into node coordinates (node size s).  The
-// children's products are in R (flip = 0) or Rn (flip = 1), the node's go
-// to the other one.
-__global__ void big_lift_kernel(BigBatch B, int d, int flip)
-{
-    const BigCore &C = B.c[blockIdx.z];
-    const BigLayout &Y = B.Y;
-    const int K = 1 << B.L, s = K >> d, h = s >> 1;
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= K) return;
-    const int32_t *pp = C.ws + Y.parP + (size_t)d * K, *pq = C.ws + Y.parQ + (size_t)d * K;
-    const int32_t *R = C.ws + (flip ? Y.Rn : Y.R);
-    int32_t *Rn = C.ws + (flip ? Y.R : Y.Rn);
-    uint32_t *U = (uint32_t *)(C.ws + Y.U), *CI = (uint32_t *)(C.ws + Y.CI);
-    const int p_pos = pp[x];
-    const int cseg = x & ~(h - 1);
-    const int q_pos = pq[cseg + R[x]];
-    const int v0 = p_pos & ~(s - 1);
-    const uint32_t lo = (x & h) ? 0u : kLo31;
-    const int lr = p_pos - v0, lc = q_pos - v0;
-    U[p_pos] = (uint32_t)lc | lo;
-    CI[v0 + lc] = (uint32_t)lr | lo;
-    Rn[p_pos] = lc;
+    core_lds_body(keyP, keyQ, s0, B.L0, lds, lines,
+                  [&](int x, int c) { big_lift(B, w, d0 - 1, v0, s0, v0 + x, c); });
 }
 
 // Per histogram block (w entries of CI for y = 0, of U for y = 1): packed
@@ -781,11 +795,11 @@ __global__ void big_lift_kernel(BigBatch B, int d, int flip)
 // boundary j < nb, and the packed totals at [nb].
 __global__ __launch_bounds__(256) void big_hist_kernel(BigBatch B, int d)
 {
-    const BigCore &C = B.c[blockIdx.z];
+    int32_t *const w = B.c[blockIdx.z].core();
     const BigLayout &Y = B.Y;
     const BigDepth &D = B.D[d];
     const int K = 1 << B.L, y = blockIdx.y;
-    const uint32_t *E = (const uint32_t *)(C.ws + (y ? Y.U : Y.CI));
+    const uint32_t *E = (const uint32_t *)w + (y ? Y.U[d & 1] : Y.CI[d & 1]);
     __shared__ uint32_t h[kMaxLines];
     __shared__ uint32_t sums[4];
     for (int j = threadIdx.x; j < D.nb; j += 256) h[j] = 0;
@@ -793,7 +807,8 @@ __global__ __launch_bounds__(256) void big_hist_kernel(BigBatch B, int d)
     const size_t base = (size_t)blockIdx.x * D.w;
     for (int i = threadIdx.x; i < D.w; i += 256) {
         const uint32_t e = E[base + i];
-        const int bk = (D.s - 1 - (int)(e & ~kLo31)) >> D.glog;
+        // an aborted comb can leave entries unwritten: keep the bucket in range
+        const int bk = (D.s - 1 - (int)(e & (uint32_t)(D.s - 1))) >> D.glog;
         atomicAdd(&h[bk], (e & kLo31) ? 1u : 0x10000u);
     }
     __syncthreads();
@@ -821,7 +836,7 @@ __global__ __launch_bounds__(256) void big_hist_kernel(BigBatch B, int d)
     // writes its own row, coalesced), then the nsegs block totals in a row
     // of their own (read coalesced by the search)
     const int node = blockIdx.x / D.nsegs, g = blockIdx.x % D.nsegs, nodes = K / D.s;
-    uint32_t *rows = (uint32_t *)(C.ws + Y.hist) + ((size_t)y * nodes + node) * D.nsegs * (size_t)(D.nb + 1);
+    uint32_t *rows = (uint32_t *)(w + Y.hist) + ((size_t)y * nodes + node) * D.nsegs * (size_t)(D.nb + 1);
     uint32_t *out = rows + (size_t)g * D.nb;
     const uint32_t w1 = sums[0], w2 = w1 + (nw > 1 ? sums[1] : 0u), w3 = w2 + (nw > 2 ? sums[2] : 0u);
     for (int j = threadIdx.x; j < D.nb; j += 256) {
@@ -908,33 +923,15 @@ __device__ __forceinline__ int sweep_block(const uint32_t *E, int w, int s, int 
     return 0;
 }
 
-// One wave per (y, node, boundary j): Y_j and the block where the running
-// count reaches it (block_search, at most kSegRounds x 64 blocks per node),
-// then a sweep of that block (sweep_block) for the entry where the count
-// reaches the rank still needed; T = that entry's position + 1.
-// Boundaries with j = 0 or Y_j = 0 get T = 0.
 constexpr int kSegRounds = 16;
 static_assert(big_blocks_fit(64 * kSegRounds), "histogram blocks per node");
-#ifndef LCS_SWEEP_WAVES
-#define LCS_SWEEP_WAVES 4
-#endif
-constexpr int kSweepWaves = LCS_SWEEP_WAVES;   // waves (boundaries) per workgroup
-__global__ __launch_bounds__(64 * kSweepWaves) void big_sweep_kernel(BigBatch B, int d)
+
+// T of boundary j > 0 over the entries E of a node: Y_j and the block where
+// the running count reaches it (block_search, at most kSegRounds x 64 blocks
+// per node), then a sweep of that block for the entry where the count reaches
+// the rank still needed; T is that entry's position + 1, 0 when Y_j = 0.
+__device__ __forceinline__ int big_line(const BigDepth &D, const uint32_t *H, const uint32_t *E, int j, int lane)
 {
-    const BigCore &C = B.c[blockIdx.z];
-    const BigLayout &Y = B.Y;
-    const BigDepth &D = B.D[d];
-    const int K = 1 << B.L, nodes = K / D.s, y = blockIdx.y;
-    // the wave's boundary, made scalar so that its addresses stay in SGPRs
-    const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * kSweepWaves + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    if (t >= nodes * D.nb) return;
-    const int node = t / D.nb, j = t % D.nb;
-    int32_t *T = C.ws + Y.T + (size_t)y * nodes * D.nb + t;
-    if (j == 0) {
-        if (lane == 0) *T = 0;
-        return;
-    }
-    const uint32_t *H = (const uint32_t *)(C.ws + Y.hist) + ((size_t)y * nodes + node) * D.nsegs * (size_t)(D.nb + 1);
     const uint32_t *Hj = H + j, *Ht = H + (size_t)D.nsegs * D.nb;
     int Yj, Z, seg;
     if (D.nsegs <= 64) block_search<1>(Hj, Ht, D.nb, D.nsegs, lane, Yj, Z, seg);
@@ -942,73 +939,76 @@ __global__ __launch_bounds__(64 * kSweepWaves) void big_sweep_kernel(BigBatch B,
     else if (D.nsegs <= 256) block_search<4>(Hj, Ht, D.nb, D.nsegs, lane, Yj, Z, seg);
     else if (D.nsegs <= 512) block_search<8>(Hj, Ht, D.nb, D.nsegs, lane, Yj, Z, seg);
     else block_search<kSegRounds>(Hj, Ht, D.nb, D.nsegs, lane, Yj, Z, seg);
-    if (Yj == 0) {
-        if (lane == 0) *T = 0;
-        return;
-    }
-    const uint32_t *E = (const uint32_t *)(C.ws + (y ? Y.U : Y.CI)) + (size_t)node * D.s + (size_t)seg * D.w;
+    if (Yj == 0) return 0;
+    E += (size_t)seg * D.w;
     // w is a power of two >= 128: the whole block in one batch up to 1024 entries
     const int need = Yj - Z;
     const int pos = D.w <= 128   ? sweep_block<2>(E, D.w, D.s, D.glog, j, need, lane)
                     : D.w <= 256 ? sweep_block<4>(E, D.w, D.s, D.glog, j, need, lane)
                     : D.w <= 512 ? sweep_block<8>(E, D.w, D.s, D.glog, j, need, lane)
                                  : sweep_block<16>(E, D.w, D.s, D.glog, j, need, lane);
-    if (lane == 0 && pos) *T = seg * D.w + pos;
+    return pos ? min(seg * D.w + pos, D.s) : 0;
 }
 
-// One wave per piece of the ant's path.  Piece q < nb of a node starts at
-// row line j = q (q = 0: the start of the passage at T(s) = 0), q >= nb at
-// column line i = q - nb + 1; it stays in one g x g box (box_rows above says
-// how its rows find T).  With g above 64 the rows go 64 at a time from the
-// line upwards, carrying the rows counted so far, and the columns 64 at a
-// time.  About 200 VALU and a few coalesced loads per wave; walking the boxes
-// one lane each took 21 us per depth of a k = 2^16 product, this 3.  Whole
-// products (random, kernel time, before and after boxes and wave_product64
-// took the walks' place): k = 2^11 142 and 100 us, 2^16 344 and 215, 2^20
-// 1419 and 1178.
+// One wave per piece of the ant's path: (y = 0) from row line j = 0 .. nb - 1
+// (j = 0: the start of the passage at T(s) = 0), (y = 1) from column line i =
+// nb - j.  The wave finds its own crossing (big_line), then its box's rows
+// (box_rows), and hands every row it decides straight to the parent node
+// (big_lift), or from the top depth to the product: each row lies in exactly
+// one piece's box.  A wave's chain of dependent loads (histogram, block, box,
+// parents) is what bounds it.  Sweep, boxes, lift and output were kernels of
+// their own, each a launch (about 4 us with its gap) and a pass over U and CI;
+// with them in one and the slicing in three, a k = 2^16 product takes 24
+// launches instead of 38: 197 -> 155 us, 2^11 86 -> 71, 2^20 1178 -> 991.  With g above 64 the rows go
+// 64 at a time from the line upwards, carrying the rows counted so far, and
+// the columns 64 at a time.
 constexpr int kBoxWaves = 4;   // pieces per workgroup
-__global__ __launch_bounds__(64 * kBoxWaves) void big_box_kernel(BigBatch B, int d, int flip)
+__global__ __launch_bounds__(64 * kBoxWaves) void big_box_kernel(BigBatch B, int d)
 {
-    const BigCore &C = B.c[blockIdx.z];
+    const MulArgs &M = B.c[blockIdx.z];
+    int32_t *const w = M.core();
     const BigLayout &Y = B.Y;
     const BigDepth &D = B.D[d];
-    const int K = 1 << B.L, s = D.s, nodes = K / s, g = 1 << D.glog, nb = D.nb;
-    const int pieces = 2 * nb - 1, lane = threadIdx.x & 63;
+    const int K = 1 << B.L, s = D.s, nodes = K / s, g = 1 << D.glog, nb = D.nb, lane = threadIdx.x & 63;
     const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * kBoxWaves + (threadIdx.x >> 6));
-    if (t >= nodes * pieces) return;
-    const int node = t / pieces, q = t - node * pieces;
-    const size_t v0 = (size_t)node * s;
-    const uint32_t *U = (const uint32_t *)(C.ws + Y.U) + v0, *CI = (const uint32_t *)(C.ws + Y.CI) + v0;
-    int32_t *Rn = C.ws + (flip ? Y.R : Y.Rn) + v0;
-    // T lies in [0, s]; the clamps only keep every access inside the node
-    // after an aborted comb fed undefined input
+    if (t >= 2 * nodes * nb) return;
+    const bool col = t >= nodes * nb;
+    const int q = col ? t - nodes * nb : t, node = q / nb, j = q - node * nb;
+    if (col && j == 0) return;
+    const int v0 = node * s;
+    const uint32_t *U = (const uint32_t *)w + Y.U[d & 1] + v0, *CI = (const uint32_t *)w + Y.CI[d & 1] + v0;
+    int T0 = 0;
+    if (j) {
+        const uint32_t *H = (const uint32_t *)w + Y.hist + ((size_t)(col ? 1 : 0) * nodes + node) * D.nsegs * (size_t)(D.nb + 1);
+        T0 = big_line(D, H, col ? U : CI, j, lane);
+    }
     int r_lo, rho, cs, ce;
-    const bool col = q >= nb;
     if (!col) {
-        r_lo = s - (q + 1) * g;
+        r_lo = s - (j + 1) * g;
         rho = r_lo + g - 1;
-        cs = q == 0 ? 0 : min(max(C.ws[Y.T + (size_t)node * nb + q], 0), s);
+        cs = T0;
         ce = cs == 0 ? g : (((cs - 1) >> D.glog) + 1) << D.glog;
     } else {
-        const int i = q - nb + 1;
-        const int Tc = min(max(C.ws[Y.T + (size_t)nodes * nb + (size_t)node * nb + nb - i], 0), s);
-        if (Tc == 0) return;   // the ant never reaches this column line
-        rho = Tc - 1;
+        if (T0 == 0) return;   // the ant never reaches this column line
+        rho = T0 - 1;
         r_lo = rho & ~(g - 1);
-        cs = i * g;
+        cs = (nb - j) * g;
         ce = cs + g;
     }
+    auto finish = [&](int r, int c) {
+        if (d) big_lift(B, w, d - 1, v0, s, v0 + r, c);
+        else M.put(r, c);
+    };
     auto entry = [&](int c) { return CI[c]; };
     if (g == kBox) {
-        if (r_lo) ce = min(ce, min(max(C.ws[Y.T + (size_t)node * nb + nb - (r_lo >> D.glog)], 0), s));
         const uint32_t u = U[r_lo + lane];
         const int c = col ? box_rows<31, true>(u, entry, r_lo, rho, cs, ce, lane)
                           : box_rows<31, false>(u, entry, r_lo, rho, cs, ce, lane);
-        if (c >= 0) Rn[r_lo + lane] = c;
+        if (c >= 0) finish(r_lo + lane, c);
         return;
     }
     int below = col ? 1 : 0;   // -delta(r, cs) just below the rows in hand
-    for (int rb = (rho & ~63); rb >= r_lo; rb -= 64) {
+    for (int rb = rho & ~63; rb >= r_lo; rb -= 64) {
         const int r = rb + lane;
         const uint32_t u = U[r];
         const bool uc = counted<31>(u, cs);
@@ -1017,209 +1017,146 @@ __global__ __launch_bounds__(64 * kBoxWaves) void big_box_kernel(BigBatch B, int
         below += (int)__popcll(m);
         int T = need ? -1 : cs;
         for (int c0 = cs; c0 < ce; c0 += 64) {
-            uint32_t q[4];
+            uint32_t qm[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int c = c0 + 16 * i + (lane & 15);
-                q[i] = counted_row16(c < ce ? entry(c) : ~kLo31, (uint32_t)r, lane);
+                qm[i] = counted_row16(c < ce ? entry(c) : ~kLo31, (uint32_t)r, lane);
             }
-            const uint32_t lo = q[0] | q[1] << 16, hi = q[2] | q[3] << 16;
+            const uint32_t lo = qm[0] | qm[1] << 16, hi = qm[2] | qm[3] << 16;
             const int cnt = __popc(lo) + __popc(hi);
             if (T < 0 && need <= cnt) T = c0 + 1 + select64(lo, hi, need);
             need -= cnt;
         }
-        if ((!col || r <= rho) && T > 0 && counted<31>(u, T)) Rn[r] = T - 1;
+        if ((!col || r <= rho) && T >= 0) finish(r, T > 0 && counted<31>(u, T) ? T - 1 : (int)(u & ~kLo31));
     }
-}
-
-// the product of the last depth is in R (flip = 0) or Rn (flip = 1)
-__global__ void big_out_kernel(BigBatch B, int flip)
-{
-    const BigCore &C = B.c[blockIdx.z];
-    const BigLayout &Y = B.Y;
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x < C.k) C.R[x] = C.ws[(flip ? Y.Rn : Y.R) + x];
 }
 
 // ---------------------------------------------------------------- slicing
-// Device-wide stable compaction in three kernels: per-block counts, a scan
-// of the counts in one block, per-block scatter.  The products of one merge
-// level go through each kernel in one launch: blockIdx.y picks the slice
-// (two per product, p's rows at even y and q's columns at odd y).
-constexpr int kScanBlock = 256, kScanPer = 8, kScanTile = kScanBlock * kScanPer;
-constexpr int kMulBatch = 32;   // products per slicing / assembly launch
-
-struct SliceSpec {
-    // selects element i of `src` (size n) when lo <= src[i] < hi; per-block
-    // counts (then their exclusive scan) in `counts`; records, for slice j of
-    // the selected elements (j < cap):
-    //   even slice (vertical slice of p, rows in order):   map[j] = i, val[j] = src[i] - lo
-    //   odd slice (horizontal slice of q, cols in order):  map[j] = i (a column), val[src[i] - lo] = j
+// The points of p in the glued columns (p's rows in order) and those of q in
+// the glued rows (q's columns in order) become the core's keys; every other
+// point goes to the product unchanged (braid_multiplication.hpp:353-401).
+// Device-wide stable compaction: per-block counts, then a scatter whose
+// blocks sum the counts before them themselves.  The products of one merge
+// level go through each kernel in one launch: blockIdx.y / 2 picks the
+// product, blockIdx.y & 1 its side (0: p by rows, 1: q by columns).
+struct SliceSide {
     const int32_t *src;
-    int32_t *counts, *map, *val;
-    int32_t n, lo, hi, cap;
+    int32_t n, lo, hi;
+    __device__ bool sel(int i) const { return src[i] >= lo && src[i] < hi; }
 };
-struct SliceBatch {
-    SliceSpec s[2 * kMulBatch];
-};
-
-__device__ __forceinline__ bool sel(const SliceSpec &S, int i) { const int v = S.src[i]; return v >= S.lo && v < S.hi; }
-
-__global__ void slice_count_kernel(SliceBatch B)
+__device__ __forceinline__ SliceSide slice_side(const MulArgs &M, int side)
 {
-    const SliceSpec &S = B.s[blockIdx.y];
-    if ((int64_t)blockIdx.x * kScanTile >= S.n) return;   // past this slice's blocks (whole block)
-    __shared__ int32_t red[kScanBlock];
-    const int base = blockIdx.x * kScanTile + threadIdx.x * kScanPer;
-    int c = 0;
-    for (int q = 0; q < kScanPer; ++q) c += (base + q < S.n) && sel(S, base + q);
-    red[threadIdx.x] = c;
-    __syncthreads();
-    for (int off = kScanBlock / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) S.counts[blockIdx.x] = red[0];
+    if (side == 0) return {M.p, M.p_size, M.row_glue ? 0 : M.p_size - M.k, M.row_glue ? M.k : M.p_size};
+    return {M.q_c2r(), M.q_size, M.row_glue ? M.q_size - M.k : 0, M.row_glue ? M.q_size : M.k};
 }
 
-__global__ void scan_counts_kernel(SliceBatch B)
+__device__ __forceinline__ int block_sum256(int x, int *red)
 {
-    // exclusive scan of slice blockIdx.x's block counts in place, one block of 1024
-    const SliceSpec &S = B.s[blockIdx.x];
-    int32_t *counts = S.counts;
-    const int nblocks = (S.n + kScanTile - 1) / kScanTile;
-    __shared__ int32_t s[1024];
-    const int t = threadIdx.x;
-    const int per = (nblocks + 1023) / 1024;
-    const int lo = min(t * per, nblocks), hi = min(lo + per, nblocks);
-    int run = 0;
-    for (int i = lo; i < hi; ++i) run += counts[i];
-    s[t] = run;
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
     __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int v = t >= off ? s[t - off] : 0;
-        __syncthreads();
-        s[t] += v;
-        __syncthreads();
-    }
-    int acc = s[t] - run;
-    for (int i = lo; i < hi; ++i) { const int c = counts[i]; counts[i] = acc; acc += c; }
+    return red[0] + red[1] + red[2] + red[3];
 }
 
-__global__ void slice_scatter_kernel(SliceBatch B)
+__global__ __launch_bounds__(kScanBlock) void slice_count_kernel(MulBatch B)
 {
-    const SliceSpec &S = B.s[blockIdx.y];
+    const MulArgs &M = B.m[blockIdx.y >> 1];
+    const int side = blockIdx.y & 1;
+    const SliceSide S = slice_side(M, side);
     if ((int64_t)blockIdx.x * kScanTile >= S.n) return;   // past this slice's blocks (whole block)
-    const bool rows = (blockIdx.y & 1) == 0;
-    __shared__ int32_t s[kScanBlock];
-    const int base = blockIdx.x * kScanTile + threadIdx.x * kScanPer;
+    __shared__ int red[kScanBlock / 64];
+    const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x * kScanPer;
     int c = 0;
-    for (int q = 0; q < kScanPer; ++q) c += (base + q < S.n) && sel(S, base + q);
-    s[threadIdx.x] = c;
-    __syncthreads();
-    for (int off = 1; off < kScanBlock; off <<= 1) {
-        int v = (int)threadIdx.x >= off ? s[threadIdx.x - off] : 0;
-        __syncthreads();
-        s[threadIdx.x] += v;
-        __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kScanPer; ++q) c += base + q < S.n && S.sel((int)base + q);
+    c = block_sum256(c, red);
+    if (threadIdx.x == 0) M.counts(side)[blockIdx.x] = c;
+}
+
+// also pads the keys of a core smaller than 2^L with fixed points, and zeroes
+// the tile counts of a big core's depths 1 and 2, which the partitions before
+// them accumulate
+__global__ __launch_bounds__(kScanBlock) void slice_scatter_kernel(MulBatch B)
+{
+    const MulArgs &M = B.m[blockIdx.y >> 1];
+    const int side = blockIdx.y & 1;
+    const SliceSide S = slice_side(M, side);
+    const int K = 1 << M.L, k = M.k, ps = M.p_size, qs = M.q_size;
+    int32_t *const key = M.core() + (side ? K : 0), *const map = side ? M.map_col() : M.map_row();
+    for (int64_t x = k + (int64_t)blockIdx.x * kScanBlock + threadIdx.x; x < K; x += (int64_t)gridDim.x * kScanBlock)
+        key[x] = (int32_t)x;
+    if (M.L >= kBigMinL) {
+        const int ntiles = K / kSplitTile;
+        const size_t cnt = big_layout_cnt(M.L) + (size_t)ntiles * 2;
+        for (int x = blockIdx.x * kScanBlock + threadIdx.x; x < 2 * ntiles; x += gridDim.x * kScanBlock)
+            M.core()[cnt + (size_t)side * 2 * ntiles + x] = 0;
     }
-    int j = S.counts[blockIdx.x] + s[threadIdx.x] - c;
+    if ((int64_t)blockIdx.x * kScanTile >= S.n) return;   // past this slice's blocks (whole block)
+    __shared__ int red[kScanBlock / 64], wsum[kScanBlock / 64];
+    const int32_t *counts = M.counts(side);
+    int before = 0;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanBlock) before += counts[i];
+    before = block_sum256(before, red);
+    const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x * kScanPer;
+    int32_t v[kScanPer];
+    int c = 0;
+#pragma unroll
     for (int q = 0; q < kScanPer; ++q) {
-        const int i = base + q;
-        if (i < S.n && sel(S, i) && j < S.cap) {
-            S.map[j] = i;
-            if (rows) S.val[j] = S.src[i] - S.lo;
-            else S.val[S.src[i] - S.lo] = j;
+        v[q] = base + q < S.n ? S.src[base + q] : -1;
+        c += v[q] >= S.lo && v[q] < S.hi;
+    }
+    const int incl = wave_incl_scan(c);
+    if ((threadIdx.x & 63) == 63) wsum[threadIdx.x >> 6] = incl;
+    __syncthreads();
+    int j = before + incl - c;
+    for (int q = 0; q < (int)(threadIdx.x >> 6); ++q) j += wsum[q];
+#pragma unroll
+    for (int q = 0; q < kScanPer; ++q) {
+        const int i = (int)base + q;
+        if (base + q >= S.n) break;
+        if (v[q] >= S.lo && v[q] < S.hi) {
+            if (j < k) {
+                map[j] = i;
+                key[j] = v[q] - S.lo;
+            }
             ++j;
+            continue;
         }
+        // an untouched point (row, col) of p or q; the range test only matters
+        // after an aborted comb fed undefined input
+        int row = side ? v[q] : i, col = side ? i : v[q];
+        if (side == 0 && M.row_glue) { row += qs - k; col += qs - k; }
+        if (side == 1 && !M.row_glue) { row += ps - k; col += ps - k; }
+        if ((uint32_t)row < (uint32_t)(ps + qs - k)) M.out[row] = col;
     }
 }
 
-struct InvertBatch {
-    struct {
-        const int32_t *r2c;
-        int32_t *c2r;
-        int32_t n;
-    } s[kMulBatch];
-};
-
-__global__ void invert_kernel(InvertBatch B)
+__global__ void invert_kernel(MulBatch B)
 {
-    const auto &S = B.s[blockIdx.y];
+    const MulArgs &M = B.m[blockIdx.y];
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;   // no wrap near 2^31
-    if (i < S.n && (uint32_t)S.r2c[i] < (uint32_t)S.n) S.c2r[S.r2c[i]] = (int32_t)i;
+    if (i < M.q_size && (uint32_t)M.q[i] < (uint32_t)M.q_size) M.q_c2r()[M.q[i]] = (int32_t)i;
 }
 
-struct AssembleBatch {
-    AssembleArgs a[kMulBatch];
-};
-
-// Writes the product (row -> col) from the core result and the untouched
-// points of p and q (braid_multiplication.hpp:353-401).
-__global__ void assemble_kernel(AssembleBatch B)
+// A product with no glued strands: p's points, then q's.
+__global__ void juxtapose_kernel(MulBatch B)
 {
-    const AssembleArgs &A = B.a[blockIdx.y];
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;   // no wrap near 2^31
-    const int k = A.k, ps = A.p_size, qs = A.q_size;
-    // the range tests only matter after an aborted comb fed undefined input
-    if (i < k && (uint32_t)A.core[i] < (uint32_t)k) {
-        const int row = A.map_row[i], col = A.map_col[A.core[i]];
-        if ((uint32_t)row < (uint32_t)ps) {
-            if (A.row_glue) A.out[qs - k + row] = col;
-            else A.out[row] = col + ps - k;
-        }
-    }
-    if (i < ps) {
-        const int c = A.p[i];
-        if (A.row_glue) { if (c >= k) A.out[i + qs - k] = c + qs - k; }
-        else { if (c < ps - k) A.out[i] = c; }
-    }
-    if (i < qs) {
-        const int c = A.q[i];
-        if (A.row_glue) { if (i < qs - k) A.out[i] = c; }
-        else { if (i >= k) A.out[i - k + ps] = c - k + ps; }
-    }
+    const MulArgs &M = B.m[blockIdx.y];
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int ps = M.p_size, qs = M.q_size;
+    if (i < ps) M.out[M.row_glue ? i + qs : i] = M.p[i] + (M.row_glue ? qs : 0);
+    if (i < qs) M.out[M.row_glue ? i : i + ps] = M.q[i] + (M.row_glue ? 0 : ps);
 }
 
 }  // namespace lcsb
 
 using namespace lcsb;
 
-// Cores of 2^L points with L >= kBigMinL run over the whole GPU, with
-// leaves of at most 2^kBigLeafMaxL points (at least 2^10: the device-wide
-// partitions work on tiles of 2048 keys inside nodes of 2^(leaf+1); at most
-// 2^kLdsCoreL: a leaf is one workgroup's LDS core).
-// Measured on the Zipf pair's five merge levels (k = 2^14, 16 .. 1 products
-// per level): one workgroup per core 15.6 ms for the whole pair; whole-GPU
-// cores with leaves of 2^10 / 2^11 / 2^12 points 12.5 / 12.3 / 12.5 ms.
-#ifndef LCS_BIG_MIN_L
-#define LCS_BIG_MIN_L 12
-#endif
-#ifndef LCS_BIG_LEAF_L
-#define LCS_BIG_LEAF_L 11
-#endif
-// cores of 2^16 points and more take leaves of up to 2^LCS_BIG_LEAF_L_LARGE
-#ifndef LCS_BIG_LEAF_L_LARGE
-#define LCS_BIG_LEAF_L_LARGE 11
-#endif
-constexpr int kBigMinL = LCS_BIG_MIN_L;
-constexpr int kBigLeafMaxL = LCS_BIG_LEAF_L;
-constexpr int kBigLeafLargeL = LCS_BIG_LEAF_L_LARGE;
-static_assert(kBigMinL >= 11 && kBigMinL <= kLdsCoreL + 1 && kBigLeafMaxL >= 10 && kBigLeafMaxL <= kLdsCoreL &&
-                  kBigLeafLargeL >= 10 && kBigLeafLargeL <= kLdsCoreL,
-              "big-core leaf sizes");
-static int big_leaf_L(int L)
-{
-    const int lim = L >= 16 ? kBigLeafLargeL : kBigLeafMaxL;
-    return L - 1 < lim ? L - 1 : lim;
-}
-static bool is_big(int L) { return L >= kBigMinL; }
-
 size_t lcsb_core_scratch_words(int32_t k)
 {
     const int L = lcsb_core_L(k);
-    if (!is_big(L)) return 0;   // the one-workgroup core keeps everything in LDS
-    return big_layout(L, big_leaf_L(L)).total;
+    return L >= kBigMinL ? big_layout(L, big_leaf_L(L)).total : (size_t)2 << L;   // small cores: the keys
 }
 
 // Padded core size 2^L: at least 64 (the LDS kernel ranks keys by wave
@@ -1231,12 +1168,11 @@ int lcsb_core_L(int32_t k)
     return L;
 }
 
-// The big-core sequence for up to kBigBatch products of one padded size.
+// The big-core sequence for up to kMulBatch products of one padded size.
 static int launch_big(const BigBatch &B, int cnt, hipStream_t stream)
 {
     const int L = B.L, L0 = B.L0, d0 = L - L0, K = 1 << L;
-    const dim3 lin((unsigned)(K / 256), 1, (unsigned)cnt), tiles((unsigned)(K / kSplitTile), 2, (unsigned)cnt);
-    hipLaunchKernelGGL(big_init_kernel, lin, dim3(256), 0, stream, B);
+    const dim3 tiles((unsigned)(K / kSplitTile), 2, (unsigned)cnt);
     hipLaunchKernelGGL(big_split_count_kernel, tiles, dim3(256), 0, stream, B, 0);
     for (int d = 0; d < d0; ++d) {
         if (d + 1 < d0) hipLaunchKernelGGL(big_split_scatter_kernel<true>, tiles, dim3(256), 0, stream, B, d);
@@ -1244,20 +1180,13 @@ static int launch_big(const BigBatch &B, int cnt, hipStream_t stream)
     }
     hipLaunchKernelGGL(big_leaf_kernel, dim3(1u << d0, 1, (unsigned)cnt), dim3(kThreads), lds_core_bytes(L0),
                        stream, B);
-    int flip = 0;
     for (int d = d0 - 1; d >= 0; --d) {
         const BigDepth D = big_depth(L, d);
-        const int lines = (K / D.s) * D.nb, pieces = (K / D.s) * (2 * D.nb - 1);
-        hipLaunchKernelGGL(big_lift_kernel, lin, dim3(256), 0, stream, B, d, flip);
+        const int pieces = 2 * (K / D.s) * D.nb;
         hipLaunchKernelGGL(big_hist_kernel, dim3((unsigned)(K / D.w), 2, (unsigned)cnt), dim3(256), 0, stream, B, d);
-        hipLaunchKernelGGL(big_sweep_kernel, dim3((unsigned)((lines + kSweepWaves - 1) / kSweepWaves), 2, (unsigned)cnt),
-                           dim3(64 * kSweepWaves), 0, stream,
-                           B, d);
         hipLaunchKernelGGL(big_box_kernel, dim3((unsigned)((pieces + kBoxWaves - 1) / kBoxWaves), 1, (unsigned)cnt),
-                           dim3(64 * kBoxWaves), 0, stream, B, d, flip);
-        flip ^= 1;
+                           dim3(64 * kBoxWaves), 0, stream, B, d);
     }
-    hipLaunchKernelGGL(big_out_kernel, lin, dim3(256), 0, stream, B, flip);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -1277,119 +1206,52 @@ int lcsb_init(void)
     return rc;
 }
 
-int lcsb_launch_core(const BraidCoreDesc *descs, int count, hipStream_t stream)
-{
-    if (lcsb_init()) return -5;
-    // small cores: one workgroup each, descriptors by value in the arguments
-    std::vector<BraidCoreDesc> small;
-    std::vector<BraidCoreDesc> big;
-    for (int i = 0; i < count; ++i) {
-        if (descs[i].L > kMaxCoreL) return -34;
-        (is_big(descs[i].L) ? big : small).push_back(descs[i]);
-    }
-    for (size_t base = 0; base < small.size(); base += kCoreBatch) {
-        CoreBatch batch{};
-        const int cnt = (int)std::min<size_t>(small.size() - base, kCoreBatch);
-        int max_L = 0;
-        for (int i = 0; i < cnt; ++i) {
-            batch.d[i] = small[base + (size_t)i];
-            max_L = std::max(max_L, (int)batch.d[i].L);
-        }
-        if (max_L > kLdsCoreL) return -34;
-        hipLaunchKernelGGL(braid_core_lds_kernel, dim3(cnt), dim3(kThreads), lds_core_bytes(max_L), stream, batch);
-    }
-    // big cores: products of one padded size share each launch of the sequence
-    std::sort(big.begin(), big.end(), [](const BraidCoreDesc &x, const BraidCoreDesc &y) { return x.L < y.L; });
-    for (size_t i = 0; i < big.size();) {
-        BigBatch B{};
-        B.L = big[i].L;
-        B.L0 = big_leaf_L(B.L);
-        B.Y = big_layout(B.L, B.L0);
-        for (int d = 0; d < B.L - B.L0; ++d) B.D[d] = big_depth(B.L, d);
-        int cnt = 0;
-        while (i < big.size() && big[i].L == B.L && cnt < kBigBatch) {
-            B.c[cnt++] = BigCore{big[i].P, big[i].Q, big[i].R, big[i].scratch, big[i].k};
-            ++i;
-        }
-        const int rc = launch_big(B, cnt, stream);
-        if (rc) return rc;
-    }
-    return hipGetLastError() == hipSuccess ? 0 : -5;
-}
-
 // staggered_multiply for `count` independent products on device pointers.
-// Their slicing, cores and assembly each go to one launch per kind (in
-// groups of kMulBatch products for the slicing and assembly), so the
-// products of a merge-tree level run side by side.  specs[i].ws holds
+// The products of one padded core size go through each kernel of the
+// sequence side by side (in groups of kMulBatch), so the products of a
+// merge-tree level share their launches.  specs[i].ws holds
 // lcsb_multiply_ws_words(p_size, q_size, k) words.
 int lcsb_multiply_many_device(const MulSpec *specs, int count, hipStream_t stream)
 {
-    std::vector<BraidCoreDesc> cores;
-    cores.reserve((size_t)count);
-    auto nblocks = [](int32_t n) { return (n + kScanTile - 1) / kScanTile; };
-    for (int base = 0; base < count; base += kMulBatch) {
-        const int cnt = count - base < kMulBatch ? count - base : kMulBatch;
-        InvertBatch ib{};
-        SliceBatch sb{};
-        int ni = 0, inv_blocks = 0, slice_blocks = 0;
-        for (int i = 0; i < cnt; ++i) {
-            const MulSpec &M = specs[base + i];
-            const int32_t p_size = M.p_size, q_size = M.q_size, k = M.k;
-            if (k == 0) continue;
-            const int nmax = p_size > q_size ? p_size : q_size;
-            const int nblocks_max = nblocks(nmax) + 1;
-            int32_t *q_c2r = M.ws;                // q_size
-            int32_t *map_row = q_c2r + q_size;    // k
-            int32_t *map_col = map_row + k;       // k
-            int32_t *Pred = map_col + k;          // k
-            int32_t *Qred = Pred + k;             // k
-            int32_t *core = Qred + k;             // k
-            int32_t *counts_p = core + k;         // nblocks_max
-            int32_t *counts_q = counts_p + nblocks_max;
-            int32_t *core_ws = counts_q + nblocks_max;
-            ib.s[ni].r2c = M.q;
-            ib.s[ni].c2r = q_c2r;
-            ib.s[ni].n = q_size;
-            // vertical slice of p: rows whose column lies in the glued range
-            sb.s[2 * ni] = SliceSpec{M.p, counts_p, map_row, Pred, p_size, M.row_glue ? 0 : p_size - k,
-                                     M.row_glue ? k : p_size, k};
-            // horizontal slice of q: columns whose row lies in the glued range
-            sb.s[2 * ni + 1] = SliceSpec{q_c2r, counts_q, map_col, Qred, q_size, M.row_glue ? q_size - k : 0,
-                                         M.row_glue ? q_size : k, k};
-            ++ni;
-            inv_blocks = std::max(inv_blocks, (q_size + 255) / 256);
-            slice_blocks = std::max(slice_blocks, std::max(nblocks(p_size), nblocks(q_size)));
-            BraidCoreDesc h{};
-            h.P = Pred;
-            h.Q = Qred;
-            h.R = core;
-            h.k = k;
-            h.L = lcsb_core_L(k);
-            h.scratch = core_ws;
-            cores.push_back(h);
-        }
-        if (ni == 0) continue;
-        hipLaunchKernelGGL(invert_kernel, dim3(inv_blocks, ni), dim3(256), 0, stream, ib);
-        hipLaunchKernelGGL(slice_count_kernel, dim3(slice_blocks, 2 * ni), dim3(kScanBlock), 0, stream, sb);
-        hipLaunchKernelGGL(scan_counts_kernel, dim3(2 * ni), dim3(1024), 0, stream, sb);
-        hipLaunchKernelGGL(slice_scatter_kernel, dim3(slice_blocks, 2 * ni), dim3(kScanBlock), 0, stream, sb);
+    if (lcsb_init()) return -5;
+    std::vector<MulArgs> mul((size_t)count);
+    for (int i = 0; i < count; ++i) {
+        const MulSpec &M = specs[i];
+        mul[(size_t)i] = MulArgs{M.p, M.q, M.out, M.ws, M.p_size, M.q_size, M.k, M.row_glue ? 1 : 0,
+                                 M.k ? lcsb_core_L(M.k) : 0, 0};
+        if (mul[(size_t)i].L > kMaxCoreL) return -34;
     }
-    if (!cores.empty()) {
-        const int rc = lcsb_launch_core(cores.data(), (int)cores.size(), stream);
+    std::stable_sort(mul.begin(), mul.end(), [](const MulArgs &x, const MulArgs &y) { return x.L < y.L; });
+    for (size_t i = 0; i < mul.size();) {
+        MulBatch B{};
+        const int L = mul[i].L;
+        int cnt = 0, q_max = 0, n_max = 0;
+        while (i < mul.size() && mul[i].L == L && cnt < kMulBatch) {
+            q_max = std::max(q_max, mul[i].q_size);
+            n_max = std::max(n_max, std::max(mul[i].p_size, mul[i].q_size));
+            B.m[cnt++] = mul[i++];
+        }
+        const dim3 by_point((unsigned)((n_max + 255) / 256), (unsigned)cnt);
+        if (L == 0) {
+            if (n_max) hipLaunchKernelGGL(juxtapose_kernel, by_point, dim3(256), 0, stream, B);
+            continue;
+        }
+        const dim3 slices((unsigned)(n_max / kScanTile + 1), 2 * (unsigned)cnt);
+        hipLaunchKernelGGL(invert_kernel, dim3((unsigned)((q_max + 255) / 256), (unsigned)cnt), dim3(256), 0, stream, B);
+        hipLaunchKernelGGL(slice_count_kernel, slices, dim3(kScanBlock), 0, stream, B);
+        hipLaunchKernelGGL(slice_scatter_kernel, slices, dim3(kScanBlock), 0, stream, B);
+        if (L < kBigMinL) {
+            hipLaunchKernelGGL(braid_core_lds_kernel, dim3((unsigned)cnt), dim3(kThreads), lds_core_bytes(L), stream, B);
+            continue;
+        }
+        BigBatch G{};
+        for (int c = 0; c < cnt; ++c) G.c[c] = B.m[c];
+        G.L = L;
+        G.L0 = big_leaf_L(L);
+        G.Y = big_layout(L, G.L0);
+        for (int d = 0; d < L - G.L0; ++d) G.D[d] = big_depth(L, d);
+        const int rc = launch_big(G, cnt, stream);
         if (rc) return rc;
-    }
-    for (int base = 0; base < count; base += kMulBatch) {
-        const int cnt = count - base < kMulBatch ? count - base : kMulBatch;
-        AssembleBatch ab{};
-        int blocks = 1;
-        for (int i = 0; i < cnt; ++i) {
-            const MulSpec &M = specs[base + i];
-            int32_t *map_row = M.ws + M.q_size, *map_col = map_row + M.k, *core = map_col + 3 * (size_t)M.k;
-            ab.a[i] = AssembleArgs{M.p, M.q, M.out, map_row, map_col, core, M.p_size, M.q_size, M.k, M.row_glue};
-            const int n = std::max(std::max(M.p_size, M.q_size), M.k);
-            blocks = std::max(blocks, (n + 255) / 256);
-        }
-        hipLaunchKernelGGL(assemble_kernel, dim3(blocks, cnt), dim3(256), 0, stream, ab);
     }
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
@@ -1404,7 +1266,9 @@ int lcsb_multiply_device(const int32_t *p, int32_t p_size, const int32_t *q, int
 
 size_t lcsb_multiply_ws_words(int32_t p_size, int32_t q_size, int32_t k)
 {
-    const int nmax = p_size > q_size ? p_size : q_size;
-    const size_t nblocks_max = (size_t)(nmax + kScanTile - 1) / kScanTile + 1;
-    return (size_t)q_size + 5 * (size_t)k + 2 * nblocks_max + lcsb_core_scratch_words(k > 0 ? k : 1);
+    MulArgs M{};
+    M.p_size = p_size;
+    M.q_size = q_size;
+    M.k = k;
+    return (size_t)q_size + 2 * (size_t)k + 2 * (size_t)M.blocks() + lcsb_core_scratch_words(k > 0 ? k : 1);
 }
