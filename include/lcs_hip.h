@@ -55,15 +55,17 @@ typedef struct lcs_schedule {
     int32_t tile_m;          /* rows per lane: 1, 2, 4, 8, 16 or 32          */
     int32_t waves_per_simd;  /* resident waves per SIMD the launch aims at   */
     int32_t variant;         /* LCS_VARIANT_*                                */
-    int32_t strips;          /* column strips merged by the steady ant       */
+    int32_t strips;          /* column strips merged by the steady ant; 0: a
+                                single pair is cut into the grid of rows and
+                                columns that is predicted fastest          */
 } lcs_schedule;
 
 #define LCS_VARIANT_AUTO 0
 #define LCS_VARIANT_CHAIN 1      /* wave64 band chain, registers only         */
-/* The register chain reads b as bytes when every symbol of b lies in
- * [0, 255] (checked on the device per call): each lane then holds its own
- * column symbols and none move between lanes.  The bytes are staged (two
- * small launches) for pairs of 2^22 cells or more, and at any size with
+/* The band chains read b as bytes when every symbol of b lies in [0, 255]
+ * (checked on the device per call): each lane then holds its own column
+ * symbols and none move between lanes.  Single pairs always stage the bytes;
+ * the server does for pairs of 2^22 cells or more, and at any size with
  * LCS_VARIANT_CHAIN_BYTES; the results are the same either way. */
 #define LCS_VARIANT_CHAIN_LDS 2  /* band chain, four bands linked through LDS */
 /* Batches only: pairs of a batch with this variant are combed two per wave
@@ -77,7 +79,7 @@ typedef struct lcs_schedule {
  * Elsewhere it means LCS_VARIANT_CHAIN. */
 #define LCS_VARIANT_PACKED16 3
 /* LCS_VARIANT_CHAIN with the byte symbols staged whatever the pair's size
- * (single pairs; in a batch it means LCS_VARIANT_CHAIN). */
+ * (served requests; elsewhere it means LCS_VARIANT_CHAIN). */
 #define LCS_VARIANT_CHAIN_BYTES 4
 
 /* ---- context ------------------------------------------------------------

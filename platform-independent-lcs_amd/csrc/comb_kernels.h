@@ -52,8 +52,9 @@ struct TileGrid {
 // window starts at byte x0 reads copy x0 % 4 from a word boundary.
 constexpr int32_t kSym8Pad = 128;
 // flags of a staged string: a symbol outside [0, 255]; a symbol 255, the
-// padding of the copies
-constexpr int32_t kSym8Bad = 1, kSym8Has255 = 2;
+// padding of the copies; bit 8 + i: the symbol -1 - i (i < 24), so that a
+// 32-bit chain can pad its rows with one of them that is absent
+constexpr int32_t kSym8Bad = 1, kSym8Has255 = 2, kSym8RowPads = 24;
 inline int32_t lcsk_sym8_stride(int32_t n) { return (int32_t)((((int64_t)n + 2 * kSym8Pad + 15) / 16) * 4); }
 // Writes the four copies of b into `out` (4 * stride words) and b's flags.
 int lcsk_launch_sym8(const int32_t *b, int32_t n, uint32_t *out, int32_t stride, int32_t *flags, hipStream_t stream);

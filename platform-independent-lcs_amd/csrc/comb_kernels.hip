@@ -455,7 +455,7 @@ constexpr int kSymWords = 0, kSymBytes = 1, kSymBytesPadded = 2;
 // as they are now, 0.85 (2 rows per lane: 1.18, 0.93, 0.73).
 template <int TM, int C, bool ROWMASK, bool PK, typename Desc, int S8 = kSymWords, bool OH = false, bool LK = false>
 __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int g, int lane, int t_id,
-                                          const BandLink &K = BandLink{})
+                                          const BandLink &K = BandLink{}, int32_t row_pad = 0)
 {
     static_assert(!LK || (!PK && C == 32), "linked bands");
     constexpr bool PAD = PK || S8 == kSymBytesPadded || (!S8 && !ROWMASK);
@@ -492,8 +492,10 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
             if (S8 == kSymBytesPadded && a[k] == 255) a[k] = -1;   // b holds no 255
             h[k] = valid[k] ? (P.h_in ? (uint32_t)P.h_in[m - 1 - r] : (uint32_t)(m - 1 - r)) : 0u;
         } else {
-            valid[k] = ROWMASK ? (r < m) : true;
-            a[k] = valid[k] ? P.a[r] : 0;
+            // rows past m: masked, or (row_pad) a symbol that b does not hold and
+            // strand 0, as in the byte chain
+            valid[k] = r < m;
+            a[k] = valid[k] ? P.a[r] : row_pad;
             h[k] = valid[k] ? (P.h_in ? (uint32_t)P.h_in[m - 1 - r] : (uint32_t)(m - 1 - r)) : 0u;
         }
     }
@@ -767,9 +769,10 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
 }
 
 // One band of a pair, by what its column symbols are: bytes when the pair has
-// byte copies and all of b fits in a byte (they pad a partial band's rows
-// instead of masking them), else 32-bit words, masked in the band that has
-// rows past m (only a pair's last one does).
+// byte copies and all of b fits in a byte, else 32-bit words.  A partial band
+// (only a pair's last one) pads its rows; 32-bit words without a known absent
+// symbol mask them, and as the chain's last band that one sets the pace of
+// the whole launch.
 template <int TM, int C, bool LK>
 __device__ __forceinline__ bool band_dispatch(const ChainArgs &A, const PairDesc &P, int g, int lane, int t_id,
                                               const BandLink &K)
@@ -780,9 +783,12 @@ __device__ __forceinline__ bool band_dispatch(const ChainArgs &A, const PairDesc
             return band_pass<TM, C, false, false, PairDesc, kSymBytesPadded, false, LK>(A, P, g, lane, t_id, K);
         return band_pass<TM, C, false, false, PairDesc, kSymBytes, false, LK>(A, P, g, lane, t_id, K);
     }
-    const bool rowmask = (long long)(g + 1) * (kWave * TM) > (long long)P.m;
+    // rows past m take a symbol that b does not hold, when the flags know one
+    const uint32_t absent = P.sym8 ? ~(uint32_t)flags >> 8 : 0u;
+    const bool rowmask = (long long)(g + 1) * (kWave * TM) > (long long)P.m && absent == 0;
+    const int32_t row_pad = absent ? -1 - (int32_t)__builtin_ctz(absent) : 0;
     return rowmask ? band_pass<TM, C, true, false, PairDesc, kSymWords, false, LK>(A, P, g, lane, t_id, K)
-                   : band_pass<TM, C, false, false, PairDesc, kSymWords, false, LK>(A, P, g, lane, t_id, K);
+                   : band_pass<TM, C, false, false, PairDesc, kSymWords, false, LK>(A, P, g, lane, t_id, K, row_pad);
 }
 
 // Tile p of a grid as a pair of its own.
@@ -921,6 +927,7 @@ __device__ __forceinline__ void stage_sym8(const int32_t *b, int32_t ns, uint32_
             if (c >= 0 && c < ns) {
                 sym = (uint32_t)b[c];
                 seen |= sym > 255u ? kSym8Bad : sym == 255u ? kSym8Has255 : 0;
+                if (~sym < (uint32_t)kSym8RowPads) seen |= 0x100 << ~sym;
             }
             word |= (sym & 0xffu) << (8 * i);
         }

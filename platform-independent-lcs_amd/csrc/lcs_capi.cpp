@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -53,37 +54,7 @@ void DevBuf::release(lcs_ctx *ctx)
     bytes = 0;
 }
 
-// Default tile height: the largest power of two <= 16 that still gives every
-// SIMD of the device at least one band of 64*tile_m rows.
-int default_tile_m(const lcs_ctx *ctx, int32_t m)
-{
-    const long long simds = 4LL * ctx->num_cus;
-    int tm = 16;
-    while (tm > 1 && (long long)m < simds * 64LL * tm) tm >>= 1;
-    return tm;
-}
-
 bool valid_tile_m(int tm) { return tm == 1 || tm == 2 || tm == 4 || tm == 8 || tm == 16 || tm == 32; }
-
-// One strip whose bands cannot fill the SIMDs at one row per lane (m below
-// 64 rows per SIMD): the launch is the pipeline fill, (bands - 1) lags, plus
-// one band's sweep of n columns, so taller bands pay off unless the pair is
-// wide.  Measured on MI355X (one strip, byte symbols, m = 1024 .. 32768):
-// 4 rows per lane is fastest for n < 1.4 m (m = n = 4096: 0.301 ms against
-// 0.343 at one row, 0.321 at two), two rows between 1.4 m and 1.7 m by the
-// fitted per-height costs, and one row from n = 1.7 m (n = 4m: one row
-// 0.511 ms, four 0.722).  Taller bands are taken only where no partial band
-// would need the masked 32-bit loop (byte symbols pad their partial bands).
-int small_pair_tile_m(int variant, int32_t m, int32_t n)
-{
-    if (m < 1024) return 1;
-    const bool bytes = (variant == LCS_VARIANT_AUTO || variant == LCS_VARIANT_CHAIN ||
-                        variant == LCS_VARIANT_CHAIN_BYTES) && use_sym8(variant, m, n);
-    const long long n10 = 10LL * n;
-    if (n10 < 14LL * m && (bytes || m % 256 == 0)) return 4;
-    if (n10 < 17LL * m && (bytes || m % 128 == 0)) return 2;
-    return 1;
-}
 
 int32_t bands_of(int32_t m, int32_t n, int tm)
 {
@@ -310,71 +281,56 @@ int launch_prepared(const PreparedLaunch &L, hipStream_t stream)
     return lcsk_launch_chain(L.args, L.args.pairs, L.npairs, L.max_n, L.tile_m, L.blocks, L.threads, stream);
 }
 
-// Strips a single pair is cut into.  A thin pair (m <= kDefaultStripMaxM)
-// whose bands alone would leave SIMDs idle is cut until the strips' bands
-// fill them.  A tall pair whose bands already fill every SIMD is cut when it
-// is wide: the persistent waves then comb each strip's lower bands as later
-// rounds, so the chain's fill (one band-to-band lag per band before the
-// last band starts) is paid for a fraction of the bands, at the price of
-// whole-GPU steady-ant merges with k = m (S - 1 of them).  At m = n = 2^20
-// (the same kernels, same box): one strip 145.0 ms, two 138.0 (chain 136.0
-// + merge 2.0), four 136.7 (131.6 + 5.1), eight 140.3 (129.3 + 11.0).
-constexpr int32_t kDefaultStripMaxM = 32768;
-constexpr double kLargeThinCells = 34359738368.0;   // 2^35
-constexpr int32_t kTallStripMinN = 1 << 18;    // two strips from here
-constexpr int32_t kTallStrip4MinN = 1 << 20;   // four strips from here
-int default_strips(const lcs_ctx *ctx, int32_t m, int32_t n, int tm)
-{
-    const long long simds = 4LL * ctx->num_cus;
-    const long long bands = bands_of(m, n, tm);
-    if (m > kDefaultStripMaxM) {
-        if (m > kMaxCoreK || bands < simds || n < kTallStripMinN) return 1;
-        return n >= kTallStrip4MinN ? 4 : 2;
-    }
-    if (n < 2 * 8192) return 1;
-    int s = 1;
-    while ((long long)s * bands < simds && s < 64 && (long long)n / (2 * s) >= 8192) s *= 2;
-    return s;
-}
-
-// Byte symbols for the register chain (lcsk_launch_sym8): the pairs, all
-// reading columns of the one string d_b (pair p from column col0[p]), get
-// the byte copies of d_b; a chain band then takes each lane's symbols from
-// them when every symbol of d_b lies in [0, 255] (which the conversion
-// kernel finds out on the device) and from d_b otherwise.  A b longer than
-// kSym8MaxN, or a context whose budget cannot hold the 4(n + 256) bytes,
-// keeps the 32-bit symbols.  The staging is two small launches (about 8 us
-// of device time at n = 16384); a pair below kSym8MinCells cells, whose
-// comb that would not repay it, skips it unless its schedule asks for
-// LCS_VARIANT_CHAIN_BYTES.  Besides the per-step saving, bytes let a
-// partial last band (m not a multiple of 64 * tile_m) pad its rows and run
-// the unmasked loop, where with 32-bit symbols it masks every cell and, as
-// the chain's last band, sets the pace of the whole launch (TM=1,
-// n = 103691: m = 1387 took 2.75 ms against 2.14 for the full-band
-// m = 1408; with bytes 1.84).
-#ifndef LCS_SYM8
-#define LCS_SYM8 1
-#endif
+// Byte symbols: a chain band takes each lane's column symbols from byte copies
+// of b when every symbol of b lies in [0, 255] (which the staging finds out on
+// the device), and pads the rows of a partial band with a symbol that b does
+// not hold.  A single pair's copies are written by the launch's seeding
+// kernel, whatever its size; a b longer than kSym8MaxN, or a context whose
+// budget cannot hold them, keeps the 32-bit symbols.  The server stages them
+// in two launches of their own (about 8 us of device time at n = 16384), which
+// pays from kSym8MinCells cells.
 constexpr int32_t kSym8MaxN = 1 << 30;
 constexpr double kSym8MinCells = 4194304.0;   // 2^22
 bool use_sym8(int variant, int32_t m, int32_t n)
 {
-    if (!LCS_SYM8 || n <= 0 || n > kSym8MaxN) return false;
+    if (n <= 0 || n > kSym8MaxN) return false;
     return variant == LCS_VARIANT_CHAIN_BYTES || (double)m * (double)n >= kSym8MinCells;
 }
-// How one pair is cut and combed.
+
+// How one pair is cut and combed: GR x GC tiles of tm rows per lane.
 struct GridPlan {
     int32_t tm, wps, group_w, GR, GC;
-    bool sym8;
 };
 
-// Words of one merge workspace (the largest product of the tree).
-static size_t grid_merge_ws(int32_t m, int32_t n, const GridPlan &G)
+// The merge tree over a grid of tiles: every level joins neighbours along the
+// shorter side of the current tiles (two tiles side by side glue on their
+// common rows, one above the other on their common columns).
+// level(products, k, p_size) sees each level with its largest product.
+template <typename Level>
+static void merge_levels(int32_t m, int32_t n, int32_t GR, int32_t GC, Level level)
 {
-    size_t w = 0;
-    if (G.GC > 1) w = std::max(w, lcsb_multiply_ws_words(m + n, m + n, m));
-    if (G.GR > 1) w = std::max(w, lcsb_multiply_ws_words(m + n, m + n, n));
-    return w;
+    int32_t gr = GR, gc = GC, h = (m + GR - 1) / GR, w = (n + GC - 1) / GC;
+    while (gr * gc > 1) {
+        const bool side = gc > 1 && (gr == 1 || h <= w);
+        level(side ? gr * (gc / 2) : gc * (gr / 2), side ? h : w, h + w);
+        if (side) {
+            gc = (gc + 1) / 2;
+            w = std::min(n, 2 * w);
+        } else {
+            gr = (gr + 1) / 2;
+            h = std::min(m, 2 * h);
+        }
+    }
+}
+
+// Words of the merge workspaces (the level that needs most).
+static size_t grid_merge_words(int32_t m, int32_t n, const GridPlan &G)
+{
+    size_t most = 0;
+    merge_levels(m, n, G.GR, G.GC, [&](int32_t products, int32_t k, int32_t size) {
+        most = std::max(most, (size_t)products * lcsb_multiply_ws_words(size, size, k));
+    });
+    return most;
 }
 
 // Words of the tiles' permutations: every tile row holds its rows once per
@@ -384,12 +340,75 @@ static size_t grid_perm_words(int32_t m, int32_t n, const GridPlan &G)
     return (size_t)G.GC * m + (size_t)G.GR * n;
 }
 
-// Merges the tiles' permutations to the whole pair's and writes its strands.
-// Every level joins neighbours along the shorter side of the current tiles
-// (two tiles side by side glue on their common rows, one above the other on
-// their common columns), all its products in one launch sequence.
-static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_t *ws, size_t ws_words, int32_t *d_h,
-                       int32_t *d_v, hipStream_t stream)
+// Predicted microseconds of a plan.  The chain: one wave per band and SIMD; a
+// band starts kLagSteps steps after the one above it (64 of lane skew, a chunk
+// of 32 published, a chunk prefetched) and takes W + 64 steps of kStepNs[tm];
+// bands beyond the SIMDs run in further rounds.  Measured on MI355X, one
+// strip, byte symbols (m = 64 tm bands, n = 65536): 12.9 / 21.4 / 33.3 /
+// 61.4 / 114.4 ns a step at 1 / 2 / 4 / 8 / 16 rows per lane (one row: 17.4
+// from 16 bands, where the ring word's trip takes longer than a chunk) and
+// 130 to 138 steps from band to band.  The merges: a level's products share
+// its launches, about 60 us for a core of 2^11 points plus 8 per doubling, and
+// about 0.6 ns per point (k = 2^16 155 us, 2^18 285, eight of 2^16 390).
+// Checked against the whole grid of plans at 2^14, 50021 x 70207, 2^16,
+// 200000 and 2^18: the chain within 8 %, the plan it picks within 3 % of the
+// best one measured (200000^2: 20 tiles of 16 rows 7.1 ms, one 10.6).
+constexpr double kLagSteps = 130.0;
+static double plan_us(const lcs_ctx *ctx, int32_t m, int32_t n, const GridPlan &G)
+{
+    const int32_t H = (m + G.GR - 1) / G.GR, W = (n + G.GC - 1) / G.GC, tiles = G.GR * G.GC;
+    const double bands = bands_of(H, W, G.tm), waves = bands * tiles, simds = 4.0 * ctx->num_cus * G.wps;
+    const double step_ns = G.tm == 1   ? (bands * tiles < 16 ? 12.9 : 17.4)
+                           : G.tm == 2 ? 21.4
+                           : G.tm == 4 ? 33.3
+                           : G.tm == 8 ? 61.4
+                                       : 114.4 / 16 * G.tm;
+    const double rounds = std::ceil(waves / simds), last = std::fmod(waves - 1, simds) / tiles;
+    const double steps = std::max(rounds * (W + 64.0) + last * kLagSteps, W + 64.0 + (bands - 1) * kLagSteps);
+    double us = steps * step_ns * 1e-3;
+    merge_levels(m, n, G.GR, G.GC, [&](int32_t products, int32_t k, int32_t) {
+        const int L = std::max(6, lcsb_core_L(k));
+        us += 60.0 + 8.0 * std::max(0, L - 11) + 0.6e-3 * products * (double)(1LL << L);
+    });
+    return us + (tiles > 1 ? 10.0 : 0.0);
+}
+
+// The plan of a pair: the cheapest predicted one with the fields that the
+// schedule fixes (tm, strips; 0 = open).  A pair below kGridMinCells cells, or
+// one with explicit strands, is one tile.
+constexpr double kGridMinCells = 67108864.0;   // 2^26: below it no merge pays (8192^2 0.36 ms as one tile)
+static GridPlan choose_grid(const lcs_ctx *ctx, int32_t m, int32_t n, int tm, int strips, bool whole, GridPlan G)
+{
+    static const int32_t kCols[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64}, kRows[] = {1, 2, 3, 4, 6, 8};
+    const bool open = !whole && !strips && (double)m * n >= kGridMinCells;
+    double best = 0.0;
+    GridPlan B = G;
+    B.tm = 0;
+    for (int32_t t = 1; t <= 16; t *= 2) {
+        if (tm && t != (tm < 16 ? tm : 16)) continue;
+        for (const int32_t r : kRows) {
+            if (r > 1 && (!open || m / r < 2048 || n > kMaxCoreK)) break;
+            for (int32_t c : kCols) {
+                if (c > 1 && (!open || n / c < 2048 || m > kMaxCoreK)) break;
+                GridPlan T = G;
+                T.tm = tm ? tm : t;
+                T.GR = r;
+                T.GC = strips ? strips : c;
+                const double us = plan_us(ctx, m, n, T);
+                if (!B.tm || us < best) {
+                    best = us;
+                    B = T;
+                }
+            }
+        }
+    }
+    return B;
+}
+
+// Merges the tiles' permutations to the whole pair's and writes its strands,
+// all products of a level (merge_levels) in one launch sequence.
+static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_t *ws, int32_t *d_h, int32_t *d_v,
+                       hipStream_t stream)
 {
     const int32_t m = T.pair.m, n = T.pair.n;
     struct Tile {
@@ -402,7 +421,8 @@ static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_
         for (int32_t j = 0; j < gc; ++j) cur[(size_t)i * gc + j] = Tile{permA + T.perm_off(i, j), T.rows(i), T.cols(j)};
     int32_t *dst_base = permB;
     while (gr * gc > 1) {
-        const bool side = gc > 1 && (gr == 1 || cur[0].m <= cur[0].n);   // glue columns of tiles (on rows) or rows
+        const bool side = gc > 1 && (gr == 1 || cur[0].m <= cur[0].n);
+        int32_t *next_ws = ws;
         const int32_t nr = side ? gr : (gr + 1) / 2, nc = side ? (gc + 1) / 2 : gc;
         std::vector<Tile> nxt((size_t)nr * nc);
         std::vector<MulSpec> specs;
@@ -414,8 +434,9 @@ static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_
                 o = Tile{dst, p.m, p.n};
                 if (side ? 2 * j + 1 < gc : 2 * i + 1 < gr) {
                     const Tile &q = side ? cur[(size_t)i * gc + 2 * j + 1] : cur[(size_t)(2 * i + 1) * gc + j];
-                    specs.push_back(MulSpec{p.p, p.m + p.n, q.p, q.m + q.n, side ? p.m : p.n, side ? 0 : 1, dst,
-                                            ws + specs.size() * ws_words});
+                    const int32_t k = side ? p.m : p.n;
+                    specs.push_back(MulSpec{p.p, p.m + p.n, q.p, q.m + q.n, k, side ? 0 : 1, dst, next_ws});
+                    next_ws += lcsb_multiply_ws_words(p.m + p.n, q.m + q.n, k);
                     if (side) o.n += q.n;
                     else o.m += q.m;
                 } else if (lcsk_launch_copy(dst, p.p, (long long)p.m + p.n, stream)) {
@@ -450,7 +471,7 @@ static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, hipStrea
     int rc = ctx->ring.reserve(ctx, (size_t)tiles * lcsk_ring_words(T.W) * sizeof(unsigned long long));
     if (rc) return rc;
     T.pair.E = (unsigned long long *)ctx->ring.ptr;
-    if (G.sym8) {
+    if (n <= kSym8MaxN) {
         const int32_t stride = lcsk_sym8_stride(T.W);
         if (ctx->sym8.reserve(ctx, (size_t)T.GC * 16 * (size_t)stride) == LCS_OK) {
             T.pair.sym8 = (const uint32_t *)ctx->sym8.ptr;
@@ -459,14 +480,11 @@ static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, hipStrea
             T.pair.sym8_flags = T.sym8_flags;
         }
     }
-    size_t perm_words = 0, ws_words = 0;
-    int32_t *ws = nullptr;
+    size_t perm_words = 0;
     if (tiles > 1) {
         perm_words = grid_perm_words(m, n, G);
-        ws_words = grid_merge_ws(m, n, G);
-        if ((rc = ctx->strip_ws.reserve(ctx, (2 * perm_words + (size_t)(tiles / 2) * ws_words) * 4))) return rc;
+        if ((rc = ctx->strip_ws.reserve(ctx, (2 * perm_words + grid_merge_words(m, n, G)) * 4))) return rc;
         T.perm = (int32_t *)ctx->strip_ws.ptr;
-        ws = T.perm + 2 * perm_words;
     }
     ChainArgs A{};
     const long long units = (T.pair.nbands + G.group_w - 1) / G.group_w * (long long)tiles;
@@ -487,7 +505,7 @@ static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, hipStrea
     if (hipEventRecord(ctx->evc1, stream) != hipSuccess) return LCS_EIO;
     ctx->chain_timed = true;
     if (tiles == 1) return LCS_OK;
-    return merge_tiles(T, T.perm, T.perm + perm_words, ws, ws_words, pair.h_out, pair.v_out, stream);
+    return merge_tiles(T, T.perm, T.perm + perm_words, T.perm + 2 * perm_words, pair.h_out, pair.v_out, stream);
 }
 
 int ws_acquire(lcs_ctx *ctx, hipStream_t s)
@@ -541,31 +559,10 @@ static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const i
     if (strips_req < 0) return LCS_EINVAL;
     const int group_w = group_width(sched ? sched->variant : LCS_VARIANT_AUTO);
     if (!group_w) return LCS_EINVAL;
-    if (!tm) {
-        tm = default_tile_m(ctx, m);
-        if (strips_req != 1 && !d_h_in && !d_v_in && tm < 4 && default_strips(ctx, m, n, 4) > 1) {
-            // a thin pair cut into strips: 16 rows per lane for a large pair
-            // (2^35 cells or more) when at most 64 strips of such bands fill
-            // every SIMD -- on the Zipf pair (m = 2^14, n = 2^22) 64 strips of
-            // 16 rows took 10.64 ms against 10.91 for 32 strips of 8 rows: the
-            // chain's 0.9 ms outweighs a sixth merge level; else 8 rows when
-            // at most 32 strips of them fill every SIMD (fewer merge levels
-            // than with 4 rows per lane would cost), else 4
-            const long long simds = 4LL * ctx->num_cus;
-            const int s16 = default_strips(ctx, m, n, 16), s8 = default_strips(ctx, m, n, 8);
-            if ((double)m * n >= kLargeThinCells && s16 <= 64 && (long long)s16 * bands_of(m, n, 16) >= simds)
-                tm = 16;
-            else
-                tm = (s8 <= 32 && (long long)s8 * bands_of(m, n, 8) >= simds) ? 8 : 4;
-        } else if (tm == 1) {
-            tm = small_pair_tile_m(sched ? sched->variant : LCS_VARIANT_AUTO, m, n);
-        }
-    }
-    int strips = strips_req ? strips_req : ((d_h_in || d_v_in) ? 1 : default_strips(ctx, m, n, tm));
-    if (strips > 1 && (d_h_in || d_v_in)) return LCS_EINVAL;  // fixups use explicit strands: one strip
-    if (strips > 1 && m > kMaxCoreK) return LCS_ERANGE;
-    if (strips > n) strips = n;
-    GridPlan G{tm, wps, group_w, 1, strips, use_sym8(sched ? sched->variant : LCS_VARIANT_AUTO, m, n)};
+    const bool whole = d_h_in || d_v_in;   // fixups use explicit strands: one tile
+    if (strips_req > 1 && whole) return LCS_EINVAL;
+    if (strips_req > 1 && m > kMaxCoreK) return LCS_ERANGE;
+    const GridPlan G = choose_grid(ctx, m, n, tm, std::min(strips_req, n), whole, GridPlan{0, wps, group_w, 1, 1});
     PairDesc P{};
     P.a = d_a;
     P.b = d_b;
@@ -575,7 +572,11 @@ static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const i
     P.v_out = d_v;
     P.m = m;
     P.n = n;
-    return enqueue_grid(ctx, P, G, stream);
+    const int rc = enqueue_grid(ctx, P, G, stream);
+    if (rc != LCS_ENOMEM || strips_req || G.GR * G.GC == 1) return rc;
+    // the budget cannot hold the library's own cut (its workspaces are reserved
+    // before anything is launched): one tile
+    return enqueue_grid(ctx, P, choose_grid(ctx, m, n, tm, 1, whole, G), stream);
 }
 
 // The abort flag of the last launch on the context's own ctrl words (the
