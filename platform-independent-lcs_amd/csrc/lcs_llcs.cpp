@@ -20,20 +20,23 @@ struct LlcsPair {
     int32_t *out;           // device int32
 };
 
-// Steps from the first band's start to the last band's end: a band lags the
-// one below by about kLag steps (63 of skew, two chunks of hand-off, the
-// fetch round trip), and bands beyond the resident ones run in later rounds.
-constexpr double kLag = 160.0;
-
-double pipeline_steps(int64_t rows, int64_t cols, int64_t resident)
+// Microseconds from the first band's start to the last band's end with blocks
+// of B columns: a band lags the one below by 64 blocks of skew, the chunk that
+// a carry word fills, two chunks of prefetch and the word's trip (measured 390
+// columns at 4, 260 at 2), and bands beyond the resident ones run in later
+// rounds.  A column takes 15.0 ns at 4 and 17.0 at 2.
+double pipeline_us(int64_t rows, int64_t cols, int64_t resident, int B)
 {
     const int64_t bands = (rows + lcsl::kBandRows - 1) / lcsl::kBandRows;
     const int64_t rounds = (bands + resident - 1) / std::max<int64_t>(resident, 1);
-    return (double)rounds * (double)(cols + lcsl::kWave - 1) + (double)bands * kLag;
+    return ((double)rounds * ((double)cols + lcsl::kWave * B) + (double)bands * (130.0 + 65.0 * B)) *
+           (B == 4 ? 0.0150 : 0.0170);
 }
 
-// bands in flight: a band is a workgroup of two waves (comb + fetch), four per CU
-int resident_bands(const lcs_ctx *ctx) { return 4 * ctx->num_cus; }
+// LDS of a CU, and the bands it holds at once: one per SIMD, fewer when the
+// match-mask tables fill the LDS
+constexpr int kCuLdsBytes = 160 * 1024;
+int bands_per_cu(int sigma) { return (int)std::min<size_t>(4, kCuLdsBytes / lcsl::llcs_lds_bytes(sigma)); }
 
 // Enqueues one launch over `pairs` on `s`: the longer-pipelined orientation
 // is chosen per pair (LCS is symmetric).  Rings and descriptors live in the
@@ -53,43 +56,55 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
 {
     const int np = (int)pairs.size();
     if (np == 0) return LCS_OK;
-    const int64_t resident = resident_bands(ctx);
+    const int64_t resident = (int64_t)ctx->num_cus * bands_per_cu(sigma);
     std::vector<lcsl::LlcsDesc> descs((size_t)np);
-    size_t ring_words = 0;
-    int max_ring = 0;
+    size_t ring_words = 0, code_bytes = 0;
+    int max_words = 0;
+    double us[2] = {0.0, 0.0};   // blocks of 4, of 2: the slowest pair
+    int64_t all_bands = 0;
     for (int p = 0; p < np; ++p) {
         const LlcsPair &P = pairs[(size_t)p];
-        const bool swap = pipeline_steps(P.n, P.m, resident) < pipeline_steps(P.m, P.n, resident);
+        const bool swap = std::min(pipeline_us(P.n, P.m, resident, 4), pipeline_us(P.n, P.m, resident, 2)) <
+                          std::min(pipeline_us(P.m, P.n, resident, 4), pipeline_us(P.m, P.n, resident, 2));
         lcsl::LlcsDesc &D = descs[(size_t)p];
         D = lcsl::LlcsDesc{};
         D.rows = swap ? P.b : P.a;
         D.cols = swap ? P.a : P.b;
         D.nrows = swap ? P.n : P.m;
         D.ncols = swap ? P.m : P.n;
-        // the band loop counts columns up to ncols + 3 chunks in int
+        // the widest b of the ABI; the band loop itself counts chunks
         if (D.ncols > 0x7fffffff - 4096) return LCS_ERANGE;
         D.nbands = lcsl::llcs_nbands(D.nrows);
-        D.nchunks = lcsl::llcs_nchunks(D.ncols);
+        D.nwords = lcsl::llcs_nwords(D.ncols);
+        us[0] = std::max(us[0], pipeline_us(D.nrows, D.ncols, resident, 4));
+        us[1] = std::max(us[1], pipeline_us(D.nrows, D.ncols, resident, 2));
+        all_bands += D.nbands;
         D.out = P.out;
-        ring_words += 2 * (size_t)D.nchunks;
-        max_ring = std::max(max_ring, 2 * D.nchunks);
+        ring_words += 2 * ((size_t)D.nwords + lcsl::kSpare);
+        code_bytes += lcsl::llcs_code_bytes(D.ncols, sigma);
+        max_words = std::max(max_words, D.nwords);
     }
     int rc = ctx->ring.reserve(ctx, ring_words * sizeof(unsigned long long));
+    if (!rc) rc = ctx->sym8.reserve(ctx, code_bytes);
     if (rc) return rc;
     std::vector<int2> tasks;
     for (int p = 0; p < np; ++p)
         for (int32_t g = 0; g < descs[(size_t)p].nbands; ++g) tasks.push_back(make_int2(p, g));
     const size_t desc_bytes = sizeof(lcsl::LlcsDesc) * (size_t)np, task_bytes = sizeof(int2) * tasks.size();
+    // the error words travel with the descriptors, as zeros
     const size_t err_off = (desc_bytes + task_bytes + 255) / 256 * 256;
     if ((rc = ctx->descs.reserve(ctx, err_off + 4 * (size_t)np + 256))) return rc;
+    uint8_t *codes = (uint8_t *)ctx->sym8.ptr;
     unsigned long long *ring = (unsigned long long *)ctx->ring.ptr;
     int32_t *err = (int32_t *)((unsigned char *)ctx->descs.ptr + err_off);
     for (int p = 0; p < np; ++p) {
         descs[(size_t)p].ring = ring;
-        ring += 2 * (size_t)descs[(size_t)p].nchunks;
+        ring += 2 * ((size_t)descs[(size_t)p].nwords + lcsl::kSpare);
+        descs[(size_t)p].codes = codes;
+        codes += lcsl::llcs_code_bytes(descs[(size_t)p].ncols, sigma);
         descs[(size_t)p].err = err + p;
     }
-    std::vector<unsigned char> blob(desc_bytes + task_bytes);
+    std::vector<unsigned char> blob(err_off + 4 * (size_t)np, 0);
     std::memcpy(blob.data(), descs.data(), desc_bytes);
     if (task_bytes) std::memcpy(blob.data() + desc_bytes, tasks.data(), task_bytes);
     if ((rc = upload(ctx, ctx->descs.ptr, blob.data(), blob.size(), s))) return rc;
@@ -104,8 +119,14 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
     A.timeout_ticks = ctx->timeout_ticks;
     A.trace = ctx->band_trace;
     A.trace_cap = ctx->band_trace_cap;
+    // more bands than SIMDs over several pairs: the time per column counts
+    A.block = us[1] < us[0] && (np == 1 || all_bands <= resident) ? 2 : 4;
     const int blocks = (int)std::min<int64_t>((int64_t)tasks.size(), resident);
-    return lcsl_launch(A, A.descs, np, max_ring, blocks, s) == 0 ? LCS_OK : LCS_EIO;
+    // as much LDS per band as leaves each CU its share of them: the dispatcher
+    // then spreads the bands over the CUs, and a band has its SIMD to itself
+    const int share = std::max(1, (blocks + ctx->num_cus - 1) / ctx->num_cus);
+    const int lds = std::max((int)lcsl::llcs_lds_bytes(sigma), kCuLdsBytes / share / 512 * 512);
+    return lcsl_launch(A, A.descs, np, max_words, blocks, lds, s) == 0 ? LCS_OK : LCS_EIO;
 }
 
 bool valid_sigma(int32_t sigma) { return sigma >= 1 && sigma <= lcsl::kMaxSigma; }

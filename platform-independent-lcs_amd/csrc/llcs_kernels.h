@@ -8,26 +8,51 @@ namespace lcsl {
 constexpr int kWave = 64;
 constexpr int kWordRows = 32;                    // rows of the row string per lane
 constexpr int kBandRows = kWave * kWordRows;     // 2048 rows per band (one wave)
-constexpr int kChunk = 32;                       // steps per chunk = bits per ring word
-constexpr int kMaxSigma = 200;              // table, staging and rings stay under 64 KiB of LDS
+constexpr int kChunk = 32;                       // columns per carry word
+constexpr int kMaxBlock = 4;                     // columns a lane takes per turn: 4 or 2
+constexpr int kMaxSigma = 200;                   // one table row per symbol, 51 KB of LDS
+// Up to this alphabet a table row serves two columns: (sigma + 1)^2 rows of
+// 512 bytes, lanes 0 .. 31 in one half of the table and 32 .. 63 in the other,
+// 128 rows of 256 bytes on (58 KB at 9).
+constexpr int kMaxPairSigma = 9;
 
 // One LCS-length problem: `rows` (nrows symbols) is cut into bands of 2048
 // rows, one 32-bit word per lane; `cols` (ncols symbols) streams through the
-// band.  Band g reads the carry words of band g-1 from ring slot g&1 (tag g)
-// and writes its own to slot (g+1)&1 (tag g+1).
+// band as codes.  Band g reads the carry words of band g-1 from ring slot g&1
+// (tag g) and writes its own to slot (g+1)&1; the seeding kernel fills slot 0
+// with empty words of tag 0 for band 0.  A slot has nwords words and kSpare
+// that the last prefetches read.
+constexpr int kSpare = 24;
 struct LlcsDesc {
     const int32_t *rows;
     const int32_t *cols;
-    int32_t nrows, ncols, nbands, nchunks;
-    unsigned long long *ring;    // 2 * nchunks words (tag << 32 | 32 carry bits)
+    int32_t nrows, ncols, nbands, nwords;
+    unsigned long long *ring;    // 2 * (nwords + kSpare) words (tag << 32 | 32 carry bits)
+    uint8_t *codes;              // llcs_code_bytes(ncols, sigma), 16-byte aligned
     int32_t *out;                // LCS length (zeroed by the prep kernel); -1 on a symbol outside [0, sigma)
-    int32_t *err;                // set to 1 on a symbol outside [0, sigma)
+    int32_t *err;                // zero before the launch; set on a symbol outside [0, sigma)
 };
 
 inline int32_t llcs_nbands(int32_t nrows) { return (int32_t)(((int64_t)nrows + kBandRows - 1) / kBandRows); }
-// Chunks a band runs: lane 63 takes the last symbol at step ncols+62 and its
-// carry-out is collected one step later, in word (ncols-1)/32 + 2.
-inline int32_t llcs_nchunks(int32_t ncols) { return ncols > 0 ? (ncols - 1) / kChunk + 3 : 0; }
+inline int32_t llcs_nwords(int32_t ncols) { return ncols > 0 ? (ncols - 1) / kChunk + 1 : 0; }
+// Chunks between the column word q of a band and the one in which it is whole:
+// with blocks of B columns a chunk has 32 / B turns and lane 63 takes block b
+// in turn b + 63, so word q is whole after the last turn but one of chunk q +
+// word_lag(B).
+__host__ __device__ constexpr int word_lag(int B) { return kWave * B / kChunk; }
+__host__ __device__ inline bool llcs_pairs(int sigma) { return sigma <= kMaxPairSigma; }
+// Codes: 64 blocks of padding (lane 63 starts 63 blocks back), the string, and
+// padding up to the last prefetch (three chunks past the last, in steps of
+// six); a byte per column, or per two.
+constexpr int kFrontPad = kWave * kMaxBlock;   // columns
+__host__ __device__ inline int64_t llcs_code_columns(int32_t nwords)
+{
+    return kFrontPad + (int64_t)kChunk * (nwords + word_lag(kMaxBlock) + 10);
+}
+inline size_t llcs_code_bytes(int32_t ncols, int sigma)
+{
+    return ((size_t)llcs_code_columns(llcs_nwords(ncols)) / (llcs_pairs(sigma) ? 2 : 1) + 31) & ~(size_t)15;
+}
 
 struct LlcsArgs {
     const LlcsDesc *descs;
@@ -39,21 +64,20 @@ struct LlcsArgs {
     unsigned long long timeout_ticks;
     unsigned long long *trace;   // nullable: [2t] start, [2t+1] end of task t (realtime ticks)
     int32_t trace_cap;
-    int32_t pad;
+    int32_t block;               // columns per turn, 4 or 2
     unsigned *sticky;            // nullable: the prep kernel ORs the abort flag into it before clearing it
 };
 
-constexpr int kLdsSymRing = 2048, kLdsInRing = 128;
-// LDS: two buffers of 96 staged addresses, one all-zero row (padding
-// symbols), sigma rows, the symbol and carry-in rings, 16 control words
+// LDS of one band: the match-mask table, a zero row for the padding included
 inline size_t llcs_lds_bytes(int sigma)
 {
-    return (size_t)(2 * 96 + kWave + sigma * kWave + kLdsSymRing + kLdsInRing + 16) * 4;
+    return llcs_pairs(sigma) ? (size_t)32768 + (size_t)(sigma + 1) * (sigma + 1) * 256 : (size_t)(sigma + 1) * 256;
 }
 
 }  // namespace lcsl
 
-// Clears outputs, error words, ticket and abort flag and invalidates every
-// ring word; runs the band chain; marks pairs with a bad symbol (-1).
-int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int npairs, int max_ring_words,
-                int grid_blocks, hipStream_t stream);
+// Clears outputs, ticket and abort flag, invalidates every ring word and
+// writes the codes; runs the band chain (lds_bytes >= llcs_lds_bytes(sigma)
+// per workgroup); marks pairs with a bad symbol (-1).
+int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int npairs, int max_words,
+                int grid_blocks, int lds_bytes, hipStream_t stream);

@@ -10,32 +10,44 @@
 // row i to row i+1, which is the only coupling between rows.
 //
 // MI355X mapping: one wave64 per band of 2048 rows, one 32-bit word of V per
-// lane (rows 32l..32l+31 of the band).  Lanes are skewed like the seaweed
-// band chain: lane l takes column symbol k-l at step k, so the carry leaving
-// lane l-1 at step k-1 is the carry entering lane l at step k.  Carries live
-// as a 64-bit lane mask in SGPRs: one v_addc_co_u32 per step takes the
-// shifted mask as carry-in and writes the new carry-out mask, and the shift
-// and the band's own carry-in/carry-out bits are scalar work.  A step is one
-// v_and, one v_addc_co, one 3-input bit op and two LDS reads per 2048 cells.
+// lane.  Lane l takes the columns in blocks of B = 4, block k - l in turn k, so
+// what it needs from lane l-1 -- the four carries of that block -- was
+// finished the turn before and moves as one register by one DPP per turn.
+// Inside a turn everything is VALU and lane-private: per column
+//     cin:  shift the carry word left, its top bit to an SGPR pair (v_add_co)
+//     U, sum with carry in and out (v_and, v_addc_co), V (v_bitop3)
+//     cout: shift the carry out into the outgoing word (v_addc_co),
+// five VALU for 2048 cells.  The columns of one band are a serial chain, so
+// the kernel's time is columns x time per column plus the bands' fill, and a
+// lone wave issues an instruction of any kind every four to five cycles: the
+// count per column is what matters.  With one column per step, carries in
+// lane-skewed SGPR masks and a second wave fetching through LDS a column took
+// 30.5 ns and m = n = 2^20 38.0 ms; now 15.0 and 19.9.  A band follows the one
+// below by 64 blocks, so blocks of two (15 instead of 12 issues a turn for two
+// columns, 17 ns a column) halve the skew where bands, not columns, make the
+// time: the caller picks by that.
 //
-//  * Match masks: each band builds M[c][lane] for c in [0, sigma) in LDS
-//    once; the all-zero row just below the table (row -1) serves the
-//    padding symbols before and after the column string.
-//  * Column symbols: per chunk of 32 steps the 95 symbols the lanes need are
-//    staged in LDS as ready-made table addresses (c*256 + const - 4p), so a
-//    lane's mask read is two dependent ds_reads with immediate offsets and no
-//    address arithmetic.
-//  * Band hand-off: lane 63's carry-out bits, 32 per chunk, go to the band
-//    above as one tagged 64-bit word (tag << 32 | bits) that the comb wave
-//    stores with an agent-scope relaxed atomic; the fetch wave of the band
-//    above polls for its tag, bounded in time, with the abort flag of the
-//    comb kernels.  A carry-out bit is
-//    collected one step late, which aligns producer word c with symbols
-//    32(c-2) .. 32(c-2)+31: consumer chunk q reads word q+2.
+//  * Match masks: a table in LDS, built once per band: one row of 64 words per
+//    symbol, or (alphabets of at most 9) one row of 64 pairs of words per two
+//    consecutive symbols, so that one address (a v_perm of the code byte and
+//    the lane) and one ds_read_b64 serve two columns.  A zero row serves the
+//    padding before and after the column string.
+//  * Column symbols: the seeding kernel writes them as code bytes; a lane
+//    loads its own 32 columns of codes per chunk (32 / B turns), two chunks
+//    before their masks are read, and those are read a chunk before use.
+//  * Band hand-off: after the last turn but one of chunk q + 2 B lane 63's
+//    outgoing word holds exactly the 32 carries of columns 32q ..; it goes to the band above as
+//    one tagged 64-bit word (tag << 32 | bits), stored with an agent-scope
+//    relaxed atomic.  The band above loads each word two chunks ahead and
+//    polls, bounded in time, when it comes too early.
 //  * Bands are handed out by an atomic ticket in order, so every wait is on a
 //    band that a resident wave already holds.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
+#include <mutex>
+#include <type_traits>
 
 #include "llcs_kernels.h"
 
@@ -44,27 +56,15 @@ namespace lcsl {
 #define LCSL_GLOBAL __attribute__((address_space(1)))
 typedef LCSL_GLOBAL unsigned long long gword;
 typedef LCSL_GLOBAL const unsigned long long gcword;
-typedef LCSL_GLOBAL const int32_t gsym;     // global, not flat: a flat load also counts against lgkmcnt,
-                                            // so every LDS wait would wait for it too
+typedef LCSL_GLOBAL const int32_t gsym;
+typedef LCSL_GLOBAL const uint8_t gbyte;
+typedef uint32_t unaligned_u32 __attribute__((aligned(1)));
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
-typedef __attribute__((address_space(3))) volatile uint32_t lds_vu32;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
 
-constexpr int kStage = kChunk + kWave - 1;   // 95 symbols staged per chunk
-constexpr int kStageWords = 96;              // one staging buffer (two are used)
-constexpr int kZeroRowWords = kWave;         // row -1 of the table, all zero
 constexpr unsigned kNoTag = 0xffffffffu;
-constexpr int kSymRing = kLdsSymRing;        // LDS rings (powers of two): column symbols,
-constexpr int kInRing = kLdsInRing;          // carry words of the band below
-constexpr int kSymBatch = 1024;              // symbols per fetch round
-// LDS control words of a workgroup
-constexpr int kTask = 0, kGo = 1, kStop = 2, kInAvail = 3, kInUsed = 4, kSymAvail = 5, kSymUsed = 6;
-
-// The workgroup's LDS: staging buffers, the zero row and the match-mask
-// table (comb wave), the two rings and the control words (shared).
-struct Lds {
-    lds_u32 *stage, *tab, *sym, *in;
-    lds_vu32 *ctl;
-};
+constexpr int kMaxLdsBytes = 160 * 1024;
 
 __device__ __forceinline__ unsigned long long ld_relaxed(gcword *p)
 {
@@ -79,394 +79,297 @@ __device__ __forceinline__ unsigned ld_flag(const unsigned *p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Waits (bounded in time) until control word `w` of the workgroup exceeds
-// `need`; `cache` keeps the last value seen.  False when the band must stop
-// (the other wave gave up, or the time ran out).
-__device__ __forceinline__ bool wait_ctl(const LlcsArgs &A, lds_vu32 *ctl, int w, uint32_t need, uint32_t &cache)
+// One turn: the B columns of a lane's block, their match masks in M.
+// First the carries move: lane l-1's cout of the turn before (its low B
+// bits), left-aligned, becomes cin; lane 0, which the DPP leaves alone, keeps
+// shifting the band's own input word out of its cin.  Column k: N(k) u = V &
+// m, A(k) cin <<= 1 with its top bit to sA[k % 2], S(k) sum = V + u + sA with
+// the carry to sB[k % 2], B(k) V = sum | (V & ~m), O(k) cout = cout << 1 | sB.
+// A VALU-written SGPR mask, and a VGPR that a DPP reads, want two issues in
+// between, so A runs a column ahead and O a column behind, and the two table
+// addresses of the caller's next reads (bytes sel0, sel1 of w over the lane's
+// place in a row) fill the turn's head: no s_nop, 24 issues for four columns
+// (14 for two).
+#define LCSL_N(K) "v_and_b32 %[u], %[v], %[m" #K "]\n\t"
+#define LCSL_A(X) "v_add_co_u32_e64 %[ci], %[a" #X "], %[ci], %[ci]\n\t"
+#define LCSL_S(X) "v_addc_co_u32_e64 %[s], %[b" #X "], %[v], %[u], %[a" #X "]\n\t"
+#define LCSL_B(K) "v_bitop3_b32 %[v], %[s], %[v], %[m" #K "] bitop3:0xf4\n\t"
+#define LCSL_O(X) "v_addc_co_u32_e64 %[co], %[d], %[co], %[co], %[b" #X "]\n\t"
+__device__ __forceinline__ void turn(uint32_t &V, uint32_t &cout, uint32_t &cin, const uint32_t (&M)[4], uint32_t w,
+                                     uint32_t lane_off, uint32_t sel0, uint32_t sel1, uint32_t &p0, uint32_t &p1)
 {
-    if (cache > need) return true;
-    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-    for (;;) {
-        cache = __builtin_amdgcn_readfirstlane(ctl[w]);
-        if (cache > need) return true;
-        if (__builtin_amdgcn_readfirstlane(ctl[kStop])) return false;
-        if (__builtin_amdgcn_s_memrealtime() - t0 > A.timeout_ticks) {
-            __hip_atomic_store(A.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-        __builtin_amdgcn_s_sleep(0);
-    }
+    uint32_t t, u, sum;
+    uint64_t a0, a1, b0, b1, d;
+    asm volatile("v_lshlrev_b32 %[t], 28, %[co]\n\t"
+                 LCSL_N(0)
+                 "v_perm_b32 %[p0], %[w], %[l], %[s0]\n\t"
+                 "v_mov_b32_dpp %[ci], %[t] wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                 LCSL_A(0) LCSL_A(1)
+                 "v_perm_b32 %[p1], %[w], %[l], %[s1]\n\t"
+                 LCSL_S(0) LCSL_B(0)
+                 LCSL_N(1) LCSL_A(0) LCSL_S(1) LCSL_B(1) LCSL_O(0)
+                 LCSL_N(2) LCSL_A(1) LCSL_S(0) LCSL_B(2) LCSL_O(1)
+                 LCSL_N(3) LCSL_S(1) LCSL_B(3) LCSL_O(0) LCSL_O(1)
+                 : [v] "+v"(V), [co] "+v"(cout), [ci] "+v"(cin), [t] "=&v"(t), [u] "=&v"(u), [s] "=&v"(sum),
+                   [a0] "=&s"(a0), [a1] "=&s"(a1), [b0] "=&s"(b0), [b1] "=&s"(b1), [d] "=&s"(d), [p0] "=&v"(p0),
+                   [p1] "=&v"(p1)
+                 : [w] "v"(w), [l] "v"(lane_off), [s0] "s"(sel0), [s1] "s"(sel1), [m0] "v"(M[0]), [m1] "v"(M[1]),
+                   [m2] "v"(M[2]), [m3] "v"(M[3]));
 }
 
-// Sixteen steps of one lane's 32 rows.  Per step: the band's carry-in bit
-// for lane 0 (bit B of w) goes to SCC; VCC, the previous step's carry-out
-// mask, doubles into the carry-in mask (lane l-1's carry enters lane l) with
-// SCC as bit 0, and its old bit 63 (lane 63's carry-out of the previous
-// step) doubles into `o`; then U = V & M, (s, VCC) = V + U + VCC and
-// V = s | (V & ~M) (v_bitop3 table 0xf4 over (s, V, M)).  Four SALU and
-// three VALU issues.  VCC is written by VALU and read by SALU and the
-// reverse, which needs no wait states on gfx950; the carry state enters and
-// leaves in `c` so that no compiled code between blocks can disturb VCC.
-#define LCSL_STEP(B, K)                                   \
-    "s_bitcmp1_b32 %[w], " #B "\n\t"                    \
-    "s_addc_u32 vcc_lo, vcc_lo, vcc_lo\n\t"              \
-    "s_addc_u32 vcc_hi, vcc_hi, vcc_hi\n\t"              \
-    "s_addc_u32 %[o], %[o], %[o]\n\t"                    \
-    "v_and_b32 %[u], %[v], %[m" #K "]\n\t"               \
-    "v_addc_co_u32_e32 %[s], vcc, %[v], %[u], vcc\n\t"   \
-    "v_bitop3_b32 %[v], %[s], %[v], %[m" #K "] bitop3:0xf4\n\t"
-
-#define LCSL_OPERANDS(M, OFF)                                                                          \
-    : [v] "+v"(V), [o] "+s"(wout), [c] "+s"(carry), [u] "=&v"(u), [s] "=&v"(sum)                       \
-    : [w] "s"(win), [m0] "v"(M[OFF + 0]), [m1] "v"(M[OFF + 1]), [m2] "v"(M[OFF + 2]),                  \
-      [m3] "v"(M[OFF + 3]), [m4] "v"(M[OFF + 4]), [m5] "v"(M[OFF + 5]), [m6] "v"(M[OFF + 6]),           \
-      [m7] "v"(M[OFF + 7])                                                                              \
-    : "vcc", "scc"
-
-// (readfirstlane returns int: each half goes through uint32_t so the low
-// half is not sign-extended into the high one)
-__device__ __forceinline__ uint64_t uniform64(uint64_t x)
+__device__ __forceinline__ void turn(uint32_t &V, uint32_t &cout, uint32_t &cin, const uint32_t (&M)[2], uint32_t w,
+                                     uint32_t lane_off, uint32_t sel0, uint32_t sel1, uint32_t &p0, uint32_t &p1)
 {
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)x);
-    return ((uint64_t)hi << 32) | lo;
+    uint32_t t, u, sum;
+    uint64_t a0, a1, b0, b1, d;
+    asm volatile("v_lshlrev_b32 %[t], 30, %[co]\n\t"
+                 LCSL_N(0)
+                 "v_perm_b32 %[p0], %[w], %[l], %[s0]\n\t"
+                 "v_mov_b32_dpp %[ci], %[t] wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                 LCSL_A(0) LCSL_A(1)
+                 "v_perm_b32 %[p1], %[w], %[l], %[s1]\n\t"
+                 LCSL_S(0) LCSL_B(0)
+                 LCSL_N(1) LCSL_S(1) LCSL_B(1) LCSL_O(0) LCSL_O(1)
+                 : [v] "+v"(V), [co] "+v"(cout), [ci] "+v"(cin), [t] "=&v"(t), [u] "=&v"(u), [s] "=&v"(sum),
+                   [a0] "=&s"(a0), [a1] "=&s"(a1), [b0] "=&s"(b0), [b1] "=&s"(b1), [d] "=&s"(d), [p0] "=&v"(p0),
+                   [p1] "=&v"(p1)
+                 : [w] "v"(w), [l] "v"(lane_off), [s0] "s"(sel0), [s1] "s"(sel1), [m0] "v"(M[0]), [m1] "v"(M[1]));
 }
 
-// Eight steps (quarter Q of a chunk): carry-in bits come from w (bit 31 - t
-// at step t of the chunk), carry-out bits of the previous step are
-// collected into wout.  Volatile, so the LDS reads the chunk loop places
-// between quarters stay there: at most a quarter's reads are outstanding at
-// each block, well under lgkmcnt's limit of 15 (a wait for an older read
-// then never waits for the newer ones).
-template <int Q>
-__device__ __forceinline__ void quarter_steps(uint32_t &V, const uint32_t (&M)[kChunk], uint32_t win, uint32_t &wout,
-                                              unsigned long long &carry)
+// One band.  PAIRS: a code byte stands for two columns; B: columns per turn.
+template <bool PAIRS, int B>
+__device__ bool band(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, lds_u32 *tab)
 {
-    uint32_t u, sum;
-    if constexpr (Q == 0)
-        asm volatile("s_mov_b64 vcc, %[c]\n\t"
-                     LCSL_STEP(31, 0) LCSL_STEP(30, 1) LCSL_STEP(29, 2) LCSL_STEP(28, 3)
-                     LCSL_STEP(27, 4) LCSL_STEP(26, 5) LCSL_STEP(25, 6) LCSL_STEP(24, 7)
-                     "s_mov_b64 %[c], vcc"
-                     LCSL_OPERANDS(M, 0));
-    else if constexpr (Q == 1)
-        asm volatile("s_mov_b64 vcc, %[c]\n\t"
-                     LCSL_STEP(23, 0) LCSL_STEP(22, 1) LCSL_STEP(21, 2) LCSL_STEP(20, 3)
-                     LCSL_STEP(19, 4) LCSL_STEP(18, 5) LCSL_STEP(17, 6) LCSL_STEP(16, 7)
-                     "s_mov_b64 %[c], vcc"
-                     LCSL_OPERANDS(M, 8));
-    else if constexpr (Q == 2)
-        asm volatile("s_mov_b64 vcc, %[c]\n\t"
-                     LCSL_STEP(15, 0) LCSL_STEP(14, 1) LCSL_STEP(13, 2) LCSL_STEP(12, 3)
-                     LCSL_STEP(11, 4) LCSL_STEP(10, 5) LCSL_STEP(9, 6) LCSL_STEP(8, 7)
-                     "s_mov_b64 %[c], vcc"
-                     LCSL_OPERANDS(M, 16));
-    else
-        asm volatile("s_mov_b64 vcc, %[c]\n\t"
-                     LCSL_STEP(7, 0) LCSL_STEP(6, 1) LCSL_STEP(5, 2) LCSL_STEP(4, 3)
-                     LCSL_STEP(3, 4) LCSL_STEP(2, 5) LCSL_STEP(1, 6) LCSL_STEP(0, 7)
-                     "s_mov_b64 %[c], vcc"
-                     LCSL_OPERANDS(M, 24));
-}
-
-// Column symbol j as a table row: [0, sigma) as is, -1 (the zero row) for
-// padding (j outside the string); a symbol outside [0, sigma) sets `bad`.
-__device__ __forceinline__ int32_t code_of(int32_t s, bool inside, int sigma, bool &bad)
-{
-    if (!inside) return -1;
-    if ((uint32_t)s >= (uint32_t)sigma) {
-        bad = true;
-        return -1;
-    }
-    return s;
-}
-
-// Comb wave of a band.  Column symbols come from the LDS symbol ring and the
-// band below's carry words from the LDS in-ring, both filled by the fetch
-// wave; its own carry words go straight to the global ring, one store by
-// lane 0 per chunk.  The loop issues no global load, so nothing ever waits
-// for those stores (on gfx950 vmcnt counts loads and stores alike); staging
-// them through an LDS out-ring and the fetch wave instead cost 3 ms at
-// m = n = 2^20, in the chunk's own LDS traffic and in the longer hand-off.
-__device__ bool band_compute(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, const Lds &L)
-{
+    constexpr int kBlock = B, kTurns = kChunk / B, kWordLag = word_lag(B);
+    constexpr int kCodeWords = PAIRS ? kChunk / 8 : kChunk / 4;   // code words of a lane's chunk
     const int sigma = A.sigma;
-    lds_u32 *tab = L.tab;
-    const uint32_t tab_addr = (uint32_t)(uintptr_t)tab;
-    lds_vu32 *ctl = L.ctl;
-
-    // match masks of this lane's 32 rows (each lane owns column `lane`)
-    for (int c = -1; c < sigma; ++c) tab[c * kWave + lane] = 0u;
-    const int64_t r0 = ((int64_t)g * kWave + lane) * kWordRows;
     bool bad = false;
-    for (int i = 0; i < kWordRows; ++i) {
-        const int64_t r = r0 + i;
-        if (r < D.nrows) {
-            const int32_t s = ((gsym *)D.rows)[r];
-            if ((uint32_t)s < (uint32_t)sigma)
-                tab[s * kWave + lane] |= 1u << i;
-            else
-                bad = true;
+    // the masks of this lane's 32 rows; row `sigma` stays zero (padding)
+    {
+        // the single-symbol rows: in the table itself, or in its first words
+        // while the pair rows are written from the last one down
+        const int rows1 = sigma + 1;
+        for (int c = 0; c < rows1; ++c) tab[c * kWave + lane] = 0u;
+        const int64_t r0 = ((int64_t)g * kWave + lane) * kWordRows;
+        for (int i = 0; i < kWordRows; ++i) {
+            const int64_t r = r0 + i;
+            if (r < D.nrows) {
+                const int32_t s = ((gsym *)D.rows)[r];
+                if ((uint32_t)s < (uint32_t)sigma) tab[s * kWave + lane] |= 1u << i;
+                else bad = true;
+            }
         }
+        if constexpr (PAIRS) {
+            uint32_t one[kMaxPairSigma + 1];
+#pragma unroll
+            for (int c = 0; c <= kMaxPairSigma; ++c) one[c] = c < rows1 ? tab[c * kWave + lane] : 0u;
+            __syncthreads();   // one wave: only keeps the reads before the writes
+            for (int c = 0; c < rows1; ++c) {
+                uint32_t mc = 0;
+#pragma unroll
+                for (int x = 0; x <= kMaxPairSigma; ++x) mc = x == c ? one[x] : mc;
+#pragma unroll
+                for (int x = 0; x <= kMaxPairSigma; ++x)
+                    if (x < rows1)
+                        *((lds_u32x2 *)tab + (c * rows1 + x + (lane & 32) * 4) * 32 + (lane & 31)) = u32x2{mc, one[x]};
+            }
+        }
+        __syncthreads();
     }
-
-    const int32_t ncols = D.ncols, nchunks = D.nchunks;
-    const bool has_in = g > 0, has_out = g + 1 < D.nbands;
-    gword *rout = (gword *)(D.ring + (size_t)((g + 1) & 1) * D.nchunks);
+    const int32_t nwords = D.nwords, nchunks = nwords > 0 ? nwords + kWordLag : 0;
+    gcword *rin = (gcword *)(D.ring + (size_t)(g & 1) * ((size_t)nwords + kSpare));
+    gword *rout = (gword *)(D.ring + (size_t)((g + 1) & 1) * ((size_t)nwords + kSpare));
+    const uint32_t tag_in = (uint32_t)g;
     const unsigned long long tag_out = (unsigned long long)(g + 1) << 32;
-    uint32_t in_avail = 0, sym_avail = 0;
-    bool ok = true;
-
-    // Chunk c covers steps [32c, 32c+32); lane l takes column symbol k - l at
-    // step k, so the chunk needs symbols 32c-63 .. 32c+31: staged position
-    // p = lane (symbol 32c-63+lane) and p = 64+lane (symbol 32c+1+lane).
-    auto raw_syms = [&](int c, int32_t &sa, int32_t &sb) -> bool {
-        const int64_t hi = min((int64_t)c * kChunk + kChunk, (int64_t)ncols);
-        if (hi > 0 && !wait_ctl(A, ctl, kSymAvail, (uint32_t)(hi - 1), sym_avail)) return false;
-        const int64_t ja = (int64_t)c * kChunk - (kWave - 1) + lane, jb = ja + kWave;
-        // unconditional reads (every index is a ring slot); stage_chunk
-        // ignores the values of positions outside the string
-        sa = (int32_t)L.sym[ja & (kSymRing - 1)];
-        sb = (int32_t)L.sym[jb & (kSymRing - 1)];
-        return true;
+    // lane l's codes of chunk q start at column kFrontPad + 32 q - B l
+    gbyte *codes = (gbyte *)D.codes + (size_t)(kFrontPad - B * lane) / (PAIRS ? 2 : 1);
+    auto load_codes = [&](int q, uint32_t (&c)[kCodeWords]) {
+        typedef LCSL_GLOBAL const unaligned_u32 gcode;
+#pragma unroll
+        for (int i = 0; i < kCodeWords; ++i) c[i] = ((gcode *)(codes + (size_t)q * kCodeWords * 4))[i];
     };
-    auto stage_chunk = [&](int c, lds_u32 *buf, int32_t sa, int32_t sb) {
-        const int64_t ja = (int64_t)c * kChunk - (kWave - 1) + lane, jb = ja + kWave;
-        // table address of row code, lane l, minus 4t for t = p + l - 63:
-        // lane l reads position t - l + 63 at step t and adds 4t
-        const int32_t ca = code_of(sa, ja >= 0 && ja < ncols, sigma, bad);
-        buf[lane] = (uint32_t)((int32_t)tab_addr + ca * (kWave * 4) + (kWave - 1) * 4 - 4 * lane);
-        if (lane < kStage - kWave) {
-            const int32_t cb = code_of(sb, jb >= 0 && jb < ncols, sigma, bad);
-            buf[kWave + lane] = (uint32_t)((int32_t)tab_addr + cb * (kWave * 4) + (kWave - 1) * 4 - 4 * (kWave + lane));
+    // The masks of turn i of a chunk from its codes: per code byte the LDS
+    // address byte * 256 + the lane's place in a row (the table is the
+    // kernel's only LDS and starts at address 0), put together by v_perm, the
+    // first two of a turn inside turn().
+    const uint32_t lane_off = PAIRS ? (uint32_t)(lane & 31) * 8u : (uint32_t)lane * 4u;
+    const uint32_t half = PAIRS && lane >= 32 ? 0x80808080u : 0u;
+    constexpr int kPerTurn = PAIRS ? B / 2 : B;   // code bytes
+    auto code_word = [&](const uint32_t (&c)[kCodeWords], int i) {
+        return PAIRS ? c[i * kPerTurn / 4] | half : c[i * kPerTurn / 4];
+    };
+    auto sel = [](int i, int k) { return 0x0c0c0000u | (uint32_t)(4 + i * kPerTurn % 4 + k) << 8; };
+    auto read_masks = [&](uint32_t w, int i, uint32_t p0, uint32_t p1, uint32_t (&M)[B]) {
+        if constexpr (PAIRS) {
+            const u32x2 x = *(const lds_u32x2 *)(uintptr_t)p0;
+            M[0] = x.x;
+            M[1] = x.y;
+            if constexpr (B == 4) {
+                const u32x2 y = *(const lds_u32x2 *)(uintptr_t)p1;
+                M[2] = y.x;
+                M[3] = y.y;
+            }
+        } else {
+            M[0] = *(const lds_u32 *)(uintptr_t)p0;
+            M[1] = *(const lds_u32 *)(uintptr_t)p1;
+#pragma unroll
+            for (int k = 2; k < B; ++k) M[k] = *(const lds_u32 *)(uintptr_t)__builtin_amdgcn_perm(w, lane_off, sel(i, k));
         }
     };
-    // staged addresses of a chunk (32 reads, 16 ds_read2), then its masks
-    // in quarters of 8 dependent reads
-    auto read_addrs = [&](const lds_u32 *buf, uint32_t (&M)[kChunk]) {
-        const lds_u32 *sp = buf + (kWave - 1) - lane;
-#pragma unroll
-        for (int t = 0; t < kChunk; ++t) M[t] = sp[t];
-    };
-    auto read_quarter = [&](uint32_t (&M)[kChunk], int qtr) {
-#pragma unroll
-        for (int i = 0; i < kChunk / 4; ++i) {
-            const int t = qtr * (kChunk / 4) + i;
-            M[t] = *((const lds_u32 *)(uintptr_t)M[t] + t);
+    auto sel1 = [&](int i) { return PAIRS && B == 2 ? sel(i, 0) : sel(i, 1); };   // (a turn of one pair has no second byte)
+    int dead = 0;   // set when a wait gave up: nothing is waited for after that
+    // the word of chunk q as loaded ahead (all lanes load the same one), once
+    // it carries this band's tag
+    auto take_word = [&](int q, unsigned long long e) -> uint32_t {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane((uint32_t)(e >> 32)) != tag_in, 0)) {
+            unsigned long long t0 = 0;
+#pragma nounroll
+            for (int polls = 0; !dead; ++polls) {
+                e = ld_relaxed(rin + q);
+                if (__builtin_amdgcn_readfirstlane((uint32_t)(e >> 32)) == tag_in) break;
+                if (polls % 8 == 0) {
+                    const unsigned long long now = __builtin_amdgcn_s_memrealtime();
+                    if (polls == 0) t0 = now;
+                    const bool late = A.timeout_ticks == 0 || now - t0 > A.timeout_ticks;
+                    if (late) __hip_atomic_store(A.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    dead = late || __builtin_amdgcn_readfirstlane(ld_flag(A.abort_flag)) != 0;
+                }
+            }
         }
-    };
-    auto read_masks = [&](const lds_u32 *buf, uint32_t (&M)[kChunk]) {
-        read_addrs(buf, M);
-        read_quarter(M, 0);
-        read_quarter(M, 1);
-        read_quarter(M, 2);
-        read_quarter(M, 3);
+        return __builtin_amdgcn_readfirstlane((uint32_t)e);
     };
 
-    uint32_t V = 0xffffffffu, wout = 0;
-    unsigned long long carry = 0;
-    uint32_t MA[kChunk], MB[kChunk];
-    int32_t s0 = 0, s1 = 0;
+    uint32_t V = 0xffffffffu, cout = 0;
+    uint32_t cA[kCodeWords], cB[kCodeWords], cC[kCodeWords];
+    uint32_t MA[kTurns][kBlock], MB[kTurns][kBlock];
+    unsigned long long wA = 0, wB = 0;
     if (nchunks > 0) {
-        if (!raw_syms(0, s0, s1)) return false;
-        stage_chunk(0, L.stage, s0, s1);
-        read_masks(L.stage, MA);
-        if (nchunks > 1 && !raw_syms(1, s0, s1)) return false;
+        load_codes(0, cA);
+        load_codes(1, cB);
+        load_codes(2, cC);
+        wA = ld_relaxed(rin);
+        wB = ld_relaxed(rin + 1);
+#pragma unroll
+        for (int i = 0; i < kTurns; ++i) {
+            const uint32_t w = code_word(cA, i);
+            read_masks(w, i, __builtin_amdgcn_perm(w, lane_off, sel(i, 0)), __builtin_amdgcn_perm(w, lane_off, sel1(i)),
+                       MA[i]);
+        }
     }
-    // chunk q: stage and read chunk q+1 (raw symbols of chunk q+2 ahead)
-    // while chunk q combs; Mc and Mn swap roles, two chunks per iteration.
-    // The band below's word q+2 holds the carry-out bits of symbols 32q ..
-    // 32q+31 (it collects each bit one step late).
-    // the band below's word for chunk q is read during chunk q-1 (before
-    // that chunk's last quarter of mask reads, so waiting for it never waits
-    // for them)
-    // (the read itself is unconditional and masked only where the chunk
-    // uses it, so that waiting for it never waits for later reads)
-    auto ring_word = [&](int q, uint32_t &w, bool &use) -> bool {
-        use = has_in && q + 2 < nchunks;
-        if (use && !wait_ctl(A, ctl, kInAvail, (uint32_t)q + 2, in_avail)) return false;
-        w = L.in[(q + 2) & (kInRing - 1)];
-        if (use && (q & 15) == 15 && lane == 0) ctl[kInUsed] = (uint32_t)q + 3;
-        return true;
+    // Chunk q: its masks are in M; the next chunk's are read between the turns
+    // from cN into N; the codes of chunk q + 3 and the word of chunk q + 2 take
+    // the place of this chunk's.  Chunks before kWordLag publish nothing and
+    // those from nwords on have no input (EDGE); the others run without a test
+    // on q, six per iteration, so that no register that a load is still to fill
+    // is copied.
+    auto chunk = [&](auto edge, int q, uint32_t (&cur)[kCodeWords], unsigned long long &word,
+                     const uint32_t (&cN)[kCodeWords], uint32_t (&M)[kTurns][kBlock], uint32_t (&N)[kTurns][kBlock]) {
+        constexpr bool EDGE = decltype(edge)::value;
+        uint32_t cin = 0;   // lane 0's; the others take theirs from the lane below each turn
+        if (!EDGE || q < nwords) cin = take_word(q, word);
+        load_codes(q + 3, cur);
+        word = ld_relaxed(rin + (EDGE ? min(q + 2, nwords + 1) : q + 2));
+#pragma unroll
+        for (int i = 0; i < kTurns; ++i) {
+            const uint32_t w = code_word(cN, i);
+            uint32_t p0, p1;
+            turn(V, cout, cin, M[i], w, lane_off, sel(i, 0), sel1(i), p0, p1);
+            if (i == kTurns - 2 && (!EDGE || q >= kWordLag)) {
+                // lane 63: the carries of columns 32 (q - kWordLag) ..; all
+                // lanes store the same word, so no lane mask puts a branch
+                // between the loads and their waits
+                uint32_t bits;   // (a v_readlane wants an issue between it and the VALU write)
+                asm volatile("s_nop 0\n\tv_readlane_b32 %0, %1, 63" : "=s"(bits) : "v"(cout));
+                st_relaxed(rout + (q - kWordLag), tag_out | bits);
+            }
+            read_masks(w, i, p0, p1, N[i]);
+        }
     };
-    uint32_t win_next = 0;
-    bool use_next = false;
-    if (!ring_word(0, win_next, use_next)) return false;
-    auto do_chunk = [&](int q, uint32_t (&Mc)[kChunk], uint32_t (&Mn)[kChunk]) -> bool {
-        uint32_t win = use_next ? win_next : 0u;
-        // chunk q combs in four quarters; between them the next chunk's
-        // masks are read a quarter at a time (addresses first).  After the
-        // last chunk this stages chunk nchunks, all padding (zero-row
-        // addresses), and reads nothing else.
-        lds_u32 *nb = L.stage + ((q + 1) & 1) * kStageWords;
-        stage_chunk(q + 1, nb, s0, s1);
-        read_addrs(nb, Mn);
-        // wave-uniform by construction; readfirstlane lets the compiler see
-        // it across the early exits of the chunk loop
-        win = __builtin_amdgcn_readfirstlane(win);
-        wout = __builtin_amdgcn_readfirstlane(wout);
-        carry = uniform64(carry);
-        quarter_steps<0>(V, Mc, win, wout, carry);
-        read_quarter(Mn, 0);
-        quarter_steps<1>(V, Mc, win, wout, carry);
-        read_quarter(Mn, 1);
-        quarter_steps<2>(V, Mc, win, wout, carry);
-        read_quarter(Mn, 2);
-        if (!raw_syms(q + 2, s0, s1)) return false;
-        if ((q & 15) == 15 && lane == 0) ctl[kSymUsed] = (uint32_t)max(0, (q + 3) * kChunk - (kWave - 1));
-        if (!ring_word(q + 1, win_next, use_next)) return false;
-        quarter_steps<3>(V, Mc, win, wout, carry);
-        read_quarter(Mn, 3);
-        if (has_out && lane == 0) st_relaxed(rout + q, tag_out | wout);
-        return true;
+    using Edge = std::integral_constant<bool, true>;
+    using Inner = std::integral_constant<bool, false>;
+    auto edges = [&](int q, int end) {   // q a multiple of six, where the sets' roles start over
+        for (; q < end; q += 6) {
+            chunk(Edge{}, q, cA, wA, cB, MA, MB);
+            if (q + 1 < end) chunk(Edge{}, q + 1, cB, wB, cC, MB, MA);
+            if (q + 2 < end) chunk(Edge{}, q + 2, cC, wA, cA, MA, MB);
+            if (q + 3 < end) chunk(Edge{}, q + 3, cA, wB, cB, MB, MA);
+            if (q + 4 < end) chunk(Edge{}, q + 4, cB, wA, cC, MA, MB);
+            if (q + 5 < end) chunk(Edge{}, q + 5, cC, wB, cA, MB, MA);
+        }
     };
-    int q = 0;
-    for (; q + 1 < nchunks && ok; q += 2) {
-        if (!do_chunk(q, MA, MB)) return false;
-        if (!do_chunk(q + 1, MB, MA)) return false;
+    constexpr int kRampChunks = (kWordLag + 5) / 6 * 6;
+    int q = min(kRampChunks, nchunks);
+    edges(0, q);
+    for (; q + 6 <= nwords; q += 6) {
+        chunk(Inner{}, q, cA, wA, cB, MA, MB);
+        chunk(Inner{}, q + 1, cB, wB, cC, MB, MA);
+        chunk(Inner{}, q + 2, cC, wA, cA, MA, MB);
+        chunk(Inner{}, q + 3, cA, wB, cB, MB, MA);
+        chunk(Inner{}, q + 4, cB, wA, cC, MA, MB);
+        chunk(Inner{}, q + 5, cC, wB, cA, MB, MA);
     }
-    if (q < nchunks && !do_chunk(q, MA, MB)) return false;
+    edges(q, nchunks);
 
     if (__any(bad) && lane == 0) *D.err = 1;
-    const int64_t live = D.nrows - r0;
+    const int64_t live = (int64_t)D.nrows - ((int64_t)g * kWave + lane) * kWordRows;
     const uint32_t valid = live >= kWordRows ? 0xffffffffu : live <= 0 ? 0u : ((1u << live) - 1u);
     int zeros = __popc(~V & valid);
     for (int off = 32; off > 0; off >>= 1) zeros += __shfl_xor(zeros, off);
     if (lane == 0) atomicAdd(D.out, zeros);
-    return true;
+    return !dead;
 }
 
-// Fetch wave of a band: the band's global loads after its table is built.
-// Each round it
-//  * loads the next column symbols (up to kSymBatch, 16 per lane) into the
-//    LDS symbol ring, as far as the comb wave's progress frees slots;
-//  * loads the band below's next 64 carry words from the global ring and
-//    copies the leading run that carries this band's tag to the LDS in-ring
-//    (one load brings every word published so far).
-// Both loads are issued before either result is awaited, so a round costs
-// about one memory round trip.  Every wait is bounded in time.
-__device__ void band_fetch(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, const Lds &L)
-{
-    lds_vu32 *ctl = L.ctl;
-    const int32_t ncols = D.ncols, nchunks = D.nchunks;
-    const bool need_in = g > 0 && nchunks > 2;
-    gcword *rin = (gcword *)(D.ring + (size_t)(g & 1) * nchunks);
-    const uint32_t tag_in = (uint32_t)g;
-    gsym *cols = (gsym *)D.cols;
-    int32_t next_s = 0, next_w = 2;
-    unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-    for (;;) {
-        const bool done_s = next_s >= ncols, done_w = !need_in || next_w >= nchunks;
-        if (done_s && done_w) return;
-        if (__builtin_amdgcn_readfirstlane(ctl[kStop])) return;
-        bool progress = false;
-
-        // issue: symbols, carry words in
-        int32_t scnt = 0;
-        int32_t sv[kSymBatch / kWave];
-        if (!done_s) {
-            const int32_t sym_used = (int32_t)__builtin_amdgcn_readfirstlane(ctl[kSymUsed]);
-            scnt = min(min(sym_used + kSymRing - next_s, kSymBatch), ncols - next_s);
-#pragma unroll
-            for (int k = 0; k < kSymBatch / kWave; ++k) {
-                const int32_t i = lane + k * kWave;
-                sv[k] = i < scnt ? cols[next_s + i] : 0;
-            }
-        }
-        int32_t want = 0;
-        unsigned long long e = 0;
-        if (!done_w) {
-            const int32_t used = (int32_t)__builtin_amdgcn_readfirstlane(ctl[kInUsed]);
-            want = min(min(used + kInRing - next_w, kWave), nchunks - next_w);
-            if (want > 0 && lane < want) e = ld_relaxed(rin + next_w + lane);
-        }
-        // land the loads
-        if (scnt > 0) {
-#pragma unroll
-            for (int k = 0; k < kSymBatch / kWave; ++k) {
-                const int32_t i = lane + k * kWave;
-                if (i < scnt) L.sym[(next_s + i) & (kSymRing - 1)] = (uint32_t)sv[k];
-            }
-            next_s += scnt;
-            if (lane == 0) ctl[kSymAvail] = (uint32_t)next_s;   // after the symbols
-            progress = true;
-        }
-        if (want > 0) {
-            const unsigned long long fresh = __ballot(lane < want && (uint32_t)(e >> 32) == tag_in);
-            const int k = ~fresh ? (int)__builtin_ctzll(~fresh) : kWave;   // leading run of fresh words
-            if (k > 0) {
-                if (lane < k) L.in[(next_w + lane) & (kInRing - 1)] = (uint32_t)e;
-                next_w += k;
-                if (lane == 0) ctl[kInAvail] = (uint32_t)next_w;   // after the words
-                progress = true;
-            }
-        }
-        if (progress) {
-            t0 = __builtin_amdgcn_s_memrealtime();
-        } else {
-            if (__builtin_amdgcn_s_memrealtime() - t0 > A.timeout_ticks) {
-                __hip_atomic_store(A.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (lane == 0) ctl[kStop] = 1u;
-                return;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-    }
-}
-
-// One workgroup of two waves per band: wave 0 combs, wave 1 fetches.  Thread
-// 0 takes the ticket and publishes it (and whether to go on) in LDS; the
-// barriers keep both waves on the same band.
-__global__ __launch_bounds__(2 * kWave) void llcs_chain_kernel(LlcsArgs A)
+template <bool PAIRS, int B>
+__global__ __launch_bounds__(kWave) void llcs_chain_kernel(LlcsArgs A)
 {
     extern __shared__ uint32_t lds_dyn[];
-    Lds L;
-    L.stage = (lds_u32 *)lds_dyn;
-    L.tab = L.stage + 2 * kStageWords + kZeroRowWords;
-    L.sym = L.tab + A.sigma * kWave;
-    L.in = L.sym + kSymRing;
-    L.ctl = (lds_vu32 *)(L.in + kInRing);
-    lds_vu32 *ctl = L.ctl;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
+    const int lane = threadIdx.x;
     for (;;) {
-        if (threadIdx.x == 0) {
-            const unsigned t = atomicAdd(A.ticket, 1u);
-            ctl[kTask] = t;
-            ctl[kGo] = ((int)t < A.ntasks && !ld_flag(A.abort_flag)) ? 1u : 0u;
-            ctl[kStop] = 0u;
-            ctl[kInAvail] = 2u;
-            ctl[kInUsed] = 2u;
-            ctl[kSymAvail] = 0u;
-            ctl[kSymUsed] = 0u;
-        }
-        __syncthreads();
-        if (!__builtin_amdgcn_readfirstlane(ctl[kGo])) break;
-        const unsigned t = __builtin_amdgcn_readfirstlane(ctl[kTask]);
+        unsigned t = 0;
+        if (lane == 0) t = atomicAdd(A.ticket, 1u);
+        t = __builtin_amdgcn_readfirstlane(t);
+        if ((int)t >= A.ntasks) break;
+        if (__builtin_amdgcn_readfirstlane(ld_flag(A.abort_flag))) break;
         const int2 task = A.tasks[t];
         const LlcsDesc D = A.descs[task.x];
-        if (wave == 0) {
-            const bool traced = A.trace && (int)t < A.trace_cap;
-            if (traced && lane == 0) A.trace[2 * (size_t)t] = __builtin_amdgcn_s_memrealtime();
-            if (!band_compute(A, D, task.y, lane, L) && lane == 0) ctl[kStop] = 1u;
-            if (traced && lane == 0) A.trace[2 * (size_t)t + 1] = __builtin_amdgcn_s_memrealtime();
-        } else {
-            band_fetch(A, D, task.y, lane, L);
-        }
-        __syncthreads();
+        const bool traced = A.trace && (int)t < A.trace_cap && lane == 0;
+        if (traced) A.trace[2 * (size_t)t] = __builtin_amdgcn_s_memrealtime();
+        if (!band<PAIRS, B>(A, D, task.y, lane, (lds_u32 *)lds_dyn)) break;
+        if (traced) A.trace[2 * (size_t)t + 1] = __builtin_amdgcn_s_memrealtime();
+        __syncthreads();   // the table is rebuilt
     }
 }
 
-// grid (x: ring words, y: pair); block (0,0) clears the ticket and abort
-// words, after folding the previous launch's abort flag into `sticky`
-__global__ void llcs_prep_kernel(const LlcsDesc *descs, unsigned *ticket, unsigned *abort_flag, unsigned *sticky)
+// grid (x: columns / 4, y: pair): ring words (band 0's empty input, and no tag any
+// band waits for), the column string as codes (one thread per four columns); block (0,0) clears
+// the ticket and abort words, after folding the previous launch's abort flag
+// into `sticky`
+__global__ void llcs_prep_kernel(const LlcsDesc *descs, int sigma, unsigned *ticket, unsigned *abort_flag,
+                                 unsigned *sticky)
 {
     const LlcsDesc D = descs[blockIdx.y];
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 2 * (int64_t)D.nchunks) D.ring[i] = (unsigned long long)kNoTag << 32;
-    if (i == 0) {
-        *D.out = 0;
-        *D.err = 0;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t slot = (int64_t)D.nwords + kSpare;
+    for (int64_t i = i0; i < 2 * slot; i += stride) D.ring[i] = i < slot ? 0ull : (unsigned long long)kNoTag << 32;
+    const bool pairs = llcs_pairs(sigma);
+    bool bad = false;
+    auto code = [&](int64_t c) -> uint32_t {
+        if (c < 0 || c >= D.ncols) return (uint32_t)sigma;
+        const uint32_t s = (uint32_t)D.cols[c];
+        bad = bad || s >= (uint32_t)sigma;
+        return s < (uint32_t)sigma ? s : (uint32_t)sigma;
+    };
+    if (D.nwords > 0) {
+        const int64_t quads = llcs_code_columns(D.nwords) / 4;
+        for (int64_t b = i0; b < quads; b += stride) {
+            const int64_t c0 = 4 * b - kFrontPad;
+            const uint32_t x = code(c0), y = code(c0 + 1), z = code(c0 + 2), w = code(c0 + 3), row = (uint32_t)sigma + 1;
+            if (pairs) ((uint16_t *)D.codes)[b] = (uint16_t)((x * row + y) | (z * row + w) << 8);
+            else ((uint32_t *)D.codes)[b] = x | y << 8 | z << 16 | w << 24;
+        }
     }
+    if (bad) *D.err = 1;
+    if (i0 == 0) *D.out = 0;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
         if (sticky && *abort_flag) *sticky = 1u;
         *ticket = 0u;
@@ -484,18 +387,36 @@ __global__ void llcs_finish_kernel(const LlcsDesc *descs, int npairs)
 
 }  // namespace lcsl
 
-int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int npairs, int max_ring_words,
-                int grid_blocks, hipStream_t stream)
+int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int npairs, int max_words,
+                int grid_blocks, int lds_bytes, hipStream_t stream)
 {
     using namespace lcsl;
     if (npairs <= 0) return 0;
-    if (args.sigma < 1 || args.sigma > kMaxSigma) return -22;
-    const unsigned px = (unsigned)(((long long)max_ring_words + 255) / 256);
-    hipLaunchKernelGGL(llcs_prep_kernel, dim3(px > 0 ? px : 1, npairs), dim3(256), 0, stream, d_descs, args.ticket,
-                       args.abort_flag, args.sticky);
-    if (args.ntasks > 0 && grid_blocks > 0)
-        hipLaunchKernelGGL(llcs_chain_kernel, dim3(grid_blocks), dim3(2 * kWave), llcs_lds_bytes(args.sigma), stream,
-                           args);
+    if (args.sigma < 1 || args.sigma > kMaxSigma || lds_bytes < (int)llcs_lds_bytes(args.sigma)) return -22;
+    const bool pairs = llcs_pairs(args.sigma);
+    static std::once_flag once;   // per process, and no stream operation
+    static bool ready = false;
+    std::call_once(once, [] {
+        ready = true;
+        for (const void *k : {(const void *)llcs_chain_kernel<true, 4>, (const void *)llcs_chain_kernel<false, 4>,
+                              (const void *)llcs_chain_kernel<true, 2>, (const void *)llcs_chain_kernel<false, 2>})
+            ready = ready && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes) == hipSuccess;
+    });
+    if (!ready) return -5;
+    // one thread per four columns
+    const unsigned px = (unsigned)std::min<long long>(4096, ((long long)max_words * (kChunk / 4) + 512) / 256);
+    for (int base = 0; base < npairs; base += 65535) {   // grid y is at most 65535
+        const int cnt = std::min(65535, npairs - base);
+        hipLaunchKernelGGL(llcs_prep_kernel, dim3(px, (unsigned)cnt), dim3(256), 0, stream, d_descs + base, args.sigma,
+                           args.ticket, args.abort_flag, base ? nullptr : args.sticky);
+    }
+    if (args.ntasks > 0 && grid_blocks > 0) {
+        const dim3 grid(grid_blocks), block(kWave);
+        if (pairs && args.block == 4) llcs_chain_kernel<true, 4><<<grid, block, lds_bytes, stream>>>(args);
+        else if (pairs) llcs_chain_kernel<true, 2><<<grid, block, lds_bytes, stream>>>(args);
+        else if (args.block == 4) llcs_chain_kernel<false, 4><<<grid, block, lds_bytes, stream>>>(args);
+        else llcs_chain_kernel<false, 2><<<grid, block, lds_bytes, stream>>>(args);
+    }
     hipLaunchKernelGGL(llcs_finish_kernel, dim3((npairs + 255) / 256), dim3(256), 0, stream, d_descs, npairs);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }

@@ -1,0 +1,39 @@
+"""The bit-parallel LCS kernel at the edges of its table and block rules:
+alphabets around the two-column table's largest (9), blocks of two columns
+(tall pairs) and of four (wide ones), column counts around the 32-column word,
+batches; against the oracle's word-parallel recurrence."""
+import numpy as np
+import pytest
+
+import lcs_amd
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sigma", [1, 8, 9, 10, 200])
+def test_words_bands_and_blocks(sigma):
+    rng = np.random.default_rng(sigma)
+    with lcs_amd.Context(0) as ctx:
+        # rows (bands of 2048) x columns either way round: few bands and many
+        for m, n in ((2048, 31), (2049, 32), (4096, 33), (2047, 2048), (40000, 3000), (30001, 257), (9000, 64),
+                     (6145, 6143), (12289, 40001)):
+            a = rng.integers(0, sigma, m).astype(np.int32)
+            b = rng.integers(0, sigma, n).astype(np.int32)
+            want = oracle.llcs_bitpar(a, b)
+            assert ctx.llcs(a, b, sigma) == want, (m, n)
+            assert ctx.llcs(b, a, sigma) == want, (n, m)
+
+
+def test_symbols_outside_the_alphabet_next_to_the_table_rows():
+    with lcs_amd.Context(0) as ctx:
+        a = np.zeros(3000, np.int32)
+        for sigma in (9, 10):
+            for bad in (sigma, -1, 255, 1 << 30):
+                for where in (0, 1, 2999):
+                    b = a.copy()
+                    b[where] = bad
+                    for x, y in ((a, b), (b, a)):
+                        with pytest.raises(lcs_amd.LcsError):
+                            ctx.llcs(x, y, sigma)
+            assert ctx.llcs(a, a, sigma) == 3000
