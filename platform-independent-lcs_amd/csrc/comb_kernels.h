@@ -21,8 +21,8 @@ struct PairDesc {
     const uint32_t *sym8;
     const int32_t *sym8_flags;
     int32_t sym8_stride, pad;
-    // Nullable: the pair's permutation (row_to_col, m + n entries), written
-    // instead of h_out and v_out.
+    // Nullable, as are h_out and v_out: the pair's permutation (row_to_col,
+    // m + n entries).
     int32_t *perm;
 };
 
@@ -31,13 +31,14 @@ struct PairDesc {
 // launch arguments, so that a single-pair call uploads nothing.  Tile (i, j)
 // combs a[iH ..) against b[jW ..) with ring slot iGC + j of `pair.E` and the
 // byte copies of strip j of `pair.sym8`.  With one tile the pair's own
-// h_in, v_in, h_out and v_out are used; with more, each tile writes its
-// permutation at `perm` + tile_perm_off(i, j).
+// h_in, v_in, h_out, v_out and perm are used; with more, each tile writes only
+// its permutation, at `perm` + perm_off(i, j).
 struct TileGrid {
     PairDesc pair;
     int32_t H, W, GR, GC;
     int32_t *perm;
     int32_t *sym8_flags;   // pair.sym8_flags, cleared by the extract kernel for the next launch
+    int32_t *status;       // nullable: receives the launch's abort flag
     __host__ __device__ int32_t rows(int32_t i) const { return pair.m - i * H < H ? pair.m - i * H : H; }
     __host__ __device__ int32_t cols(int32_t j) const { return pair.n - j * W < W ? pair.n - j * W : W; }
     __host__ __device__ int64_t perm_off(int32_t i, int32_t j) const
@@ -108,7 +109,10 @@ int lcsk_launch_grid(const ChainArgs &args, int grid_blocks, int block_threads, 
 // chain for tile height tile_m; then extracts v_out.  All on `stream`.
 int lcsk_launch_chain(const ChainArgs &args, const PairDesc *d_pairs, int npairs, int max_n, int tile_m,
                       int grid_blocks, int block_threads, hipStream_t stream);
-int lcsk_launch_identity(int32_t *h_out, int32_t m, int32_t *v_out, int32_t n, hipStream_t stream);
+// Strands (and, when perm is given, the permutation) of an empty grid (m == 0
+// or n == 0).
+int lcsk_launch_identity(int32_t *h_out, int32_t m, int32_t *v_out, int32_t n, hipStream_t stream,
+                         int32_t *perm = nullptr);
 // A string whose symbols the packed chain needs in [0, 0xfffd]: bit 0 of
 // bad[item] is set when one is outside, bit 1 when one is above 15 (the
 // one-hot cells then cannot take the pair).
@@ -126,12 +130,10 @@ int lcsk_launch_chain16(const ChainArgs &args, const CoupleDesc *d_couples, int 
 // each, written at perm + perm_off[p]).
 int lcsk_launch_from_strands(const PairDesc *d_pairs, int npairs, int max_len, int32_t *perm,
                              const int64_t *d_perm_off, hipStream_t stream);
-// row_to_col (size m+n) of one pair's permutation from its device strands.
-int lcsk_launch_r2c_from_strands(const int32_t *h, int32_t m, const int32_t *v, int32_t n, int32_t *r2c,
-                                 hipStream_t stream);
 // dst[0..count) = src[0..count) (a kernel, so it can sit in a captured graph).
 int lcsk_launch_copy(int32_t *dst, const int32_t *src, long long count, hipStream_t stream);
 // Strands from a permutation (row_to_col, size m+n): h_out[l] = row of col
 // n+l, v_out[j] = row of col j.
+// copy (nullable) receives r2c itself.
 int lcsk_launch_strands_from_perm(const int32_t *r2c, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out,
-                                  hipStream_t stream);
+                                  int32_t *copy, hipStream_t stream);

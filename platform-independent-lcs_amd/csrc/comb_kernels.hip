@@ -760,8 +760,8 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
                 const int l = m - 1 - (r0 + k);
                 // ids are below m+n after a completed comb; the test keeps an
                 // aborted one (whose strands are undefined) from writing out of range
-                if (P.perm == nullptr) P.h_out[l] = (int32_t)h[k];
-                else if (h[k] < (uint32_t)(m + n)) P.perm[h[k]] = n + l;
+                if (P.h_out) P.h_out[l] = (int32_t)h[k];
+                if (P.perm && h[k] < (uint32_t)(m + n)) P.perm[h[k]] = n + l;
             }
     }
     if (A.trace && t_id < A.trace_cap && lane == 0) A.trace[2 * (size_t)t_id + 1] = __builtin_amdgcn_s_memrealtime();
@@ -803,6 +803,7 @@ __device__ __forceinline__ PairDesc tile_pair(const TileGrid &T, int p)
         P.n = T.cols(j);
         P.E += (size_t)p * (2 * (size_t)T.W + 64);
         if (P.sym8) P.sym8 += (size_t)j * 4 * (size_t)P.sym8_stride;
+        P.h_out = P.v_out = nullptr;
         P.perm = T.perm + T.perm_off(i, j);
         P.nbands = (P.m + kWave * P.tile_m - 1) / (kWave * P.tile_m);
     }
@@ -1048,15 +1049,18 @@ __device__ __forceinline__ void extract_pair(const PairDesc &P)
     const long long stride = (long long)gridDim.x * blockDim.x;
     for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.n; c += stride) {
         const uint32_t id = (uint32_t)slot[c];
-        if (P.perm == nullptr) P.v_out[c] = (int32_t)id;
-        else if (id < (uint32_t)(P.m + P.n)) P.perm[id] = (int32_t)c;   // always, after a completed comb
+        if (P.v_out) P.v_out[c] = (int32_t)id;
+        if (P.perm && id < (uint32_t)(P.m + P.n)) P.perm[id] = (int32_t)c;   // always, after a completed comb
     }
 }
 __global__ void comb_extract_kernel(const PairDesc *pairs) { extract_pair(pairs[blockIdx.y]); }
-__global__ void comb_extract_grid_kernel(TileGrid T)
+__global__ void comb_extract_grid_kernel(TileGrid T, const unsigned *abort_flag)
 {
     extract_pair(tile_pair(T, (int)blockIdx.y));
-    if (T.sym8_flags && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *T.sym8_flags = 0;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+        if (T.sym8_flags) *T.sym8_flags = 0;
+        if (T.status) *T.status = (int32_t)*abort_flag;
+    }
 }
 
 // row_to_col of each pair's permutation (blockIdx.y = pair): the strand that
@@ -1076,26 +1080,15 @@ __global__ void from_strands_kernel(const PairDesc *pairs, int32_t *perm, const 
     }
 }
 
-// row_to_col of one pair's permutation from its device strands (FromStrands,
-// src/permutation_matrix.hpp:88-115): h[l] -> n+l, v[j] -> j.
-__global__ void r2c_from_strands_kernel(const int32_t *h, int32_t m, const int32_t *v, int32_t n, int32_t *r2c)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t size = (uint32_t)(m + n);
-    if (i >= (long long)size) return;
-    // ids are always < m+n after a completed comb; the test keeps an aborted
-    // one (whose strands are undefined) from writing out of range
-    const uint32_t id = (uint32_t)(i < m ? h[i] : v[i - m]);
-    if (id < size) r2c[id] = (int32_t)(i < m ? n + i : i - m);
-}
-
 // h_out, v_out of a permutation: the strand that ends in column c < n leaves
 // column c at the bottom, in column n + l row l on the right.
-__global__ void strands_from_perm_kernel(const int32_t *r2c, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out)
+__global__ void strands_from_perm_kernel(const int32_t *r2c, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out,
+                                         int32_t *copy)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (long long)m + n) return;
     const uint32_t c = (uint32_t)r2c[i];
+    if (copy) copy[i] = (int32_t)c;
     if (c < (uint32_t)n) v_out[c] = (int32_t)i;
     else if (c < (uint32_t)(m + n)) h_out[c - (uint32_t)n] = (int32_t)i;
 }
@@ -1107,11 +1100,12 @@ __global__ void copy_kernel(int32_t *dst, const int32_t *src, long long count)
 }
 
 // Identity strands for empty grids (m == 0 or n == 0).
-__global__ void comb_identity_kernel(int32_t *h_out, int32_t m, int32_t *v_out, int32_t n)
+__global__ void comb_identity_kernel(int32_t *h_out, int32_t m, int32_t *v_out, int32_t n, int32_t *perm)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < m) h_out[i] = (int32_t)i;
     if (i < n) v_out[i] = (int32_t)(m + i);
+    if (perm && i < (long long)m + n) perm[i] = (int32_t)(i < m ? n + i : i - m);
 }
 
 }  // namespace lcsk
@@ -1161,7 +1155,7 @@ int lcsk_launch_grid(const ChainArgs &args, int grid_blocks, int block_threads, 
     hipLaunchKernelGGL(comb_prep_grid_kernel, dim3(fill, tiles), dim3(256), 0, stream, T, args.ticket, args.sticky);
     const int rc = launch_bands(args, T.pair.tile_m, grid_blocks, block_threads, stream);
     if (rc) return rc;
-    hipLaunchKernelGGL(comb_extract_grid_kernel, dim3(fill, tiles), dim3(256), 0, stream, T);
+    hipLaunchKernelGGL(comb_extract_grid_kernel, dim3(fill, tiles), dim3(256), 0, stream, T, args.abort_flag);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -1233,23 +1227,13 @@ int lcsk_launch_from_strands(const PairDesc *d_pairs, int npairs, int max_len, i
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-int lcsk_launch_r2c_from_strands(const int32_t *h, int32_t m, const int32_t *v, int32_t n, int32_t *r2c,
-                                 hipStream_t stream)
-{
-    const long long size = (long long)m + n;
-    if (size == 0) return 0;
-    hipLaunchKernelGGL(r2c_from_strands_kernel, dim3((unsigned)((size + 255) / 256)), dim3(256), 0, stream, h, m, v, n,
-                       r2c);
-    return hipGetLastError() == hipSuccess ? 0 : -5;
-}
-
 int lcsk_launch_strands_from_perm(const int32_t *r2c, int32_t m, int32_t n, int32_t *h_out, int32_t *v_out,
-                                  hipStream_t stream)
+                                  int32_t *copy, hipStream_t stream)
 {
     const long long size = (long long)m + n;
     if (size == 0) return 0;
     hipLaunchKernelGGL(strands_from_perm_kernel, dim3((unsigned)((size + 255) / 256)), dim3(256), 0, stream, r2c, m, n,
-                       h_out, v_out);
+                       h_out, v_out, copy);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -1261,11 +1245,11 @@ int lcsk_launch_copy(int32_t *dst, const int32_t *src, long long count, hipStrea
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-int lcsk_launch_identity(int32_t *h_out, int32_t m, int32_t *v_out, int32_t n, hipStream_t stream)
+int lcsk_launch_identity(int32_t *h_out, int32_t m, int32_t *v_out, int32_t n, hipStream_t stream, int32_t *perm)
 {
     const long long mx = m > n ? m : n;
     if (mx == 0) return 0;
     hipLaunchKernelGGL(comb_identity_kernel, dim3((unsigned)((mx + 255) / 256)), dim3(256), 0, stream, h_out, m, v_out,
-                       n);
+                       n, perm);
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }

@@ -470,7 +470,8 @@ int batch_core(lcs_ctx *ctx, Extras *X, int32_t npairs, const int32_t *da, const
         }
         for (size_t i = 0; i < sp.size(); ++i) {
             const int32_t p = sp[i].p;
-            if (lcsk_launch_strands_from_perm(cur[i].perm[0], m[p], n[p], dh + a_off[p], dv + b_off[p], st))
+            if (lcsk_launch_strands_from_perm(cur[i].perm[0], m[p], n[p], dh + a_off[p], dv + b_off[p],
+                                              nullptr, st))
                 return LCS_EIO;
         }
         return LCS_OK;

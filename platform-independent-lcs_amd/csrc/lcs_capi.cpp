@@ -21,10 +21,40 @@ namespace lcs {
 
 static int hip_status(hipError_t e) { return e == hipSuccess ? LCS_OK : LCS_EIO; }
 
+DevBuf KeptBuf::take(size_t at_least, size_t at_most)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    DevBuf out;
+    if (buf.bytes >= at_least && buf.bytes <= at_most) std::swap(out, buf);
+    return out;
+}
+
+void KeptBuf::give(lcs_ctx *ctx, DevBuf &b)
+{
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (b.bytes <= kKeptMax && b.bytes > buf.bytes) std::swap(b, buf);
+    }
+    b.release(ctx);
+}
+
+void KeptBuf::trim(lcs_ctx *ctx)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    buf.release(ctx);
+}
+
+static void trim_kept(lcs_ctx *ctx)
+{
+    ctx->scratch.trim(ctx);
+    ctx->index_mem.trim(ctx);
+}
+
 int DevBuf::reserve(lcs_ctx *ctx, size_t want)
 {
     if (want <= bytes) return LCS_OK;
     size_t grow = std::max(want, bytes + bytes / 2);
+    if (ctx->held + grow - bytes > ctx->budget) trim_kept(ctx);
     if (ctx->held + grow - bytes > ctx->budget) grow = want;
     if (ctx->held + grow - bytes > ctx->budget) return LCS_ENOMEM;
     if (ptr) {
@@ -36,7 +66,11 @@ int DevBuf::reserve(lcs_ctx *ctx, size_t want)
     void *p = nullptr;
     if (hipMalloc(&p, grow) != hipSuccess) {
         (void)hipGetLastError();
-        return LCS_ENOMEM;
+        trim_kept(ctx);
+        if (hipMalloc(&p, grow) != hipSuccess) {
+            (void)hipGetLastError();
+            return LCS_ENOMEM;
+        }
     }
     ptr = p;
     bytes = grow;
@@ -407,7 +441,7 @@ static GridPlan choose_grid(const lcs_ctx *ctx, int32_t m, int32_t n, int tm, in
 
 // Merges the tiles' permutations to the whole pair's and writes its strands,
 // all products of a level (merge_levels) in one launch sequence.
-static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_t *ws, int32_t *d_h, int32_t *d_v,
+static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_t *ws, const PairDesc &out,
                        hipStream_t stream)
 {
     const int32_t m = T.pair.m, n = T.pair.n;
@@ -451,16 +485,17 @@ static int merge_tiles(const TileGrid &T, int32_t *permA, int32_t *permB, int32_
         gc = nc;
         dst_base = dst_base == permB ? permA : permB;
     }
-    return lcsk_launch_strands_from_perm(cur[0].p, m, n, d_h, d_v, stream);
+    return lcsk_launch_strands_from_perm(cur[0].p, m, n, out.h_out, out.v_out, out.perm, stream);
 }
 
 // Combs one pair as the tiles of `G` in one chain launch and merges them.
 // The launch is described by its arguments alone: nothing is uploaded.
-static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, hipStream_t stream)
+static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, int32_t *status, hipStream_t stream)
 {
     const int32_t m = pair.m, n = pair.n;
     TileGrid T{};
     T.pair = pair;
+    T.status = status;
     T.H = (m + G.GR - 1) / G.GR;
     T.W = (n + G.GC - 1) / G.GC;
     T.GR = G.GR = (m + T.H - 1) / T.H;   // no empty tile
@@ -504,8 +539,12 @@ static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, hipStrea
     if ((rc = lcsk_launch_grid(A, (int)blocks, 256, stream))) return rc;
     if (hipEventRecord(ctx->evc1, stream) != hipSuccess) return LCS_EIO;
     ctx->chain_timed = true;
+    ctx->time_from = ctx->evc0;
+    ctx->time_to = ctx->evc1;
     if (tiles == 1) return LCS_OK;
-    return merge_tiles(T, T.perm, T.perm + perm_words, T.perm + 2 * perm_words, pair.h_out, pair.v_out, stream);
+    if ((rc = merge_tiles(T, T.perm, T.perm + perm_words, T.perm + 2 * perm_words, pair, stream))) return rc;
+    ctx->time_to = ctx->ev1;
+    return hipEventRecord(ctx->ev1, stream) == hipSuccess ? LCS_OK : LCS_EIO;
 }
 
 int ws_acquire(lcs_ctx *ctx, hipStream_t s)
@@ -523,32 +562,39 @@ int ws_release(lcs_ctx *ctx, hipStream_t s)
 
 static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_b, int32_t n,
                             const lcs_schedule *sched, int32_t *d_h, int32_t *d_v, hipStream_t stream,
-                            const int32_t *d_h_in, const int32_t *d_v_in);
+                            const int32_t *d_h_in, const int32_t *d_v_in, int32_t *d_r2c, int32_t *d_status);
 
 // Enqueue one pair on `stream` with device pointers, following `sched`,
 // after the previous user of the context's workspace.
 int enqueue_chain(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_b, int32_t n,
                   const lcs_schedule *sched, int32_t *d_h, int32_t *d_v, hipStream_t stream,
-                  const int32_t *d_h_in, const int32_t *d_v_in)
+                  const int32_t *d_h_in, const int32_t *d_v_in, int32_t *d_r2c, int32_t *d_status)
 {
     int rc = ws_acquire(ctx, stream);
     if (rc) return rc;
-    rc = enqueue_chain_ws(ctx, d_a, m, d_b, n, sched, d_h, d_v, stream, d_h_in, d_v_in);
+    rc = enqueue_chain_ws(ctx, d_a, m, d_b, n, sched, d_h, d_v, stream, d_h_in, d_v_in, d_r2c, d_status);
     const int rc2 = ws_release(ctx, stream);
     return rc ? rc : rc2;
 }
 
 static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_b, int32_t n,
                             const lcs_schedule *sched, int32_t *d_h, int32_t *d_v, hipStream_t stream,
-                            const int32_t *d_h_in, const int32_t *d_v_in)
+                            const int32_t *d_h_in, const int32_t *d_v_in, int32_t *d_r2c, int32_t *d_status)
 {
     if (m == 0 || n == 0) {
+        ctx->time_from = ctx->ev0;
+        ctx->time_to = ctx->ev1;
+        bool ok = hipEventRecord(ctx->ev0, stream) == hipSuccess;
+        if (ok && d_status)
+            ok = hipMemcpyAsync(d_status, ctx->ctrl + kZeroWord, 4, hipMemcpyDeviceToDevice, stream) == hipSuccess;
         if (d_h_in || d_v_in) {
-            if (m && hipMemcpyAsync(d_h, d_h_in, (size_t)m * 4, hipMemcpyDeviceToDevice, stream) != hipSuccess) return LCS_EIO;
-            if (n && hipMemcpyAsync(d_v, d_v_in, (size_t)n * 4, hipMemcpyDeviceToDevice, stream) != hipSuccess) return LCS_EIO;
-            return LCS_OK;
+            if (ok && m) ok = hipMemcpyAsync(d_h, d_h_in, (size_t)m * 4, hipMemcpyDeviceToDevice, stream) == hipSuccess;
+            if (ok && n) ok = hipMemcpyAsync(d_v, d_v_in, (size_t)n * 4, hipMemcpyDeviceToDevice, stream) == hipSuccess;
+        } else if (ok) {
+            const int rc = lcsk_launch_identity(d_h, m, d_v, n, stream, d_r2c);
+            if (rc) return rc;
         }
-        return lcsk_launch_identity(d_h, m, d_v, n, stream);
+        return ok && hipEventRecord(ctx->ev1, stream) == hipSuccess ? LCS_OK : LCS_EIO;
     }
     if (n > kMaxChainN) return LCS_ERANGE;   // before any buffer is reserved
     const int strips_req = sched ? sched->strips : 0;
@@ -570,13 +616,31 @@ static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const i
     P.v_in = d_v_in;
     P.h_out = d_h;
     P.v_out = d_v;
+    P.perm = d_r2c;
     P.m = m;
     P.n = n;
-    const int rc = enqueue_grid(ctx, P, G, stream);
+    const int rc = enqueue_grid(ctx, P, G, d_status, stream);
     if (rc != LCS_ENOMEM || strips_req || G.GR * G.GC == 1) return rc;
     // the budget cannot hold the library's own cut (its workspaces are reserved
     // before anything is launched): one tile
-    return enqueue_grid(ctx, P, choose_grid(ctx, m, n, tm, 1, whole, G), stream);
+    return enqueue_grid(ctx, P, choose_grid(ctx, m, n, tm, 1, whole, G), d_status, stream);
+}
+
+void *pinned_staging(lcs_ctx *ctx, size_t bytes)
+{
+    if (bytes <= ctx->pinned_bytes) return ctx->pinned;
+    if (ctx->pinned) (void)hipHostFree(ctx->pinned);   // its last user has waited for its copies
+    ctx->pinned = nullptr;
+    ctx->pinned_bytes = 0;
+    void *p = nullptr;
+    const size_t want = std::min(kPinnedMax, bytes * 2);
+    if (hipHostMalloc(&p, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    ctx->pinned = p;
+    ctx->pinned_bytes = want;
+    return p;
 }
 
 // The abort flag of the last launch on the context's own ctrl words (the
@@ -664,11 +728,11 @@ int lcs_ctx_destroy(lcs_ctx *ctx)
     ctx->sym8.release(ctx);
     ctx->staging.destroy();
     if (ctx->ws_done) (void)hipEventDestroy(ctx->ws_done);
-    ctx->in_a.release(ctx);
-    ctx->in_b.release(ctx);
-    ctx->out_h.release(ctx);
-    ctx->out_v.release(ctx);
-    ctx->perm.release(ctx);
+    ctx->alive->store(false);
+    ctx->strings.release(ctx);
+    ctx->results.release(ctx);
+    trim_kept(ctx);
+    if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->ctrl) (void)hipFree(ctx->ctrl);
     if (ctx->band_trace) (void)hipFree(ctx->band_trace);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
@@ -723,9 +787,9 @@ int lcs_ctx_set_timeout(lcs_ctx *ctx, uint64_t ticks)
 int lcs_ctx_info(lcs_ctx *ctx, int32_t *num_cus, double *last_kernel_ms)
 {
     if (!ctx) return LCS_EINVAL;
-    if (ctx->pending_timing && hipEventQuery(ctx->ev1) == hipSuccess) {
+    if (ctx->pending_timing && hipEventQuery(ctx->time_to) == hipSuccess) {
         float ms = 0.f;
-        if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess) ctx->last_kernel_ms = ms;
+        if (hipEventElapsedTime(&ms, ctx->time_from, ctx->time_to) == hipSuccess) ctx->last_kernel_ms = ms;
         ctx->pending_timing = false;
     }
     if (num_cus) *num_cus = ctx->num_cus;
@@ -745,35 +809,67 @@ int lcs_ctx_chain_ms(lcs_ctx *ctx, double *chain_ms)
     return LCS_OK;
 }
 
-int lcs_comb(lcs_ctx *ctx, const int32_t *a, int32_t m, const int32_t *b, int32_t n,
-             const lcs_schedule *sched, int32_t *h_out, int32_t *v_out, int32_t *llcs_out)
+// The host single-pair calls.  Strings and results each lie in one device
+// buffer, so that a call makes one copy in and one out, through pinned host
+// memory up to kPinnedMax bytes: a small call's time is its copies, launches
+// and waits, and a copy from or to pageable memory costs a wait of its own.
+// 300 x 500 took 127 us with 2 copies in, 2 out, one of the abort flag and
+// 5 events, and takes 66 us.  The limit bounds the pinned memory a context
+// holds; past it the two waits are small beside the call.
+// Results on the device: kStatusWords words (the launch's abort flag in the
+// first), row_to_col (if asked for), v, h -- col_to_row is v then h.
+static int comb_host(lcs_ctx *ctx, const int32_t *a, int32_t m, const int32_t *b, int32_t n, const lcs_schedule *sched,
+                     int32_t *r2c, int32_t *v_out, int32_t *h_out, int32_t *llcs_out)
 {
-    if (!ctx || m < 0 || n < 0) return LCS_EINVAL;
-    if ((m > 0 && (!a || !h_out)) || (n > 0 && (!b || !v_out))) return LCS_EINVAL;
-    if ((long long)m + n > 0x7fffffffLL) return LCS_ERANGE;
+    constexpr size_t kStatusWords = 16;
     if (hipSetDevice(ctx->device) != hipSuccess) return LCS_EIO;
     int rc;
     lcs_schedule chosen{};
     if ((rc = single_schedule(ctx, a, m, b, n, sched, chosen))) return rc;
-    sched = &chosen;
-    if ((rc = ctx->in_a.reserve(ctx, (size_t)std::max(m, 1) * 4))) return rc;
-    if ((rc = ctx->in_b.reserve(ctx, (size_t)std::max(n, 1) * 4))) return rc;
-    if ((rc = ctx->out_h.reserve(ctx, (size_t)std::max(m, 1) * 4))) return rc;
-    if ((rc = ctx->out_v.reserve(ctx, (size_t)std::max(n, 1) * 4))) return rc;
-    int32_t *da = (int32_t *)ctx->in_a.ptr, *db = (int32_t *)ctx->in_b.ptr;
-    int32_t *dh = (int32_t *)ctx->out_h.ptr, *dv = (int32_t *)ctx->out_v.ptr;
+    const size_t mm = (size_t)m, nn = (size_t)n, a_words = (mm + 15) & ~(size_t)15;   // b 64-byte aligned
+    const size_t in_bytes = (a_words + nn) * 4, perm_words = r2c ? mm + nn : 0;
+    const size_t out_bytes = (kStatusWords + perm_words + mm + nn) * 4;
+    if ((rc = ctx->strings.reserve(ctx, std::max<size_t>(in_bytes, 4)))) return rc;
+    if ((rc = ctx->results.reserve(ctx, out_bytes))) return rc;
+    int32_t *da = (int32_t *)ctx->strings.ptr, *db = da + a_words;
+    int32_t *dstatus = (int32_t *)ctx->results.ptr, *dr2c = dstatus + kStatusWords, *dv = dr2c + perm_words, *dh = dv + n;
     hipStream_t s = ctx->stream;
-    if (m && hipMemcpyAsync(da, a, (size_t)m * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
-    if (n && hipMemcpyAsync(db, b, (size_t)n * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
-    if (hipEventRecord(ctx->ev0, s) != hipSuccess) return LCS_EIO;
-    if ((rc = enqueue_chain(ctx, da, m, db, n, sched, dh, dv, s))) return rc;
-    if (hipEventRecord(ctx->ev1, s) != hipSuccess) return LCS_EIO;
-    if (m && hipMemcpyAsync(h_out, dh, (size_t)m * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
-    if (n && hipMemcpyAsync(v_out, dv, (size_t)n * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
-    if (hipStreamSynchronize(s) != hipSuccess) return LCS_EIO;
+    int32_t *pin = in_bytes + out_bytes <= kPinnedMax ? (int32_t *)pinned_staging(ctx, in_bytes + out_bytes) : nullptr;
+    if (pin) {
+        if (m) std::memcpy(pin, a, mm * 4);
+        if (n) std::memcpy(pin + a_words, b, nn * 4);
+        if (in_bytes && hipMemcpyAsync(da, pin, in_bytes, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
+    } else {
+        if (m && hipMemcpyAsync(da, a, mm * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
+        if (n && hipMemcpyAsync(db, b, nn * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
+    }
+    if ((rc = enqueue_chain(ctx, da, m, db, n, &chosen, dh, dv, s, nullptr, nullptr, r2c ? dr2c : nullptr, dstatus)))
+        return rc;
+    int32_t status = 0;
+    if (pin) {
+        int32_t *res = pin + in_bytes / 4;
+        if (hipMemcpyAsync(res, dstatus, out_bytes, hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess)
+            return LCS_EIO;
+        status = res[0];
+        if (!status) {
+            res += kStatusWords;
+            if (perm_words) std::memcpy(r2c, res, perm_words * 4);
+            if (n) std::memcpy(v_out, res + perm_words, nn * 4);
+            if (m) std::memcpy(h_out, res + perm_words + nn, mm * 4);
+        }
+    } else {
+        if (perm_words && hipMemcpyAsync(r2c, dr2c, perm_words * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
+        if (n && hipMemcpyAsync(v_out, dv, nn * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
+        if (m && hipMemcpyAsync(h_out, dh, mm * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
+        if (hipMemcpyAsync(&status, dstatus, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess)
+            return LCS_EIO;
+    }
     float ms = 0.f;
-    if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess) ctx->last_kernel_ms = ms;
-    if ((rc = check_abort(ctx))) return rc;
+    if (hipEventElapsedTime(&ms, ctx->time_from, ctx->time_to) == hipSuccess) ctx->last_kernel_ms = ms;
+    ctx->pending_timing = false;
+    if (status) return (rc = check_abort(ctx)) ? rc : LCS_ETIMEDOUT;   // clears the flag
     if (llcs_out) {
         int32_t c = 0;
         for (int32_t j = 0; j < n; ++j) c += v_out[j] < m;
@@ -782,47 +878,23 @@ int lcs_comb(lcs_ctx *ctx, const int32_t *a, int32_t m, const int32_t *b, int32_
     return LCS_OK;
 }
 
+int lcs_comb(lcs_ctx *ctx, const int32_t *a, int32_t m, const int32_t *b, int32_t n,
+             const lcs_schedule *sched, int32_t *h_out, int32_t *v_out, int32_t *llcs_out)
+{
+    if (!ctx || m < 0 || n < 0) return LCS_EINVAL;
+    if ((m > 0 && (!a || !h_out)) || (n > 0 && (!b || !v_out))) return LCS_EINVAL;
+    if ((long long)m + n > 0x7fffffffLL) return LCS_ERANGE;
+    return comb_host(ctx, a, m, b, n, sched, nullptr, v_out, h_out, llcs_out);
+}
+
 int lcs_comb_permutation(lcs_ctx *ctx, const int32_t *a, int32_t m, const int32_t *b, int32_t n,
                          const lcs_schedule *sched, int32_t *row_to_col, int32_t *col_to_row, int32_t *llcs_out)
 {
     if (!ctx || m < 0 || n < 0) return LCS_EINVAL;
     if ((m > 0 && !a) || (n > 0 && !b) || (m + n > 0 && (!row_to_col || !col_to_row))) return LCS_EINVAL;
     if ((long long)m + n > 0x7fffffffLL) return LCS_ERANGE;
-    if (hipSetDevice(ctx->device) != hipSuccess) return LCS_EIO;
-    int rc;
-    lcs_schedule chosen{};
-    if ((rc = single_schedule(ctx, a, m, b, n, sched, chosen))) return rc;
-    sched = &chosen;
-    if ((rc = ctx->in_a.reserve(ctx, (size_t)std::max(m, 1) * 4))) return rc;
-    if ((rc = ctx->in_b.reserve(ctx, (size_t)std::max(n, 1) * 4))) return rc;
-    if ((rc = ctx->out_h.reserve(ctx, (size_t)std::max(m, 1) * 4))) return rc;
-    if ((rc = ctx->out_v.reserve(ctx, (size_t)std::max(n, 1) * 4))) return rc;
-    if ((rc = ctx->perm.reserve(ctx, (size_t)std::max(m + n, 1) * 4))) return rc;
-    int32_t *da = (int32_t *)ctx->in_a.ptr, *db = (int32_t *)ctx->in_b.ptr;
-    int32_t *dh = (int32_t *)ctx->out_h.ptr, *dv = (int32_t *)ctx->out_v.ptr, *dr2c = (int32_t *)ctx->perm.ptr;
-    hipStream_t s = ctx->stream;
-    if (m && hipMemcpyAsync(da, a, (size_t)m * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
-    if (n && hipMemcpyAsync(db, b, (size_t)n * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
-    if (hipEventRecord(ctx->ev0, s) != hipSuccess) return LCS_EIO;
-    if ((rc = enqueue_chain(ctx, da, m, db, n, sched, dh, dv, s))) return rc;
-    if (hipEventRecord(ctx->ev1, s) != hipSuccess) return LCS_EIO;
-    if (lcsk_launch_r2c_from_strands(dh, m, dv, n, dr2c, s)) return LCS_EIO;
     // col_to_row is v then h (FromStrands: col j <- v[j], col n+l <- h[l])
-    if (n && hipMemcpyAsync(col_to_row, dv, (size_t)n * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
-    if (m && hipMemcpyAsync(col_to_row + n, dh, (size_t)m * 4, hipMemcpyDeviceToHost, s) != hipSuccess)
-        return LCS_EIO;
-    if (m + n && hipMemcpyAsync(row_to_col, dr2c, (size_t)(m + n) * 4, hipMemcpyDeviceToHost, s) != hipSuccess)
-        return LCS_EIO;
-    if (hipStreamSynchronize(s) != hipSuccess) return LCS_EIO;
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess) ctx->last_kernel_ms = ms;
-    if ((rc = check_abort(ctx))) return rc;
-    if (llcs_out) {
-        int32_t c = 0;
-        for (int32_t j = 0; j < n; ++j) c += col_to_row[j] < m;
-        *llcs_out = c;
-    }
-    return LCS_OK;
+    return comb_host(ctx, a, m, b, n, sched, row_to_col, col_to_row, col_to_row ? col_to_row + n : nullptr, llcs_out);
 }
 
 int lcs_comb_device(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_b, int32_t n,
@@ -836,10 +908,8 @@ int lcs_comb_device(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *
     lcs_schedule chosen{};
     int rc = single_schedule(ctx, nullptr, m, nullptr, n, sched, chosen);
     if (rc) return rc;
-    if (hipEventRecord(ctx->ev0, s) != hipSuccess) return LCS_EIO;
     rc = enqueue_chain(ctx, d_a, m, d_b, n, &chosen, d_h_out, d_v_out, s);
     if (rc) return rc;
-    if (hipEventRecord(ctx->ev1, s) != hipSuccess) return LCS_EIO;
     ctx->pending_timing = true;
     return LCS_OK;
 }

@@ -2,7 +2,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <map>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -18,6 +21,20 @@ struct DevBuf {
     size_t bytes = 0;
     int reserve(lcs_ctx *ctx, size_t want);
     void release(lcs_ctx *ctx);
+};
+
+// Device memory kept between calls that each need some for their own time.  A
+// caller takes it, reserves what it needs, and gives it back once the device
+// is done with it; what is kept is at most kKeptMax bytes and is freed when
+// another buffer needs its share of the budget or of the device's memory.
+// Any thread may give back (an index is destroyed by whoever drops it).
+constexpr size_t kKeptMax = (size_t)256 << 20;
+struct KeptBuf {
+    std::mutex mu;
+    DevBuf buf;
+    DevBuf take(size_t at_least, size_t at_most);   // empty when what is kept does not fit
+    void give(lcs_ctx *ctx, DevBuf &b);
+    void trim(lcs_ctx *ctx);
 };
 
 struct Extras;  // batch / server resources, created on first use
@@ -67,6 +84,7 @@ constexpr int kStickyWord = 63;
 // ctrl word of the byte-symbol flags of single-pair launches; zero between
 // launches (each one's extract kernel clears it)
 constexpr int kSym8FlagWord = 62;
+constexpr int kZeroWord = 61;   // always zero
 }  // namespace lcs
 
 struct lcs_ctx {
@@ -85,7 +103,15 @@ struct lcs_ctx {
     unsigned long long timeout_ticks = 500000000ull;  // 5 s at 100 MHz
     double last_kernel_ms = 0.0;
     bool pending_timing = false;
-    lcs::DevBuf ring, in_a, in_b, out_h, out_v, descs, strip_ws, perm;
+    // events around the last timed call's kernels (of ev0, ev1, evc0, evc1)
+    hipEvent_t time_from = nullptr, time_to = nullptr;
+    lcs::DevBuf ring, strings, results, descs, strip_ws;   // strings, results: of the host calls
+    void *pinned = nullptr;              // host staging of strings and results, at most lcs::kPinnedMax bytes
+    size_t pinned_bytes = 0;
+    lcs::KeptBuf scratch;                // braid products and index builds
+    lcs::KeptBuf index_mem;              // the memory of a destroyed index
+    // false once the context is destroyed: an index dropped later frees its own memory
+    std::shared_ptr<std::atomic<bool>> alive = std::make_shared<std::atomic<bool>>(true);
     lcs::DevBuf sym8;                    // byte copies of b and their range flag (single-pair chains)
     // The shared workspace (ring, descriptors, ctrl words) is used by one
     // launch at a time: a call on another stream first waits for ws_done,
@@ -102,8 +128,13 @@ struct lcs_ctx {
 namespace lcs {
 int enqueue_chain(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_b, int32_t n,
                   const lcs_schedule *sched, int32_t *d_h, int32_t *d_v, hipStream_t stream,
-                  const int32_t *d_h_in = nullptr, const int32_t *d_v_in = nullptr);
+                  const int32_t *d_h_in = nullptr, const int32_t *d_v_in = nullptr, int32_t *d_r2c = nullptr,
+                  int32_t *d_status = nullptr);
 int check_abort(lcs_ctx *ctx);
+// Host staging of host single-pair calls up to this size; larger ones are
+// copied straight from and to the caller's memory.
+constexpr size_t kPinnedMax = (size_t)4 << 20;
+void *pinned_staging(lcs_ctx *ctx, size_t bytes);
 // order a call on `s` after the previous user of the shared workspace, and
 // mark `s` as its latest user once the call's kernels are enqueued
 int ws_acquire(lcs_ctx *ctx, hipStream_t s);

@@ -141,12 +141,11 @@ int run_host(lcs_ctx *ctx, int32_t npairs, const int32_t *a_all, const int64_t *
         a_len = std::max<int64_t>(a_len, a_off[p] + m[p]);
         b_len = std::max<int64_t>(b_len, b_off[p] + n[p]);
     }
-    int rc = ctx->in_a.reserve(ctx, (size_t)std::max<int64_t>(a_len, 1) * 4);
-    if (!rc) rc = ctx->in_b.reserve(ctx, (size_t)std::max<int64_t>(b_len, 1) * 4);
-    if (!rc) rc = ctx->out_h.reserve(ctx, (size_t)std::max(npairs, 1) * 4);
+    int rc = ctx->strings.reserve(ctx, (size_t)std::max<int64_t>(a_len + b_len, 1) * 4);
+    if (!rc) rc = ctx->results.reserve(ctx, (size_t)std::max(npairs, 1) * 4);
     if (rc) return rc;
     hipStream_t s = ctx->stream;
-    int32_t *da = (int32_t *)ctx->in_a.ptr, *db = (int32_t *)ctx->in_b.ptr, *dout = (int32_t *)ctx->out_h.ptr;
+    int32_t *da = (int32_t *)ctx->strings.ptr, *db = da + a_len, *dout = (int32_t *)ctx->results.ptr;
     if (a_len && hipMemcpyAsync(da, a_all, (size_t)a_len * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
     if (b_len && hipMemcpyAsync(db, b_all, (size_t)b_len * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
     std::vector<LlcsPair> pairs((size_t)npairs);
@@ -155,6 +154,8 @@ int run_host(lcs_ctx *ctx, int32_t npairs, const int32_t *a_all, const int64_t *
     if (hipEventRecord(ctx->ev0, s) != hipSuccess) return LCS_EIO;
     if ((rc = enqueue_llcs(ctx, pairs, sigma, s))) return rc;
     if (hipEventRecord(ctx->ev1, s) != hipSuccess) return LCS_EIO;
+    ctx->time_from = ctx->ev0;
+    ctx->time_to = ctx->ev1;
     ctx->pending_timing = true;
     if (hipMemcpyAsync(out, dout, (size_t)npairs * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
@@ -186,6 +187,8 @@ extern "C" int lcs_llcs_device(lcs_ctx *ctx, const int32_t *d_a, int32_t m, cons
     int rc = enqueue_llcs(ctx, pairs, sigma, s);
     if (rc) return rc;
     if (hipEventRecord(ctx->ev1, s) != hipSuccess) return LCS_EIO;
+    ctx->time_from = ctx->ev0;
+    ctx->time_to = ctx->ev1;
     ctx->pending_timing = true;
     return LCS_OK;
 }

@@ -16,6 +16,8 @@ struct lcs_dominance_index {
     lcs_ctx *ctx = nullptr;
     int32_t size = 0;
     int levels = 0;
+    int device = 0;
+    std::shared_ptr<std::atomic<bool>> alive;
     DevBuf mem;   // RankWord words[levels * W], then uint32 zeros[levels]
     DevBuf io;    // query staging for the host entry point
     lcsq::RankWord *words() const { return (lcsq::RankWord *)mem.ptr; }
@@ -49,15 +51,24 @@ int build_index(lcs_ctx *ctx, const int32_t *src, bool src_on_host, int32_t size
     auto *idx = new (std::nothrow) lcs_dominance_index;
     if (!idx) return LCS_ENOMEM;
     idx->ctx = ctx;
+    idx->device = ctx->device;
+    idx->alive = ctx->alive;
     idx->size = size;
     idx->levels = size > 0 ? bit_length(size) : 0;
     hipStream_t s = ctx->stream;
     int rc = LCS_OK;
     if (size > 0) {
         const size_t W = ((size_t)size >> 6) + 1, nb = (W + 63) / 64;
-        rc = idx->mem.reserve(ctx, idx->words_bytes() + (size_t)idx->levels * 4);
+        // the memory of a destroyed index and the builds' scratch are kept
+        const size_t need = idx->words_bytes() + (size_t)idx->levels * 4;
+        const size_t scratch_bytes = (2 * (size_t)size + nb + 1 + (src_on_host ? (size_t)size : 0)) * 4;
+        idx->mem = ctx->index_mem.take(need, 2 * need);
+        rc = idx->mem.reserve(ctx, need);
         DevBuf scratch;
-        if (!rc) rc = scratch.reserve(ctx, (2 * (size_t)size + nb + 1 + (src_on_host ? (size_t)size : 0)) * 4);
+        if (!rc) {
+            scratch = ctx->scratch.take(scratch_bytes, kKeptMax);
+            rc = scratch.reserve(ctx, scratch_bytes);
+        }
         if (!rc) {
             int32_t *sc = (int32_t *)scratch.ptr;
             int32_t *bad = sc + 2 * (size_t)size + nb;
@@ -75,7 +86,8 @@ int build_index(lcs_ctx *ctx, const int32_t *src, bool src_on_host, int32_t size
                      hipStreamSynchronize(s) == hipSuccess;
             rc = !ok ? LCS_EIO : flag ? LCS_EINVAL : LCS_OK;
         }
-        scratch.release(ctx);
+        if (rc == LCS_EIO) scratch.release(ctx);   // waits for what was enqueued
+        ctx->scratch.give(ctx, scratch);
     }
     if (rc) {
         lcs_dominance_index_destroy(idx);
@@ -219,17 +231,24 @@ extern "C" int lcs_dominance_index_query_device(lcs_dominance_index *idx, int32_
 
 extern "C" int64_t lcs_dominance_index_bytes(const lcs_dominance_index *idx)
 {
-    return idx ? (int64_t)idx->mem.bytes : 0;
+    return idx && idx->size ? (int64_t)(idx->words_bytes() + (size_t)idx->levels * 4) : 0;
 }
 
 extern "C" void lcs_dominance_index_destroy(lcs_dominance_index *idx)
 {
     if (!idx) return;
+    if (!idx->alive->load()) {
+        (void)hipSetDevice(idx->device);
+        if (idx->mem.ptr) (void)hipFree(idx->mem.ptr);
+        if (idx->io.ptr) (void)hipFree(idx->io.ptr);
+        delete idx;
+        return;
+    }
     if (idx->mem.ptr || idx->io.ptr) {
         (void)hipSetDevice(idx->ctx->device);
         (void)hipStreamSynchronize(idx->ctx->stream);
     }
-    idx->mem.release(idx->ctx);
+    idx->ctx->index_mem.give(idx->ctx, idx->mem);
     idx->io.release(idx->ctx);
     delete idx;
 }

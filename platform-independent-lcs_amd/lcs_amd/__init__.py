@@ -226,7 +226,7 @@ class Context:
                             ctypes.byref(sched) if sched is not None else None,
                             _p(h), _p(v), ctypes.byref(llcs))
         _check("lcs_comb", rc)
-        return h[: a.size].copy(), v[: b.size].copy(), llcs.value
+        return h[: a.size], v[: b.size], llcs.value
 
     def comb_permutation(self, a, b, sched: Schedule | None = None):
         """(row_to_col, col_to_row, llcs) of a against b, the permutation built
@@ -253,7 +253,7 @@ class Context:
         out = np.empty(max(p.size + q.size - k, 1), np.int32)
         _check("lcs_braid_multiply", lib().lcs_braid_multiply(self._h, _p(p), p.size, _p(q), q.size, k,
                                                               int(bool(row_glue)), _p(out)))
-        return out[: p.size + q.size - k].copy()
+        return out[: p.size + q.size - k]
 
     def autotune(self, m: int, n: int, alphabet: int, rate: float, candidates, mode: int = 1, reps: int = 2,
                  seed: int = 1) -> np.ndarray:
@@ -295,14 +295,14 @@ class Context:
         out = np.empty(max(qi.size, 1), np.int32)
         _check("lcs_semilocal_string_substring", lib().lcs_semilocal_string_substring(
             self._h, _p(p), m, n, _p(qi), _p(qj), qi.size, _p(out)))
-        return out[: qi.size].copy()
+        return out[: qi.size]
 
     def dominance(self, row_to_col, qr, qc) -> np.ndarray:
         p, qr, qc = _i32(row_to_col), _i32(qr), _i32(qc)
         out = np.empty(max(qr.size, 1), np.int32)
         _check("lcs_permutation_dominance", lib().lcs_permutation_dominance(
             self._h, _p(p), p.size, _p(qr), _p(qc), qr.size, _p(out)))
-        return out[: qr.size].copy()
+        return out[: qr.size]
 
     def llcs(self, a, b, sigma: int) -> int:
         """LCS length by the bit-parallel kernel (symbols in [0, sigma))."""
@@ -333,7 +333,7 @@ class Context:
         _check("lcs_llcs_batch", lib().lcs_llcs_batch(
             self._h, npairs, _p(a_all), a_off.ctypes.data_as(_i64p), _p(m), _p(b_all),
             b_off.ctypes.data_as(_i64p), _p(n), sigma, _p(out)))
-        return out[:npairs].copy()
+        return out[:npairs]
 
     def semilocal(self, row_to_col, m: int, n: int, kind: int, q0, q1) -> np.ndarray:
         """Quadrant queries (SEMI_*) read from P(a, b) on the GPU."""
@@ -341,7 +341,7 @@ class Context:
         out = np.empty(max(q0.size, 1), np.int32)
         _check("lcs_semilocal_query", lib().lcs_semilocal_query(
             self._h, _p(p), m, n, kind, _p(q0), _p(q1), q0.size, _p(out)))
-        return out[: q0.size].copy()
+        return out[: q0.size]
 
     def batch_comb(self, a_list, b_list, scheds=None, use_graph: bool = True):
         """Comb every pair (a_list[p], b_list[p]) in one batched launch."""
@@ -389,7 +389,7 @@ class DominanceIndex:
         out = np.empty(max(q0.size, 1), np.int32)
         _check("lcs_dominance_index_query", lib().lcs_dominance_index_query(
             self._h, m, n, kind, _p(q0), _p(q1), q0.size, _p(out)))
-        return out[: q0.size].copy()
+        return out[: q0.size]
 
     def query_device(self, m: int, n: int, kind: int, d_q0: int, d_q1: int, nq: int, d_out: int) -> None:
         _check("lcs_dominance_index_query_device", lib().lcs_dominance_index_query_device(
@@ -560,7 +560,7 @@ class Server:
         h = np.empty(max(m, 1), np.int32)
         v = np.empty(max(n, 1), np.int32)
         _check("lcs_server_wait", lib().lcs_server_wait(self._h, rid, _p(h), _p(v), timeout_ms))
-        return h[:m].copy(), v[:n].copy()
+        return h[:m], v[:n]
 
     def times(self, rid: int):
         q, t = ctypes.c_double(), ctypes.c_double()
@@ -592,7 +592,7 @@ def from_strands(h, v):
     c2r = np.empty(max(size, 1), np.int32)
     _check("lcs_permutation_from_strands",
            lib().lcs_permutation_from_strands(_p(h), h.size, _p(v), v.size, _p(r2c), _p(c2r)))
-    return r2c[:size].copy(), c2r[:size].copy()
+    return r2c[:size], c2r[:size]
 
 
 def perm_hash(col_to_row) -> int:
