@@ -228,8 +228,9 @@ int lcs_semilocal_query(lcs_ctx *ctx, const int32_t *row_to_col, int32_t m, int3
 /* A device-resident dominance index (wavelet matrix over row_to_col + 1):
  * each query costs O(log size) dependent loads instead of a scan of the
  * permutation.  row_to_col must hold values in [-1, size) (-1 = unset);
- * anything else is LCS_EINVAL.  The index holds ceil(log2(size+1)) levels of
- * 16 bytes per 64 rows, charged to the context's HBM budget; destroy it
+ * anything else is LCS_EINVAL.  The index holds two of ceil(log2(size+1))
+ * value bits per level, 16 bytes per 32 rows (the last of an odd number of
+ * bits: 16 per 64), charged to the context's HBM budget; destroy it
  * before the context.  No counterpart in the reference (it reads no scores
  * from its permutations).
  *   _build: host row_to_col; _build_device: device row_to_col (both

@@ -18,11 +18,10 @@ struct lcs_dominance_index {
     int levels = 0;
     int device = 0;
     std::shared_ptr<std::atomic<bool>> alive;
-    DevBuf mem;   // RankWord words[levels * W], then uint32 zeros[levels]
+    DevBuf mem;
     DevBuf io;    // query staging for the host entry point
-    lcsq::RankWord *words() const { return (lcsq::RankWord *)mem.ptr; }
-    uint32_t *zeros() const { return (uint32_t *)((char *)mem.ptr + words_bytes()); }
-    size_t words_bytes() const { return (size_t)levels * (((size_t)size >> 6) + 1) * sizeof(lcsq::RankWord); }
+    lcsq::IndexView view() const { return lcsq::index_view(mem.ptr, size, levels); }
+    size_t mem_bytes() const { return size > 0 ? lcsq::index_bytes(size, levels) : 0; }
 };
 
 namespace {
@@ -58,10 +57,9 @@ int build_index(lcs_ctx *ctx, const int32_t *src, bool src_on_host, int32_t size
     hipStream_t s = ctx->stream;
     int rc = LCS_OK;
     if (size > 0) {
-        const size_t W = ((size_t)size >> 6) + 1, nb = (W + 63) / 64;
         // the memory of a destroyed index and the builds' scratch are kept
-        const size_t need = idx->words_bytes() + (size_t)idx->levels * 4;
-        const size_t scratch_bytes = (2 * (size_t)size + nb + 1 + (src_on_host ? (size_t)size : 0)) * 4;
+        const size_t need = idx->mem_bytes(), words = lcsq::build_scratch_words(size);
+        const size_t scratch_bytes = (words + (src_on_host ? (size_t)size : 0)) * 4;
         idx->mem = ctx->index_mem.take(need, 2 * need);
         rc = idx->mem.reserve(ctx, need);
         DevBuf scratch;
@@ -71,15 +69,15 @@ int build_index(lcs_ctx *ctx, const int32_t *src, bool src_on_host, int32_t size
         }
         if (!rc) {
             int32_t *sc = (int32_t *)scratch.ptr;
-            int32_t *bad = sc + 2 * (size_t)size + nb;
+            int32_t *bad = sc + words - 1;
             const int32_t *perm = src;
-            bool ok = hipMemsetAsync(bad, 0, 4, s) == hipSuccess;
-            if (ok && src_on_host) {
+            bool ok = true;
+            if (src_on_host) {
                 int32_t *staged = bad + 1;
                 ok = hipMemcpyAsync(staged, src, (size_t)size * 4, hipMemcpyHostToDevice, s) == hipSuccess;
                 perm = staged;
             }
-            if (ok) ok = lcsq_launch_index_build(perm, size, idx->levels, idx->words(), idx->zeros(), sc, s) == 0;
+            if (ok) ok = lcsq_launch_index_build(perm, idx->view(), sc, s) == 0;
             int32_t flag = 0;
             if (ok)
                 ok = hipMemcpyAsync(&flag, bad, 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
@@ -109,8 +107,7 @@ int query_index_host(lcs_dominance_index *idx, int32_t m, int32_t n, int32_t kin
     bool ok = hipMemcpyAsync(d0, q0, (size_t)nq * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
               hipMemcpyAsync(d1, q1, (size_t)nq * 4, hipMemcpyHostToDevice, s) == hipSuccess;
     if (ok)
-        ok = lcsq_launch_index_query(idx->words(), idx->zeros(), idx->levels, idx->size, kind, m, n, d0, d1, nq, dout,
-                                     s) == 0;
+        ok = lcsq_launch_index_query(idx->view(), kind, m, n, d0, d1, nq, dout, s) == 0;
     if (ok)
         ok = hipMemcpyAsync(out, dout, (size_t)nq * 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
              hipStreamSynchronize(s) == hipSuccess;
@@ -139,7 +136,7 @@ int query_scan_host(lcs_ctx *ctx, const int32_t *row_to_col, int32_t m, int32_t 
 }
 
 // A direct count reads every row per query (about 30 us per query at 2^21
-// rows on MI355X); the index costs 0.3-0.6 ms to build and then answers
+// rows on MI355X); the index costs 0.1 ms to build at 2^19 rows and then answers
 // billions of queries per second.  Past ~2^25 scanned rows the index wins.
 bool prefer_index(int32_t size, int32_t nq) { return (double)size * nq > (double)(1 << 25); }
 
@@ -223,15 +220,14 @@ extern "C" int lcs_dominance_index_query_device(lcs_dominance_index *idx, int32_
     if (!valid_kind(kind) || m < 0 || n < 0 || (int64_t)m + n != idx->size) return LCS_EINVAL;
     if (nq == 0) return LCS_OK;
     if (hipSetDevice(idx->ctx->device) != hipSuccess) return LCS_EIO;
-    return lcsq_launch_index_query(idx->words(), idx->zeros(), idx->levels, idx->size, kind, m, n, d_q0, d_q1, nq,
-                                   d_out, idx->ctx->stream) == 0
+    return lcsq_launch_index_query(idx->view(), kind, m, n, d_q0, d_q1, nq, d_out, idx->ctx->stream) == 0
                ? LCS_OK
                : LCS_EIO;
 }
 
 extern "C" int64_t lcs_dominance_index_bytes(const lcs_dominance_index *idx)
 {
-    return idx && idx->size ? (int64_t)(idx->words_bytes() + (size_t)idx->levels * 4) : 0;
+    return idx ? (int64_t)idx->mem_bytes() : 0;
 }
 
 extern "C" void lcs_dominance_index_destroy(lcs_dominance_index *idx)
