@@ -387,16 +387,15 @@ static size_t grid_perm_words(int32_t m, int32_t n, const GridPlan &G)
 // Checked against the whole grid of plans at 2^14, 50021 x 70207, 2^16,
 // 200000 and 2^18: the chain within 8 %, the plan it picks within 3 % of the
 // best one measured (200000^2: 20 tiles of 16 rows 7.1 ms, one 10.6).
-constexpr double kLagSteps = 130.0;
+double chain_step_ns(int tm, double bands)
+{
+    return tm == 1 ? (bands < 16 ? 12.9 : 17.4) : tm == 2 ? 21.4 : tm == 4 ? 33.3 : tm == 8 ? 61.4 : 114.4 / 16 * tm;
+}
 static double plan_us(const lcs_ctx *ctx, int32_t m, int32_t n, const GridPlan &G)
 {
     const int32_t H = (m + G.GR - 1) / G.GR, W = (n + G.GC - 1) / G.GC, tiles = G.GR * G.GC;
     const double bands = bands_of(H, W, G.tm), waves = bands * tiles, simds = 4.0 * ctx->num_cus * G.wps;
-    const double step_ns = G.tm == 1   ? (bands * tiles < 16 ? 12.9 : 17.4)
-                           : G.tm == 2 ? 21.4
-                           : G.tm == 4 ? 33.3
-                           : G.tm == 8 ? 61.4
-                                       : 114.4 / 16 * G.tm;
+    const double step_ns = chain_step_ns(G.tm, waves);
     const double rounds = std::ceil(waves / simds), last = std::fmod(waves - 1, simds) / tiles;
     const double steps = std::max(rounds * (W + 64.0) + last * kLagSteps, W + 64.0 + (bands - 1) * kLagSteps);
     double us = steps * step_ns * 1e-3;

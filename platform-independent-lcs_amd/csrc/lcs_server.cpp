@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <condition_variable>
 #include <cstring>
 #include <deque>
@@ -125,6 +126,12 @@ struct Slot {
     Staging staging;               // this slot's own pinned upload buffer
     std::vector<std::shared_ptr<Request>> reqs;
     bool busy = false;
+    double work_us = 0, us = 0;    // SIMD time of its chains, and their time, both predicted
+    Clock::time_point t_launch;
+    double us_left() const
+    {
+        return busy ? std::max(0.0, us - std::chrono::duration<double, std::micro>(Clock::now() - t_launch).count()) : 0.0;
+    }
 };
 
 // A cost model handed over by lcs_server_set_cost_model: the parameters are
@@ -168,6 +175,68 @@ struct lcs_server {
 
 namespace {
 
+// How a slot's requests that bring no schedule are cut: `tile` rows per lane
+// for every pair, or (keep_short) for those longer than one band of it while
+// the others keep the height of their own single band, in a launch of their
+// own before (a slot's launches run one after another).
+struct SlotPlan {
+    int tile;
+    bool keep_short;
+    int tile_of(const Request &R) const
+    {
+        if (R.sched.tile_m) return R.sched.tile_m;
+        return keep_short ? std::min(tile, default_batch_tile_m((int32_t)R.a.size())) : tile;
+    }
+};
+
+// A pair is as slow as its longest band and the lag of the bands above it, so
+// few rows per lane finish it sooner; many rows cost less SIMD time per cell
+// (7.2 ns a row and step at 16, 7.7 at 8, 8.3 at 4, 10.7 at 2).  The plan with
+// the shortest predicted end, given what the other slots still have to do, of
+// those that cost at most a quarter more SIMD time than the cheapest: later
+// requests share the chip.  24 requests with lengths of 1024 to 262144 took
+// 48 ms with 16 rows for every pair of more than 512, 31 with 8, and take 29
+// as planned here.
+SlotPlan plan_slot(lcs_server *S, Slot &slot)
+{
+    const double simds = 4.0 * S->ctx->num_cus;
+    double others = 0;
+    for (auto &o : S->slots)
+        if (o.us > 0) others += o.work_us * o.us_left() / o.us;
+    struct Cost {
+        SlotPlan plan;
+        double work, us;
+    };
+    std::vector<Cost> costs;
+    double cheapest = 0;
+    for (int i = 4; i >= 0; --i)
+        for (const bool keep : {true, false}) {
+            const SlotPlan plan{kTiles[i], keep};
+            double work[kNumTiles] = {}, span[kNumTiles] = {}, all = 0, us = 0;
+            for (auto &R : slot.reqs) {
+                const double m = (double)R->a.size(), n = (double)R->b.size();
+                if (m == 0 || n == 0) continue;
+                const int tm = plan.tile_of(*R), c = class_index(tm, 1);
+                const double bands = std::ceil(m / (64.0 * tm)), us_step = chain_step_ns(tm, bands) * 1e-3;
+                work[c] += bands * (n + 64) * us_step;
+                span[c] = std::max(span[c], (n + 64 + (bands - 1) * kLagSteps) * us_step);
+            }
+            for (int c = 0; c < kNumTiles; ++c) {
+                all += work[c];
+                us += std::max(span[c], work[c] / simds);
+            }
+            costs.push_back(Cost{plan, all, std::max(us, (all + others) / simds)});
+            cheapest = costs.size() > 1 ? std::min(cheapest, all) : all;
+        }
+    const Cost *best = nullptr;
+    for (const Cost &c : costs)
+        if (c.work <= 1.25 * cheapest && (!best || c.us < 0.97 * best->us)) best = &c;
+    slot.work_us = best->work;
+    slot.us = best->us;
+    slot.t_launch = Clock::now();
+    return best->plan;
+}
+
 // Launch the admitted requests of one slot (worker thread).
 int launch_slot(lcs_server *S, Slot &slot)
 {
@@ -189,6 +258,11 @@ int launch_slot(lcs_server *S, Slot &slot)
                         slot.reqs[idx[j]]->sched = S->candidates[(size_t)choice[j]];
         }
     }
+    // the longest first: its bands take the first tickets
+    std::stable_sort(slot.reqs.begin(), slot.reqs.end(), [](const auto &x, const auto &y) {
+        return (double)x->a.size() * x->b.size() > (double)y->a.size() * y->b.size();
+    });
+    const SlotPlan plan = plan_slot(S, slot);
     std::vector<std::vector<PairDesc>> groups(kClasses);
     char *base = (char *)S->arena_base;
     for (auto &R : slot.reqs) {
@@ -200,7 +274,7 @@ int launch_slot(lcs_server *S, Slot &slot)
             return LCS_EIO;
         if (n && hipMemcpyAsync(db, R->b.data(), (size_t)n * 4, hipMemcpyHostToDevice, slot.stream) != hipSuccess)
             return LCS_EIO;
-        const int tm = R->sched.tile_m ? R->sched.tile_m : default_batch_tile_m(m);
+        const int tm = plan.tile_of(*R);
         const int c = class_index(tm, group_width(R->sched.variant));
         if (c < 0) return LCS_EINVAL;
         PairDesc P{};
@@ -238,7 +312,8 @@ int launch_slot(lcs_server *S, Slot &slot)
         if (rc) return rc;
     }
     if (blob.empty()) return hipEventRecord(slot.done, slot.stream) == hipSuccess ? LCS_OK : LCS_EIO;
-    int rc = slot.descs.reserve(ctx, blob.size() + 256);
+    // growing it later would wait for every slot's kernels
+    int rc = slot.descs.reserve(ctx, std::max<size_t>(blob.size() + 256, (size_t)1 << 20));
     if (rc) return rc;
     if ((rc = upload_via(slot.staging, slot.descs.ptr, blob.data(), blob.size(), slot.stream))) return rc;
     for (int c = 0; c < kClasses; ++c) {
