@@ -258,10 +258,6 @@ int launch_slot(lcs_server *S, Slot &slot)
                         slot.reqs[idx[j]]->sched = S->candidates[(size_t)choice[j]];
         }
     }
-    // the longest first: its bands take the first tickets
-    std::stable_sort(slot.reqs.begin(), slot.reqs.end(), [](const auto &x, const auto &y) {
-        return (double)x->a.size() * x->b.size() > (double)y->a.size() * y->b.size();
-    });
     const SlotPlan plan = plan_slot(S, slot);
     std::vector<std::vector<PairDesc>> groups(kClasses);
     char *base = (char *)S->arena_base;
