@@ -598,6 +598,16 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     // made the compiler carry the band's registers over every exit (about 20
     // copies and several branches a chunk).
     int dead = 0;
+    // Byte chains of one or two rows per lane: a chunk of 32 steps is shorter
+    // than the trips through memory, and a band that is just in time prefetches
+    // the words of a chunk before the band above has stored them.  The lines it
+    // then holds make that band's stores slow, and a store two chunks back is
+    // what its next loads queue behind (vmcnt counts both in order), so the
+    // whole chain falls to the pace of its stores and stays there: one row, 16
+    // bands, 100000 columns 1.75 to 2.5 ms, some runs 1.3.  So a band that had
+    // to wait waits for one chunk more (band_slack, comb_kernels.h): 1.33 ms
+    // (50000 columns and 32 bands 1.25 -> 0.73, two rows 1.29 -> 1.09).
+    const int slack = S8 != kSymWords && band_slack(TM, P.nbands, n) ? C : 0;
     auto take_inputs = [&](int t, uint32_t &I, auto inside) {
         const int c = t + (lane & (C - 1));   // lanes >= C repeat lanes < C
         const bool need = decltype(inside)::value || c < n;
@@ -612,13 +622,17 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
             // flag and the clock every few rounds only (each is a memory
             // round trip of its own).
             unsigned long long t_start = 0;
+            int ahead = slack;
 #pragma nounroll
             for (int polls = 0; !dead; ++polls) {
                 // a wave that shares its SIMD with other launches' waves
                 // gives up its issue slots between polls
                 if (A.poll_sleep) __builtin_amdgcn_s_sleep(2);
-                e = ld_relaxed(Ein + min(c, nm1));
-                if (__builtin_amdgcn_ballot_w64(need && (uint32_t)(e >> 32) != tag_in) == 0) break;
+                e = ld_relaxed(Ein + min(c + ahead, nm1));
+                if (__builtin_amdgcn_ballot_w64(need && (uint32_t)(e >> 32) != tag_in) == 0) {
+                    if (ahead == 0) break;
+                    ahead = 0;
+                }
                 if (polls % kRingPolls == 0) {
                     const unsigned long long now = __builtin_amdgcn_s_memrealtime();
                     if (polls == 0) t_start = now;

@@ -28,3 +28,11 @@ def test_wide_symbols_wait_for_no_load_before_the_steps():
     # symbols before the steps, 20
     with lcs_amd.Context(0) as ctx:
         assert chain_ms(ctx, 1, 1, 300) < 1.5 * chain_ms(ctx, 1, 1, 4)
+
+
+@pytest.mark.parametrize("bands", [16, 32])
+def test_a_chain_of_bands_keeps_the_pace_of_one(bands):
+    # 32 bands add 31 lags of about 162 steps to 100064: 1.05 of one band's
+    # time; in step with the stores of the band above them 1.4 to 2.0
+    with lcs_amd.Context(0) as ctx:
+        assert chain_ms(ctx, bands, 1, 4) < 1.3 * chain_ms(ctx, 1, 1, 4)
