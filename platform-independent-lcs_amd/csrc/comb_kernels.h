@@ -63,12 +63,12 @@ int lcsk_launch_sym8(const int32_t *b, int32_t n, uint32_t *out, int32_t stride,
 // Whether a byte chain's bands keep one chunk more than they need between
 // themselves and the band above (band_pass).  It costs 32 steps a band and
 // spares up to half of every step, so it is for bands that are long beside
-// their number.  Measured at 1 row per lane: 32 bands of 16384 columns 0.48 ms
+// their number.  Measured: 32 bands of 16384 columns 0.48 ms
 // without, 0.32 with; 64 of 16384 0.40 and 0.39; 256 of 50000 1.18 and 1.37.
 constexpr int kSlackColumns = 384;   // per band
 __host__ __device__ inline bool band_slack(int tile_m, int32_t nbands, int32_t n)
 {
-    return tile_m <= 2 && n / kSlackColumns > nbands;
+    return tile_m == 1 && n / kSlackColumns > nbands;
 }
 
 // Two pairs combed together by the 16-bit packed chain

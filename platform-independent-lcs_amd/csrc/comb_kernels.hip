@@ -598,7 +598,7 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     // made the compiler carry the band's registers over every exit (about 20
     // copies and several branches a chunk).
     int dead = 0;
-    // Byte chains of one or two rows per lane: a chunk of 32 steps is shorter
+    // Byte chains of one row per lane: a chunk of 32 steps is shorter
     // than the trips through memory, and a band that is just in time prefetches
     // the words of a chunk before the band above has stored them.  The lines it
     // then holds make that band's stores slow, and a store two chunks back is
@@ -606,8 +606,10 @@ __device__ __forceinline__ bool band_pass(const ChainArgs &A, const Desc &P, int
     // whole chain falls to the pace of its stores and stays there: one row, 16
     // bands, 100000 columns 1.75 to 2.5 ms, some runs 1.3.  So a band that had
     // to wait waits for one chunk more (band_slack, comb_kernels.h): 1.33 ms
-    // (50000 columns and 32 bands 1.25 -> 0.73, two rows 1.29 -> 1.09).
-    const int slack = S8 != kSymWords && band_slack(TM, P.nbands, n) ? C : 0;
+    // (50000 columns and 32 bands 1.25 -> 0.73).  Two rows fall to 24 ns a step
+    // from 20 at worst, but the longer poll loop costs them 1 % where it does
+    // not help (50021 x 70207 as a grid 1540 -> 1551 us), so they have none.
+    const int slack = TM == 1 && S8 != kSymWords && band_slack(TM, P.nbands, n) ? C : 0;
     auto take_inputs = [&](int t, uint32_t &I, auto inside) {
         const int c = t + (lane & (C - 1));   // lanes >= C repeat lanes < C
         const bool need = decltype(inside)::value || c < n;

@@ -374,31 +374,42 @@ static size_t grid_perm_words(int32_t m, int32_t n, const GridPlan &G)
     return (size_t)G.GC * m + (size_t)G.GR * n;
 }
 
-// Predicted microseconds of a plan.  The chain: one wave per band and SIMD; a
-// band starts kLagSteps steps after the one above it (64 of lane skew, a chunk
-// of 32 published, a chunk prefetched) and takes W + 64 steps of kStepNs[tm];
-// bands beyond the SIMDs run in further rounds.  Measured on MI355X, one
-// strip, byte symbols (m = 64 tm bands, n = 65536): 12.9 / 21.4 / 33.3 /
-// 61.4 / 114.4 ns a step at 1 / 2 / 4 / 8 / 16 rows per lane (one row: 17.4
-// from 16 bands, where the ring word's trip takes longer than a chunk) and
-// 130 to 138 steps from band to band.  The merges: a level's products share
-// its launches, about 60 us for a core of 2^11 points plus 8 per doubling, and
-// about 0.6 ns per point (k = 2^16 155 us, 2^18 285, eight of 2^16 390).
-// Checked against the whole grid of plans at 2^14, 50021 x 70207, 2^16,
-// 200000 and 2^18: the chain within 8 %, the plan it picks within 3 % of the
-// best one measured (200000^2: 20 tiles of 16 rows 7.1 ms, one 10.6).
-double chain_step_ns(int tm, double bands)
+// The pace of a byte chain: nanoseconds a step, and steps from one band's
+// start to the next one's (64 of lane skew, a chunk of 32 published, a chunk
+// prefetched, and with band_slack a chunk more).  `bands` of one pair with
+// `columns` each, `waves` bands in the whole launch.  Measured on MI355X, one
+// strip, n = 65536, 1 / 8 / 64 bands: 12.6 / 12.6 / 13.7 ns at 1 row per lane,
+// 19.3 / 19.5 / 20.1 at 2, 32.3 / 32.3 / 32.8 at 4, 59.3 / 59.4 / 60.0 at 8 and
+// 112.7 / 112.8 / 113.6 at 16; from 4 rows on 2 % more with every SIMD busy.
+// Without the slack one row takes about 17.4 once
+// a launch's bands lie on several XCDs (n = 4096 .. 50000, from 16 bands), two
+// 20 to 24 in chains of 8 to 64 bands.
+ChainPace chain_pace(int tm, double waves, double bands, double columns)
 {
-    return tm == 1 ? (bands < 16 ? 12.9 : 17.4) : tm == 2 ? 21.4 : tm == 4 ? 33.3 : tm == 8 ? 61.4 : 114.4 / 16 * tm;
+    const bool slack = band_slack(tm, (int32_t)bands, (int32_t)columns);
+    const double lag = slack ? 162.0 : 130.0;
+    if (tm == 1) return {slack ? 13.3 : waves < 16 ? 12.9 : 17.4, lag};
+    return {tm == 2 ? 21.4 : tm == 4 ? 33.3 : tm == 8 ? 61.4 : 114.4 / 16 * tm, lag};
 }
+
+// Predicted microseconds of a plan.  The chain: one wave per band and SIMD, at
+// chain_pace; bands beyond the SIMDs run in further rounds.  The merges: a
+// level's products share its launches, about 60 us for a core of 2^11 points
+// plus 8 per doubling, and about 0.6 ns per point (k = 2^16 155 us, 2^18 285,
+// eight of 2^16 390).  Checked against the whole grid of plans at 2^14,
+// 50021 x 70207, 2^16, 200000 and 2^18: the chain within 8 %, the plan it
+// picks within 3 % of the best one measured (200000^2: 20 tiles of 16 rows
+// 7.1 ms, one 10.6).  Small cores merge faster than that (k = 64 about 15 us a
+// level), so a short a is cut into fewer strips than would be best (64 x
+// 100000: 8 strips 223 us, 32 136, one 1254).
 static double plan_us(const lcs_ctx *ctx, int32_t m, int32_t n, const GridPlan &G)
 {
     const int32_t H = (m + G.GR - 1) / G.GR, W = (n + G.GC - 1) / G.GC, tiles = G.GR * G.GC;
     const double bands = bands_of(H, W, G.tm), waves = bands * tiles, simds = 4.0 * ctx->num_cus * G.wps;
-    const double step_ns = chain_step_ns(G.tm, waves);
+    const ChainPace pace = chain_pace(G.tm, waves, bands, W);
     const double rounds = std::ceil(waves / simds), last = std::fmod(waves - 1, simds) / tiles;
-    const double steps = std::max(rounds * (W + 64.0) + last * kLagSteps, W + 64.0 + (bands - 1) * kLagSteps);
-    double us = steps * step_ns * 1e-3;
+    const double steps = std::max(rounds * (W + 64.0) + last * pace.lag, W + 64.0 + (bands - 1) * pace.lag);
+    double us = steps * pace.step_ns * 1e-3;
     merge_levels(m, n, G.GR, G.GC, [&](int32_t products, int32_t k, int32_t) {
         const int L = std::max(6, lcsb_core_L(k));
         us += 60.0 + 8.0 * std::max(0, L - 11) + 0.6e-3 * products * (double)(1LL << L);
@@ -407,22 +418,28 @@ static double plan_us(const lcs_ctx *ctx, int32_t m, int32_t n, const GridPlan &
 }
 
 // The plan of a pair: the cheapest predicted one with the fields that the
-// schedule fixes (tm, strips; 0 = open).  A pair below kGridMinCells cells, or
-// one with explicit strands, is one tile.
-constexpr double kGridMinCells = 67108864.0;   // 2^26: below it no merge pays (8192^2 0.36 ms as one tile)
+// schedule fixes (tm, strips; 0 = open).  A pair with explicit strands is one
+// tile.  Below kGridMinCells cells a pair is cut only into columns, and from
+// kWideMinN of them: m is then so small that its merges are short beside the
+// columns (64 x 16384 216 us as one tile, 103 as four; 512 x 100000 1268 and
+// 261; 4000 x 16400 446 and 371), while a square one gains nothing (8192^2
+// 0.36 ms as one tile).
+constexpr double kGridMinCells = 67108864.0;   // 2^26
+constexpr int32_t kWideMinN = 16384;
 static GridPlan choose_grid(const lcs_ctx *ctx, int32_t m, int32_t n, int tm, int strips, bool whole, GridPlan G)
 {
     static const int32_t kCols[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64}, kRows[] = {1, 2, 3, 4, 6, 8};
-    const bool open = !whole && !strips && (double)m * n >= kGridMinCells;
+    const bool open_rows = !whole && !strips && (double)m * n >= kGridMinCells;
+    const bool open_cols = open_rows || (!whole && !strips && n >= kWideMinN);
     double best = 0.0;
     GridPlan B = G;
     B.tm = 0;
     for (int32_t t = 1; t <= 16; t *= 2) {
         if (tm && t != (tm < 16 ? tm : 16)) continue;
         for (const int32_t r : kRows) {
-            if (r > 1 && (!open || m / r < 2048 || n > kMaxCoreK)) break;
+            if (r > 1 && (!open_rows || m / r < 2048 || n > kMaxCoreK)) break;
             for (int32_t c : kCols) {
-                if (c > 1 && (!open || n / c < 2048 || m > kMaxCoreK)) break;
+                if (c > 1 && (!open_cols || n / c < 2048 || m > kMaxCoreK)) break;
                 GridPlan T = G;
                 T.tm = tm ? tm : t;
                 T.GR = r;

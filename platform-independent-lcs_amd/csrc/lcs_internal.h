@@ -132,9 +132,11 @@ int enqueue_chain(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_
                   int32_t *d_status = nullptr);
 int check_abort(lcs_ctx *ctx);
 // The register chain's time per step and the steps from one band's start to
-// the next one's, as plan_us (lcs_capi.cpp) measured them.
-double chain_step_ns(int tm, double bands);
-constexpr double kLagSteps = 130.0;
+// the next one's (lcs_capi.cpp).
+struct ChainPace {
+    double step_ns, lag;
+};
+ChainPace chain_pace(int tm, double waves, double bands, double columns);
 // Host staging of host single-pair calls up to this size; larger ones are
 // copied straight from and to the caller's memory.
 constexpr size_t kPinnedMax = (size_t)4 << 20;

@@ -217,9 +217,14 @@ SlotPlan plan_slot(lcs_server *S, Slot &slot)
                 const double m = (double)R->a.size(), n = (double)R->b.size();
                 if (m == 0 || n == 0) continue;
                 const int tm = plan.tile_of(*R), c = class_index(tm, 1);
-                const double bands = std::ceil(m / (64.0 * tm)), us_step = chain_step_ns(tm, bands) * 1e-3;
+                const double bands = std::ceil(m / (64.0 * tm));
+                // (without band_slack, whatever n: its pace would rule one row out of
+                // plans that need it; 20 requests of 100 x 200000 take 11.6 ms
+                // with one row and 15.7 with two)
+                const ChainPace pace = chain_pace(tm, bands, bands, 0);
+                const double us_step = pace.step_ns * 1e-3;
                 work[c] += bands * (n + 64) * us_step;
-                span[c] = std::max(span[c], (n + 64 + (bands - 1) * kLagSteps) * us_step);
+                span[c] = std::max(span[c], (n + 64 + (bands - 1) * pace.lag) * us_step);
             }
             for (int c = 0; c < kNumTiles; ++c) {
                 all += work[c];

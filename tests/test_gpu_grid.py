@@ -61,3 +61,10 @@ def test_plans_agree_with_one_tile(ctx):
         whole = ctx.comb(a, b, lcs_amd.schedule(4, 1, lcs_amd.VARIANT_CHAIN, 1))
         cut = ctx.comb(a, b)
         assert np.array_equal(whole[0], cut[0]) and np.array_equal(whole[1], cut[1])
+
+
+@pytest.mark.parametrize("m,n,alphabet", [(1, 16384, 2), (5, 40001, 300), (64, 100003, 4), (300, 60000, 256),
+                                          (1024, 16385, 40000), (4000, 16400, 20)])
+def test_wide_short_pairs_match_oracle(ctx, m, n, alphabet):
+    # below the cells from which a pair is cut both ways: columns only
+    check(ctx, *pair(m + n, m, n, alphabet))

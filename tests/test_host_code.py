@@ -1,0 +1,65 @@
+"""The library's host code without a GPU: liblcs_hip.so on the recording
+runtime of tests/host_runtime, in a process of its own.  What a call launches,
+what it leaves pending when it returns and what it charges to its budget is
+checked here; the kernels do not run."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PKG = os.path.join(os.path.dirname(HERE), "platform-independent-lcs_amd")
+
+PRELUDE = """
+import ctypes, json, sys
+rec = ctypes.CDLL({rec!r}, mode=ctypes.RTLD_GLOBAL)
+rec.rec_launches.restype = ctypes.c_char_p
+rec.rec_clock.restype = ctypes.c_double
+rec.rec_live.restype = ctypes.c_size_t
+sys.path.insert(0, {pkg!r})
+import numpy as np
+import lcs_amd
+from lcs_amd import lib
+
+def launches(name):
+    return [tuple(map(int, l.split()[1:])) for l in rec.rec_launches().decode().splitlines() if name in l]
+
+def zeros(n):
+    return np.zeros(n, np.int32)
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    if not shutil.which("g++") or not os.path.exists("/opt/rocm/include/hip/hip_runtime.h"):
+        pytest.skip("needs g++ and the HIP headers")
+    rec = str(tmp_path_factory.mktemp("runtime") / "librecording_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", os.path.join(HERE, "host_runtime", "recording_hip.cpp"), "-o", rec], check=True)
+
+    def run(code):
+        """The value that `code` leaves in `result`."""
+        script = PRELUDE.format(rec=rec, pkg=PKG) + code + "\nprint('RESULT', json.dumps(result))\n"
+        done = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=300)
+        assert done.returncode == 0, done.stderr
+        return json.loads([l for l in done.stdout.splitlines() if l.startswith("RESULT ")][-1][7:])
+    return run
+
+
+def test_wide_short_pairs_are_cut(host):
+    # tiles of the launch (grid.y of its seeding kernel): a wide pair is cut
+    # though it has few cells, a square or tall one of that size is not
+    sizes = [(64, 16384), (64, 100000), (1, 1000000), (512, 100000), (2000, 33000), (4000, 16400),
+             (64, 16383), (300, 500), (4096, 4096), (8000, 8000), (100000, 64)]
+    tiles = host(f"""
+result = []
+with lcs_amd.Context(0) as c:
+    for m, n in {sizes}:
+        rec.rec_clear()
+        c.comb(zeros(m), zeros(n))
+        result.append(launches('comb_prep_grid_kernel')[0][1])
+""")
+    assert all(t > 1 for t in tiles[:6]) and tiles[6:] == [1] * 5, tiles
