@@ -850,23 +850,28 @@ static int comb_host(lcs_ctx *ctx, const int32_t *a, int32_t m, const int32_t *b
     int32_t *da = (int32_t *)ctx->strings.ptr, *db = da + a_words;
     int32_t *dstatus = (int32_t *)ctx->results.ptr, *dr2c = dstatus + kStatusWords, *dv = dr2c + perm_words, *dh = dv + n;
     hipStream_t s = ctx->stream;
+    // an error leaves no copy of the staging or the caller's memory queued
+    const auto drained = [s](int rc) {
+        (void)hipStreamSynchronize(s);
+        return rc;
+    };
     int32_t *pin = in_bytes + out_bytes <= kPinnedMax ? (int32_t *)pinned_staging(ctx, in_bytes + out_bytes) : nullptr;
     if (pin) {
         if (m) std::memcpy(pin, a, mm * 4);
         if (n) std::memcpy(pin + a_words, b, nn * 4);
-        if (in_bytes && hipMemcpyAsync(da, pin, in_bytes, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
+        if (in_bytes && hipMemcpyAsync(da, pin, in_bytes, hipMemcpyHostToDevice, s) != hipSuccess) return drained(LCS_EIO);
     } else {
-        if (m && hipMemcpyAsync(da, a, mm * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
-        if (n && hipMemcpyAsync(db, b, nn * 4, hipMemcpyHostToDevice, s) != hipSuccess) return LCS_EIO;
+        if (m && hipMemcpyAsync(da, a, mm * 4, hipMemcpyHostToDevice, s) != hipSuccess) return drained(LCS_EIO);
+        if (n && hipMemcpyAsync(db, b, nn * 4, hipMemcpyHostToDevice, s) != hipSuccess) return drained(LCS_EIO);
     }
     if ((rc = enqueue_chain(ctx, da, m, db, n, &chosen, dh, dv, s, nullptr, nullptr, r2c ? dr2c : nullptr, dstatus)))
-        return rc;
+        return drained(rc);
     int32_t status = 0;
     if (pin) {
         int32_t *res = pin + in_bytes / 4;
         if (hipMemcpyAsync(res, dstatus, out_bytes, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess)
-            return LCS_EIO;
+            return drained(LCS_EIO);
         status = res[0];
         if (!status) {
             res += kStatusWords;
@@ -875,12 +880,12 @@ static int comb_host(lcs_ctx *ctx, const int32_t *a, int32_t m, const int32_t *b
             if (m) std::memcpy(h_out, res + perm_words + nn, mm * 4);
         }
     } else {
-        if (perm_words && hipMemcpyAsync(r2c, dr2c, perm_words * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
-        if (n && hipMemcpyAsync(v_out, dv, nn * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
-        if (m && hipMemcpyAsync(h_out, dh, mm * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return LCS_EIO;
+        if (perm_words && hipMemcpyAsync(r2c, dr2c, perm_words * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return drained(LCS_EIO);
+        if (n && hipMemcpyAsync(v_out, dv, nn * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return drained(LCS_EIO);
+        if (m && hipMemcpyAsync(h_out, dh, mm * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return drained(LCS_EIO);
         if (hipMemcpyAsync(&status, dstatus, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess)
-            return LCS_EIO;
+            return drained(LCS_EIO);
     }
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, ctx->time_from, ctx->time_to) == hipSuccess) ctx->last_kernel_ms = ms;

@@ -63,3 +63,18 @@ with lcs_amd.Context(0) as c:
         result.append(launches('comb_prep_grid_kernel')[0][1])
 """)
     assert all(t > 1 for t in tiles[:6]) and tiles[6:] == [1] * 5, tiles
+
+
+def test_a_refused_pair_leaves_no_copy_queued(host):
+    # the schedule is looked at after the strings are staged
+    assert host("""
+result = []
+with lcs_amd.Context(0) as c:
+    for m, sched in ((300, lcs_amd.schedule(3, 1, lcs_amd.VARIANT_CHAIN, 1)), (300, lcs_amd.schedule(4, 1, 99, 1)),
+                     (300, lcs_amd.schedule(4, 9, lcs_amd.VARIANT_CHAIN, 1))):
+        for call in (c.comb, c.comb_permutation):
+            try:
+                call(zeros(m), zeros(500), sched)
+            except lcs_amd.LcsError:
+                result.append(rec.rec_pending())
+""") == [0] * 6
