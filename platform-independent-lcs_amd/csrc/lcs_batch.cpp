@@ -477,6 +477,7 @@ int batch_core(lcs_ctx *ctx, Extras *X, int32_t npairs, const int32_t *da, const
         return LCS_OK;
     };
     if (hipStreamSynchronize(s) != hipSuccess) return LCS_EIO;
+    ctx->pending_timing = false;   // of an asynchronous call before, whose events the launches record anew
     if ((rc = run_launches(ctx, X, classes, launches, use_graph != 0, merges))) return rc;
     if (hipStreamSynchronize(s) != hipSuccess) return LCS_EIO;
     float ms = 0.f;

@@ -59,6 +59,7 @@ extern "C" int lcs_braid_multiply(lcs_ctx *ctx, const int32_t *p_row_to_col, int
         ok = (!p_size || hipMemcpyAsync(dp, p_row_to_col, (size_t)p_size * 4, hipMemcpyHostToDevice, s) == hipSuccess) &&
              (!q_size || hipMemcpyAsync(dq, q_row_to_col, (size_t)q_size * 4, hipMemcpyHostToDevice, s) == hipSuccess);
     }
+    ctx->pending_timing = false;   // its events are recorded anew
     if (!ok || hipEventRecord(ctx->ev0, s) != hipSuccess) { buf.release(ctx); return LCS_EIO; }
     rc = lcsb_multiply_device(dp, p_size, dq, q_size, k, row_glue ? 1 : 0, dout, dws, s);
     if (!rc) {
@@ -68,7 +69,6 @@ extern "C" int lcs_braid_multiply(lcs_ctx *ctx, const int32_t *p_row_to_col, int
         rc = ok ? LCS_OK : LCS_EIO;
         float ms = 0.f;
         if (ok && pin) std::memcpy(out_row_to_col, pin + in_words, (size_t)out_size * 4);
-        if (ok) ctx->pending_timing = false;
         if (ok && hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess) ctx->last_kernel_ms = ms;
     }
     if (rc) buf.release(ctx);   // waits for what was enqueued

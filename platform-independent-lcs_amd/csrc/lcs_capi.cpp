@@ -551,6 +551,7 @@ static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, int32_t 
     A.trace_cap = ctx->band_trace_cap;
     const long long per_cu = G.group_w == 1 ? 4LL : 1LL, resident = per_cu * ctx->num_cus * G.wps;
     const long long blocks = (std::min(units, resident) + per_cu - 1) / per_cu;
+    ctx->pending_timing = false;   // its events are recorded anew
     if (hipEventRecord(ctx->evc0, stream) != hipSuccess) return LCS_EIO;
     if ((rc = lcsk_launch_grid(A, (int)blocks, 256, stream))) return rc;
     if (hipEventRecord(ctx->evc1, stream) != hipSuccess) return LCS_EIO;
@@ -598,6 +599,7 @@ static int enqueue_chain_ws(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const i
                             const int32_t *d_h_in, const int32_t *d_v_in, int32_t *d_r2c, int32_t *d_status)
 {
     if (m == 0 || n == 0) {
+        ctx->pending_timing = false;   // its events are recorded anew
         ctx->time_from = ctx->ev0;
         ctx->time_to = ctx->ev1;
         bool ok = hipEventRecord(ctx->ev0, stream) == hipSuccess;
@@ -657,6 +659,17 @@ void *pinned_staging(lcs_ctx *ctx, size_t bytes)
     ctx->pinned = p;
     ctx->pinned_bytes = want;
     return p;
+}
+
+// Reads the time of an asynchronous call off its events (waiting for them),
+// before a call that times nothing itself records into the same ones.
+void settle_timing(lcs_ctx *ctx)
+{
+    float ms = 0.f;
+    if (ctx->pending_timing && hipEventSynchronize(ctx->time_to) == hipSuccess &&
+        hipEventElapsedTime(&ms, ctx->time_from, ctx->time_to) == hipSuccess)
+        ctx->last_kernel_ms = ms;
+    ctx->pending_timing = false;
 }
 
 // The abort flag of the last launch on the context's own ctrl words (the
@@ -803,11 +816,7 @@ int lcs_ctx_set_timeout(lcs_ctx *ctx, uint64_t ticks)
 int lcs_ctx_info(lcs_ctx *ctx, int32_t *num_cus, double *last_kernel_ms)
 {
     if (!ctx) return LCS_EINVAL;
-    if (ctx->pending_timing && hipEventQuery(ctx->time_to) == hipSuccess) {
-        float ms = 0.f;
-        if (hipEventElapsedTime(&ms, ctx->time_from, ctx->time_to) == hipSuccess) ctx->last_kernel_ms = ms;
-        ctx->pending_timing = false;
-    }
+    if (ctx->pending_timing && hipEventQuery(ctx->time_to) == hipSuccess) settle_timing(ctx);
     if (num_cus) *num_cus = ctx->num_cus;
     if (last_kernel_ms) *last_kernel_ms = ctx->last_kernel_ms;
     return LCS_OK;

@@ -34,6 +34,7 @@ extern "C" int lcs_comb_fixup(lcs_ctx *ctx, const int32_t *a_prepared, int32_t m
               hipMemcpyAsync(db, b + j0, (size_t)jsize * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
               hipMemcpyAsync(dvin, v + j0, (size_t)jsize * 4, hipMemcpyHostToDevice, s) == hipSuccess;
     if (!ok) { tmp.release(ctx); return LCS_EIO; }
+    settle_timing(ctx);
     rc = enqueue_chain(ctx, da, isize, db, jsize, nullptr, dhout, dvout, s, dhin, dvin);
     if (!rc) {
         ok = hipMemcpyAsync(h + i0, dhout, (size_t)isize * 4, hipMemcpyDeviceToHost, s) == hipSuccess &&

@@ -131,6 +131,7 @@ int enqueue_chain(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_
                   const int32_t *d_h_in = nullptr, const int32_t *d_v_in = nullptr, int32_t *d_r2c = nullptr,
                   int32_t *d_status = nullptr);
 int check_abort(lcs_ctx *ctx);
+void settle_timing(lcs_ctx *ctx);
 // The register chain's time per step and the steps from one band's start to
 // the next one's (lcs_capi.cpp).
 struct ChainPace {

@@ -78,3 +78,32 @@ with lcs_amd.Context(0) as c:
             except lcs_amd.LcsError:
                 result.append(rec.rec_pending())
 """) == [0] * 6
+
+
+@pytest.mark.parametrize("n", [500, 100000])   # one tile; columns cut and merged
+def test_the_time_reported_is_the_last_calls_own(host, n):
+    # 1 ms a launch.  A device pair's time is read off its events later; a
+    # batch or a product after it reports its own, a fixup (which reports
+    # none) leaves the pair's
+    got = host(f"""
+def after(call, pair):
+    with lcs_amd.Context(0) as c:
+        if pair:
+            dev = [np.zeros({n} + 300, np.int32) for _ in range(4)]
+            lcs_amd._check("lcs_comb_device", lib().lcs_comb_device(
+                c.handle, dev[0].ctypes.data, 300, dev[1].ctypes.data, {n}, None, dev[2].ctypes.data, dev[3].ctypes.data, None))
+            if call is None:
+                return c.info()[1]
+        call(c)
+        return c.info()[1]
+
+def fixup(c):
+    h, v = np.arange(70, dtype=np.int32), np.arange(70, 150, dtype=np.int32)
+    c.comb_fixup(zeros(70), zeros(80), h, v, 0, 70, 0, 80)
+
+batch = lambda c: c.batch_comb([zeros(100)] * 3, [zeros(200)] * 3, use_graph=False)
+product = lambda c: c.braid_multiply(np.arange(50, dtype=np.int32), np.arange(60, dtype=np.int32), 20, False)
+result = [after(batch, False), after(batch, True), after(product, False), after(product, True), after(None, True),
+          after(fixup, True)]
+""")
+    assert got[0] == got[1] and got[2] == got[3] and got[4] == got[5] and min(got) > 0, got
