@@ -44,18 +44,32 @@ void KeptBuf::trim(lcs_ctx *ctx)
     buf.release(ctx);
 }
 
-static void trim_kept(lcs_ctx *ctx)
+// Frees what the context keeps for later calls and no call is using: products'
+// and index builds' memory, and the single-pair workspaces that the call under
+// way has not reserved.  (hipFree waits for the kernels that still use them.)
+static void trim_kept(lcs_ctx *ctx, const DevBuf *reserving)
 {
     ctx->scratch.trim(ctx);
     ctx->index_mem.trim(ctx);
+    DevBuf *const bufs[] = {&ctx->ring, &ctx->strip_ws, &ctx->sym8};
+    for (int i = 0; i < 3; ++i)
+        if (!(ctx->ws_reserved >> i & 1) && bufs[i] != reserving) bufs[i]->release(ctx);
+}
+
+int reserve_ws(lcs_ctx *ctx, PairWs which, size_t bytes)
+{
+    DevBuf &buf = which == kWsRing ? ctx->ring : which == kWsStrips ? ctx->strip_ws : ctx->sym8;
+    const int rc = buf.reserve(ctx, bytes);
+    if (!rc) ctx->ws_reserved |= 1u << which;
+    return rc;
 }
 
 int DevBuf::reserve(lcs_ctx *ctx, size_t want)
 {
     if (want <= bytes) return LCS_OK;
     size_t grow = std::max(want, bytes + bytes / 2);
-    if (ctx->held + grow - bytes > ctx->budget) trim_kept(ctx);
     if (ctx->held + grow - bytes > ctx->budget) grow = want;
+    if (ctx->held + grow - bytes > ctx->budget) trim_kept(ctx, this);
     if (ctx->held + grow - bytes > ctx->budget) return LCS_ENOMEM;
     if (ptr) {
         (void)hipFree(ptr);
@@ -66,7 +80,7 @@ int DevBuf::reserve(lcs_ctx *ctx, size_t want)
     void *p = nullptr;
     if (hipMalloc(&p, grow) != hipSuccess) {
         (void)hipGetLastError();
-        trim_kept(ctx);
+        trim_kept(ctx, this);
         if (hipMalloc(&p, grow) != hipSuccess) {
             (void)hipGetLastError();
             return LCS_ENOMEM;
@@ -519,23 +533,25 @@ static int enqueue_grid(lcs_ctx *ctx, const PairDesc &pair, GridPlan G, int32_t 
     const int32_t tiles = T.GR * T.GC;
     T.pair.tile_m = G.tm;
     T.pair.nbands = bands_of(T.H, T.W, G.tm);
-    int rc = ctx->ring.reserve(ctx, (size_t)tiles * lcsk_ring_words(T.W) * sizeof(unsigned long long));
+    // what the call cannot do without first; the byte copies take what is left
+    ctx->ws_reserved = 0;
+    int rc = reserve_ws(ctx, kWsRing, (size_t)tiles * lcsk_ring_words(T.W) * sizeof(unsigned long long));
     if (rc) return rc;
+    size_t perm_words = 0;
+    if (tiles > 1) {
+        perm_words = grid_perm_words(m, n, G);
+        if ((rc = reserve_ws(ctx, kWsStrips, (2 * perm_words + grid_merge_words(m, n, G)) * 4))) return rc;
+        T.perm = (int32_t *)ctx->strip_ws.ptr;
+    }
     T.pair.E = (unsigned long long *)ctx->ring.ptr;
     if (n <= kSym8MaxN) {
         const int32_t stride = lcsk_sym8_stride(T.W);
-        if (ctx->sym8.reserve(ctx, (size_t)T.GC * 16 * (size_t)stride) == LCS_OK) {
+        if (reserve_ws(ctx, kWsSym8, (size_t)T.GC * 16 * (size_t)stride) == LCS_OK) {
             T.pair.sym8 = (const uint32_t *)ctx->sym8.ptr;
             T.pair.sym8_stride = stride;
             T.sym8_flags = (int32_t *)ctx->ctrl + kSym8FlagWord;
             T.pair.sym8_flags = T.sym8_flags;
         }
-    }
-    size_t perm_words = 0;
-    if (tiles > 1) {
-        perm_words = grid_perm_words(m, n, G);
-        if ((rc = ctx->strip_ws.reserve(ctx, (2 * perm_words + grid_merge_words(m, n, G)) * 4))) return rc;
-        T.perm = (int32_t *)ctx->strip_ws.ptr;
     }
     ChainArgs A{};
     const long long units = (T.pair.nbands + G.group_w - 1) / G.group_w * (long long)tiles;
@@ -591,6 +607,7 @@ int enqueue_chain(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_
     if (rc) return rc;
     rc = enqueue_chain_ws(ctx, d_a, m, d_b, n, sched, d_h, d_v, stream, d_h_in, d_v_in, d_r2c, d_status);
     const int rc2 = ws_release(ctx, stream);
+    ctx->ws_reserved = 0;
     return rc ? rc : rc2;
 }
 
@@ -760,7 +777,7 @@ int lcs_ctx_destroy(lcs_ctx *ctx)
     ctx->alive->store(false);
     ctx->strings.release(ctx);
     ctx->results.release(ctx);
-    trim_kept(ctx);
+    trim_kept(ctx, nullptr);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->ctrl) (void)hipFree(ctx->ctrl);
     if (ctx->band_trace) (void)hipFree(ctx->band_trace);

@@ -113,6 +113,7 @@ struct lcs_ctx {
     // false once the context is destroyed: an index dropped later frees its own memory
     std::shared_ptr<std::atomic<bool>> alive = std::make_shared<std::atomic<bool>>(true);
     lcs::DevBuf sym8;                    // byte copies of b and their range flag (single-pair chains)
+    unsigned ws_reserved = 0;            // bit per lcs::PairWs: reserved by the single-pair call being enqueued
     // The shared workspace (ring, descriptors, ctrl words) is used by one
     // launch at a time: a call on another stream first waits for ws_done,
     // recorded after the last call's kernels on ws_stream.
@@ -126,6 +127,10 @@ struct lcs_ctx {
 };
 
 namespace lcs {
+// Reserves one of the single-pair workspaces for the call being enqueued; those
+// that it has not reserved are freed where the budget or the device runs short.
+enum PairWs { kWsRing, kWsStrips, kWsSym8 };
+int reserve_ws(lcs_ctx *ctx, PairWs which, size_t bytes);
 int enqueue_chain(lcs_ctx *ctx, const int32_t *d_a, int32_t m, const int32_t *d_b, int32_t n,
                   const lcs_schedule *sched, int32_t *d_h, int32_t *d_v, hipStream_t stream,
                   const int32_t *d_h_in = nullptr, const int32_t *d_v_in = nullptr, int32_t *d_r2c = nullptr,

@@ -49,6 +49,7 @@ int enqueue_llcs(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int32_t sigma
     if (rc) return rc;
     rc = enqueue_llcs_ws(ctx, pairs, sigma, s);
     const int rc2 = ws_release(ctx, s);
+    ctx->ws_reserved = 0;
     return rc ? rc : rc2;
 }
 
@@ -84,8 +85,9 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
         code_bytes += lcsl::llcs_code_bytes(D.ncols, sigma);
         max_words = std::max(max_words, D.nwords);
     }
-    int rc = ctx->ring.reserve(ctx, ring_words * sizeof(unsigned long long));
-    if (!rc) rc = ctx->sym8.reserve(ctx, code_bytes);
+    ctx->ws_reserved = 0;
+    int rc = reserve_ws(ctx, kWsRing, ring_words * sizeof(unsigned long long));
+    if (!rc) rc = reserve_ws(ctx, kWsSym8, code_bytes);
     if (rc) return rc;
     std::vector<int2> tasks;
     for (int p = 0; p < np; ++p)

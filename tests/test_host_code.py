@@ -107,3 +107,24 @@ result = [after(batch, False), after(batch, True), after(product, False), after(
           after(fixup, True)]
 """)
     assert got[0] == got[1] and got[2] == got[3] and got[4] == got[5] and min(got) > 0, got
+
+
+def test_workspaces_of_one_pair_give_way_to_the_next(host):
+    # strings, results and ring of the second pair fill the budget, so the
+    # first one's tiles, permutations and byte copies have to go
+    got = host("""
+def need(m, n):
+    return 8 * (m + n) + 16 * n + 100000
+
+result = []
+for first, second, sched in (((9000, 9000), (30000, 30000), lcs_amd.schedule(4, 1, lcs_amd.VARIANT_CHAIN, 1)),
+                             ((60000, 60000), (100, 200000), lcs_amd.schedule(1, 1, lcs_amd.VARIANT_CHAIN, 1))):
+    with lcs_amd.Context(0, hbm_budget=need(*second)) as c:
+        for (m, n), s in ((first, None), (second, sched), (second, sched)):
+            try:
+                c.comb(zeros(m), zeros(n), s)
+                result.append(0)
+            except lcs_amd.LcsError as e:
+                result.append(e.args)
+""")
+    assert got[1:3] == got[4:6] == [0, 0], got
