@@ -116,7 +116,8 @@ int lcs_ctx_status(lcs_ctx *ctx);
  * up at once (a way to exercise the error path). */
 int lcs_ctx_set_timeout(lcs_ctx *ctx, uint64_t ticks);
 /* Device bytes the context holds now (workspaces grow on demand and stay
- * until lcs_ctx_destroy) and its budget. */
+ * until lcs_ctx_destroy, or until another call needs their share of the
+ * budget) and its budget. */
 int lcs_ctx_memory(lcs_ctx *ctx, size_t *held, size_t *budget);
 
 /* Diagnostics (no counterpart in the reference): record the start and end
@@ -267,7 +268,11 @@ int lcs_braid_multiply(lcs_ctx *ctx, const int32_t *p_row_to_col, int32_t p_size
  * alphabet of at most 200 symbols.  Symbols of a and b must lie in
  * [0, sigma), 1 <= sigma <= 200; a symbol outside gives LCS_ERANGE (host
  * entry points) or a length of -1 (device entry point).  Equal to
- * #{v_out[j] < m} of lcs_comb on the same pair.  The string combed as
+ * #{v_out[j] < m} of lcs_comb on the same pair.  Device memory: the strings
+ * (host entry points), half a byte a column for the hand-off between bands,
+ * and, where the budget has room for it, the column string as codes: half a
+ * byte or a byte a column and under 1 KB a pair.  Without the codes a length
+ * takes about three times as long.  The string combed as
  * columns (the longer one, as a rule) may hold at most 2^31 - 4097
  * symbols, else LCS_ERANGE.
  *   lcs_llcs: host pointers, synchronous.

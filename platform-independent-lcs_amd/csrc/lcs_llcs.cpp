@@ -75,35 +75,34 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
         D.ncols = swap ? P.m : P.n;
         // the widest b of the ABI; the band loop itself counts chunks
         if (D.ncols > 0x7fffffff - 4096) return LCS_ERANGE;
-        D.nbands = lcsl::llcs_nbands(D.nrows);
-        D.nwords = lcsl::llcs_nwords(D.ncols);
         us[0] = std::max(us[0], pipeline_us(D.nrows, D.ncols, resident, 4));
         us[1] = std::max(us[1], pipeline_us(D.nrows, D.ncols, resident, 2));
-        all_bands += D.nbands;
+        all_bands += lcsl::llcs_nbands(D.nrows);
         D.out = P.out;
-        ring_words += 2 * ((size_t)D.nwords + lcsl::kSpare);
+        ring_words += 2 * (size_t)lcsl::llcs_slot_words(D.ncols);
         code_bytes += lcsl::llcs_code_bytes(D.ncols, sigma);
-        max_words = std::max(max_words, D.nwords);
+        max_words = std::max(max_words, lcsl::llcs_nwords(D.ncols));
     }
     ctx->ws_reserved = 0;
     int rc = reserve_ws(ctx, kWsRing, ring_words * sizeof(unsigned long long));
-    if (!rc) rc = reserve_ws(ctx, kWsSym8, code_bytes);
     if (rc) return rc;
     std::vector<int2> tasks;
     for (int p = 0; p < np; ++p)
-        for (int32_t g = 0; g < descs[(size_t)p].nbands; ++g) tasks.push_back(make_int2(p, g));
+        for (int32_t g = 0; g < lcsl::llcs_nbands(descs[(size_t)p].nrows); ++g) tasks.push_back(make_int2(p, g));
     const size_t desc_bytes = sizeof(lcsl::LlcsDesc) * (size_t)np, task_bytes = sizeof(int2) * tasks.size();
     // the error words travel with the descriptors, as zeros
     const size_t err_off = (desc_bytes + task_bytes + 255) / 256 * 256;
     if ((rc = ctx->descs.reserve(ctx, err_off + 4 * (size_t)np + 256))) return rc;
-    uint8_t *codes = (uint8_t *)ctx->sym8.ptr;
+    // a budget that does not hold the codes: the bands read the symbols themselves
+    const bool coded = reserve_ws(ctx, kWsSym8, code_bytes) == LCS_OK;
+    uint8_t *codes = coded ? (uint8_t *)ctx->sym8.ptr : nullptr;
     unsigned long long *ring = (unsigned long long *)ctx->ring.ptr;
     int32_t *err = (int32_t *)((unsigned char *)ctx->descs.ptr + err_off);
     for (int p = 0; p < np; ++p) {
         descs[(size_t)p].ring = ring;
-        ring += 2 * ((size_t)descs[(size_t)p].nwords + lcsl::kSpare);
+        ring += 2 * (size_t)lcsl::llcs_slot_words(descs[(size_t)p].ncols);
         descs[(size_t)p].codes = codes;
-        codes += lcsl::llcs_code_bytes(descs[(size_t)p].ncols, sigma);
+        if (coded) codes += lcsl::llcs_code_bytes(descs[(size_t)p].ncols, sigma);
         descs[(size_t)p].err = err + p;
     }
     std::vector<unsigned char> blob(err_off + 4 * (size_t)np, 0);
@@ -121,6 +120,7 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
     A.timeout_ticks = ctx->timeout_ticks;
     A.trace = ctx->band_trace;
     A.trace_cap = ctx->band_trace_cap;
+    A.codes = coded;
     // more bands than SIMDs over several pairs: the time per column counts
     A.block = us[1] < us[0] && (np == 1 || all_bands <= resident) ? 2 : 4;
     const int blocks = (int)std::min<int64_t>((int64_t)tasks.size(), resident);

@@ -20,21 +20,21 @@ constexpr int kMaxPairSigma = 9;
 // rows, one 32-bit word per lane; `cols` (ncols symbols) streams through the
 // band as codes.  Band g reads the carry words of band g-1 from ring slot g&1
 // (tag g) and writes its own to slot (g+1)&1; the seeding kernel fills slot 0
-// with empty words of tag 0 for band 0.  A slot has nwords words and kSpare
-// that the last prefetches read.
-constexpr int kSpare = 24;
+// with empty words of tag 0 for band 0.  A slot has a word per 32 columns and
+// two that the last prefetches read.
 struct LlcsDesc {
     const int32_t *rows;
     const int32_t *cols;
-    int32_t nrows, ncols, nbands, nwords;
-    unsigned long long *ring;    // 2 * (nwords + kSpare) words (tag << 32 | 32 carry bits)
-    uint8_t *codes;              // llcs_code_bytes(ncols, sigma), 16-byte aligned
+    int32_t nrows, ncols;
+    unsigned long long *ring;    // 2 * llcs_slot_words(ncols) words (tag << 32 | 32 carry bits)
+    uint8_t *codes;              // llcs_code_bytes(ncols, sigma), 16-byte aligned; null in a launch without codes
     int32_t *out;                // LCS length (zeroed by the prep kernel); -1 on a symbol outside [0, sigma)
     int32_t *err;                // zero before the launch; set on a symbol outside [0, sigma)
 };
 
 inline int32_t llcs_nbands(int32_t nrows) { return (int32_t)(((int64_t)nrows + kBandRows - 1) / kBandRows); }
-inline int32_t llcs_nwords(int32_t ncols) { return ncols > 0 ? (ncols - 1) / kChunk + 1 : 0; }
+__host__ __device__ inline int32_t llcs_nwords(int32_t ncols) { return ncols > 0 ? (ncols - 1) / kChunk + 1 : 0; }
+__host__ __device__ inline int64_t llcs_slot_words(int32_t ncols) { return ncols > 0 ? (int64_t)llcs_nwords(ncols) + 2 : 0; }
 // Chunks between the column word q of a band and the one in which it is whole:
 // with blocks of B columns a chunk has 32 / B turns and lane 63 takes block b
 // in turn b + 63, so word q is whole after the last turn but one of chunk q +
@@ -65,6 +65,7 @@ struct LlcsArgs {
     unsigned long long *trace;   // nullable: [2t] start, [2t+1] end of task t (realtime ticks)
     int32_t trace_cap;
     int32_t block;               // columns per turn, 4 or 2
+    int32_t codes;               // 0: no descriptor has codes, the bands read `cols`
     unsigned *sticky;            // nullable: the prep kernel ORs the abort flag into it before clearing it
 };
 

@@ -137,10 +137,13 @@ __device__ __forceinline__ void turn(uint32_t &V, uint32_t &cout, uint32_t &cin,
 }
 
 // One band.  PAIRS: a code byte stands for two columns; B: columns per turn.
-template <bool PAIRS, int B>
+// RAW: no codes (a budget that does not hold them): a lane turns the 32
+// symbols of its chunk into codes itself (m = n = 2^20: 57.8 ms against 20.1).
+template <bool PAIRS, int B, bool RAW = false>
 __device__ bool band(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, lds_u32 *tab)
 {
     constexpr int kBlock = B, kTurns = kChunk / B, kWordLag = word_lag(B);
+    static_assert(!(PAIRS && RAW), "raw symbols have a code each");
     constexpr int kCodeWords = PAIRS ? kChunk / 8 : kChunk / 4;   // code words of a lane's chunk
     const int sigma = A.sigma;
     bool bad = false;
@@ -176,17 +179,35 @@ __device__ bool band(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, lds_
         }
         __syncthreads();
     }
-    const int32_t nwords = D.nwords, nchunks = nwords > 0 ? nwords + kWordLag : 0;
-    gcword *rin = (gcword *)(D.ring + (size_t)(g & 1) * ((size_t)nwords + kSpare));
-    gword *rout = (gword *)(D.ring + (size_t)((g + 1) & 1) * ((size_t)nwords + kSpare));
+    const int32_t nwords = llcs_nwords(D.ncols), nchunks = nwords > 0 ? nwords + kWordLag : 0;
+    gcword *rin = (gcword *)(D.ring + (g & 1) * llcs_slot_words(D.ncols));
+    gword *rout = (gword *)(D.ring + ((g + 1) & 1) * llcs_slot_words(D.ncols));
     const uint32_t tag_in = (uint32_t)g;
     const unsigned long long tag_out = (unsigned long long)(g + 1) << 32;
     // lane l's codes of chunk q start at column kFrontPad + 32 q - B l
     gbyte *codes = (gbyte *)D.codes + (size_t)(kFrontPad - B * lane) / (PAIRS ? 2 : 1);
     auto load_codes = [&](int q, uint32_t (&c)[kCodeWords]) {
-        typedef LCSL_GLOBAL const unaligned_u32 gcode;
+        if constexpr (RAW) {
+            // all loads, from clamped addresses, before the first symbol is used
+            const int32_t c0 = q * kChunk - B * lane;
+            uint32_t x[kChunk];
 #pragma unroll
-        for (int i = 0; i < kCodeWords; ++i) c[i] = ((gcode *)(codes + (size_t)q * kCodeWords * 4))[i];
+            for (int k = 0; k < kChunk; ++k) x[k] = (uint32_t)((gsym *)D.cols)[min(max(c0 + k, 0), D.ncols - 1)];
+#pragma unroll
+            for (int i = 0; i < kCodeWords; ++i) {
+                c[i] = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int32_t col = c0 + 4 * i + k;
+                    const uint32_t s = col >= 0 && col < D.ncols ? x[4 * i + k] : (uint32_t)sigma;
+                    c[i] |= min(s, (uint32_t)sigma) << (8 * k);
+                }
+            }
+        } else {
+            typedef LCSL_GLOBAL const unaligned_u32 gcode;
+#pragma unroll
+            for (int i = 0; i < kCodeWords; ++i) c[i] = ((gcode *)(codes + (size_t)q * kCodeWords * 4))[i];
+        }
     };
     // The masks of turn i of a chunk from its codes: per code byte the LDS
     // address byte * 256 + the lane's place in a row (the table is the
@@ -319,7 +340,7 @@ __device__ bool band(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, lds_
     return !dead;
 }
 
-template <bool PAIRS, int B>
+template <bool PAIRS, int B, bool RAW = false>
 __global__ __launch_bounds__(kWave) void llcs_chain_kernel(LlcsArgs A)
 {
     extern __shared__ uint32_t lds_dyn[];
@@ -334,7 +355,7 @@ __global__ __launch_bounds__(kWave) void llcs_chain_kernel(LlcsArgs A)
         const LlcsDesc D = A.descs[task.x];
         const bool traced = A.trace && (int)t < A.trace_cap && lane == 0;
         if (traced) A.trace[2 * (size_t)t] = __builtin_amdgcn_s_memrealtime();
-        if (!band<PAIRS, B>(A, D, task.y, lane, (lds_u32 *)lds_dyn)) break;
+        if (!band<PAIRS, B, RAW>(A, D, task.y, lane, (lds_u32 *)lds_dyn)) break;
         if (traced) A.trace[2 * (size_t)t + 1] = __builtin_amdgcn_s_memrealtime();
         __syncthreads();   // the table is rebuilt
     }
@@ -349,7 +370,7 @@ __global__ void llcs_prep_kernel(const LlcsDesc *descs, int sigma, unsigned *tic
 {
     const LlcsDesc D = descs[blockIdx.y];
     const int64_t stride = (int64_t)gridDim.x * blockDim.x, i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t slot = (int64_t)D.nwords + kSpare;
+    const int64_t slot = llcs_slot_words(D.ncols);
     for (int64_t i = i0; i < 2 * slot; i += stride) D.ring[i] = i < slot ? 0ull : (unsigned long long)kNoTag << 32;
     const bool pairs = llcs_pairs(sigma);
     bool bad = false;
@@ -359,11 +380,12 @@ __global__ void llcs_prep_kernel(const LlcsDesc *descs, int sigma, unsigned *tic
         bad = bad || s >= (uint32_t)sigma;
         return s < (uint32_t)sigma ? s : (uint32_t)sigma;
     };
-    if (D.nwords > 0) {
-        const int64_t quads = llcs_code_columns(D.nwords) / 4;
+    if (D.ncols > 0) {
+        const int64_t quads = llcs_code_columns(llcs_nwords(D.ncols)) / 4;
         for (int64_t b = i0; b < quads; b += stride) {
             const int64_t c0 = 4 * b - kFrontPad;
             const uint32_t x = code(c0), y = code(c0 + 1), z = code(c0 + 2), w = code(c0 + 3), row = (uint32_t)sigma + 1;
+            if (!D.codes) continue;   // only checked
             if (pairs) ((uint16_t *)D.codes)[b] = (uint16_t)((x * row + y) | (z * row + w) << 8);
             else ((uint32_t *)D.codes)[b] = x | y << 8 | z << 16 | w << 24;
         }
@@ -393,13 +415,14 @@ int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int n
     using namespace lcsl;
     if (npairs <= 0) return 0;
     if (args.sigma < 1 || args.sigma > kMaxSigma || lds_bytes < (int)llcs_lds_bytes(args.sigma)) return -22;
-    const bool pairs = llcs_pairs(args.sigma);
+    const bool pairs = llcs_pairs(args.sigma) && args.codes;
     static std::once_flag once;   // per process, and no stream operation
     static bool ready = false;
     std::call_once(once, [] {
         ready = true;
         for (const void *k : {(const void *)llcs_chain_kernel<true, 4>, (const void *)llcs_chain_kernel<false, 4>,
-                              (const void *)llcs_chain_kernel<true, 2>, (const void *)llcs_chain_kernel<false, 2>})
+                              (const void *)llcs_chain_kernel<true, 2>, (const void *)llcs_chain_kernel<false, 2>,
+                              (const void *)llcs_chain_kernel<false, 4, true>})
             ready = ready && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes) == hipSuccess;
     });
     if (!ready) return -5;
@@ -412,7 +435,8 @@ int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int n
     }
     if (args.ntasks > 0 && grid_blocks > 0) {
         const dim3 grid(grid_blocks), block(kWave);
-        if (pairs && args.block == 4) llcs_chain_kernel<true, 4><<<grid, block, lds_bytes, stream>>>(args);
+        if (!args.codes) llcs_chain_kernel<false, 4, true><<<grid, block, lds_bytes, stream>>>(args);
+        else if (pairs && args.block == 4) llcs_chain_kernel<true, 4><<<grid, block, lds_bytes, stream>>>(args);
         else if (pairs) llcs_chain_kernel<true, 2><<<grid, block, lds_bytes, stream>>>(args);
         else if (args.block == 4) llcs_chain_kernel<false, 4><<<grid, block, lds_bytes, stream>>>(args);
         else llcs_chain_kernel<false, 2><<<grid, block, lds_bytes, stream>>>(args);

@@ -37,3 +37,23 @@ def test_symbols_outside_the_alphabet_next_to_the_table_rows():
                         with pytest.raises(lcs_amd.LcsError):
                             ctx.llcs(x, y, sigma)
             assert ctx.llcs(a, a, sigma) == 3000
+
+
+@pytest.mark.parametrize("sigma", [4, 9, 10, 200])
+def test_a_budget_without_room_for_codes(sigma):
+    # the bands then read the symbols themselves; edges of the 32-column chunk
+    # and of the string, unaligned starts of a pair's columns, and bad symbols
+    rng = np.random.default_rng(sigma)
+    sizes = [(0, 5), (5, 0), (1, 1), (31, 33), (2047, 65), (4097, 64), (70, 2049), (3000, 3001)]
+    A = [rng.integers(0, sigma, m).astype(np.int32) for m, _ in sizes]
+    B = [rng.integers(0, sigma, n).astype(np.int32) for _, n in sizes]
+    want = [oracle.llcs_bitpar(a, b) if a.size and b.size else 0 for a, b in zip(A, B)]
+    with lcs_amd.Context(0) as free:
+        assert free.llcs_batch(A, B, sigma).tolist() == want
+        budget = free.memory()[0] - 1024   # short by a part of the codes
+    with lcs_amd.Context(0, hbm_budget=budget) as ctx:
+        assert ctx.llcs_batch(A, B, sigma).tolist() == want
+        assert ctx.memory()[0] < budget   # none kept
+        B[4][7] = sigma
+        with pytest.raises(lcs_amd.LcsError):
+            ctx.llcs_batch(A, B, sigma)

@@ -128,3 +128,20 @@ for first, second, sched in (((9000, 9000), (30000, 30000), lcs_amd.schedule(4, 
                 result.append(e.args)
 """)
     assert got[1:3] == got[4:6] == [0, 0], got
+
+
+def test_lcs_length_fits_where_its_rings_do(host):
+    # half a byte a column for each pair's rings, the strings and a fixed part:
+    # the codes (a byte or half a byte a column) are kept only where they fit
+    need = {"300 x 500": 3912, "100000^2": 850808, "1000 of 50^2": 536256, "empty": 1332}
+    got = host(f"""
+need = {need!r}
+calls = {{"300 x 500": (1, 300, 500), "100000^2": (1, 100000, 100000), "1000 of 50^2": (1000, 50, 50), "empty": (3, 0, 50)}}
+result = []
+for name, (pairs, m, n) in calls.items():
+    for sigma in (4, 20):
+        with lcs_amd.Context(0, hbm_budget=need[name]) as c:
+            c.llcs_batch([zeros(m)] * pairs, [zeros(n)] * pairs, sigma)
+            result.append(c.memory()[0] <= need[name])
+""")
+    assert got == [True] * 8
