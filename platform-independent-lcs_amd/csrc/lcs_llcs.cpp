@@ -21,22 +21,29 @@ struct LlcsPair {
 };
 
 // Microseconds from the first band's start to the last band's end with blocks
-// of B columns: a band lags the one below by 64 blocks of skew, the chunk that
-// a carry word fills, two chunks of prefetch and the word's trip (measured 390
-// columns at 4, 260 at 2), and bands beyond the resident ones run in later
-// rounds.  A column takes 15.0 ns at 4 and 17.0 at 2.
-double pipeline_us(int64_t rows, int64_t cols, int64_t resident, int B)
+// of 4 and of 2 columns: a band lags the one below by 64 blocks of skew, the
+// chunk that a carry word fills, two chunks of prefetch and the word's trip
+// (measured 390 columns at 4, 260 at 2), and bands beyond the resident ones run
+// in later rounds.  A column takes 15.0 ns at 4 and 17.0 at 2.
+struct PipelineUs {
+    double of4, of2;
+    double best() const { return std::min(of4, of2); }
+};
+PipelineUs pipeline_us(int32_t rows, int32_t cols, int64_t resident)
 {
-    const int64_t bands = (rows + lcsl::kBandRows - 1) / lcsl::kBandRows;
-    const int64_t rounds = (bands + resident - 1) / std::max<int64_t>(resident, 1);
-    return ((double)rounds * ((double)cols + lcsl::kWave * B) + (double)bands * (130.0 + 65.0 * B)) *
-           (B == 4 ? 0.0150 : 0.0170);
+    const int64_t bands = lcsl::llcs_nbands(rows);
+    const double rounds = bands <= resident ? 1.0 : (double)((bands + resident - 1) / resident);
+    return {(rounds * ((double)cols + lcsl::kWave * 4) + (double)bands * 390.0) * 0.0150,
+            (rounds * ((double)cols + lcsl::kWave * 2) + (double)bands * 260.0) * 0.0170};
 }
 
 // LDS of a CU, and the bands it holds at once: one per SIMD, fewer when the
 // match-mask tables fill the LDS
 constexpr int kCuLdsBytes = 160 * 1024;
-int bands_per_cu(int sigma) { return (int)std::min<size_t>(4, kCuLdsBytes / lcsl::llcs_lds_bytes(sigma)); }
+int bands_per_cu(int sigma, bool pairs)
+{
+    return (int)std::min<size_t>(4, kCuLdsBytes / lcsl::llcs_lds_bytes(sigma, pairs));
+}
 
 // Enqueues one launch over `pairs` on `s`: the longer-pipelined orientation
 // is chosen per pair (LCS is symmetric).  Rings and descriptors live in the
@@ -57,7 +64,18 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
 {
     const int np = (int)pairs.size();
     if (np == 0) return LCS_OK;
-    const int64_t resident = (int64_t)ctx->num_cus * bands_per_cu(sigma);
+    // tables of column pairs while every band still has its SIMD, or the tables
+    // are small enough for four to a CU: of 5 to 9 symbols, 20 pairs of 100000
+    // take 3.87 ms with them and 2.34 without
+    bool two_columns = sigma <= lcsl::kMaxPairSigma;
+    int64_t bands_a = 0, bands_b = 0;
+    for (const LlcsPair &P : pairs) {
+        bands_a += lcsl::llcs_nbands(P.m);
+        bands_b += lcsl::llcs_nbands(P.n);
+    }
+    const int tables = two_columns ? bands_per_cu(sigma, true) : 0;
+    if (tables < 4 && std::min(bands_a, bands_b) > (int64_t)ctx->num_cus * tables) two_columns = false;
+    const int64_t resident = (int64_t)ctx->num_cus * bands_per_cu(sigma, two_columns);
     std::vector<lcsl::LlcsDesc> descs((size_t)np);
     size_t ring_words = 0, code_bytes = 0;
     int max_words = 0;
@@ -65,8 +83,8 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
     int64_t all_bands = 0;
     for (int p = 0; p < np; ++p) {
         const LlcsPair &P = pairs[(size_t)p];
-        const bool swap = std::min(pipeline_us(P.n, P.m, resident, 4), pipeline_us(P.n, P.m, resident, 2)) <
-                          std::min(pipeline_us(P.m, P.n, resident, 4), pipeline_us(P.m, P.n, resident, 2));
+        const PipelineUs as_given = pipeline_us(P.m, P.n, resident), swapped = pipeline_us(P.n, P.m, resident);
+        const bool swap = swapped.best() < as_given.best();
         lcsl::LlcsDesc &D = descs[(size_t)p];
         D = lcsl::LlcsDesc{};
         D.rows = swap ? P.b : P.a;
@@ -75,12 +93,12 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
         D.ncols = swap ? P.m : P.n;
         // the widest b of the ABI; the band loop itself counts chunks
         if (D.ncols > 0x7fffffff - 4096) return LCS_ERANGE;
-        us[0] = std::max(us[0], pipeline_us(D.nrows, D.ncols, resident, 4));
-        us[1] = std::max(us[1], pipeline_us(D.nrows, D.ncols, resident, 2));
+        us[0] = std::max(us[0], swap ? swapped.of4 : as_given.of4);
+        us[1] = std::max(us[1], swap ? swapped.of2 : as_given.of2);
         all_bands += lcsl::llcs_nbands(D.nrows);
         D.out = P.out;
         ring_words += 2 * (size_t)lcsl::llcs_slot_words(D.ncols);
-        code_bytes += lcsl::llcs_code_bytes(D.ncols, sigma);
+        code_bytes += lcsl::llcs_code_bytes(D.ncols, two_columns);
         max_words = std::max(max_words, lcsl::llcs_nwords(D.ncols));
     }
     ctx->ws_reserved = 0;
@@ -102,7 +120,7 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
         descs[(size_t)p].ring = ring;
         ring += 2 * (size_t)lcsl::llcs_slot_words(descs[(size_t)p].ncols);
         descs[(size_t)p].codes = codes;
-        if (coded) codes += lcsl::llcs_code_bytes(descs[(size_t)p].ncols, sigma);
+        if (coded) codes += lcsl::llcs_code_bytes(descs[(size_t)p].ncols, two_columns);
         descs[(size_t)p].err = err + p;
     }
     std::vector<unsigned char> blob(err_off + 4 * (size_t)np, 0);
@@ -120,6 +138,7 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
     A.timeout_ticks = ctx->timeout_ticks;
     A.trace = ctx->band_trace;
     A.trace_cap = ctx->band_trace_cap;
+    A.pairs = two_columns;
     A.codes = coded;
     // more bands than SIMDs over several pairs: the time per column counts
     A.block = us[1] < us[0] && (np == 1 || all_bands <= resident) ? 2 : 4;
@@ -127,7 +146,7 @@ static int enqueue_llcs_ws(lcs_ctx *ctx, const std::vector<LlcsPair> &pairs, int
     // as much LDS per band as leaves each CU its share of them: the dispatcher
     // then spreads the bands over the CUs, and a band has its SIMD to itself
     const int share = std::max(1, (blocks + ctx->num_cus - 1) / ctx->num_cus);
-    const int lds = std::max((int)lcsl::llcs_lds_bytes(sigma), kCuLdsBytes / share / 512 * 512);
+    const int lds = std::max((int)lcsl::llcs_lds_bytes(sigma, two_columns), kCuLdsBytes / share / 512 * 512);
     return lcsl_launch(A, A.descs, np, max_words, blocks, lds, s) == 0 ? LCS_OK : LCS_EIO;
 }
 

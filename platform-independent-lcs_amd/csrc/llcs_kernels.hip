@@ -28,7 +28,7 @@
 // time: the caller picks by that.
 //
 //  * Match masks: a table in LDS, built once per band: one row of 64 words per
-//    symbol, or (alphabets of at most 9) one row of 64 pairs of words per two
+//    symbol, or (alphabets of at most 9, the caller's choice) one row of 64 pairs of words per two
 //    consecutive symbols, so that one address (a v_perm of the code byte and
 //    the lane) and one ds_read_b64 serve two columns.  A zero row serves the
 //    padding before and after the column string.
@@ -149,8 +149,8 @@ __device__ bool band(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, lds_
     bool bad = false;
     // the masks of this lane's 32 rows; row `sigma` stays zero (padding)
     {
-        // the single-symbol rows: in the table itself, or in its first words
-        // while the pair rows are written from the last one down
+        // the single-symbol rows: the table itself, or in its first words until
+        // the lane holds them in registers, before the first pair row is written
         const int rows1 = sigma + 1;
         for (int c = 0; c < rows1; ++c) tab[c * kWave + lane] = 0u;
         const int64_t r0 = ((int64_t)g * kWave + lane) * kWordRows;
@@ -179,7 +179,10 @@ __device__ bool band(const LlcsArgs &A, const LlcsDesc &D, int g, int lane, lds_
         }
         __syncthreads();
     }
-    const int32_t nwords = llcs_nwords(D.ncols), nchunks = nwords > 0 ? nwords + kWordLag : 0;
+    // (readfirstlane: with the word count's range known to it the compiler
+    // computes every chunk's addresses anew, 1 % of the time)
+    const int32_t nwords = __builtin_amdgcn_readfirstlane(llcs_nwords(D.ncols));
+    const int32_t nchunks = nwords > 0 ? nwords + kWordLag : 0;
     gcword *rin = (gcword *)(D.ring + (g & 1) * llcs_slot_words(D.ncols));
     gword *rout = (gword *)(D.ring + ((g + 1) & 1) * llcs_slot_words(D.ncols));
     const uint32_t tag_in = (uint32_t)g;
@@ -365,14 +368,13 @@ __global__ __launch_bounds__(kWave) void llcs_chain_kernel(LlcsArgs A)
 // band waits for), the column string as codes (one thread per four columns); block (0,0) clears
 // the ticket and abort words, after folding the previous launch's abort flag
 // into `sticky`
-__global__ void llcs_prep_kernel(const LlcsDesc *descs, int sigma, unsigned *ticket, unsigned *abort_flag,
+__global__ void llcs_prep_kernel(const LlcsDesc *descs, int sigma, bool pairs, unsigned *ticket, unsigned *abort_flag,
                                  unsigned *sticky)
 {
     const LlcsDesc D = descs[blockIdx.y];
     const int64_t stride = (int64_t)gridDim.x * blockDim.x, i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t slot = llcs_slot_words(D.ncols);
     for (int64_t i = i0; i < 2 * slot; i += stride) D.ring[i] = i < slot ? 0ull : (unsigned long long)kNoTag << 32;
-    const bool pairs = llcs_pairs(sigma);
     bool bad = false;
     auto code = [&](int64_t c) -> uint32_t {
         if (c < 0 || c >= D.ncols) return (uint32_t)sigma;
@@ -414,8 +416,10 @@ int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int n
 {
     using namespace lcsl;
     if (npairs <= 0) return 0;
-    if (args.sigma < 1 || args.sigma > kMaxSigma || lds_bytes < (int)llcs_lds_bytes(args.sigma)) return -22;
-    const bool pairs = llcs_pairs(args.sigma) && args.codes;
+    if (args.sigma < 1 || args.sigma > kMaxSigma || (args.pairs && args.sigma > kMaxPairSigma) ||
+        lds_bytes < (int)llcs_lds_bytes(args.sigma, args.pairs))
+        return -22;
+    const bool pairs = args.pairs && args.codes;
     static std::once_flag once;   // per process, and no stream operation
     static bool ready = false;
     std::call_once(once, [] {
@@ -426,12 +430,12 @@ int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int n
             ready = ready && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes) == hipSuccess;
     });
     if (!ready) return -5;
-    // one thread per four columns
-    const unsigned px = (unsigned)std::min<long long>(4096, ((long long)max_words * (kChunk / 4) + 512) / 256);
+    // one thread per four columns, the padding among them
+    const unsigned px = (unsigned)std::min<int64_t>(4096, (llcs_code_columns(max_words) / 4 + 255) / 256);
     for (int base = 0; base < npairs; base += 65535) {   // grid y is at most 65535
         const int cnt = std::min(65535, npairs - base);
         hipLaunchKernelGGL(llcs_prep_kernel, dim3(px, (unsigned)cnt), dim3(256), 0, stream, d_descs + base, args.sigma,
-                           args.ticket, args.abort_flag, base ? nullptr : args.sticky);
+                           pairs, args.ticket, args.abort_flag, base ? nullptr : args.sticky);
     }
     if (args.ntasks > 0 && grid_blocks > 0) {
         const dim3 grid(grid_blocks), block(kWave);

@@ -57,3 +57,30 @@ def test_a_budget_without_room_for_codes(sigma):
         B[4][7] = sigma
         with pytest.raises(lcs_amd.LcsError):
             ctx.llcs_batch(A, B, sigma)
+
+
+@pytest.mark.parametrize("sigma", [4, 5, 9, 10])
+@pytest.mark.parametrize("shape", ["tall", "many"])
+def test_batches(sigma, shape):
+    # tall: few pairs whose bands outnumber their words of columns, blocks of
+    # two; many: more bands than the chip holds at once (of tables of column
+    # pairs, and of four to a CU), blocks of four and, for 5 to 9 symbols, one
+    # column a table row.  Word edges and empty strings among them.
+    rng = np.random.default_rng(sigma)
+    edges = [0, 1, 31, 32, 33]
+    if shape == "tall":
+        sizes = [(40000, 40000), (30001, 33000)] + [(20000 + n, n) for n in edges]
+    else:
+        sizes = [(int(m), int(n)) for m, n in rng.integers(1, 3000, (1300, 2))] + [(2049, n) for n in edges]
+    A = [rng.integers(0, sigma, m).astype(np.int32) for m, _ in sizes]
+    B = [rng.integers(0, sigma, n).astype(np.int32) for _, n in sizes]
+    want = [oracle.llcs_bitpar(a, b) if a.size and b.size else 0 for a, b in zip(A, B)]
+    with lcs_amd.Context(0) as ctx:
+        assert ctx.llcs_batch(A, B, sigma).tolist() == want
+        assert ctx.llcs_batch(B, A, sigma).tolist() == want
+        B[1][5] = sigma
+        with pytest.raises(lcs_amd.LcsError):
+            ctx.llcs_batch(A, B, sigma)
+        B[1][5] = 0
+        want[1] = oracle.llcs_bitpar(A[1], B[1])
+        assert ctx.llcs_batch(A, B, sigma).tolist() == want   # the error does not stay
