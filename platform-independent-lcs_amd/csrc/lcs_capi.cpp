@@ -765,6 +765,10 @@ int lcs_ctx_create(int device, size_t hbm_budget, lcs_ctx **out)
 int lcs_ctx_destroy(lcs_ctx *ctx)
 {
     if (!ctx) return LCS_EINVAL;
+    {
+        const std::lock_guard<std::mutex> lock(ctx->life->mu);   // of an index being dropped: after it
+        ctx->life->alive = false;
+    }
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     destroy_extras(ctx);
@@ -774,7 +778,6 @@ int lcs_ctx_destroy(lcs_ctx *ctx)
     ctx->sym8.release(ctx);
     ctx->staging.destroy();
     if (ctx->ws_done) (void)hipEventDestroy(ctx->ws_done);
-    ctx->alive->store(false);
     ctx->strings.release(ctx);
     ctx->results.release(ctx);
     trim_kept(ctx, nullptr);

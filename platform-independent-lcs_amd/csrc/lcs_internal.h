@@ -27,7 +27,7 @@ struct DevBuf {
 // caller takes it, reserves what it needs, and gives it back once the device
 // is done with it; what is kept is at most kKeptMax bytes and is freed when
 // another buffer needs its share of the budget or of the device's memory.
-// Any thread may give back (an index is destroyed by whoever drops it).
+// A thread other than the context's may give back, under ContextLife.
 constexpr size_t kKeptMax = (size_t)256 << 20;
 struct KeptBuf {
     std::mutex mu;
@@ -35,6 +35,14 @@ struct KeptBuf {
     DevBuf take(size_t at_least, size_t at_most);   // empty when what is kept does not fit
     void give(lcs_ctx *ctx, DevBuf &b);
     void trim(lcs_ctx *ctx);
+};
+
+// Whether a context is there still, for what may be dropped after it and on
+// another thread (an index, by whoever collects it).  The lock is held for a
+// whole give-back, and by lcs_ctx_destroy to mark the context gone.
+struct ContextLife {
+    std::mutex mu;
+    bool alive = true;
 };
 
 struct Extras;  // batch / server resources, created on first use
@@ -92,7 +100,7 @@ struct lcs_ctx {
     int num_cus = 0;
     std::string name, arch;
     size_t budget = 0;
-    size_t held = 0;
+    std::atomic<size_t> held{0};         // device bytes; freed on any thread, reserved on the context's
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // around the band-chain launch (seed, chain, extract) of the last
@@ -110,8 +118,7 @@ struct lcs_ctx {
     size_t pinned_bytes = 0;
     lcs::KeptBuf scratch;                // braid products and index builds
     lcs::KeptBuf index_mem;              // the memory of a destroyed index
-    // false once the context is destroyed: an index dropped later frees its own memory
-    std::shared_ptr<std::atomic<bool>> alive = std::make_shared<std::atomic<bool>>(true);
+    std::shared_ptr<lcs::ContextLife> life = std::make_shared<lcs::ContextLife>();
     lcs::DevBuf sym8;                    // byte copies of b and their range flag (single-pair chains)
     unsigned ws_reserved = 0;            // bit per lcs::PairWs: reserved by the single-pair call being enqueued
     // The shared workspace (ring, descriptors, ctrl words) is used by one

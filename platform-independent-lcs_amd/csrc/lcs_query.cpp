@@ -17,7 +17,7 @@ struct lcs_dominance_index {
     int32_t size = 0;
     int levels = 0;
     int device = 0;
-    std::shared_ptr<std::atomic<bool>> alive;
+    std::shared_ptr<ContextLife> life;
     DevBuf mem;
     DevBuf io;    // query staging for the host entry point
     lcsq::IndexView view() const { return lcsq::index_view(mem.ptr, size, levels); }
@@ -51,7 +51,7 @@ int build_index(lcs_ctx *ctx, const int32_t *src, bool src_on_host, int32_t size
     if (!idx) return LCS_ENOMEM;
     idx->ctx = ctx;
     idx->device = ctx->device;
-    idx->alive = ctx->alive;
+    idx->life = ctx->life;
     idx->size = size;
     idx->levels = size > 0 ? bit_length(size) : 0;
     hipStream_t s = ctx->stream;
@@ -233,7 +233,9 @@ extern "C" int64_t lcs_dominance_index_bytes(const lcs_dominance_index *idx)
 extern "C" void lcs_dominance_index_destroy(lcs_dominance_index *idx)
 {
     if (!idx) return;
-    if (!idx->alive->load()) {
+    const std::shared_ptr<ContextLife> life = idx->life;
+    const std::lock_guard<std::mutex> lock(life->mu);
+    if (!life->alive) {
         (void)hipSetDevice(idx->device);
         if (idx->mem.ptr) (void)hipFree(idx->mem.ptr);
         if (idx->io.ptr) (void)hipFree(idx->io.ptr);

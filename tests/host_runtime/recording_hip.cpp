@@ -5,12 +5,15 @@
 // library binds.  rec_* are the tests' own entry points.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <set>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace {
@@ -26,7 +29,8 @@ std::map<const void *, std::string> names;
 std::string launches;   // "name grid.x grid.y\n"
 std::map<std::string, std::set<int>> lds_set;
 double clock_ms = 0.0;
-size_t live = 0, most_live = 0;
+size_t live = 0;
+std::atomic<int> slow_sync{0};
 std::map<void *, size_t> device_mem;
 thread_local int device = 0;
 
@@ -54,6 +58,7 @@ double rec_clock() { return clock_ms; }
 const char *rec_launches() { return launches.c_str(); }
 void rec_clear() { Lock l(mu); launches.clear(); }
 size_t rec_live() { return live; }
+void rec_slow_next_sync(int ms) { slow_sync = ms; }
 int rec_lds_devices(const char *name)   // how many devices the kernel's LDS limit was raised on
 {
     size_t most = 0;
@@ -128,7 +133,13 @@ hipError_t hipMemset(void *d, int v, size_t n) { std::memset(d, v, n); return hi
 
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)std::malloc(8); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { std::free(s); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { Lock l(mu); run_pending(); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    if (const int ms = slow_sync.exchange(0)) std::this_thread::sleep_for(std::chrono::milliseconds(ms));
+    Lock l(mu);
+    run_pending();
+    return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *e) { *e = (hipEvent_t)std::calloc(1, 8); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }

@@ -43,7 +43,7 @@ def host(tmp_path_factory):
     def run(code):
         """The value that `code` leaves in `result`."""
         script = PRELUDE.format(rec=rec, pkg=PKG) + code + "\nprint('RESULT', json.dumps(result))\n"
-        done = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=300)
+        done = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=60)
         assert done.returncode == 0, done.stderr
         return json.loads([l for l in done.stdout.splitlines() if l.startswith("RESULT ")][-1][7:])
     return run
@@ -145,3 +145,49 @@ for name, (pairs, m, n) in calls.items():
             result.append(c.memory()[0] <= need[name])
 """)
     assert got == [True] * 8
+
+
+def test_an_index_dropped_on_another_thread_keeps_the_account(host):
+    # the context's bytes stay those that the runtime has allocated for it,
+    # with indexes dropped on one thread while another reserves and frees
+    assert host("""
+import queue, threading
+result = []
+for rounds in range(8):
+    c = lcs_amd.Context(0)
+    besides = rec.rec_live() - c.memory()[0]
+    dropped = queue.Queue()
+
+    def drop():
+        for idx in iter(dropped.get, None):
+            idx.close()
+
+    thread = threading.Thread(target=drop, daemon=True)
+    thread.start()
+    perm = np.arange(300, dtype=np.int32)
+    for i in range(1500):
+        dropped.put(lcs_amd.DominanceIndex(c, perm))
+        c.semilocal(perm, 20, 280, 0, zeros(4), zeros(4))   # a buffer of its own for the call
+    dropped.put(None)
+    thread.join()
+    result.append(int(rec.rec_live() - c.memory()[0] - besides))
+    c.close()
+""") == [0] * 8
+
+
+def test_a_context_waits_for_an_index_being_dropped(host):
+    # the drop is inside its wait for the stream when the context is closed
+    waited = host("""
+import threading, time
+c = lcs_amd.Context(0)
+idx = lcs_amd.DominanceIndex(c, np.arange(300, dtype=np.int32))
+rec.rec_slow_next_sync(1000)
+drop = threading.Thread(target=idx.close, daemon=True)
+drop.start()
+time.sleep(0.2)
+t = time.monotonic()
+c.close()
+result = time.monotonic() - t
+drop.join()
+""")
+    assert waited > 0.5
