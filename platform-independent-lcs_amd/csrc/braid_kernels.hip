@@ -33,10 +33,10 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <mutex>
 #include <vector>
 
 #include "braid_kernels.h"
+#include "per_device.h"
 
 namespace lcsb {
 
@@ -1190,20 +1190,18 @@ static int launch_big(const BigBatch &B, int cnt, hipStream_t stream)
     return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-// The dynamic LDS limit of the core kernels, set once per process (before
-// any capture: it is not a stream operation).
+// The dynamic LDS limit of the core kernels, set once per device (before any
+// capture: it is not a stream operation).
 int lcsb_init(void)
 {
-    static std::once_flag once;
-    static int rc = 0;
-    std::call_once(once, [] {
-        if (hipFuncSetAttribute((const void *)braid_core_lds_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds_core_bytes(kLdsCoreL)) != hipSuccess ||
-            hipFuncSetAttribute((const void *)big_leaf_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds_core_bytes(kLdsCoreL)) != hipSuccess)
-            rc = -5;
+    static PerDevice lds;
+    return lds.once([] {
+        for (const void *k : {(const void *)braid_core_lds_kernel, (const void *)big_leaf_kernel})
+            if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_core_bytes(kLdsCoreL)) !=
+                hipSuccess)
+                return -5;
+        return 0;
     });
-    return rc;
 }
 
 // staggered_multiply for `count` independent products on device pointers.

@@ -46,10 +46,10 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <mutex>
 #include <type_traits>
 
 #include "llcs_kernels.h"
+#include "per_device.h"
 
 namespace lcsl {
 
@@ -420,16 +420,15 @@ int lcsl_launch(const lcsl::LlcsArgs &args, const lcsl::LlcsDesc *d_descs, int n
         lds_bytes < (int)llcs_lds_bytes(args.sigma, args.pairs))
         return -22;
     const bool pairs = args.pairs && args.codes;
-    static std::once_flag once;   // per process, and no stream operation
-    static bool ready = false;
-    std::call_once(once, [] {
-        ready = true;
+    static PerDevice lds;   // no stream operation
+    const int rc = lds.once([] {
         for (const void *k : {(const void *)llcs_chain_kernel<true, 4>, (const void *)llcs_chain_kernel<false, 4>,
                               (const void *)llcs_chain_kernel<true, 2>, (const void *)llcs_chain_kernel<false, 2>,
                               (const void *)llcs_chain_kernel<false, 4, true>})
-            ready = ready && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes) == hipSuccess;
+            if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes) != hipSuccess) return -5;
+        return 0;
     });
-    if (!ready) return -5;
+    if (rc) return rc;
     // one thread per four columns, the padding among them
     const unsigned px = (unsigned)std::min<int64_t>(4096, (llcs_code_columns(max_words) / 4 + 255) / 256);
     for (int base = 0; base < npairs; base += 65535) {   // grid y is at most 65535

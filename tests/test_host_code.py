@@ -191,3 +191,16 @@ result = time.monotonic() - t
 drop.join()
 """)
     assert waited > 0.5
+
+
+def test_lds_limits_are_raised_on_every_device(host):
+    # kernels that ask for more than 64 KB of LDS, on the first device and then
+    # on a second one in the same process
+    assert host("""
+p = np.arange(3000, dtype=np.int32)
+for device in (0, 1):
+    with lcs_amd.Context(device) as c:
+        c.braid_multiply(p, p, 2000, False)
+        c.llcs_batch([zeros(100)], [zeros(100)], 4)
+result = [rec.rec_lds_devices(k) for k in (b"llcs_chain_kernel", b"big_leaf_kernel", b"braid_core_lds_kernel")]
+""") == [2, 2, 2]
