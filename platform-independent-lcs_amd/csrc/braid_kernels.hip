@@ -423,19 +423,29 @@ __device__ __forceinline__ void split_depth_pq(const uint16_t *keyP, uint16_t *k
 // begin with the keys: keyP[x] = shared strand of the core's row x, keyQ[x] =
 // shared strand of its column x.
 constexpr int kScanBlock = 256, kScanPer = 8, kScanTile = kScanBlock * kScanPer;
+// Every workgroup of a slice adds up the counts of those before it, so their
+// number is bounded (2^26 points a side, k = 64: 2.47 ms with a workgroup per
+// tile, 2.36 with at most 4096, 2.18 with whole lines stored as well).
+constexpr int kMaxSliceBlocks = 4096;
+constexpr int kLinesMin = 1 << 18;   // points from which a slice stores whole lines (slice_scatter_kernel)
+static_assert(kLinesMin / kScanTile < kMaxSliceBlocks, "one tile a workgroup below");
 constexpr int kMulBatch = 32;   // products per launch
 struct MulArgs {
     const int32_t *p, *q;
     int32_t *out, *ws;
-    int32_t p_size, q_size, k, row_glue, L, pad;
+    int32_t p_size, q_size, k, row_glue, L;
+    int32_t run, blocks;   // tiles of kScanTile points that a workgroup of a slice takes, and the workgroups
     __host__ __device__ int32_t *q_c2r() const { return ws; }
     __host__ __device__ int32_t *map_row() const { return ws + q_size; }
     __host__ __device__ int32_t *map_col() const { return map_row() + k; }
-    __host__ __device__ int32_t blocks() const
+    // (on the host: a division in every kernel of a product took 6 of 155 us)
+    void set_blocks()
     {
-        return (p_size > q_size ? p_size : q_size) / kScanTile + 1;
+        const int32_t tiles = (p_size > q_size ? p_size : q_size) / kScanTile + 1;
+        run = (tiles + kMaxSliceBlocks - 1) / kMaxSliceBlocks;
+        blocks = (tiles + run - 1) / run;
     }
-    __host__ __device__ int32_t *counts(int side) const { return map_col() + k + side * blocks(); }
+    __host__ __device__ int32_t *counts(int side) const { return map_col() + k + side * blocks; }
     __host__ __device__ int32_t *core() const { return counts(2); }
     // row i of the core goes to column c: the product's point
     // (braid_multiplication.hpp:353-401); the range tests only matter after an
@@ -1059,24 +1069,36 @@ __device__ __forceinline__ int block_sum256(int x, int *red)
     return red[0] + red[1] + red[2] + red[3];
 }
 
+template <bool LINES>
 __global__ __launch_bounds__(kScanBlock) void slice_count_kernel(MulBatch B)
 {
     const MulArgs &M = B.m[blockIdx.y >> 1];
-    const int side = blockIdx.y & 1;
+    const int side = blockIdx.y & 1, run = LINES ? M.run : 1;
     const SliceSide S = slice_side(M, side);
-    if ((int64_t)blockIdx.x * kScanTile >= S.n) return;   // past this slice's blocks (whole block)
+    const int64_t first = (int64_t)blockIdx.x * run * kScanTile;
+    if (first >= S.n) return;   // past this slice's blocks (whole block)
     __shared__ int red[kScanBlock / 64];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x * kScanPer;
     int c = 0;
+    for (int t = 0; t < run; ++t) {
+        constexpr int kStep = LINES ? kScanBlock : 1;
+        const int64_t base = first + (int64_t)t * kScanTile + threadIdx.x * (LINES ? 1 : kScanPer);
 #pragma unroll
-    for (int q = 0; q < kScanPer; ++q) c += base + q < S.n && S.sel((int)base + q);
+        for (int q = 0; q < kScanPer; ++q) c += base + q * kStep < S.n && S.sel((int)(base + q * kStep));
+    }
     c = block_sum256(c, red);
     if (threadIdx.x == 0) M.counts(side)[blockIdx.x] = c;
 }
 
-// also pads the keys of a core smaller than 2^L with fixed points, and zeroes
+// LINES: consecutive threads take consecutive points, so that those passed on
+// unchanged leave in whole lines, and a workgroup takes as many tiles as keep
+// their number bounded; else each thread takes kScanPer consecutive points,
+// whose ranks are one scan.  Kernel time of a product, else / LINES: 5000
+// points, k = 64 19 / 22 us; 100000, 65000 153 / 156; 2^20, 1 49 / 45; 2^22,
+// 64 159 / 142; 2^26, 64 2470 / 2180.
+// Also pads the keys of a core smaller than 2^L with fixed points, and zeroes
 // the tile counts of a big core's depths 1 and 2, which the partitions before
 // them accumulate
+template <bool LINES>
 __global__ __launch_bounds__(kScanBlock) void slice_scatter_kernel(MulBatch B)
 {
     const MulArgs &M = B.m[blockIdx.y >> 1];
@@ -1092,43 +1114,80 @@ __global__ __launch_bounds__(kScanBlock) void slice_scatter_kernel(MulBatch B)
         for (int x = blockIdx.x * kScanBlock + threadIdx.x; x < 2 * ntiles; x += gridDim.x * kScanBlock)
             M.core()[cnt + (size_t)side * 2 * ntiles + x] = 0;
     }
-    if ((int64_t)blockIdx.x * kScanTile >= S.n) return;   // past this slice's blocks (whole block)
-    __shared__ int red[kScanBlock / 64], wsum[kScanBlock / 64];
+    const int run = LINES ? M.run : 1;
+    const int64_t first = (int64_t)blockIdx.x * run * kScanTile;
+    if (first >= S.n) return;   // past this slice's blocks (whole block)
+    constexpr int kWaves = kScanBlock / 64, kGroups = kScanPer * kWaves;   // groups of 64 points, in order
+    static_assert(kGroups <= 64, "one wave scans the groups' counts");
+    __shared__ int red[kWaves], group[LINES ? kGroups : kWaves];
     const int32_t *counts = M.counts(side);
     int before = 0;
     for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanBlock) before += counts[i];
     before = block_sum256(before, red);
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x * kScanPer;
-    int32_t v[kScanPer];
-    int c = 0;
-#pragma unroll
-    for (int q = 0; q < kScanPer; ++q) {
-        v[q] = base + q < S.n ? S.src[base + q] : -1;
-        c += v[q] >= S.lo && v[q] < S.hi;
-    }
-    const int incl = wave_incl_scan(c);
-    if ((threadIdx.x & 63) == 63) wsum[threadIdx.x >> 6] = incl;
-    __syncthreads();
-    int j = before + incl - c;
-    for (int q = 0; q < (int)(threadIdx.x >> 6); ++q) j += wsum[q];
-#pragma unroll
-    for (int q = 0; q < kScanPer; ++q) {
-        const int i = (int)base + q;
-        if (base + q >= S.n) break;
-        if (v[q] >= S.lo && v[q] < S.hi) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // point i (value v) goes to place j of the core's, or on unchanged
+    auto place = [&](int i, int32_t v, bool selected, int j) {
+        if (selected) {
             if (j < k) {
                 map[j] = i;
-                key[j] = v[q] - S.lo;
+                key[j] = v - S.lo;
             }
-            ++j;
-            continue;
+            return;
         }
         // an untouched point (row, col) of p or q; the range test only matters
         // after an aborted comb fed undefined input
-        int row = side ? v[q] : i, col = side ? i : v[q];
+        int row = side ? v : i, col = side ? i : v;
         if (side == 0 && M.row_glue) { row += qs - k; col += qs - k; }
         if (side == 1 && !M.row_glue) { row += ps - k; col += ps - k; }
         if ((uint32_t)row < (uint32_t)(ps + qs - k)) M.out[row] = col;
+    };
+    int32_t v[kScanPer];
+    if constexpr (!LINES) {
+        const int64_t base = first + threadIdx.x * kScanPer;
+        int c = 0;
+#pragma unroll
+        for (int q = 0; q < kScanPer; ++q) {
+            v[q] = base + q < S.n ? S.src[base + q] : -1;
+            c += v[q] >= S.lo && v[q] < S.hi;
+        }
+        const int incl = wave_incl_scan(c);
+        if (lane == 63) group[wave] = incl;
+        __syncthreads();
+        int j = before + incl - c;
+        for (int q = 0; q < wave; ++q) j += group[q];
+#pragma unroll
+        for (int q = 0; q < kScanPer; ++q) {
+            if (base + q >= S.n) break;
+            const bool selected = v[q] >= S.lo && v[q] < S.hi;
+            place((int)(base + q), v[q], selected, j);
+            j += selected;
+        }
+    } else {
+        for (int t = 0; t < run; ++t) {
+            const int64_t base = first + (int64_t)t * kScanTile + threadIdx.x;
+            unsigned long long mask[kScanPer];
+#pragma unroll
+            for (int q = 0; q < kScanPer; ++q) v[q] = base + q * kScanBlock < S.n ? S.src[base + q * kScanBlock] : -1;
+#pragma unroll
+            for (int q = 0; q < kScanPer; ++q) {
+                mask[q] = __ballot(v[q] >= S.lo && v[q] < S.hi);
+                if (lane == 0) group[q * kWaves + wave] = __popcll(mask[q]);
+            }
+            __syncthreads();
+            const int c = lane < kGroups ? group[lane] : 0, incl = wave_incl_scan(c);
+            if (t + 1 < run) __syncthreads();   // before the next tile's counts
+            int start[kScanPer];   // read here, where every lane is there to be read
+#pragma unroll
+            for (int q = 0; q < kScanPer; ++q)
+                start[q] = before + __builtin_amdgcn_readlane(incl - c, q * kWaves + wave);
+            before += __builtin_amdgcn_readlane(incl, 63);
+#pragma unroll
+            for (int q = 0; q < kScanPer; ++q) {
+                if (base + q * kScanBlock >= S.n) break;
+                place((int)(base + q * kScanBlock), v[q], mask[q] >> lane & 1,
+                      start[q] + __popcll(mask[q] & ((1ull << lane) - 1)));
+            }
+        }
     }
 }
 
@@ -1216,7 +1275,8 @@ int lcsb_multiply_many_device(const MulSpec *specs, int count, hipStream_t strea
     for (int i = 0; i < count; ++i) {
         const MulSpec &M = specs[i];
         mul[(size_t)i] = MulArgs{M.p, M.q, M.out, M.ws, M.p_size, M.q_size, M.k, M.row_glue ? 1 : 0,
-                                 M.k ? lcsb_core_L(M.k) : 0, 0};
+                                 M.k ? lcsb_core_L(M.k) : 0, 0, 0};
+        mul[(size_t)i].set_blocks();
         if (mul[(size_t)i].L > kMaxCoreL) return -34;
     }
     std::stable_sort(mul.begin(), mul.end(), [](const MulArgs &x, const MulArgs &y) { return x.L < y.L; });
@@ -1234,10 +1294,17 @@ int lcsb_multiply_many_device(const MulSpec *specs, int count, hipStream_t strea
             if (n_max) hipLaunchKernelGGL(juxtapose_kernel, by_point, dim3(256), 0, stream, B);
             continue;
         }
-        const dim3 slices((unsigned)(n_max / kScanTile + 1), 2 * (unsigned)cnt);
+        int slice_blocks = 0;
+        for (int c = 0; c < cnt; ++c) slice_blocks = std::max(slice_blocks, B.m[c].blocks);
+        const dim3 slices((unsigned)slice_blocks, 2 * (unsigned)cnt);
         hipLaunchKernelGGL(invert_kernel, dim3((unsigned)((q_max + 255) / 256), (unsigned)cnt), dim3(256), 0, stream, B);
-        hipLaunchKernelGGL(slice_count_kernel, slices, dim3(kScanBlock), 0, stream, B);
-        hipLaunchKernelGGL(slice_scatter_kernel, slices, dim3(kScanBlock), 0, stream, B);
+        if (n_max >= kLinesMin) {
+            hipLaunchKernelGGL(slice_count_kernel<true>, slices, dim3(kScanBlock), 0, stream, B);
+            hipLaunchKernelGGL(slice_scatter_kernel<true>, slices, dim3(kScanBlock), 0, stream, B);
+        } else {
+            hipLaunchKernelGGL(slice_count_kernel<false>, slices, dim3(kScanBlock), 0, stream, B);
+            hipLaunchKernelGGL(slice_scatter_kernel<false>, slices, dim3(kScanBlock), 0, stream, B);
+        }
         if (L < kBigMinL) {
             hipLaunchKernelGGL(braid_core_lds_kernel, dim3((unsigned)cnt), dim3(kThreads), lds_core_bytes(L), stream, B);
             continue;
@@ -1268,5 +1335,6 @@ size_t lcsb_multiply_ws_words(int32_t p_size, int32_t q_size, int32_t k)
     M.p_size = p_size;
     M.q_size = q_size;
     M.k = k;
-    return (size_t)q_size + 2 * (size_t)k + 2 * (size_t)M.blocks() + lcsb_core_scratch_words(k > 0 ? k : 1);
+    M.set_blocks();
+    return (size_t)q_size + 2 * (size_t)k + 2 * (size_t)M.blocks + lcsb_core_scratch_words(k > 0 ? k : 1);
 }

@@ -150,3 +150,13 @@ def test_strips_above_32768_rows(ctx, m, n, strips):
     h, v, _ = ctx.comb(a, b, lcs_amd.schedule(strips=strips))
     ho, vo = oracle.comb(a, b, order="simd")
     assert np.array_equal(h, ho) and np.array_equal(v, vo)
+
+
+@pytest.mark.parametrize("p_size,q_size,k", [(4096 * 2048, 3000, 64), (3000, 4096 * 2048 - 1, 2100),
+                                             (9000011, 8400001, 3), ((1 << 18) - 1, 7001, 300), (1 << 18, 7001, 300),
+                                             (5003, (1 << 18) + 77, 1500)])
+def test_slices_of_several_tiles_per_workgroup(ctx, p_size, q_size, k):
+    rng = np.random.default_rng(k)
+    p, q = rng.permutation(p_size).astype(np.int32), rng.permutation(q_size).astype(np.int32)
+    for glue in (False, True):
+        assert np.array_equal(ctx.braid_multiply(p, q, k, glue), oracle.staggered_multiply(p, q, k, glue))

@@ -204,3 +204,17 @@ for device in (0, 1):
         c.llcs_batch([zeros(100)], [zeros(100)], 4)
 result = [rec.rec_lds_devices(k) for k in (b"llcs_chain_kernel", b"big_leaf_kernel", b"braid_core_lds_kernel")]
 """) == [2, 2, 2]
+
+
+def test_a_slice_has_a_bounded_number_of_workgroups(host):
+    # each adds up the counts of those before it
+    blocks = host("""
+result = []
+with lcs_amd.Context(0) as c:
+    for size in (2047, 2048, 4096 * 2048 - 1, 4096 * 2048, 1 << 24):
+        p = np.arange(size, dtype=np.int32)
+        rec.rec_clear()
+        c.braid_multiply(p, p[:100], 64, False)
+        result += [g[0] for g in launches('slice_count_kernel') + launches('slice_scatter_kernel')]
+""")
+    assert blocks == [1, 1, 2, 2, 4096, 4096, 2049, 2049, 2731, 2731], blocks
