@@ -1331,10 +1331,8 @@ int lcsb_multiply_device(const int32_t *p, int32_t p_size, const int32_t *q, int
 
 size_t lcsb_multiply_ws_words(int32_t p_size, int32_t q_size, int32_t k)
 {
-    MulArgs M{};
-    M.p_size = p_size;
-    M.q_size = q_size;
-    M.k = k;
-    M.set_blocks();
-    return (size_t)q_size + 2 * (size_t)k + 2 * (size_t)M.blocks + lcsb_core_scratch_words(k > 0 ? k : 1);
+    // at least MulArgs::blocks counts a side, and no fewer for a larger product:
+    // merges reserve for the largest of a level
+    const int32_t tiles = std::max(p_size, q_size) / kScanTile + 1;
+    return (size_t)q_size + 2 * (size_t)k + 2 * (size_t)std::min(tiles, kMaxSliceBlocks) + lcsb_core_scratch_words(k > 0 ? k : 1);
 }

@@ -218,3 +218,18 @@ with lcs_amd.Context(0) as c:
         result += [g[0] for g in launches('slice_count_kernel') + launches('slice_scatter_kernel')]
 """)
     assert blocks == [1, 1, 2, 2, 4096, 4096, 2049, 2049, 2731, 2731], blocks
+
+
+def test_a_larger_product_needs_no_smaller_workspace(host):
+    # a merge level reserves for its largest product, whichever has more
+    # workgroups to a slice
+    words = host("""
+f = lib()._Z22lcsb_multiply_ws_wordsiii
+f.restype = ctypes.c_size_t
+tile, most = 2048, 4096
+sizes = [s + d for s in (tile, tile * most, 2 * tile * most, 3 * tile * most) for d in (-tile - 1, -tile, -1, 0, 1, tile)]
+result = [[f(p, q, k) for p, q in zip(sizes, sizes)] for k in (1, 300)]
+result += [[f(s, 400, 300) for s in sizes], [f(400, s, 300) for s in sizes]]
+""")
+    for row in words:
+        assert row == sorted(row), row
