@@ -435,6 +435,7 @@ struct MulArgs {
     int32_t *out, *ws;
     int32_t p_size, q_size, k, row_glue, L;
     int32_t run, blocks;   // tiles of kScanTile points that a workgroup of a slice takes, and the workgroups
+    int32_t big;           // the core runs over the whole GPU
     __host__ __device__ int32_t *q_c2r() const { return ws; }
     __host__ __device__ int32_t *map_row() const { return ws + q_size; }
     __host__ __device__ int32_t *map_col() const { return map_row() + k; }
@@ -1108,7 +1109,7 @@ __global__ __launch_bounds__(kScanBlock) void slice_scatter_kernel(MulBatch B)
     int32_t *const key = M.core() + (side ? K : 0), *const map = side ? M.map_col() : M.map_row();
     for (int64_t x = k + (int64_t)blockIdx.x * kScanBlock + threadIdx.x; x < K; x += (int64_t)gridDim.x * kScanBlock)
         key[x] = (int32_t)x;
-    if (M.L >= kBigMinL) {
+    if (M.big) {
         const int ntiles = K / kSplitTile;
         const size_t cnt = big_layout_cnt(M.L) + (size_t)ntiles * 2;
         for (int x = blockIdx.x * kScanBlock + threadIdx.x; x < 2 * ntiles; x += gridDim.x * kScanBlock)
@@ -1212,10 +1213,12 @@ __global__ void juxtapose_kernel(MulBatch B)
 
 using namespace lcsb;
 
-size_t lcsb_core_scratch_words(int32_t k)
+static bool core_is_big(int L, bool in_lds) { return L >= kBigMinL && !(in_lds && L <= kLdsCoreL); }
+
+size_t lcsb_core_scratch_words(int32_t k, bool in_lds)
 {
     const int L = lcsb_core_L(k);
-    return L >= kBigMinL ? big_layout(L, big_leaf_L(L)).total : (size_t)2 << L;   // small cores: the keys
+    return core_is_big(L, in_lds) ? big_layout(L, big_leaf_L(L)).total : (size_t)2 << L;   // small cores: the keys
 }
 
 // Padded core size 2^L: at least 64 (the LDS kernel ranks keys by wave
@@ -1268,14 +1271,15 @@ int lcsb_init(void)
 // sequence side by side (in groups of kMulBatch), so the products of a
 // merge-tree level share their launches.  specs[i].ws holds
 // lcsb_multiply_ws_words(p_size, q_size, k) words.
-int lcsb_multiply_many_device(const MulSpec *specs, int count, hipStream_t stream)
+int lcsb_multiply_many_device(const MulSpec *specs, int count, hipStream_t stream, bool in_lds)
 {
     if (lcsb_init()) return -5;
     std::vector<MulArgs> mul((size_t)count);
     for (int i = 0; i < count; ++i) {
         const MulSpec &M = specs[i];
         mul[(size_t)i] = MulArgs{M.p, M.q, M.out, M.ws, M.p_size, M.q_size, M.k, M.row_glue ? 1 : 0,
-                                 M.k ? lcsb_core_L(M.k) : 0, 0, 0};
+                                 M.k ? lcsb_core_L(M.k) : 0, 0, 0, 0};
+        mul[(size_t)i].big = core_is_big(mul[(size_t)i].L, in_lds);
         mul[(size_t)i].set_blocks();
         if (mul[(size_t)i].L > kMaxCoreL) return -34;
     }
@@ -1305,7 +1309,7 @@ int lcsb_multiply_many_device(const MulSpec *specs, int count, hipStream_t strea
             hipLaunchKernelGGL(slice_count_kernel<false>, slices, dim3(kScanBlock), 0, stream, B);
             hipLaunchKernelGGL(slice_scatter_kernel<false>, slices, dim3(kScanBlock), 0, stream, B);
         }
-        if (L < kBigMinL) {
+        if (!B.m[0].big) {
             hipLaunchKernelGGL(braid_core_lds_kernel, dim3((unsigned)cnt), dim3(kThreads), lds_core_bytes(L), stream, B);
             continue;
         }
@@ -1323,16 +1327,16 @@ int lcsb_multiply_many_device(const MulSpec *specs, int count, hipStream_t strea
 
 // staggered_multiply on device pointers; ws must hold lcsb_multiply_ws_words(...)
 int lcsb_multiply_device(const int32_t *p, int32_t p_size, const int32_t *q, int32_t q_size, int32_t k,
-                         int32_t row_glue, int32_t *out, int32_t *ws, hipStream_t stream)
+                         int32_t row_glue, int32_t *out, int32_t *ws, hipStream_t stream, bool in_lds)
 {
     const MulSpec M{p, p_size, q, q_size, k, row_glue, out, ws};
-    return lcsb_multiply_many_device(&M, 1, stream);
+    return lcsb_multiply_many_device(&M, 1, stream, in_lds);
 }
 
-size_t lcsb_multiply_ws_words(int32_t p_size, int32_t q_size, int32_t k)
+size_t lcsb_multiply_ws_words(int32_t p_size, int32_t q_size, int32_t k, bool in_lds)
 {
     // at least MulArgs::blocks counts a side, and no fewer for a larger product:
     // merges reserve for the largest of a level
     const int32_t tiles = std::max(p_size, q_size) / kScanTile + 1;
-    return (size_t)q_size + 2 * (size_t)k + 2 * (size_t)std::min(tiles, kMaxSliceBlocks) + lcsb_core_scratch_words(k > 0 ? k : 1);
+    return (size_t)q_size + 2 * (size_t)k + 2 * (size_t)std::min(tiles, kMaxSliceBlocks) + lcsb_core_scratch_words(k > 0 ? k : 1, in_lds);
 }

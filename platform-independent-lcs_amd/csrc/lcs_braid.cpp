@@ -38,12 +38,17 @@ extern "C" int lcs_braid_multiply(lcs_ctx *ctx, const int32_t *p_row_to_col, int
     if (k > kMaxCoreK) return LCS_ERANGE;
     if (out_size == 0) return LCS_OK;
     if (hipSetDevice(ctx->device) != hipSuccess) return LCS_EIO;
-    const size_t ws_words = lcsb_multiply_ws_words(p_size, q_size, k);
-    const size_t words = (size_t)p_size + q_size + out_size + ws_words + 16;
+    const size_t io_words = (size_t)p_size + q_size + out_size;
+    size_t words = io_words + lcsb_multiply_ws_words(p_size, q_size, k) + 16;
     // kept between calls: with it, the staged copies and the results returned
     // uncopied, a product with k = 65000 fell from 430 to 320 us
     DevBuf buf = ctx->scratch.take(words * 4, kKeptMax);
     int rc = buf.reserve(ctx, words * 4);
+    const bool in_lds = rc == LCS_ENOMEM;   // a workspace that may still fit
+    if (in_lds) {
+        words = io_words + lcsb_multiply_ws_words(p_size, q_size, k, true);
+        rc = buf.reserve(ctx, words * 4);
+    }
     if (rc) return rc;
     int32_t *dp = (int32_t *)buf.ptr, *dq = dp + p_size, *dout = dq + q_size, *dws = dout + out_size;
     hipStream_t s = ctx->stream;
@@ -61,7 +66,7 @@ extern "C" int lcs_braid_multiply(lcs_ctx *ctx, const int32_t *p_row_to_col, int
     }
     ctx->pending_timing = false;   // its events are recorded anew
     if (!ok || hipEventRecord(ctx->ev0, s) != hipSuccess) { buf.release(ctx); return LCS_EIO; }
-    rc = lcsb_multiply_device(dp, p_size, dq, q_size, k, row_glue ? 1 : 0, dout, dws, s);
+    rc = lcsb_multiply_device(dp, p_size, dq, q_size, k, row_glue ? 1 : 0, dout, dws, s, in_lds);
     if (!rc) {
         (void)hipEventRecord(ctx->ev1, s);
         ok = hipMemcpyAsync(pin ? pin + in_words : out_row_to_col, dout, (size_t)out_size * 4, hipMemcpyDeviceToHost, s) == hipSuccess &&

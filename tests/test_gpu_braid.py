@@ -160,3 +160,12 @@ def test_slices_of_several_tiles_per_workgroup(ctx, p_size, q_size, k):
     p, q = rng.permutation(p_size).astype(np.int32), rng.permutation(q_size).astype(np.int32)
     for glue in (False, True):
         assert np.array_equal(ctx.braid_multiply(p, q, k, glue), oracle.staggered_multiply(p, q, k, glue))
+
+
+@pytest.mark.parametrize("k", [1025, 2047, 2048])
+def test_core_of_2048_in_lds_under_a_small_budget(k):
+    rng = np.random.default_rng(k)
+    p, q = rng.permutation(4096).astype(np.int32), rng.permutation(4000).astype(np.int32)
+    with lcs_amd.Context(0, hbm_budget=114776) as small:
+        for glue in (False, True):
+            assert np.array_equal(small.braid_multiply(p, q, k, glue), oracle.staggered_multiply(p, q, k, glue))

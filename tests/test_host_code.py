@@ -224,12 +224,27 @@ def test_a_larger_product_needs_no_smaller_workspace(host):
     # a merge level reserves for its largest product, whichever has more
     # workgroups to a slice
     words = host("""
-f = lib()._Z22lcsb_multiply_ws_wordsiii
+f = lib()._Z22lcsb_multiply_ws_wordsiiib
 f.restype = ctypes.c_size_t
 tile, most = 2048, 4096
 sizes = [s + d for s in (tile, tile * most, 2 * tile * most, 3 * tile * most) for d in (-tile - 1, -tile, -1, 0, 1, tile)]
-result = [[f(p, q, k) for p, q in zip(sizes, sizes)] for k in (1, 300)]
-result += [[f(s, 400, 300) for s in sizes], [f(400, s, 300) for s in sizes]]
+result = [[f(p, q, k, False) for p, q in zip(sizes, sizes)] for k in (1, 300)]
+result += [[f(s, 400, 300, False) for s in sizes], [f(400, s, 300, False) for s in sizes]]
 """)
     for row in words:
         assert row == sorted(row), row
+
+
+def test_a_product_of_2048_strands_fits_where_it_did(host):
+    # one workgroup's LDS holds the core where the budget does not hold the
+    # workspace of a core spread over the GPU
+    got = host("""
+result = []
+p = np.arange(4096, dtype=np.int32)
+for budget in (0, 114776):
+    with lcs_amd.Context(0, hbm_budget=budget) as c:
+        rec.rec_clear()
+        c.braid_multiply(p, p, 2048, True)
+        result.append([len(launches('braid_core_lds_kernel')), len(launches('big_leaf_kernel'))])
+""")
+    assert got == [[0, 1], [1, 0]]
