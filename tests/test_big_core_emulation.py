@@ -1,12 +1,13 @@
 """CPU emulation of the whole-GPU steady ant's index arithmetic
 (platform-independent-lcs_amd/csrc/braid_kernels.hip, the "big cores" kernels:
-big_split_count/scatter, big_lift_kernel, big_hist_kernel, block_search, sweep_block,
-big_walk_kernel), step for step in Python, checked against the oracle's
-steady ant (orc_steady_ant, braid_multiplication.hpp:204-270).  The leaves
-(one workgroup each on the GPU) are taken from the oracle here; the GPU tests
-check the leaf kernel itself.  Small line and block constants make small
-cores exercise what only large cores meet on the GPU: several histogram
-blocks per node, blocks of 512 entries, boxes wider than 64."""
+big_split_count/scatter, the leaves' big_lift, big_hist_kernel, and
+big_box_kernel with its line search, row rule, 64 x 64 steps of wider boxes
+and lift into the parents), step for step in Python, checked against the
+oracle's steady ant (orc_steady_ant, braid_multiplication.hpp:204-270).  The
+leaves (one workgroup each on the GPU) are taken from the oracle here; the GPU
+tests check the leaf kernel itself.  Small line, wave and block constants make
+small cores exercise what only large cores meet on the GPU: several histogram
+blocks per node, blocks of 512 entries, boxes wider than a wave."""
 import numpy as np
 import pytest
 
@@ -16,11 +17,8 @@ LO = 1 << 31
 
 
 def counted31(e, r):
-    return (((e - r) & 0xFFFFFFFF) >> 31) & 1
-
-
-def counted16(e, r):
-    return (((e - r) & 0xFFFFFFFF) >> 15) & 1
+    """counted<31>: bit 31 of e - r (numbers or arrays)."""
+    return ((e - r) & 0xFFFFFFFF) >> 31
 
 
 def w_log(e):
@@ -98,7 +96,60 @@ def block_search(Hj, Ht, nsegs, Yj):
     return nsegs - 1, Z
 
 
+def select(counts, need):
+    """Position of the need-th counted column of a row (select64), need >= 1."""
+    return int(np.nonzero(np.cumsum(counts) == need)[0][0])
+
+
+def box_rows(u, CI, r_lo, rho, cs, ce, col, wave):
+    """The rows of a box of one wave that this piece decides, as (row, column)."""
+    r = r_lo + np.arange(wave)
+    m = counted31(u, cs)
+    if col:
+        m = m & (r < rho)
+    need = int(col) + np.cumsum(m[::-1])[::-1]
+    assert ce - cs <= wave
+    out = []
+    for i in range(wave):
+        c = counted31(CI[cs:ce], int(r[i]))
+        if (col and r[i] > rho) or need[i] > c.sum():
+            continue
+        T = cs + 1 + select(c, need[i]) if need[i] else cs
+        out.append((int(r[i]), T - 1 if T > 0 and counted31(int(u[i]), T) else int(u[i]) & (LO - 1)))
+    return out
+
+
+def wide_box_rows(U, CI, r_lo, rho, cs, ce, col, wave):
+    """The same in a box wider than a wave: `wave` rows at a time from rho
+    upwards, the rows counted so far carried in `below`; `wave` columns at a
+    time, the columns still needed carried in `need`."""
+    out, below = [], int(col)
+    for rb in range(rho & ~(wave - 1), r_lo - 1, -wave):
+        r = rb + np.arange(wave)
+        u = U[rb:rb + wave]
+        m = counted31(u, cs)
+        if col:
+            m = m & (r < rho)
+        need = below + np.cumsum(m[::-1])[::-1]
+        below += int(m.sum())
+        T = np.where(need > 0, -1, cs)
+        for c0 in range(cs, ce, wave):
+            e = np.full(wave, LO - 1, np.int64)   # past ce: counted at no line
+            e[:min(wave, ce - c0)] = CI[c0:min(c0 + wave, ce)]
+            for i in range(wave):
+                c = counted31(e, int(r[i]))
+                if T[i] < 0 and need[i] <= c.sum():
+                    T[i] = c0 + 1 + select(c, need[i])
+                need[i] -= c.sum()
+        for i in range(wave):
+            if (not col or r[i] <= rho) and T[i] >= 0:
+                t = int(T[i])
+                out.append((int(r[i]), t - 1 if t > 0 and counted31(int(u[i]), t) else int(u[i]) & (LO - 1)))
+    return out
+
+
 def emulate(P, Q, k, L, L0, box_g=64, max_lines=8192, w_fixed=None):
+    """box_g: rows and columns of a wave (64 on the GPU)."""
     K = 1 << L
     d0 = L - L0
     keyP = np.array([P[x] if x < k else x for x in range(K)], np.int64)
@@ -117,31 +168,33 @@ def emulate(P, Q, k, L, L0, box_g=64, max_lines=8192, w_fixed=None):
             cP, cQ = nP, nQ
         parP.append(pp)
         parQ.append(pq)
+    # U and CI alternate between two sets: a depth's boxes read one and lift
+    # into the other
+    U2, CI2 = [np.full(K, -1, np.int64) for _ in range(2)], [np.full(K, -1, np.int64) for _ in range(2)]
+
+    def lift(d, v0, h, x, c):
+        p_pos, q_pos = int(parP[d][x]), int(parQ[d][v0 + (c & (h - 1))])
+        p0 = p_pos & ~(2 * h - 1)
+        lo = 0 if x & h else LO
+        U2[d & 1][p_pos] = (q_pos - p0) | lo
+        CI2[d & 1][q_pos] = (p_pos - p0) | lo
+
     s0 = 1 << L0
-    R = np.empty(K, np.int64)
+    R = np.full(K, -1, np.int64)
     for v in range(K >> L0):
         kp = keyP[v * s0:(v + 1) * s0] & (s0 - 1)
         kq = keyQ[v * s0:(v + 1) * s0] & (s0 - 1)   # column -> shared row
         qr2c = np.empty(s0, np.int32)
         qr2c[kq] = np.arange(s0)
-        R[v * s0:(v + 1) * s0] = oracle.steady_ant(kp.astype(np.int32), qr2c)
+        for x, c in enumerate(oracle.steady_ant(kp.astype(np.int32), qr2c)):
+            lift(d0 - 1, v * s0, s0, v * s0 + x, int(c))
     for d in range(d0 - 1, -1, -1):
         s, nb, glog, w, nsegs = depth(L, d, box_g, max_lines, w_fixed)
         g = 1 << glog
-        h = s >> 1
         nodes = K // s
-        # big_lift_kernel
-        U = np.zeros(K, np.int64)
-        CI = np.zeros(K, np.int64)
-        Rn = np.zeros(K, np.int64)
-        for x in range(K):
-            p_pos = int(parP[d][x])
-            q_pos = int(parQ[d][(x & ~(h - 1)) + int(R[x])])
-            v0 = p_pos & ~(s - 1)
-            lo = 0 if (x & h) else LO
-            U[p_pos] = (q_pos - v0) | lo
-            CI[v0 + q_pos - v0] = (p_pos - v0) | lo
-            Rn[p_pos] = q_pos - v0
+        U, CI = U2[d & 1], CI2[d & 1]
+        assert (U >= 0).all() and (CI >= 0).all()
+        U2[1 - (d & 1)][:] = CI2[1 - (d & 1)][:] = -1   # what a depth reads was written for it
         # big_hist_kernel: per (y, node) an nb x nsegs prefix matrix, then totals
         H = {}
         for y, E in ((0, CI), (1, U)):
@@ -156,7 +209,7 @@ def emulate(P, Q, k, L, L0, box_g=64, max_lines=8192, w_fixed=None):
                     M[:nb, gg] = np.concatenate([[0], np.cumsum(hh)[:-1]])
                     M[nb, gg] = hh.sum()
                 H[(y, node)] = M
-        # big_sweep_kernel: block_search + sweep_block
+        # big_line: block_search + sweep_block
         T = {}
         for y, E in ((0, CI), (1, U)):
             for node in range(nodes):
@@ -178,61 +231,31 @@ def emulate(P, Q, k, L, L0, box_g=64, max_lines=8192, w_fixed=None):
                                 T[(y, node, j)] = seg * w + r + 1
                                 break
                     assert need == 0
-        # big_walk_kernel: one lane per piece, 16-bit entries relative to the box
-        for node in range(nodes):
+        # big_box_kernel: one wave per piece (row lines, then column lines)
+        seen = np.zeros(K, int)
+        for t in range(2 * nodes * nb):
+            col = t >= nodes * nb
+            node, j = divmod(t - nodes * nb if col else t, nb)
+            T0 = T[(int(col), node, j)] if j else 0
+            if col and (j == 0 or T0 == 0):
+                continue
+            if col:
+                rho, cs = T0 - 1, (nb - j) * g
+                r_lo, ce = rho & ~(g - 1), cs + g
+            else:
+                r_lo, cs = s - (j + 1) * g, T0
+                rho, ce = r_lo + g - 1, g if cs == 0 else (((cs - 1) >> glog) + 1) << glog
             v0 = node * s
-            for q in range(2 * nb - 1):
-                if q < nb:
-                    Dr = s - q * g
-                    dc = 0 if q == 0 else min(max(T[(0, node, q)], 0), s)
-                    dr, r_lo = Dr - 1, Dr - g
-                    cb = 0 if dc == 0 else (dc - 1) >> glog
+            Un, CIn = U[v0:v0 + s], CI[v0:v0 + s]
+            rows = (box_rows(Un[r_lo:r_lo + g], CIn, r_lo, rho, cs, ce, col, box_g) if g == box_g
+                    else wide_box_rows(Un, CIn, r_lo, rho, cs, ce, col, box_g))
+            for r, c in rows:
+                seen[v0 + r] += 1
+                if d:
+                    lift(d - 1, v0, s, v0 + r, c)
                 else:
-                    i = q - nb + 1
-                    Tc = min(max(T[(1, node, nb - i)], 0), s)
-                    if Tc == 0:
-                        continue
-                    dr, dc = Tc - 1, i * g + 1
-                    r_lo = s - (((s - 1 - dr) >> glog) + 1) * g
-                    cb = i
-                c_lo = cb * g + 1 if cb else 0
-                c_hi = s + 1 if cb == nb - 1 else (cb + 1) * g + 1
-                nc = c_hi - c_lo + 1
-                assert nc <= g + 2
-
-                def box_entry(e, base, top):
-                    return (0x8000 if (e & LO) else 0) | (min(max(e & 0x7FFFFFFF, base), top) - base)
-
-                bu = [box_entry(int(U[v0 + min(max(r_lo - 1 + i, 0), s - 1)]), c_lo - 1, c_hi) for i in range(g + 1)]
-                bc = [box_entry(int(CI[v0 + min(max(c_lo - 1 + i, 0), s - 1)]), r_lo - 1, r_lo + g) for i in range(nc)]
-                box = bu + bc
-                Rr, X, Xs = dr - r_lo + 1, dc - c_lo + 1, s - c_lo + 1
-                assert 1 <= Rr <= g and 1 <= X < nc
-                # the same entry values as the node-level (absolute) form
-                if q < nb:
-                    assert counted16(bu[Rr], X) == counted31(int(U[v0 + dr]), dc)
-                    delta = -counted16(bu[Rr], X)
-                else:
-                    assert counted16(bc[0], Rr) == counted31(int(CI[v0 + i * g]), dr)
-                    delta = -1 + counted16(bc[0], Rr)
-                cl, cc, ud, ur = bc[X - 1], bc[X], bu[Rr], bu[Rr - 1]
-                while Rr >= 1 and X < nc:
-                    d_left = delta - counted16(cl, Rr)
-                    d_down = delta + counted16(ud, X)
-                    if X + c_lo > 1 and d_left < 0 and d_down > 0:
-                        Rn[v0 + Rr + r_lo - 1] = X + c_lo - 2
-                    right = delta < 0 and X < Xs
-                    d_right = counted16(cc, Rr)
-                    d_up = counted16(ur, X) if Rr + r_lo > 1 else 0
-                    delta = delta + d_right if right else delta - d_up
-                    X += 1 if right else 0
-                    Rr -= 0 if right else 1
-                    cl = cc if right else cl
-                    ud = ud if right else ur
-                    nx = box[g + 1 + min(X, nc - 1)] if right else box[max(Rr - 1, 0)]
-                    cc = nx if right else cc
-                    ur = ur if right else nx
-        R = Rn
+                    R[r] = c
+        assert (seen == 1).all()   # every row lies in exactly one piece's box
     return R[:k].astype(np.int32)
 
 
@@ -240,9 +263,10 @@ CASES = [
     # (k, L, L0, box side, max lines, fixed block width)
     (4096, 12, 10, 64, 8192, None),     # the library's constants: one block per node
     (4000, 12, 11, 64, 8192, None),     # padded core, leaves of 2^11
-    (6000, 13, 11, 32, 8192, None),     # boxes of 32
+    (6000, 13, 11, 32, 8192, None),     # waves of 32
     (4096, 12, 10, 64, 16, 512),        # wide boxes (g = 256 at the top) and 8 blocks per node
-    (8192, 13, 10, 16, 8192, 512),      # boxes of 16, 16 blocks per node
+    (4000, 12, 10, 32, 16, 512),        # boxes of 4 and 8 waves a side
+    (8192, 13, 10, 16, 8192, 512),      # waves of 16, 16 blocks per node
     (16384, 14, 10, 32, 8192, None),    # four device-wide depths, 8 partition tiles per segment
 ]
 
@@ -273,7 +297,7 @@ def test_big_core_structured():
 
 def test_block_width_bounds():
     """Blocks are 512 .. 8192 entries, at most 1024 per node up to 2^22 points
-    (what big_sweep_kernel's block search holds in registers)."""
+    (what big_line's block search holds in registers)."""
     for e in range(11, 23):
         w = min(1 << e, 1 << w_log(e))
         assert 512 <= w <= 8192 and (1 << e) // w <= 1024
