@@ -576,8 +576,8 @@ def main():
     cells = float(m) * float(n)
     ms_step = wall / args.steps * 1e3
     gcups = cells * args.steps / wall / 1e9
-    # the dominant kernel is the band chain (one launch combs every strip);
-    # the rest of a step is the strip permutations and steady-ant merges
+    # the dominant kernel is the band chain (one launch combs every tile);
+    # the rest of a step is the steady-ant merges of the tiles' permutations
     k_ms = float(np.mean([t for t, _ in kernel_ms]))
     chain_ms = float(np.mean([c for _, c in kernel_ms]))
     peak_ops = cus * 64 * PEAK_CLOCK_HZ
@@ -607,7 +607,7 @@ def main():
         "dtype": "int32",
         "data": "synthetic (seeded mt19937_64: uniform alphabet-4 A, B = A + 10% subs + 2% indels)",
         "config": {"workload": f"single pair m=n=2^{args.log2n}, tiled band-chain comb + steady-ant merge "
-                               "(library default schedule: four column strips, three merges with k = m)",
+                               "(library default schedule: tiles by predicted time, 4 x 2 with seven merges at 2^20)",
                    "m": m, "n": n, "alphabet": 4, "tile_m": args.tile_m or None, "variant": args.variant or None,
                    "llcs": llcs},
         "roofline": {"bound": "valu", "achieved": round(achieved_ops / 1e12, 3), "peak": round(peak_ops / 1e12, 3),

@@ -531,7 +531,7 @@ __global__ __launch_bounds__(kThreads) void braid_core_lds_kernel(MulBatch B)
 }
 
 // ---------------------------------------------------------------- big cores
-// Cores above kLdsCoreK run the same recursion spread over the whole GPU
+// Cores from 2^kBigMinL on run the same recursion spread over the whole GPU
 // (the one-workgroup core finishes its top depths in the same boxes):
 //  * the top d0 = L - L0 depths of the top-down split are device-wide
 //    stable partitions (count, scan, scatter per depth);

@@ -18,11 +18,13 @@
 //     U, sum with carry in and out (v_and, v_addc_co), V (v_bitop3)
 //     cout: shift the carry out into the outgoing word (v_addc_co),
 // five VALU for 2048 cells.  The columns of one band are a serial chain, so
-// the kernel's time is columns x time per column plus the bands' fill, and a
-// lone wave issues an instruction of any kind every four to five cycles: the
-// count per column is what matters.  With one column per step, carries in
-// lane-skewed SGPR masks and a second wave fetching through LDS a column took
-// 30.5 ns and m = n = 2^20 38.0 ms; now 15.0 and 19.9.  A band follows the one
+// the kernel's time is columns x time per column plus the bands' fill.  By the
+// counters a lone wave's six instructions a column take 5.8 cycles each, about
+// 30 % of them stall in the turn's chain of carries (a comb wave, without such
+// a chain, issues every four): their count and that chain are what matters.
+// With one column per step, carries in lane-skewed SGPR masks and a second wave
+// fetching through LDS a column took 30.5 ns and m = n = 2^20 38.0 ms; now 15.0
+// and 19.9.  A band follows the one
 // below by 64 blocks, so blocks of two (15 instead of 12 issues a turn for two
 // columns, 17 ns a column) halve the skew where bands, not columns, make the
 // time: the caller picks by that.
