@@ -180,10 +180,7 @@ template <int TM, int C, bool ROWMASK, bool COLMASK, bool PK = false, bool OH = 
 __device__ __forceinline__ void band_steps(const int32_t (&a)[TM], uint32_t (&h)[TM], const bool (&valid)[TM],
                                            uint32_t &v, int32_t &bq, uint32_t &Q, int32_t &IB, int t0, int lane, int n)
 {
-#ifndef LCS_PACKED_CHUNK_BLOCKS
-#define LCS_PACKED_CHUNK_BLOCKS 1
-#endif
-    if constexpr (LCS_PACKED_CHUNK_BLOCKS && PK && !COLMASK && C == 32 && TM >= 4 && TM <= 16) {
+    if constexpr (PK && !COLMASK && C == 32 && TM >= 4 && TM <= 16) {
         // the packed chain's 32 steps, hand-offs included, in one asm block
         // (cell_asm.h): no step waits out a hazard with an s_nop
         uint32_t ua[TM];
@@ -261,8 +258,7 @@ __device__ __forceinline__ void column_cells8(const int32_t (&a)[TM], uint32_t (
 // An unmasked step of four or more rows runs as one asm block (cell_asm.h:
 // the strand hand-off sits behind the step's first two compares, so the DPP
 // read of v needs no s_nop after the previous step's last cell wrote it);
-// band_steps8 uses this for 32-row tiles, and for every tile height when
-// its four-step blocks are compiled out.
+// band_steps8 uses this for 32-row tiles.
 template <int TM, bool ROWMASK, bool COLMASK, int SEL>
 __device__ __forceinline__ void band_step8(const int32_t (&a)[TM], uint32_t (&h)[TM], const bool (&valid)[TM],
                                            uint32_t &v, uint32_t &Q, uint32_t word, int t, int lane, int n)
@@ -308,39 +304,21 @@ __device__ __forceinline__ void band_steps8(const int32_t (&a)[TM], uint32_t (&h
                                             int n)
 {
 // The compiler puts an s_nop 0 before every asm block that reads the strand,
-// so larger blocks pay it less often.  LCS_CHUNK_BLOCKS=0 falls back to one
-// block per symbol word and LCS_WORD_BLOCKS=0 then to one per step (m = n =
-// 2^20: 131.5 ms per comb with chunk blocks, 132.0 with word blocks on the
-// same box; 133.6 with step blocks against 132.1 for word blocks on another).
-#ifndef LCS_WORD_BLOCKS
-#define LCS_WORD_BLOCKS 1
-#endif
-#ifndef LCS_CHUNK_BLOCKS
-#define LCS_CHUNK_BLOCKS 1
-#endif
-    if constexpr (LCS_CHUNK_BLOCKS && C == 32 && !ROWMASK && !COLMASK && TM <= 16) {
+// so larger blocks pay it less often (m = n = 2^20: 131.5 ms per comb with
+// chunk blocks, 132.0 with a block per symbol word on the same box; 133.6 with
+// a block per step against 132.1 for words on another).
+    if constexpr (C == 32 && !ROWMASK && !COLMASK && TM <= 16) {
         // the whole chunk in one asm block (cell_asm.h)
         uint32_t qn;
         cell_chunk32<TM>(a, h, sym, Q, v, qn);
         Q = qn;
         return;
     }
-    if constexpr (LCS_CHUNK_BLOCKS && C == 16 && !ROWMASK && !COLMASK && TM <= 16) {
+    if constexpr (C == 16 && !ROWMASK && !COLMASK && TM <= 16) {
         // half a chunk of a linked band (cell_asm.h)
         uint32_t qn;
         cell_chunk16<TM>(a, h, sym, Q, v, qn);
         Q = qn;
-        return;
-    }
-    if constexpr (LCS_WORD_BLOCKS && !ROWMASK && !COLMASK && TM <= 16) {
-        // the four steps of a symbol word in one asm block (cell_asm.h)
-#pragma unroll
-        for (int w = 0; w < C / 4; ++w) {
-            uint32_t vw = v, vt;
-            cell_word<TM>(a, h, (int32_t)sym[w], Q, vw, vt);
-            Q = vw;
-            v = vt;
-        }
         return;
     }
 #pragma unroll

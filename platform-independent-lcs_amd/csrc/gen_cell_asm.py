@@ -67,41 +67,6 @@ def step_block(R: int, sel: int) -> str:
             f"        {body}\n        : {', '.join(outs)}\n        : {', '.join(inp)});\n}}\n")
 
 
-def word_block(R: int) -> str:
-    """Four steps of the byte-symbol band loop for R rows, one per byte of
-    the symbol word, as one block: the compiler puts its own wait state only
-    between blocks.  The strand and the conveyor rotate through w, t and u
-    (step k moves the strand into the register the conveyor was copied to
-    and the conveyor into the strand's old register), and the rows' h
-    strands alternate between the caller's registers (h, in place) and a
-    scratch set, ending back in h after the fourth step."""
-    def cmp(sel, s, a):
-        return f'"v_cmp_eq_u32_sdwa %[{s}], %[{a}], %[b] src0_sel:DWORD src1_sel:BYTE_{sel}\\n\\t"'
-    regs = [("q", "t", "w"), ("w", "u", "t"), ("t", "w", "u"), ("u", "t", "w")]   # (conveyor, copy/strand, old strand)
-    ins = []
-    for sel in range(4):
-        conv, strand, old = regs[sel]
-        src_h, dst_h = ("h", "x") if sel % 2 == 0 else ("x", "h")
-        ins += [cmp(sel, "s0", "a0")] + ([cmp(sel, "s1", "a1")] if R > 1 else []) + [
-                f'"v_mov_b32_e32 %[{strand}], %[{conv}]\\n\\t"',
-                f'"v_mov_b32_dpp %[{strand}], %[{old}] wave_shr:1 row_mask:0xf bank_mask:0xf\\n\\t"',
-                f'"v_mov_b32_dpp %[{old}], %[{conv}] wave_shl:1 row_mask:0xf bank_mask:0xf\\n\\t"']
-        for k in range(R):
-            sk = f"s{k % 2}"
-            ins.append(f'"v_min_u32_e32 %[{dst_h}{k}], %[{src_h}{k}], %[{strand}]\\n\\t"')
-            ins.append(f'"v_cndmask_b32_e64 %[{dst_h}{k}], %[{dst_h}{k}], %[{strand}], %[{sk}]\\n\\t"')
-            ins.append(f'"v_bitop3_b32 %[{strand}], %[{src_h}{k}], %[{strand}], %[{dst_h}{k}] bitop3:0x96\\n\\t"')
-            if k + 2 < R:
-                ins.append(cmp(sel, sk, f"a{k + 2}"))
-    outs = ['[w] "+v"(w)', '[t] "=&v"(t)', '[u] "=&v"(u)'] + [f'[h{k}] "+v"(h[{k}])' for k in range(R)] + \
-           [f'[x{k}] "=&v"(x[{k}])' for k in range(R)] + ['[s0] "=&s"(s0)', '[s1] "=&s"(s1)']
-    inp = ['[b] "v"(sb)', '[q] "v"(q)'] + [f'[a{k}] "v"(a[{k}])' for k in range(R)]
-    body = "\n        ".join(ins)
-    return (f"__device__ __forceinline__ void cell_word{R}(const int32_t *a, uint32_t *h, int32_t sb, uint32_t q,"
-            f" uint32_t &w, uint32_t &t)\n{{\n    uint64_t s0, s1;\n    uint32_t u, x[{R}];\n    asm volatile(\n"
-            f"        {body}\n        : {', '.join(outs)}\n        : {', '.join(inp)});\n}}\n")
-
-
 def packed_block(R: int) -> str:
     """One step of the packed (two pairs in 16-bit halves) chain for R >= 3
     rows.  Per row k: X e = a ^ b, S mk = sat(1 - e), M hx = sat(mk * 0xffff
@@ -324,8 +289,6 @@ if __name__ == "__main__":
     for R in (4, 8, 16):
         for q in range(4):
             print(step_block(R, q))
-    for R in (1, 2, 4, 8, 16):
-        print(word_block(R))
     for R in (4, 8, 16):
         print(packed_block(R))
     for R in (4, 8, 16):
@@ -353,15 +316,6 @@ if __name__ == "__main__":
     print("    else if constexpr (R == 8) cell16_block8(a, h, hn, sb, v);")
     print("    else if constexpr (R == 16) cell16_block16(a, h, hn, sb, v);")
     print('    else static_assert(R == 4 || R == 8 || R == 16, "rows per block");\n}\n')
-    print("// cell_word{R} by template argument")
-    print("template <int R>\n__device__ __forceinline__ void cell_word(const int32_t *a, uint32_t *h, int32_t sb,"
-          " uint32_t q, uint32_t &w, uint32_t &t)\n{")
-    print("    if constexpr (R == 1) cell_word1(a, h, sb, q, w, t);")
-    print("    else if constexpr (R == 2) cell_word2(a, h, sb, q, w, t);")
-    print("    else if constexpr (R == 4) cell_word4(a, h, sb, q, w, t);")
-    print("    else if constexpr (R == 8) cell_word8(a, h, sb, q, w, t);")
-    print("    else if constexpr (R == 16) cell_word16(a, h, sb, q, w, t);")
-    print('    else static_assert(R == 1 || R == 2 || R == 4 || R == 8 || R == 16, "rows per block");\n}\n')
     for R in (1, 2, 4, 8, 16):
         print(chunk_block(R, 8))
     for R in (1, 2, 4, 8, 16):
