@@ -232,7 +232,8 @@ int lcs_semilocal_query(lcs_ctx *ctx, const int32_t *row_to_col, int32_t m, int3
  * anything else is LCS_EINVAL.  The index holds two of ceil(log2(size+1))
  * value bits per level, 16 bytes per 32 rows (the last of an odd number of
  * bits: 16 per 64), charged to the context's HBM budget; destroy it
- * before the context.  No counterpart in the reference (it reads no scores
+ * before the context (on any thread; one dropped later frees its own memory
+ * and can answer nothing).  No counterpart in the reference (it reads no scores
  * from its permutations).
  *   _build: host row_to_col; _build_device: device row_to_col (both
  *     synchronous, the input may be freed on return).

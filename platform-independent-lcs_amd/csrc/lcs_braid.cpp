@@ -12,10 +12,22 @@
 using namespace lcs;
 
 namespace {
+// From kBranchMin entries the byte table misses every cache, and a branch on
+// what an earlier value stored lets the loads run ahead of the stores (2^24
+// entries 7.9 ms each with it, 8.8 without; 2^26 314 and 365); below, the loop
+// without it is the faster one (65000 entries 46 and 59 us).
+constexpr int32_t kBranchMin = 1 << 24;
 bool is_permutation(const int32_t *x, int32_t n)
 {
     std::vector<unsigned char> seen((size_t)n, 0);
-    unsigned twice = 0;   // no branch on what an earlier value stored
+    if (n >= kBranchMin) {
+        for (int32_t i = 0; i < n; ++i) {
+            if (x[i] < 0 || x[i] >= n || seen[(size_t)x[i]]) return false;
+            seen[(size_t)x[i]] = 1;
+        }
+        return true;
+    }
+    unsigned twice = 0;
     for (int32_t i = 0; i < n; ++i) {
         const uint32_t v = (uint32_t)x[i];
         if (v >= (uint32_t)n) return false;

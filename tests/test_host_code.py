@@ -248,3 +248,23 @@ for budget in (0, 114776):
         result.append([len(launches('braid_core_lds_kernel')), len(launches('big_leaf_kernel'))])
 """)
     assert got == [[0, 1], [1, 0]]
+
+
+@pytest.mark.parametrize("size", [1, 5, 70000, (1 << 24) - 1, 1 << 24])
+def test_products_refuse_what_is_no_permutation(host, size):
+    # whichever loop checks: a value twice, one past the end, a negative one
+    got = host(f"""
+p, q = np.arange({size}, dtype=np.int32)[::-1].copy(), np.arange(1, dtype=np.int32)
+result = []
+with lcs_amd.Context(0) as c:
+    for where, value in ((0, {size}), ({size} - 1, -1), ({size} // 2, None), (0, 1 if {size} > 2 else {size})):
+        old = p[where]
+        p[where] = old if value is None else value
+        try:
+            c.braid_multiply(p, q, 0, False)
+            result.append('ok')
+        except lcs_amd.LcsError as e:
+            result.append('EINVAL' if 'EINVAL' in str(e) else str(e))
+        p[where] = old
+""")
+    assert got == ["EINVAL", "EINVAL", "ok", "EINVAL"], got
