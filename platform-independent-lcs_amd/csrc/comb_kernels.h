@@ -63,12 +63,14 @@ int lcsk_launch_sym8(const int32_t *b, int32_t n, uint32_t *out, int32_t stride,
 // Whether a byte chain's bands keep one chunk more than they need between
 // themselves and the band above (band_pass).  It costs 32 steps a band and
 // spares up to half of every step, so it is for bands that are long beside
-// their number.  Measured: 32 bands of 16384 columns 0.48 ms
-// without, 0.32 with; 64 of 16384 0.40 and 0.39; 256 of 50000 1.18 and 1.37.
-constexpr int kSlackColumns = 384;   // per band
+// their number, and long enough to fall out of step at all.  Median times
+// without and with it: 8 bands of 6000 columns 103 and 108 us, of 8192 139 and
+// 134, of 12000 209 and 181; 16 of 8192 176 and 159; 32 of 16384 477 and 306;
+// 64 of 16384 404 and 395; 256 of 50000 1184 and 1367.
+constexpr int kSlackMinColumns = 8192, kSlackColumnsPerBand = 384;
 __host__ __device__ inline bool band_slack(int tile_m, int32_t nbands, int32_t n)
 {
-    return tile_m == 1 && n / kSlackColumns > nbands;
+    return tile_m == 1 && n >= kSlackMinColumns && n / kSlackColumnsPerBand > nbands;
 }
 
 // Two pairs combed together by the 16-bit packed chain
